@@ -1,0 +1,276 @@
+"""The device work of this package as its users call it, for timing.
+
+Three families, each through its public entry point:
+
+* ``orion_amd.kernels``: the bf16 matrix-core GEMM and the fp32 streaming triad,
+  the high-priority and best-effort kernels of the co-location experiments
+  (``orion_amd.kernel_pair``), on the current stream or on a stream limited to
+  some of the compute units;
+* ``transformer_xl.MemTransformerLM``: a request of the Transformer-XL inference
+  client (bf16, memory of the previous segment, per-token losses);
+* ``transformer_xl.Lamb``: the optimiser step of the Transformer-XL training
+  client.
+
+``listed`` names the cases, ``draw`` gives more of the same ranges, ``prepare``
+makes what a program holds before the call and ``run`` is one pass.
+"""
+
+import math
+
+import torch
+
+from orion_amd import kernels
+from orion_amd.benchmark_suite.transformer_trainer import MODEL_CONFIG
+from orion_amd.benchmark_suite.transformer_xl import Lamb, MemTransformerLM
+
+DEVICE = "cuda:0"
+
+# Tiles the GEMM's entry point asks for: rows of both operands, depth.
+TILE_MN, TILE_K = 256, 64
+GEMM_SIDE, GEMM_DEPTH = (256, 8192), (64, 8192)
+GEMM_FLOPS = 2 * 8192 ** 3
+TRIAD_ELEMS = (1000, 1 << 28)
+
+
+def listed():
+    return [
+        # one small product between a request's other work: launch and latency
+        _gemm("gemm_256x512x256_f32", 256, 512, 256, "f32", False),
+        # the small kernel-pair job's high-priority request
+        _gemm("gemm_1024", 1024, 1024, 1024, "bf16", True),
+        # linear layers over 8 sequences of 384 tokens: attention projection and
+        # the second feed-forward layer at hidden 1024
+        _gemm("gemm_3072x1024x1024", 3072, 1024, 1024, "bf16", False),
+        _gemm("gemm_3072x1024x4096", 3072, 1024, 4096, "bf16", False),
+        # a size that divides nothing evenly: 11 x 13 tiles, 29 k-tiles
+        _gemm("gemm_2816x3328x1856_f32", 2816, 3328, 1856, "f32", False),
+        # the stated kernel-pair job's high-priority request
+        _gemm("gemm_8192", 8192, 8192, 8192, "bf16", True),
+        # a ragged streaming update that fits the caches
+        _triad("triad_1000003", 1_000_003, 0, 0),
+        # the small kernel-pair job's best-effort kernel
+        _triad("triad_4Mi", 1 << 22, 0, 0),
+        # best-effort work confined to a quarter of the compute units, the
+        # caller's own grid
+        _triad("triad_64Mi_64cus_grid1024", (1 << 26) + 3, 1024, 64),
+        # the stated job's best-effort kernel: three arrays of 1 GiB
+        _triad("triad_256Mi", 1 << 28, 0, 0),
+        # the Transformer-XL clients of the job files: a batch-4 inference
+        # request and the optimiser step of the training client
+        _txl("txl_inference_b4", 4, 192, 192),
+        _lamb("lamb_txl", 16, MODEL_CONFIG["n_token"], 0.0),
+    ]
+
+
+def _gemm(name, m, n, k, out, keep_out):
+    return _named(name, {"kind": "gemm", "m": m, "n": n, "k": k, "out": out,
+                         "keep_out": keep_out})
+
+
+def _triad(name, n, grid_blocks, cus):
+    return _named(name, {"kind": "triad", "n": n, "grid_blocks": grid_blocks, "cus": cus})
+
+
+def _txl(name, batch, tgt_len, mem_len):
+    return _named(name, {"kind": "txl", "batch": batch, "tgt_len": tgt_len,
+                         "mem_len": mem_len})
+
+
+def _lamb(name, n_layer, n_token, weight_decay):
+    return _named(name, {"kind": "lamb", "n_layer": n_layer, "n_token": n_token,
+                         "weight_decay": weight_decay})
+
+
+def _named(name, case):
+    return dict(case, name=name) if name else case
+
+
+def _log_uniform(rng, low, high):
+    return min(high, max(low, round(math.exp(rng.uniform(math.log(low), math.log(high))))))
+
+
+def draw(rng):
+    kind = rng.choice(("gemm", "gemm", "gemm", "triad", "triad", "txl", "lamb"))
+    if kind == "gemm":
+        while True:
+            m, n = (_log_uniform(rng, *GEMM_SIDE) // TILE_MN * TILE_MN for _ in range(2))
+            k = _log_uniform(rng, *GEMM_DEPTH) // TILE_K * TILE_K
+            if 2 * m * n * k <= GEMM_FLOPS:
+                return _gemm(None, m, n, k, rng.choice(("bf16", "bf16", "f32")),
+                             rng.random() < 0.5)
+    if kind == "triad":
+        # on the whole GPU, or confined as the scheduler confines it; seldom with
+        # a grid of the caller's
+        cus = rng.choice((0, 0, 32, 64, 128))
+        n = _log_uniform(rng, *TRIAD_ELEMS)
+        if cus:
+            n = min(n, 1 << 27)
+        return _triad(None, n, rng.choice((0, 0, _log_uniform(rng, 64, 8192))), cus)
+    if kind == "txl":
+        return _txl(None, rng.randint(1, 4), rng.randint(16, 192), rng.choice((0, 192, 192)))
+    return _lamb(None, rng.randint(1, 16), _log_uniform(rng, 20000, MODEL_CONFIG["n_token"]),
+                 rng.choice((0.0, 0.01)))
+
+
+def _generator(seed):
+    return torch.Generator(device=DEVICE).manual_seed(seed)
+
+
+def _uniform(shape, g, dtype=torch.float32):
+    return torch.empty(shape, device=DEVICE, dtype=torch.float32).uniform_(
+        -1.0, 1.0, generator=g).to(dtype)
+
+
+_streams = {}
+
+
+def _stream(cus):
+    """A program makes its confined stream once and keeps it."""
+    if cus not in _streams:
+        _streams[cus] = kernels.cu_masked_stream(cus)
+    return _streams[cus]
+
+
+def _flat_views(tensors):
+    """One buffer and a view of it for each tensor, 256-byte aligned: parameters
+    (or moments) as a program that communicates or saves them in one piece lays
+    them out."""
+    sizes = [-(-t.numel() // 64) * 64 for t in tensors]
+    flat = torch.zeros(sum(sizes), device=DEVICE)
+    views, at = [], 0
+    for t, size in zip(tensors, sizes):
+        views.append(flat[at:at + t.numel()].view(t.shape))
+        at += size
+    return flat, views
+
+
+def prepare(case, seed):
+    g = _generator(seed)
+    kind = case["kind"]
+    if kind == "gemm":
+        m, n, k = case["m"], case["n"], case["k"]
+        dtype = {"bf16": torch.bfloat16, "f32": torch.float32}[case["out"]]
+        state = {"a": _uniform((m, k), g, torch.bfloat16),
+                 "b": _uniform((n, k), g, torch.bfloat16), "dtype": dtype, "out": None}
+        if case["keep_out"]:
+            state["out"] = torch.empty((m, n), device=DEVICE, dtype=dtype)
+    elif kind == "triad":
+        n = case["n"]
+        state = {"a": torch.empty(n, device=DEVICE), "b": _uniform(n, g), "c": _uniform(n, g),
+                 "grid_blocks": case["grid_blocks"],
+                 "stream": _stream(case["cus"]) if case["cus"] else None}
+    elif kind == "txl":
+        torch.manual_seed(seed)
+        with torch.device(DEVICE):
+            model = MemTransformerLM(**MODEL_CONFIG)
+        model = model.eval().to(torch.bfloat16)
+        shape = (case["tgt_len"], case["batch"])
+        state = {"model": model, "mems": None}
+        state["data"], state["target"] = (
+            torch.randint(0, MODEL_CONFIG["n_token"], shape, device=DEVICE, generator=g)
+            for _ in range(2))
+        if case["mem_len"]:
+            # layer inputs: the scaled embedding, then outputs of layer norms
+            mems = torch.empty((MODEL_CONFIG["n_layer"], case["mem_len"], case["batch"],
+                                MODEL_CONFIG["d_model"]), device=DEVICE).normal_(generator=g)
+            mems[0] *= 0.02 * math.sqrt(MODEL_CONFIG["d_model"])
+            state["mems"] = mems.to(torch.bfloat16)
+    else:
+        torch.manual_seed(seed)
+        config = dict(MODEL_CONFIG, n_layer=case["n_layer"], n_token=case["n_token"],
+                      cutoffs=[case["n_token"] // 13, case["n_token"] // 7,
+                               case["n_token"] * 3 // 4])
+        with torch.device(DEVICE):
+            model = MemTransformerLM(**config)
+        params = list(model.parameters())
+        flats = {}
+        flats["w"], views = _flat_views(params)
+        for p, view in zip(params, views):
+            view.copy_(p.detach())
+            p.data = view
+        flat_grad, views = _flat_views(params)
+        for p, view in zip(params, views):
+            view.normal_(0.0, 1e-3, generator=g)
+            p.grad = view
+        optimizer = Lamb(params, lr=0.1, weight_decay=case["weight_decay"])
+        # training under way: the moments of the steps before
+        for key, scale in (("m", 1e-3), ("v", 1e-6)):
+            flats[key], views = _flat_views(params)
+            for p, view in zip(params, views):
+                view.normal_(0.0, scale, generator=g)
+                if key == "v":
+                    view.abs_()
+                optimizer.state[p][key] = view
+        state = {"optimizer": optimizer, "flats": flats, "grad": flat_grad, "model": model}
+    state["kind"] = kind
+    return state
+
+
+def run(state):
+    kind = state["kind"]
+    if kind == "gemm":
+        return kernels.gemm_bf16_nt(state["a"], state["b"], out=state["out"],
+                                    out_dtype=state["dtype"])
+    if kind == "triad":
+        return kernels.triad(state["a"], state["b"], state["c"], 1.7,
+                             grid_blocks=state["grid_blocks"], stream=state["stream"])
+    if kind == "txl":
+        with torch.no_grad():
+            return state["model"](state["data"], state["target"], state["mems"])
+    state["optimizer"].step()
+    return state["flats"]
+
+
+def _lamb_params(n_layer, n_token):
+    d, inner = MODEL_CONFIG["d_model"], MODEL_CONFIG["d_inner"]
+    proj = MODEL_CONFIG["n_head"] * MODEL_CONFIG["d_head"]
+    layer = (3 * proj + proj + proj) * d + 2 * d + 2 * d * inner + inner + d + 2 * d
+    return n_token * (d + 1) + 2 * proj + 3 * (d + 1) + n_layer * layer
+
+
+def work(case):
+    kind = case["kind"]
+    if kind == "gemm":
+        m, n, k = case["m"], case["n"], case["k"]
+        return {"bytes": 2 * (m + n) * k + m * n * {"bf16": 2, "f32": 4}[case["out"]],
+                "flops": 2 * m * n * k}
+    if kind == "triad":
+        return {"bytes": 12 * case["n"], "flops": 2 * case["n"]}
+    if kind == "txl":
+        c = MODEL_CONFIG
+        d, inner, proj, layers = c["d_model"], c["d_inner"], c["n_head"] * c["d_head"], c["n_layer"]
+        q, b = case["tgt_len"], case["batch"]
+        rows, klen = q * b, q + case["mem_len"]
+        # keys and values of the whole context, queries of the segment; content and
+        # position scores of the pairs that the causal mask lets through
+        pairs = b * (q * case["mem_len"] + q * (q + 1) // 2)
+        layer = (2 * d * proj * (rows + 2 * klen * b) + 2 * klen * d * proj
+                 + 2 * rows * proj * d + 4 * rows * d * inner + 6 * pairs * proj)
+        # the head over the first cluster and the cluster entries for every
+        # token; a tail cluster's logits for the tokens uniform targets put there
+        edges = [0] + list(c["cutoffs"]) + [c["n_token"]]
+        head = 2 * rows * d * (edges[1] + len(c["cutoffs"]))
+        tails = sum(2 * rows * (hi - lo) / c["n_token"] * (hi - lo) * d
+                    for lo, hi in zip(edges[1:], edges[2:]))
+        weights = _lamb_params(layers, c["n_token"])
+        mems = layers * c["mem_len"] * b * d
+        return {"bytes": 2 * (weights + mems * (2 if case["mem_len"] else 1)) + 18 * rows,
+                "flops": layers * layer + head + tails}
+    n = _lamb_params(case["n_layer"], case["n_token"])
+    # weights and moments in and out, gradients in; about a dozen operations each
+    return {"bytes": 28 * n, "flops": 14 * n}
+
+
+def tolerance(case):
+    """About four times what the present code is off from the same computation in
+    64 bits: 2.4e-7 (GEMM, fp32 output), 1.7e-3 (bf16 output), 1e-7 (LAMB weights
+    and moments); 9.4e-3 for the model's memory (2e-3 for the losses), where twice
+    that is stated."""
+    kind = case["kind"]
+    if kind == "triad":
+        return "exact"
+    if kind == "gemm":
+        return {"rel": 7e-3} if case["out"] == "bf16" else {"rel": 2e-6}
+    if kind == "txl":
+        return {"rel": 2e-2}
+    return {"rel": 1e-6}
