@@ -274,3 +274,93 @@ def tolerance(case):
     if kind == "txl":
         return {"rel": 2e-2}
     return {"rel": 1e-6}
+
+
+def exact(case, seed):
+    """What ``run`` returns for these inputs, in 64 bits with plain torch."""
+    state = prepare(case, seed)
+    kind = state["kind"]
+    with torch.no_grad():
+        if kind == "gemm":
+            return torch.matmul(state["a"].double(), state["b"].double().t())
+        if kind == "triad":
+            scale = torch.tensor(1.7, dtype=torch.float32).item()
+            return state["b"].double() + scale * state["c"].double()
+        if kind == "txl":
+            return _exact_txl(state)
+        return _exact_lamb(state)
+
+
+def _exact_lamb(state):
+    group = state["optimizer"].param_groups[0]
+    lr, eps, decay, (b1, b2) = (group[key] for key in ("lr", "eps", "weight_decay", "betas"))
+    after = {key: torch.zeros(flat.shape, device=flat.device, dtype=torch.float64)
+             for key, flat in state["flats"].items()}
+    at = 0
+    for p in group["params"]:
+        w, g = p.detach().double().flatten(), p.grad.double().flatten()
+        m, v = (state["optimizer"].state[p][key].double().flatten() for key in ("m", "v"))
+        m = b1 * m + (1 - b1) * g
+        v = b2 * v + (1 - b2) * g * g
+        update = m / (v.sqrt() + eps) + decay * w
+        w_norm, u_norm = w.norm().clamp(0, 10), update.norm()
+        ratio = 1.0 if w_norm == 0 or u_norm == 0 else w_norm / (u_norm + eps)
+        for key, value in (("w", w - lr * ratio * update), ("m", m), ("v", v)):
+            after[key][at:at + w.numel()] = value
+        at += -(-w.numel() // 64) * 64
+    return after
+
+
+def _exact_txl(state):
+    config, data, target = MODEL_CONFIG, state["data"], state["target"]
+    p = {key: value.double() for key, value in state["model"].state_dict().items()}
+    heads, width, d = config["n_head"], config["d_head"], config["d_model"]
+    q_len, batch = data.shape
+    mems = None if state["mems"] is None else state["mems"].double()
+    m_len = 0 if mems is None else mems.size(1)
+    k_len = q_len + m_len
+
+    def norm(x, prefix):
+        return torch.nn.functional.layer_norm(x, (d,), p[prefix + ".weight"], p[prefix + ".bias"])
+
+    # the distance of key j from query i, and which of them a query may see
+    distance = (torch.arange(q_len, device=DEVICE)[:, None] + m_len
+                - torch.arange(k_len, device=DEVICE)[None, :])
+    hidden_keys = distance < 0
+    rate = 10000.0 ** (-torch.arange(0, d, 2, device=DEVICE, dtype=torch.float64) / d)
+    angles = torch.arange(k_len, device=DEVICE, dtype=torch.float64)[:, None] * rate
+    positions = torch.cat([angles.sin(), angles.cos()], dim=1)
+    x = p["word_emb.weight"][data] * math.sqrt(d)
+    inputs = []
+    for i in range(config["n_layer"]):
+        inputs.append(x)
+        attn, ff = f"attn.{i}.", f"ff.{i}."
+        context = x if mems is None else torch.cat([mems[i], x])
+        q, k, v = (t.reshape(k_len, batch, heads, width).permute(1, 2, 0, 3)
+                   for t in (context @ p[attn + "qkv.weight"].t()).chunk(3, dim=-1))
+        q = q[:, :, m_len:]
+        r = (positions @ p[attn + "pos.weight"].t()).view(k_len, heads, width).permute(1, 2, 0)
+        content = (q + p["u"][:, None]) @ k.transpose(-1, -2).contiguous()
+        by_distance = (q + p["v"][:, None]) @ r.contiguous()
+        position = by_distance.gather(3, distance.clamp(min=0).expand_as(content))
+        scores = ((content + position) / math.sqrt(width)).masked_fill(hidden_keys, -math.inf)
+        mixed = (scores.softmax(-1) @ v).permute(2, 0, 1, 3).reshape(q_len, batch, heads * width)
+        x = norm(x + mixed @ p[attn + "out.weight"].t(), attn + "norm")
+        inner = (x @ p[ff + "net.0.weight"].t() + p[ff + "net.0.bias"]).relu()
+        x = norm(x + inner @ p[ff + "net.3.weight"].t() + p[ff + "net.3.bias"], ff + "norm")
+    new = torch.stack(inputs)
+    if mems is not None:
+        new = torch.cat([mems, new], dim=1)
+
+    edges = [0] + list(config["cutoffs"]) + [config["n_token"]]
+    rows, wanted = x.reshape(-1, d), target.reshape(-1)
+    weight, bias = p["crit.weight"], p["crit.bias"]
+    head = torch.cat([rows @ weight[:edges[1]].t() + bias[:edges[1]],
+                      rows @ p["crit.cluster_weight"].t() + p["crit.cluster_bias"]], dim=1)
+    head = head.log_softmax(1)
+    loss = -head.gather(1, wanted.clamp(max=edges[1] - 1)[:, None]).squeeze(1)
+    for c, (lo, hi) in enumerate(zip(edges[1:], edges[2:])):
+        at = ((wanted >= lo) & (wanted < hi)).nonzero().squeeze(1)
+        tail = (rows[at] @ weight[lo:hi].t() + bias[lo:hi]).log_softmax(1)
+        loss[at] = -(head[at, edges[1] + c] + tail.gather(1, (wanted[at] - lo)[:, None]).squeeze(1))
+    return loss.view(q_len, batch), new[:, -config["mem_len"]:]
