@@ -27,6 +27,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from .. import kernels
+
 
 def relative_shift(x):
     """``x[..., i, p]`` holds query i against the p-th entry of a distance table
@@ -227,7 +229,9 @@ class Lamb(torch.optim.Optimizer):
     (related/baselines/transformer/lamb.py:79-146): Adam moments without bias
     correction, the update scaled per tensor by ||w|| (clamped to 10) over
     ||update||, ratio 1 where either norm is zero.  The whole step stays on the
-    device (the reference reads both norms back for every tensor)."""
+    device (the reference reads both norms back for every tensor): contiguous
+    fp32 tensors of one GPU through ``kernels.lamb_step``, anything else as
+    element-wise operations over the lists."""
 
     def __init__(self, params, lr=1e-3, betas=(0.9, 0.999), eps=1e-6, weight_decay=0.0):
         super().__init__(params, dict(lr=lr, betas=betas, eps=eps, weight_decay=weight_decay))
@@ -246,6 +250,12 @@ class Lamb(torch.optim.Optimizer):
             ms = [self.state[p]["m"] for p in params]
             vs = [self.state[p]["v"] for p in params]
             b1, b2 = group["betas"]
+            if (all(type(x) in (int, float)
+                    for x in (group["lr"], b1, b2, group["eps"], group["weight_decay"]))
+                    and kernels.lamb_takes(params, grads, ms, vs)):
+                kernels.lamb_step(params, grads, ms, vs, group["lr"], (b1, b2), group["eps"],
+                                  group["weight_decay"])
+                continue
             torch._foreach_mul_(ms, b1)
             torch._foreach_add_(ms, grads, alpha=1 - b1)
             torch._foreach_mul_(vs, b2)

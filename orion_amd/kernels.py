@@ -32,6 +32,12 @@ def lib():
             ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
             ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
         handle.orion_gemm_bf16_nt.restype = ctypes.c_int
+        handle.orion_lamb_workspace_bytes.argtypes = [ctypes.c_void_p, ctypes.c_int]
+        handle.orion_lamb_workspace_bytes.restype = ctypes.c_size_t
+        handle.orion_lamb_step.argtypes = [
+            ctypes.c_void_p, ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_double,
+            ctypes.c_double, ctypes.c_double, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+        handle.orion_lamb_step.restype = ctypes.c_int
         handle.orion_stream_create.argtypes = [ctypes.c_int, ctypes.POINTER(ctypes.c_void_p)]
         handle.orion_stream_create.restype = ctypes.c_int
         handle.orion_stream_destroy.argtypes = [ctypes.c_void_p]
@@ -139,3 +145,57 @@ def gemm_bf16_nt(a, b, out=None, out_dtype=torch.bfloat16, stream=None):
     if rc != 0:
         raise KernelError("orion_gemm_bf16_nt", rc)
     return out
+
+
+def plain_eager():
+    """False while something has to see every operation: a transform or a mode
+    that rewrites them, or a tracer."""
+    return (torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0
+            and not torch.jit.is_tracing()
+            and not torch.compiler.is_compiling())
+
+
+def plain_tensors(tensors, dtype, device):
+    """Whether these are ordinary contiguous tensors of the device: what a kernel
+    that takes addresses can work on."""
+    for t in tensors:
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype is not dtype
+                or t.device != device or t.layout is not torch.strided
+                or not t.is_contiguous()):
+            return False
+    return True
+
+
+def lamb_takes(params, grads, ms, vs):
+    """Whether ``lamb_step`` takes these lists: contiguous fp32 tensors of one
+    GPU, of equal shapes item by item."""
+    device = params[0].device
+    if device.type != "cuda" or not plain_eager():
+        return False
+    if not all(plain_tensors(ts, torch.float32, device) for ts in (params, grads, ms, vs)):
+        return False
+    return all(p.shape == g.shape == m.shape == v.shape
+               for p, g, m, v in zip(params, grads, ms, vs))
+
+
+def lamb_step(params, grads, ms, vs, lr, betas, eps, weight_decay):
+    """One LAMB step in place over lists that ``lamb_takes`` accepts, on the
+    current stream of their device."""
+    device = params[0].device
+    table = []
+    for p, g, m, v in zip(params, grads, ms, vs):
+        table += (p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), p.numel())
+    table = (ctypes.c_uint64 * len(table))(*table)
+    handle = lib()
+    with torch.cuda.device(device):
+        size = handle.orion_lamb_workspace_bytes(table, len(params))
+        # in stream order: the allocator hands it on only behind these kernels
+        work = torch.empty(size, dtype=torch.uint8, device=device)
+        rc = handle.orion_lamb_step(table, len(params), lr, betas[0], betas[1], eps,
+                                    weight_decay, work.data_ptr(), size, _stream_ptr(None))
+    if rc != 0:
+        raise KernelError("orion_lamb_step", rc)
+    for ts in (params, ms, vs):          # written behind autograd's back
+        torch.autograd.graph.increment_version(ts)
