@@ -117,6 +117,12 @@ class AdaptiveLogSoftmax(nn.Module):
 
     def forward(self, hidden, target):
         """hidden [n, d], target [n] -> nll [n] (in the order of the rows)."""
+        if (type(self) is AdaptiveLogSoftmax and hidden.dtype is torch.bfloat16
+                and kernels.inference_only()):
+            nll = kernels.adaptive_nll(hidden, target, self.weight, self.bias,
+                                       self.cluster_weight, self.cluster_bias, self.edges)
+            if nll is not None:
+                return nll
         head = self.head_logprob(hidden)
         short = self.edges[1]
         nll = torch.zeros_like(target, dtype=hidden.dtype)
@@ -146,6 +152,22 @@ class AdaptiveLogSoftmax(nn.Module):
             tail = F.log_softmax(F.linear(hidden, self.weight[lo:hi], self.bias[lo:hi]), dim=-1)
             parts.append(head[:, short + c - 1, None] + tail)
         return torch.cat(parts, dim=1)
+
+
+def _global_hooks():
+    module = torch.nn.modules.module
+    return module._global_forward_hooks or module._global_forward_pre_hooks
+
+
+def _plain(module):
+    """Calling the module is its class's forward and nothing else, in inference."""
+    attrs = module.__dict__
+    return type(module) in _PLAIN_TYPES and not (attrs["_forward_hooks"] or attrs["_forward_pre_hooks"] or "forward" in attrs
+                or type(module) is nn.Dropout and module.training and module.p)
+
+
+_PLAIN_TYPES = {RelativeAttention, FeedForward, nn.Sequential, nn.Linear, nn.LayerNorm,
+                nn.Dropout, nn.ReLU}
 
 
 # keys of the reference's configuration that select other variants of the
@@ -192,6 +214,10 @@ class MemTransformerLM(nn.Module):
         mlen = mems[0].size(0) if mems is not None else 0
         klen = qlen + mlen
         x = self.word_emb(data) * math.sqrt(self.d_model)
+        if x.dtype is torch.bfloat16 and kernels.inference_only():
+            fused = self._fused_hidden_states(x, mems)
+            if fused is not None:
+                return fused
         table = sinusoid_table(torch.arange(klen - 1, -1, -1, device=data.device),
                                self.d_model, x.dtype)
         # key j is visible to query i when j <= mlen + i
@@ -205,6 +231,41 @@ class MemTransformerLM(nn.Module):
                              None if mems is None else mems[i])
             x = self.ff[i](x)
         return self.drop(x), self._new_mems(inputs, mems)
+
+    def _fused_hidden_states(self, x, mems):
+        """The layers through ``kernels.txl_hidden``; None unless every module it
+        passes by is the plain one, in its inference form, with nothing attached."""
+        if (type(self) is not MemTransformerLM or not self.n_layer or _global_hooks()
+                or not _plain(self.drop)):
+            return None
+        layers, eps, inner = [], self.attn[0].norm.eps, self.ff[0].net[0].out_features
+        for attn, ff in zip(self.attn._modules.values(), self.ff._modules.values()):
+            if type(attn) is not RelativeAttention or type(ff) is not FeedForward:
+                return None
+            a, f = attn._modules, ff._modules
+            net = f["net"]
+            parts = [*a.values(), *f.values(), attn, ff]
+            if type(net) is not nn.Sequential or len(a) != 5 or len(f) != 2 or len(net) != 5:
+                return None         # not the modules their constructors make
+            parts += net._modules.values()
+            if not all(map(_plain, parts)):
+                return None
+            qkv, pos, out, drop, norm1 = a.values()
+            ff1, relu, drop1, ff2, drop2 = net._modules.values()
+            norm2 = f["norm"]
+            if not (type(qkv) is type(pos) is type(out) is type(ff1) is type(ff2) is nn.Linear
+                    and type(norm1) is type(norm2) is nn.LayerNorm and type(relu) is nn.ReLU
+                    and type(drop) is type(drop1) is type(drop2) is nn.Dropout
+                    and qkv.bias is None and pos.bias is None and out.bias is None
+                    and norm1.eps == norm2.eps == eps
+                    and norm1.normalized_shape == norm2.normalized_shape == (self.d_model,)
+                    and (attn.n_head, attn.d_head) == self.u.shape):
+                return None
+            layers.append((qkv.weight, pos.weight, out.weight, norm1.weight, norm1.bias,
+                           ff1.weight, ff1.bias, ff2.weight, ff2.bias, norm2.weight,
+                           norm2.bias))
+        return kernels.txl_hidden(x, mems, self.u, self.v, layers, inner, eps,
+                                  self.mem_len or 0)
 
     def _new_mems(self, inputs, mems):
         """The last ``mem_len`` inputs of every layer, detached."""

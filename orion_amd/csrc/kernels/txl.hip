@@ -1,0 +1,993 @@
+// Forward pass of the Transformer-XL inference client in bf16: the layers of
+// relative attention and feed-forward (Dai et al., 2019), and the per-token losses
+// of the adaptive softmax (Grave et al., 2017).  The reference's client runs the
+// same model as framework operations
+// (benchmarking/benchmark_suite/transformer_trainer.py:63-86, :144).
+//
+// A request is small (768 token rows at batch 4: 0.2 TFLOP, a third of it in the
+// vocabulary) and a chain of 16 layers, so what bounds it is the number of
+// dependent launches and the latency inside each, not a rate.  Five launches a
+// layer; whatever does not depend on the chain runs before it, for all layers at
+// once:
+//
+//   before      positions (sinusoids); keys and values of the memory and the
+//               projected positions of every layer
+//   layer i     x_i = LN(y), [q k v] = x_i Wqkv^T          ln_gemm
+//               attention                                   txl_attention
+//               y = x_i + att Wo^T                          residual_gemm
+//               x' = LN(y), h = relu(x' W1^T + b1)          ln_gemm
+//               y = x' + h W2^T + b2                        residual_gemm
+//   after       hidden = LN(y)
+//
+// The layer norm rides in the product that reads it: a workgroup's A panel is 64
+// whole rows of 512, so it normalises them itself on the way into LDS (every
+// workgroup of a row panel repeats that; the first column of workgroups also
+// writes the rows, for the residual and the memory).  y stays fp32.
+//
+// Sums are fp32 throughout; activations are rounded to bf16 where the model's
+// own operations rounded them, less y, the two query biases (added in fp32) and
+// the position scores, which stay fp32 here.
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "kernels.h"
+#include "mfma_tile.h"
+
+namespace {
+
+using namespace mfma_tile;
+
+constexpr int kD = 512;               // model width: the length of a norm's row
+constexpr int kHead = 64;             // head width
+constexpr int kPanelTiles = kD / kTileK;
+constexpr int kMaxJobs = 64;
+constexpr int kThreads = 256;
+
+__device__ __forceinline__ void store_bf16x4(uint16_t* p, const f32x4& v) {
+  u32x2 packed;
+  packed[0] = pack_bf16(v[0], v[1]);
+  packed[1] = pack_bf16(v[2], v[3]);
+  *reinterpret_cast<u32x2*>(p) = packed;
+}
+
+__device__ __forceinline__ f32x4 load_bf16x4(const uint16_t* p) {
+  const u32x2 v = *reinterpret_cast<const u32x2*>(p);
+  return f32x4{bf16_lo(v[0]), bf16_hi(v[0]), bf16_lo(v[1]), bf16_hi(v[1])};
+}
+
+__device__ __forceinline__ float sum16(float v) {
+#pragma unroll
+  for (int d = 1; d < 16; d <<= 1) v += __shfl_xor(v, d);
+  return v;
+}
+
+struct Norm {
+  const uint16_t* w;
+  const uint16_t* b;
+  float eps;
+};
+
+// Layer norm of four rows of 512 by one wave, sixteen lanes a row; lane l % 16
+// gets the 16-byte bf16 chunks l % 16 + 16 * j of its row.  Mean first, then the
+// squared distances from it.
+__device__ __forceinline__ void norm_row(const float* y, const Norm& norm, int cl,
+                                         u32x4 (&out)[4]) {
+  f32x4 v[4][2];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float* p = y + (cl + 16 * j) * 8;
+    v[j][0] = *reinterpret_cast<const f32x4*>(p);
+    v[j][1] = *reinterpret_cast<const f32x4*>(p + 4);
+  }
+  float s = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += v[j][e >> 2][e & 3];
+  const float mean = sum16(s) * (1.0f / kD);
+  float q = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float d = v[j][e >> 2][e & 3] - mean;
+      q = __builtin_fmaf(d, d, q);
+    }
+  const float rstd = 1.0f / __builtin_sqrtf(sum16(q) * (1.0f / kD) + norm.eps);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const u32x4 w = *reinterpret_cast<const u32x4*>(norm.w + (cl + 16 * j) * 8);
+    const u32x4 b = *reinterpret_cast<const u32x4*>(norm.b + (cl + 16 * j) * 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float lo = (v[j][e >> 1][(e & 1) * 2] - mean) * rstd;
+      const float hi = (v[j][e >> 1][(e & 1) * 2 + 1] - mean) * rstd;
+      out[j][e] = pack_bf16(__builtin_fmaf(lo, bf16_lo(w[e]), bf16_lo(b[e])),
+                            __builtin_fmaf(hi, bf16_hi(w[e]), bf16_hi(b[e])));
+    }
+  }
+}
+
+// Rows of the normalised (or given) input that later launches and the caller read.
+struct RowsOut {
+  uint16_t* x;         // [M, 512], may be null
+  uint16_t* mem;       // rows mem_from.. of [M, 512], may be null
+  int mem_from;
+};
+
+__device__ __forceinline__ void put_row(const RowsOut& out, int row, int chunk, const u32x4& v) {
+  if (out.x) *reinterpret_cast<u32x4*>(out.x + (size_t)row * kD + chunk * 8) = v;
+  if (out.mem && row >= out.mem_from)
+    *reinterpret_cast<u32x4*>(out.mem + (size_t)(row - out.mem_from) * kD + chunk * 8) = v;
+}
+
+// C[M, N] = A[M, 512] * W[N, 512]^T with the whole A panel of a workgroup in LDS:
+// normalised on the way from fp32 (kNorm) or loaded as it is.  W streams through
+// four stages.  N is a multiple of BN; rows past M are computed from the last row
+// and not written.
+template <int BM, int BN, bool kNorm, typename Epi>
+__device__ __forceinline__ void panel_gemm(unsigned char* lds, const void* A, const uint16_t* W,
+                                           int M, int tm, int tn, const Norm& norm,
+                                           const RowsOut& out, const Epi& epi) {
+  constexpr int NS = 4;
+  constexpr int kPanel = BM * kD * 2;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int row0 = tm * BM;
+  unsigned char* stages = lds + kPanel;
+  Rows<BN> b;
+  b.init(wave, lane, [&](int r) { return W + (size_t)(tn * BN + r) * kD; });
+  if (!kNorm) {
+    Rows<BM> a;
+    a.init(wave, lane, [&](int r) {
+      const int row = row0 + r < M ? row0 + r : M - 1;
+      return static_cast<const uint16_t*>(A) + (size_t)row * kD;
+    });
+#pragma unroll
+    for (int kt = 0; kt < kPanelTiles; ++kt) a.issue(kt * kTileK, lds + kt * Rows<BM>::kBytes);
+  }
+#pragma unroll
+  for (int s = 0; s < NS - 1; ++s) b.issue(s * kTileK, stages + s * Rows<BN>::kBytes);
+  if (kNorm) {
+    const int cl = lane & 15;
+#pragma unroll
+    for (int it = 0; it < BM / 16; ++it) {
+      const int r = wave * (BM / 4) + it * 4 + (lane >> 4);
+      const int row = row0 + r < M ? row0 + r : M - 1;
+      u32x4 v[4];
+      norm_row(static_cast<const float*>(A) + (size_t)row * kD, norm, cl, v);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int chunk = cl + 16 * j;
+        *reinterpret_cast<u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes + r * kRowBytes +
+                                  (((chunk & 7) ^ (r & 7)) << 4)) = v[j];
+        if (tn == 0 && row0 + r < M) put_row(out, row0 + r, chunk, v[j]);
+      }
+    }
+  }
+  f32x4 acc[BM / 32][BN / 32];
+  clear(acc);
+#pragma unroll
+  for (int kt = 0; kt < kPanelTiles; ++kt) {
+    if (kt + NS - 2 < kPanelTiles) wait_vm<Rows<BN>::kLoads*(NS - 2)>();
+    else wait_vm<0>();
+    block_sync();
+    if (kt + NS - 1 < kPanelTiles)
+      b.issue((kt + NS - 1) * kTileK, stages + (kt + NS - 1) % NS * Rows<BN>::kBytes);
+    tile_step<BM, BN>(acc, lds + kt * Rows<BM>::kBytes, stages + kt % NS * Rows<BN>::kBytes, wm,
+                      wn, lane);
+  }
+  if (!kNorm && tn == 0 && (out.x || out.mem)) {
+    for (int i = threadIdx.x; i < BM * (kD / 8); i += kThreads) {
+      const int r = i / (kD / 8), chunk = i % (kD / 8);
+      if (row0 + r < M)
+        put_row(out, row0 + r, chunk,
+                *reinterpret_cast<const u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes +
+                                                r * kRowBytes + (((chunk & 7) ^ (r & 7)) << 4)));
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < BM / 32; ++i) {
+    const int row = row0 + wm * (BM / 2) + i * 16 + l16;
+    if (row >= M) continue;
+#pragma unroll
+    for (int j = 0; j < BN / 32; ++j)
+      epi(row, tn * BN + wn * (BN / 2) + j * 16 + lq * 4, acc[i][j]);
+  }
+}
+
+// bf16 store of a plain product.
+struct StoreEpi {
+  uint16_t* out;
+  int ld;
+  __device__ __forceinline__ void operator()(int row, int col, const f32x4& v) const {
+    store_bf16x4(out + (size_t)row * ld + col, v);
+  }
+};
+
+// [q k v]: the query leaves twice, with each of the two learned biases.
+struct QkvEpi {
+  uint16_t *qu, *qv, *kv;
+  const uint16_t *u, *v;
+  int proj;
+  __device__ __forceinline__ void operator()(int row, int col, const f32x4& x) const {
+    if (col >= proj) {
+      store_bf16x4(kv + (size_t)row * (2 * proj) + (col - proj), x);
+    } else {
+      store_bf16x4(qu + (size_t)row * proj + col, x + load_bf16x4(u + col));
+      store_bf16x4(qv + (size_t)row * proj + col, x + load_bf16x4(v + col));
+    }
+  }
+};
+
+// h = relu(v + bias); a NaN stays one.
+struct ReluEpi {
+  uint16_t* out;
+  const uint16_t* bias;
+  int ld;
+  __device__ __forceinline__ void operator()(int row, int col, const f32x4& x) const {
+    f32x4 v = x + load_bf16x4(bias + col);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = v[e] < 0.0f ? 0.0f : v[e];
+    store_bf16x4(out + (size_t)row * ld + col, v);
+  }
+};
+
+template <int BM, int BN>
+constexpr int panel_lds() {
+  return BM * kD * 2 + 4 * Rows<BN>::kBytes;
+}
+
+// Column of tiles first: with a multiple of eight of them every XCD reads its own
+// share of W and no more.
+template <int BM, int BN, bool kNorm, typename Epi>
+__global__ __launch_bounds__(kThreads, 1) void txl_ln_gemm_kernel(const void* A, const uint16_t* W,
+                                                                  int M, int tiles_n, Norm norm,
+                                                                  RowsOut out, Epi epi) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[panel_lds<BM, BN>()];
+  panel_gemm<BM, BN, kNorm>(lds, A, W, M, blockIdx.x / tiles_n, blockIdx.x % tiles_n, norm, out,
+                            epi);
+}
+
+// Independent products with the same inner length, one launch: workgroups
+// first_block[i] .. first_block[i + 1] of the grid are job i's.
+struct Job {
+  const uint16_t *A, *W;
+  uint16_t* out;
+  int M, tiles_n, ld;
+};
+struct Jobs {
+  Job job[kMaxJobs];
+  uint32_t first_block[kMaxJobs + 1];
+  int count;
+};
+constexpr int kJobM = 64, kJobN = 128;
+
+__global__ __launch_bounds__(kThreads, 1) void txl_jobs_kernel(Jobs jobs) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[panel_lds<kJobM, kJobN>()];
+  const int lane = threadIdx.x & 63;
+  const bool before = lane < jobs.count && jobs.first_block[lane] <= blockIdx.x;
+  const int i = __builtin_amdgcn_readfirstlane(__popcll(__ballot(before)) - 1);
+  const Job job = jobs.job[i];
+  const int local = blockIdx.x - jobs.first_block[i];
+  panel_gemm<kJobM, kJobN, false>(lds, job.A, job.W, job.M, local / job.tiles_n,
+                                  local % job.tiles_n, Norm{}, RowsOut{},
+                                  StoreEpi{job.out, job.ld});
+}
+
+// y[M, 512] = x + bias + A[M, K] * W[512, K]^T in fp32.  Eight waves: two groups of
+// four take the even and the odd k-tiles, which halves the chain of barriers (2048
+// deep: 16 steps instead of 32), and their sums meet in LDS.  32 x 64 tiles give
+// 192 workgroups at 768 rows.  K is a multiple of 128.
+constexpr int kResM = 32, kResN = 64, kResStages = 4;
+
+__global__ __launch_bounds__(2 * kThreads, 1) void txl_residual_gemm_kernel(
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ W, int K,
+    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ x, float* __restrict__ y,
+    int M) {
+  constexpr int kGroup = kResStages * (Rows<kResM>::kBytes + Rows<kResN>::kBytes);
+  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kGroup];
+  const int lane = threadIdx.x & 63;
+  const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave8 & 3, group = wave8 >> 2;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int tn = blockIdx.x % (kD / kResN), tm = blockIdx.x / (kD / kResN);
+  const int row0 = tm * kResM, col0 = tn * kResN;
+  Rows<kResM> a;
+  Rows<kResN> b;
+  a.init(wave, lane, [&](int r) {
+    const int row = row0 + r < M ? row0 + r : M - 1;
+    return A + (size_t)row * K + group * kTileK;
+  });
+  b.init(wave, lane, [&](int r) { return W + (size_t)(col0 + r) * K + group * kTileK; });
+  f32x4 acc[kResM / 32][kResN / 32];
+  clear(acc);
+  stream_product<kResM, kResN, kResStages>(acc, lds + group * kGroup, K / (2 * kTileK),
+                                           2 * kTileK, a, b, wm, wn, lane);
+  block_sync();
+  f32x4* other = reinterpret_cast<f32x4*>(lds) + wave * 64 + lane;
+  if (group == 1) {
+#pragma unroll
+    for (int j = 0; j < kResN / 32; ++j) other[j * 256] = acc[0][j];
+  }
+  block_sync();
+  const int row = row0 + wm * 16 + (lane & 15);
+  if (group == 1 || row >= M) return;
+#pragma unroll
+  for (int j = 0; j < kResN / 32; ++j) {
+    const int col = col0 + wn * (kResN / 2) + j * 16 + (lane >> 4) * 4;
+    f32x4 v = acc[0][j] + other[j * 256];
+    if (bias) v += load_bf16x4(bias + col);
+    v += load_bf16x4(x + (size_t)row * kD + col);
+    *reinterpret_cast<f32x4*>(y + (size_t)row * kD + col) = v;
+  }
+}
+
+// hidden = LN(y), one wave for four rows.
+__global__ __launch_bounds__(kThreads) void txl_norm_kernel(const float* y, Norm norm,
+                                                            uint16_t* hidden, int M) {
+  const int row = blockIdx.x * (kThreads / 16) + (threadIdx.x >> 4);
+  const int at = row < M ? row : M - 1;
+  u32x4 v[4];
+  norm_row(y + (size_t)at * kD, norm, threadIdx.x & 15, v);
+  if (row >= M) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    *reinterpret_cast<u32x4*>(hidden + (size_t)row * kD + ((threadIdx.x & 15) + 16 * j) * 8) = v[j];
+}
+
+// table[distance] = [sin, cos](distance * 10000^(-2c/512)), bf16.
+__global__ __launch_bounds__(kD / 2) void txl_positions_kernel(uint16_t* table) {
+  const int c = threadIdx.x;
+  const double rate = exp2(-13.287712379549449391 * (2.0 * c / kD));   // log2(10000)
+  const double angle = blockIdx.x * rate;
+  const uint32_t v = pack_bf16((float)sin(angle), (float)cos(angle));
+  table[(size_t)blockIdx.x * kD + c] = (uint16_t)v;
+  table[(size_t)blockIdx.x * kD + kD / 2 + c] = (uint16_t)(v >> 16);
+}
+
+// Relative attention of 64 queries of one head of one sequence.
+//
+//   score(i, j) = ((q_i + u) k_j + (q_i + v) r_(m + i - j)) / 8,   j <= m + i
+//
+// with m rows of memory in front of the segment.  Eight waves: wave w takes
+// queries 16 (w % 4) .. + 15 and the first or second half of each stage of 128
+// keys (online softmax; the halves meet in LDS at the end).  K and R are the first
+// MFMA operand, so a lane's values belong to ONE query (lane % 16) and to four
+// consecutive keys or distances: the softmax needs two shuffles a maximum, and the
+// probabilities are already where the second product wants its operand, given V
+// transposed and its keys taken in the same order.
+//
+// The shift by relative distance is a shear: the wave computes the 80 distances
+// that its 16 x 64 block of pairs touches, keeps them in LDS as fp32 and each lane
+// picks entry (query - key + 63) of its row.  A stage's R rows are the 192
+// distances from the workgroup's first query to the stage's last key on.
+//
+// Bound by latency: at batch 4 (96 workgroups, 384 keys, 3 stages) the matrix
+// cores have some 150 MFMAs a wave.  The next stage's rows travel through
+// registers while this one is worked on.
+constexpr int kAttnThreads = 512;
+constexpr int kQ = 64, kKeys = 128;
+constexpr int kDistances = kQ + kKeys;         // a stage's R rows
+constexpr int kVtRow = (kKeys / 2 + 2) * 4;    // bytes of a row of V transposed
+constexpr int kShearRow = 84;                  // floats of a row of position scores
+constexpr int kAttnR = kKeys * kRowBytes;
+constexpr int kAttnV = kAttnR + kDistances * kRowBytes;
+constexpr int kAttnShear = kAttnV + kHead * kVtRow;
+constexpr int kAttnLds = kAttnShear + 8 * 16 * kShearRow * 4;
+
+__global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
+    const uint16_t* __restrict__ qu, const uint16_t* __restrict__ qv,
+    const uint16_t* __restrict__ kv_mem, const uint16_t* __restrict__ kv_x,
+    const uint16_t* __restrict__ r, uint16_t* __restrict__ out, int qlen, int mlen, int batch,
+    int heads) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kAttnLds];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int head = blockIdx.x % heads, b = blockIdx.x / heads;
+  const int q0 = blockIdx.y * kQ;
+  const int klen = mlen + qlen;
+  const int proj = heads * kHead;
+  const int w4 = wave & 3, half = wave >> 2;
+
+  auto key_row = [&](int j) {
+    j = j < klen ? j : klen - 1;
+    return (j < mlen ? kv_mem + ((size_t)j * batch + b) * (2 * proj)
+                     : kv_x + ((size_t)(j - mlen) * batch + b) * (2 * proj)) + head * kHead;
+  };
+  // this thread's share of a stage
+  u32x4 nk[2], nr[3], nv[2];
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int u = i * kAttnThreads + threadIdx.x;
+      nk[i] = *reinterpret_cast<const u32x4*>(key_row(j0 + (u >> 3)) + (u & 7) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int u = i * kAttnThreads + threadIdx.x;
+      int d = mlen + q0 - (j0 + kKeys - 1) + (u >> 3);
+      d = d < 0 ? 0 : d < klen ? d : klen - 1;
+      nr[i] = *reinterpret_cast<const u32x4*>(r + (size_t)d * proj + head * kHead + (u & 7) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      nv[i] = *reinterpret_cast<const u32x4*>(key_row(j0 + (threadIdx.x >> 3) * 2 + i) + proj +
+                                              (threadIdx.x & 7) * 8);
+  };
+  auto put = [&]() {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int u = i * kAttnThreads + threadIdx.x, row = u >> 3;
+      *reinterpret_cast<u32x4*>(lds + row * kRowBytes + (((u & 7) ^ (row & 7)) << 4)) = nk[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int u = i * kAttnThreads + threadIdx.x, row = u >> 3;
+      *reinterpret_cast<u32x4*>(lds + kAttnR + row * kRowBytes + (((u & 7) ^ (row & 7)) << 4)) =
+          nr[i];
+    }
+    // two keys of a head column side by side
+    unsigned char* vt = lds + kAttnV + (threadIdx.x & 7) * 8 * kVtRow + (threadIdx.x >> 3) * 4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      *reinterpret_cast<uint32_t*>(vt + (2 * e) * kVtRow) =
+          (nv[0][e] & 0xffffu) | (nv[1][e] << 16);
+      *reinterpret_cast<uint32_t*>(vt + (2 * e + 1) * kVtRow) =
+          (nv[0][e] >> 16) | (nv[1][e] & 0xffff0000u);
+    }
+  };
+
+  const int qi = q0 + w4 * 16 + l16;            // this lane's query
+  bf16x8 fqu[2], fqv[2];
+  {
+    const int q = qi < qlen ? qi : qlen - 1;
+    const size_t at = ((size_t)q * batch + b) * proj + head * kHead + lq * 8;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      fqu[ks] = *reinterpret_cast<const bf16x8*>(qu + at + ks * 32);
+      fqv[ks] = *reinterpret_cast<const bf16x8*>(qv + at + ks * 32);
+    }
+  }
+  auto fragment = [&](int base, int row, int ks) {
+    return *reinterpret_cast<const bf16x8*>(lds + base + row * kRowBytes +
+                                            (((ks * 4 + lq) ^ (row & 7)) << 4));
+  };
+  float* shear = reinterpret_cast<float*>(lds + kAttnShear) + (wave * 16 + l16) * kShearRow;
+
+  constexpr float kExp = 0.125f * 1.44269504088896340736f;   // 1 / sqrt(64), base 2
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 o[4] = {zero, zero, zero, zero};
+  float m = -__builtin_inff(), l = 0.0f;
+  const int last_query = q0 + kQ <= qlen ? q0 + kQ - 1 : qlen - 1;
+  const int stages = (mlen + last_query) / kKeys + 1;
+  fetch(0);
+  for (int st = 0; st < stages; ++st) {
+    const int j0 = st * kKeys;
+    if (st > 0) block_sync();                   // everyone is done with the last stage
+    put();
+    block_sync();
+    if (st + 1 < stages) fetch(j0 + kKeys);
+    const int jw = j0 + 64 * half;              // this wave's first key
+    if (jw > mlen + q0 + w4 * 16 + 15) continue;   // all of them in the future
+
+    f32x4 s[4];
+#pragma unroll
+    for (int t = 0; t < 5; ++t) {
+      f32x4 g = zero;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        g = mfma(fragment(kAttnR, 16 * w4 + 64 - 64 * half + 16 * t + l16, ks), fqv[ks], g);
+      *reinterpret_cast<f32x4*>(shear + 16 * t + lq * 4) = g;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      s[t] = zero;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+        s[t] = mfma(fragment(0, 64 * half + 16 * t + l16, ks), fqu[ks], s[t]);
+    }
+    // the rows of position scores cross lanes of this wave only
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    float top = -__builtin_inff();
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int k = 16 * t + lq * 4 + e;
+        const float v = s[t][e] + shear[l16 + 63 - k];
+        s[t][e] = jw + k <= mlen + qi ? v : -__builtin_inff();
+        top = __builtin_fmaxf(top, s[t][e]);
+      }
+    top = __builtin_fmaxf(top, __shfl_xor(top, 16));
+    top = __builtin_fmaxf(top, __shfl_xor(top, 32));
+    const float m_new = __builtin_fmaxf(m, top);
+    const float base = m_new == -__builtin_inff() ? 0.0f : m_new;
+    const float scale = __builtin_amdgcn_exp2f((m - base) * kExp);
+    m = m_new;
+    l *= scale;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) o[d] *= scale;
+    uint32_t p[4][2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        s[t][e] = __builtin_amdgcn_exp2f((s[t][e] - base) * kExp);
+        l += s[t][e];
+      }
+      p[t][0] = pack_bf16(s[t][0], s[t][1]);
+      p[t][1] = pack_bf16(s[t][2], s[t][3]);
+    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const u32x4 pg = {p[2 * g][0], p[2 * g][1], p[2 * g + 1][0], p[2 * g + 1][1]};
+      const bf16x8 fp = __builtin_bit_cast(bf16x8, pg);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const unsigned char* vt =
+            lds + kAttnV + (16 * d + l16) * kVtRow + (64 * half + 32 * g + lq * 4) * 2;
+        const u32x2 lo = *reinterpret_cast<const u32x2*>(vt);
+        const u32x2 hi = *reinterpret_cast<const u32x2*>(vt + 32);
+        const u32x4 fv = {lo[0], lo[1], hi[0], hi[1]};
+        o[d] = mfma(__builtin_bit_cast(bf16x8, fv), fp, o[d]);
+      }
+    }
+  }
+  // l holds this lane's keys only
+  l += __shfl_xor(l, 16);
+  l += __shfl_xor(l, 32);
+  block_sync();
+  float* meet = reinterpret_cast<float*>(lds) + (w4 * 64 + lane) * 20;
+  if (half == 1) {
+    meet[0] = m;
+    meet[1] = l;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) *reinterpret_cast<f32x4*>(meet + 4 + d * 4) = o[d];
+  }
+  block_sync();
+  if (half == 1 || qi >= qlen) return;
+  const float m1 = meet[0];
+  const float top = __builtin_fmaxf(m, m1);
+  const float a0 = m == top ? 1.0f : __builtin_amdgcn_exp2f((m - top) * kExp);
+  const float a1 = m1 == top ? 1.0f : __builtin_amdgcn_exp2f((m1 - top) * kExp);
+  const float inv = 1.0f / (l * a0 + meet[1] * a1);
+  uint16_t* dst = out + ((size_t)qi * batch + b) * proj + head * kHead;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const f32x4 o1 = *reinterpret_cast<const f32x4*>(meet + 4 + d * 4);
+    store_bf16x4(dst + 16 * d + lq * 4, (o[d] * a0 + o1 * a1) * inv);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Adaptive softmax losses.  The logits (n x 267,738 at the client's vocabulary)
+// never reach memory: a workgroup turns its 128 x 128 tile into one (maximum, sum
+// of exponentials) pair a row, and the last kernel joins a row's pairs.
+
+constexpr int kMaxTails = 7;
+constexpr int kCritM = 128, kCritN = 128, kCritStages = 2;
+constexpr int kGroupThreads = 1024;
+
+struct Crit {
+  const uint16_t* hidden;          // [n, 512]
+  const uint16_t *weight, *bias;   // [n_token, 512], [n_token]
+  const uint16_t *tail_weight, *tail_bias;   // the head's entries for the tails
+  const int64_t* target;
+  int n, tails;
+  int edge[kMaxTails + 2];         // 0, cutoffs, n_token
+  int tiles[kMaxTails + 1];        // column tiles of the head and of each tail
+  uint32_t first_block[kMaxTails + 2];
+  int row_tiles;                   // of n rows: what every cluster's grid is made for
+  // workspace
+  int* count;                      // [tails] rows of each tail
+  int* place;                      // [n] a row's place within its tail
+  int* rows;                       // [tails][n] the rows, in order
+  float* logit;                    // [2][n] the target's logit in the head, in its tail
+  float2* pairs[kMaxTails + 1];    // [rows][tiles]
+};
+
+// Tail of a target (0: in the head or outside the vocabulary).
+__device__ __forceinline__ int tail_of(const Crit& c, int64_t t) {
+  int tail = 0;
+  for (int k = 1; k <= c.tails; ++k)
+    if (t >= c.edge[k] && t < c.edge[k + 1]) tail = k;
+  return tail;
+}
+
+// One workgroup: the rows of every tail, in their order.
+__global__ __launch_bounds__(kGroupThreads) void crit_group_kernel(Crit c) {
+  constexpr int kWaves = kGroupThreads / 64;
+  __shared__ int wave_count[kMaxTails][kWaves];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int seen[kMaxTails] = {0};
+  for (int base = 0; base < c.n; base += kGroupThreads) {
+    const int row = base + threadIdx.x;
+    const int tail = row < c.n ? tail_of(c, c.target[row]) : 0;
+    int before = 0;
+#pragma unroll
+    for (int k = 1; k <= kMaxTails; ++k) {
+      if (k > c.tails) break;
+      const uint64_t mine = __ballot(tail == k);
+      if (tail == k) before = __popcll(mine & ((1ull << lane) - 1));
+      if (lane == 0) wave_count[k - 1][wave] = __popcll(mine);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 1; k <= kMaxTails; ++k) {
+      if (k > c.tails) break;
+      int at = seen[k - 1], all = 0;
+      for (int w = 0; w < kWaves; ++w) {
+        if (w < wave) at += wave_count[k - 1][w];
+        all += wave_count[k - 1][w];
+      }
+      if (tail == k) {
+        c.place[row] = at + before;
+        c.rows[(size_t)(k - 1) * c.n + at + before] = row;
+      }
+      seen[k - 1] += all;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int k = 0; k < kMaxTails; ++k)
+      if (k < c.tails) c.count[k] = seen[k];
+}
+
+__global__ __launch_bounds__(kThreads, 2) void crit_logits_kernel(Crit c) {
+  __shared__ __attribute__((aligned(16))) unsigned char
+      lds[kCritStages * (Rows<kCritM>::kBytes + Rows<kCritN>::kBytes)];
+  int k = 0;
+  while (k < c.tails && blockIdx.x >= c.first_block[k + 1]) ++k;
+  // eight columns of tiles, then the next row of tiles: an XCD takes the row tiles
+  // of one column of tiles one after the other and reads those weights once
+  const int local = blockIdx.x - c.first_block[k];
+  const int per = 8 * c.row_tiles;
+  const int ct = local / per * 8 + local % 8;
+  const int rt = local % per / 8;
+  const int rows = k == 0 ? c.n : c.count[k - 1];
+  if (ct >= c.tiles[k] || rt * kCritM >= rows) return;
+  const int* list = k == 0 ? nullptr : c.rows + (size_t)(k - 1) * c.n;
+  const int lo = c.edge[k];
+  const int plain = c.edge[k + 1] - lo;            // columns of the vocabulary
+  const int cols = k == 0 ? plain + c.tails : plain;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int row0 = rt * kCritM, col0 = ct * kCritN;
+  auto row_of = [&](int at) {
+    at = at < rows ? at : rows - 1;
+    return list ? list[at] : at;
+  };
+  Rows<kCritM> a;
+  Rows<kCritN> b;
+  a.init(wave, lane, [&](int r) { return c.hidden + (size_t)row_of(row0 + r) * kD; });
+  b.init(wave, lane, [&](int r) {
+    const int col = col0 + r < cols ? col0 + r : cols - 1;
+    return col < plain ? c.weight + (size_t)(lo + col) * kD
+                       : c.tail_weight + (size_t)(col - plain) * kD;
+  });
+  // what the epilogue needs, asked for ahead of the product
+  float bias[kCritN / 32][4];
+#pragma unroll
+  for (int j = 0; j < kCritN / 32; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      int col = col0 + wn * (kCritN / 2) + j * 16 + lq * 4 + e;
+      col = col < cols ? col : cols - 1;
+      const uint16_t* p = col < plain ? c.bias + lo + col : c.tail_bias + (col - plain);
+      bias[j][e] = __builtin_bit_cast(float, (uint32_t)*p << 16);
+    }
+  int row[kCritM / 32], want[kCritM / 32];         // the target's column, if it has one here
+#pragma unroll
+  for (int i = 0; i < kCritM / 32; ++i) {
+    const int at = row0 + wm * (kCritM / 2) + i * 16 + l16;
+    row[i] = row_of(at);
+    const int64_t t = c.target[row[i]];
+    if (at >= rows || t < 0 || t >= c.edge[c.tails + 1]) {
+      want[i] = -1;
+    } else if (k == 0) {
+      const int tail = tail_of(c, t);
+      want[i] = tail ? plain + tail - 1 : (int)t;
+    } else {
+      want[i] = (int)t - lo;
+    }
+  }
+  f32x4 acc[kCritM / 32][kCritN / 32];
+  clear(acc);
+  stream_product<kCritM, kCritN, kCritStages>(acc, lds, kPanelTiles, kTileK, a, b, wm, wn, lane);
+
+  block_sync();
+  float2* half_pairs = reinterpret_cast<float2*>(lds);   // [2][kCritM]
+#pragma unroll
+  for (int i = 0; i < kCritM / 32; ++i) {
+    const int r = wm * (kCritM / 2) + i * 16 + l16;
+    float top = -__builtin_inff();
+#pragma unroll
+    for (int j = 0; j < kCritN / 32; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int col = col0 + wn * (kCritN / 2) + j * 16 + lq * 4 + e;
+        const float v = acc[i][j][e] + bias[j][e];
+        if (col == want[i]) c.logit[(size_t)(k != 0) * c.n + row[i]] = v;
+        acc[i][j][e] = col < cols ? v : -__builtin_inff();
+        top = __builtin_fmaxf(top, acc[i][j][e]);
+      }
+    top = __builtin_fmaxf(top, __shfl_xor(top, 16));
+    top = __builtin_fmaxf(top, __shfl_xor(top, 32));
+    const float base = top == -__builtin_inff() ? 0.0f : top;
+    float sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < kCritN / 32; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum += __expf(acc[i][j][e] - base);
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (lq == 0) half_pairs[wn * kCritM + r] = make_float2(top, sum);
+  }
+  block_sync();
+  const int r = threadIdx.x;
+  if (r < kCritM && row0 + r < rows) {
+    const float2 x = half_pairs[r], y = half_pairs[kCritM + r];
+    const float top = __builtin_fmaxf(x.x, y.x);
+    const float fx = x.x == top ? 1.0f : __expf(x.x - top);
+    const float fy = y.x == top ? 1.0f : __expf(y.x - top);
+    c.pairs[k][(size_t)(row0 + r) * c.tiles[k] + ct] = make_float2(top, x.y * fx + y.y * fy);
+  }
+}
+
+// log of a row's sum of exponentials from its pairs, by one wave.
+__device__ __forceinline__ float join_pairs(const float2* pairs, int count, int lane) {
+  float top = -__builtin_inff(), sum = 0.0f;
+  for (int i = lane; i < count; i += 64) {
+    const float2 p = pairs[i];
+    const float t = __builtin_fmaxf(top, p.x);
+    sum = sum * (top == t ? 1.0f : __expf(top - t)) + p.y * (p.x == t ? 1.0f : __expf(p.x - t));
+    top = t;
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const float ot = __shfl_xor(top, d), os = __shfl_xor(sum, d);
+    const float t = __builtin_fmaxf(top, ot);
+    sum = sum * (top == t ? 1.0f : __expf(top - t)) + os * (ot == t ? 1.0f : __expf(ot - t));
+    top = t;
+  }
+  return top + logf(sum);
+}
+
+__global__ __launch_bounds__(kThreads) void crit_losses_kernel(Crit c, uint16_t* nll) {
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
+  if (row >= c.n) return;
+  const int64_t t = c.target[row];
+  float loss = 0.0f;                               // a target outside the vocabulary: 0
+  if (t >= 0 && t < c.edge[c.tails + 1]) {
+    loss = join_pairs(c.pairs[0] + (size_t)row * c.tiles[0], c.tiles[0], lane) - c.logit[row];
+    const int k = tail_of(c, t);
+    if (k)
+      loss += join_pairs(c.pairs[k] + (size_t)c.place[row] * c.tiles[k], c.tiles[k], lane) -
+              c.logit[(size_t)c.n + row];
+  }
+  if (lane == 0) nll[row] = (uint16_t)pack_bf16(loss, 0.0f);
+}
+
+// Pieces of a workspace, 256-byte aligned; with no base only their sizes add up.
+struct Pieces {
+  char* base;
+  size_t used = 0;
+  template <typename T>
+  T* take(size_t count) {
+    T* p = base ? reinterpret_cast<T*>(base + used) : nullptr;
+    used += (count * sizeof(T) + 255) & ~(size_t)255;
+    return p;
+  }
+};
+
+struct Buffers {
+  uint16_t *x, *x2, *qu, *qv, *att, *h, *kv_x, *kv_mem, *table, *r;
+  float* y;
+  size_t bytes;
+};
+
+Buffers buffers_of(const orion_txl_dims& d, void* base) {
+  const size_t rows = (size_t)d.q_len * d.batch, mem_rows = (size_t)d.m_len * d.batch;
+  const size_t proj = (size_t)d.heads * kHead, k_len = (size_t)d.q_len + d.m_len;
+  Pieces p{(char*)base};
+  Buffers b;
+  b.y = p.take<float>(rows * kD);
+  b.x = p.take<uint16_t>(rows * kD);
+  b.x2 = p.take<uint16_t>(rows * kD);
+  b.qu = p.take<uint16_t>(rows * proj);
+  b.qv = p.take<uint16_t>(rows * proj);
+  b.att = p.take<uint16_t>(rows * proj);
+  b.h = p.take<uint16_t>(rows * d.inner);
+  b.kv_x = p.take<uint16_t>(rows * 2 * proj);
+  b.kv_mem = p.take<uint16_t>(d.layers * mem_rows * 2 * proj);
+  b.table = p.take<uint16_t>(k_len * kD);
+  b.r = p.take<uint16_t>(d.layers * k_len * proj);
+  b.bytes = p.used;
+  return b;
+}
+
+bool dims_fit(const orion_txl_dims& d) {
+  return d.q_len > 0 && d.m_len >= 0 && d.batch > 0 && d.layers > 0 && d.heads > 0 &&
+         d.heads % 2 == 0 && d.heads <= 1024 && d.inner > 0 && d.inner % 128 == 0 &&
+         d.inner <= (1 << 20) && ((int64_t)d.q_len + d.m_len) * d.batch < (1 << 24) &&
+         d.q_len <= 65535 * kQ;
+}
+
+size_t tiles(size_t n, int tile) { return (n + tile - 1) / tile; }
+
+bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
+  if (a->rows <= 0 || a->rows >= (1 << 24) || a->tails < 0 || a->tails > kMaxTails) return false;
+  c->hidden = (const uint16_t*)a->hidden;
+  c->weight = (const uint16_t*)a->weight;
+  c->bias = (const uint16_t*)a->bias;
+  c->tail_weight = (const uint16_t*)a->tail_weight;
+  c->tail_bias = (const uint16_t*)a->tail_bias;
+  c->target = (const int64_t*)a->target;
+  c->n = a->rows;
+  c->tails = a->tails;
+  c->row_tiles = (int)tiles(a->rows, kCritM);
+  uint64_t blocks = 0;
+  for (int k = 0; k <= a->tails + 1; ++k) {
+    c->edge[k] = a->edges[k];
+    if (k == 0 ? a->edges[0] != 0 : a->edges[k] <= a->edges[k - 1]) return false;
+  }
+  Pieces p{(char*)base};
+  c->count = p.take<int>(kMaxTails);
+  c->place = p.take<int>(a->rows);
+  c->rows = p.take<int>((size_t)a->tails * a->rows);
+  c->logit = p.take<float>((size_t)2 * a->rows);
+  for (int k = 0; k <= a->tails; ++k) {
+    c->first_block[k] = (uint32_t)blocks;
+    c->tiles[k] = (int)tiles((size_t)c->edge[k + 1] - c->edge[k] + (k == 0 ? a->tails : 0), kCritN);
+    c->pairs[k] = p.take<float2>((size_t)a->rows * c->tiles[k]);
+    blocks += tiles(c->tiles[k], 8) * 8 * c->row_tiles;
+    if (blocks > 0x7fffffffu) return false;
+  }
+  c->first_block[a->tails + 1] = (uint32_t)blocks;
+  *bytes = p.used;
+  return true;
+}
+
+}  // namespace
+
+extern "C" size_t orion_txl_workspace_bytes(const orion_txl_dims* dims) {
+  return dims != nullptr && dims_fit(*dims) ? buffers_of(*dims, nullptr).bytes : 0;
+}
+
+extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_layer* layers,
+                                const void* u, const void* v, const void* x0, const void* mems,
+                                size_t mem_stride, void* new_mems, size_t new_mem_stride,
+                                int mem_rows_out, void* hidden, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  if (!dims || !layers || !u || !v || !x0 || !hidden || !workspace) return ORION_ERR_ARG;
+  const orion_txl_dims& d = *dims;
+  if (!dims_fit(d)) return ORION_ERR_SHAPE;
+  if ((d.m_len > 0 && !mems) || (new_mems && (mem_rows_out <= 0 || mem_rows_out > d.q_len)))
+    return ORION_ERR_ARG;
+  uintptr_t all = (uintptr_t)u | (uintptr_t)v | (uintptr_t)x0 | (uintptr_t)mems |
+                  (uintptr_t)new_mems | (uintptr_t)hidden | (uintptr_t)workspace |
+                  (d.m_len > 0 ? mem_stride * 2 : 0) | (new_mems ? new_mem_stride * 2 : 0);
+  for (int i = 0; i < d.layers; ++i) {
+    const void* const* p = reinterpret_cast<const void* const*>(layers + i);
+    for (size_t e = 0; e < sizeof(orion_txl_layer) / sizeof(void*); ++e) {
+      if (!p[e]) return ORION_ERR_ARG;
+      all |= (uintptr_t)p[e];
+    }
+  }
+  if ((all & 15u) != 0) return ORION_ERR_ALIGN;
+  if (workspace_bytes < buffers_of(d, nullptr).bytes) return ORION_ERR_ARG;
+
+  const Buffers w = buffers_of(d, workspace);
+  hipStream_t s = (hipStream_t)stream;
+  const int rows = d.q_len * d.batch, mem_rows = d.m_len * d.batch, k_len = d.q_len + d.m_len;
+  const int proj = d.heads * kHead;
+  typedef const uint16_t* In;
+
+  hipLaunchKernelGGL(txl_positions_kernel, dim3(k_len), dim3(kD / 2), 0, s, w.table);
+  Jobs jobs;
+  jobs.count = 0;
+  uint64_t blocks = 0;
+  auto flush = [&]() {
+    if (jobs.count == 0) return;
+    for (int i = jobs.count; i <= kMaxJobs; ++i) jobs.first_block[i] = (uint32_t)blocks;
+    hipLaunchKernelGGL(txl_jobs_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, jobs);
+    jobs.count = 0;
+    blocks = 0;
+  };
+  auto add = [&](In A, In W, uint16_t* out, int M, int N) {
+    if (M == 0) return;
+    jobs.job[jobs.count] = Job{A, W, out, M, N / kJobN, N};
+    jobs.first_block[jobs.count++] = (uint32_t)blocks;
+    blocks += tiles(M, kJobM) * (N / kJobN);
+    if (jobs.count == kMaxJobs) flush();
+  };
+  for (int i = 0; i < d.layers; ++i) {
+    add(w.table, (In)layers[i].pos, w.r + (size_t)i * k_len * proj, k_len, proj);
+    add((In)mems + i * mem_stride, (In)layers[i].qkv + (size_t)proj * kD,
+        w.kv_mem + (size_t)i * mem_rows * 2 * proj, mem_rows, 2 * proj);
+  }
+  flush();
+
+  const unsigned row_tiles = (unsigned)tiles(rows, 64);
+  const unsigned qkv_tiles = 3 * proj / 96, ff_tiles = d.inner / 128;
+  const dim3 res_grid((unsigned)tiles(rows, kResM) * (kD / kResN));
+  for (int i = 0; i < d.layers; ++i) {
+    const orion_txl_layer& p = layers[i];
+    // x_i also goes into the memory's last rows
+    RowsOut out = {};
+    if (new_mems) {
+      out.mem = (uint16_t*)new_mems + i * new_mem_stride;
+      out.mem_from = (d.q_len - mem_rows_out) * d.batch;
+    }
+    const QkvEpi qkv = {w.qu, w.qv, w.kv_x, (In)u, (In)v, proj};
+    In x = (In)x0;
+    if (i == 0) {
+      hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 96, false, QkvEpi>), dim3(row_tiles * qkv_tiles),
+                         dim3(kThreads), 0, s, x0, (In)p.qkv, rows, (int)qkv_tiles, Norm{}, out,
+                         qkv);
+    } else {
+      x = out.x = w.x;
+      const Norm norm = {(In)layers[i - 1].norm2_w, (In)layers[i - 1].norm2_b, d.eps};
+      hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 96, true, QkvEpi>), dim3(row_tiles * qkv_tiles),
+                         dim3(kThreads), 0, s, (const void*)w.y, (In)p.qkv, rows, (int)qkv_tiles,
+                         norm, out, qkv);
+    }
+    hipLaunchKernelGGL(txl_attention_kernel, dim3(d.heads * d.batch, (unsigned)tiles(d.q_len, kQ)),
+                       dim3(kAttnThreads), 0, s, (In)w.qu, (In)w.qv,
+                       (In)(w.kv_mem + (size_t)i * mem_rows * 2 * proj), (In)w.kv_x,
+                       (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
+                       d.heads);
+    hipLaunchKernelGGL(txl_residual_gemm_kernel, res_grid, dim3(2 * kThreads), 0, s, (In)w.att,
+                       (In)p.out, proj, (In) nullptr, x, w.y, rows);
+    const Norm norm = {(In)p.norm1_w, (In)p.norm1_b, d.eps};
+    RowsOut out2 = {};
+    out2.x = w.x2;
+    hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 128, true, ReluEpi>), dim3(row_tiles * ff_tiles),
+                       dim3(kThreads), 0, s, (const void*)w.y, (In)p.ff1_w, rows, (int)ff_tiles,
+                       norm, out2, ReluEpi{w.h, (In)p.ff1_b, d.inner});
+    hipLaunchKernelGGL(txl_residual_gemm_kernel, res_grid, dim3(2 * kThreads), 0, s, (In)w.h,
+                       (In)p.ff2_w, d.inner, (In)p.ff2_b, (In)w.x2, w.y, rows);
+  }
+  const orion_txl_layer& last = layers[d.layers - 1];
+  hipLaunchKernelGGL(txl_norm_kernel, dim3((unsigned)tiles(rows, kThreads / 16)), dim3(kThreads), 0,
+                     s, (const float*)w.y, (Norm{(In)last.norm2_w, (In)last.norm2_b, d.eps}),
+                     (uint16_t*)hidden, rows);
+  return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
+}
+
+extern "C" size_t orion_nll_workspace_bytes(const orion_nll* args) {
+  Crit c;
+  size_t bytes = 0;
+  return args != nullptr && lay_out(args, nullptr, &c, &bytes) ? bytes : 0;
+}
+
+extern "C" int orion_nll_bf16(const orion_nll* args, void* nll, void* workspace,
+                              size_t workspace_bytes, void* stream) {
+  if (!args || !nll || !workspace || !args->hidden || !args->weight || !args->bias ||
+      !args->target || (args->tails > 0 && (!args->tail_weight || !args->tail_bias)))
+    return ORION_ERR_ARG;
+  Crit c;
+  size_t bytes = 0;
+  if (!lay_out(args, workspace, &c, &bytes)) return ORION_ERR_SHAPE;
+  if (workspace_bytes < bytes) return ORION_ERR_ARG;
+  if ((((uintptr_t)args->hidden | (uintptr_t)args->weight | (uintptr_t)args->tail_weight |
+        (uintptr_t)workspace) & 15u) != 0)
+    return ORION_ERR_ALIGN;
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(crit_group_kernel, dim3(1), dim3(kGroupThreads), 0, s, c);
+  hipLaunchKernelGGL(crit_logits_kernel, dim3(c.first_block[c.tails + 1]), dim3(kThreads), 0, s,
+                     c);
+  hipLaunchKernelGGL(crit_losses_kernel, dim3((unsigned)tiles(c.n, kThreads / 64)), dim3(kThreads),
+                     0, s, c, (uint16_t*)nll);
+  return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
+}

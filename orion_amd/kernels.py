@@ -15,6 +15,17 @@ STATUS = {0: "ok", 1: "bad argument", 2: "shape not a multiple of the tile",
           3: "pointer not 16-byte aligned", 4: "launch rejected"}
 
 
+class _TxlDims(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_int) for name in
+                ("layers", "heads", "inner", "q_len", "m_len", "batch")] + [("eps", ctypes.c_float)]
+
+
+class _Nll(ctypes.Structure):
+    _fields_ = [(name, ctypes.c_void_p) for name in
+                ("hidden", "weight", "bias", "tail_weight", "tail_bias", "target")] + [
+                    ("rows", ctypes.c_int), ("tails", ctypes.c_int), ("edges", ctypes.c_int * 9)]
+
+
 class KernelError(RuntimeError):
     def __init__(self, name, code):
         super().__init__(f"{name}: {STATUS.get(code, code)}")
@@ -38,6 +49,16 @@ def lib():
             ctypes.c_void_p, ctypes.c_int, ctypes.c_double, ctypes.c_double, ctypes.c_double,
             ctypes.c_double, ctypes.c_double, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
         handle.orion_lamb_step.restype = ctypes.c_int
+        ptr, size = ctypes.c_void_p, ctypes.c_size_t
+        handle.orion_txl_workspace_bytes.argtypes = [ptr]
+        handle.orion_txl_workspace_bytes.restype = size
+        handle.orion_txl_hidden.argtypes = [ptr, ptr, ptr, ptr, ptr, ptr, size, ptr, size,
+                                            ctypes.c_int, ptr, ptr, size, ptr]
+        handle.orion_txl_hidden.restype = ctypes.c_int
+        handle.orion_nll_workspace_bytes.argtypes = [ptr]
+        handle.orion_nll_workspace_bytes.restype = size
+        handle.orion_nll_bf16.argtypes = [ptr, ptr, ptr, size, ptr]
+        handle.orion_nll_bf16.restype = ctypes.c_int
         handle.orion_stream_create.argtypes = [ctypes.c_int, ctypes.POINTER(ctypes.c_void_p)]
         handle.orion_stream_create.restype = ctypes.c_int
         handle.orion_stream_destroy.argtypes = [ctypes.c_void_p]
@@ -199,3 +220,116 @@ def lamb_step(params, grads, ms, vs, lr, betas, eps, weight_decay):
         raise KernelError("orion_lamb_step", rc)
     for ts in (params, ms, vs):          # written behind autograd's back
         torch.autograd.graph.increment_version(ts)
+
+
+TXL_WIDTH, TXL_HEAD, TXL_TAILS = 512, 64, 7     # what the Transformer-XL kernels are built for
+
+
+def _bf16_operand(t, shape, index):
+    """Whether a tensor is what the bf16 kernels read: plain, contiguous, on GPU
+    ``index`` and 16-byte aligned."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype is torch.bfloat16
+            and t.shape == shape and t.get_device() == index and t.layout is torch.strided
+            and t.is_contiguous() and not t.data_ptr() & 15)
+
+
+def inference_only():
+    """No gradients to record, no tracing or rewriting, no autocast."""
+    return (not torch.is_grad_enabled() and plain_eager()
+            and not torch.is_autocast_enabled("cuda"))
+
+
+def txl_hidden(x, mems, u, v, layers, inner, eps, keep):
+    """Hidden states [q, batch, 512] of the embedded tokens ``x`` behind the memory
+    ``mems`` [layers, m, batch, 512] (or None), and the last ``keep`` positions of
+    the layers' inputs, memory included (None for ``keep`` 0).  ``layers`` holds,
+    per layer, the eleven tensors of ``orion_txl_layer``.  None where the kernels
+    do not take these tensors."""
+    index = x.get_device()
+    if index < 0 or not _bf16_operand(x, x.shape, index) or x.dim() != 3 or not x.numel():
+        return None
+    q_len, batch, width = x.shape
+    heads = u.shape[0]
+    proj = heads * TXL_HEAD
+    if width != TXL_WIDTH or not (_bf16_operand(u, (heads, TXL_HEAD), index)
+                                  and _bf16_operand(v, (heads, TXL_HEAD), index)):
+        return None
+    row = (width,)
+    shapes = ((3 * proj, width), (proj, width), (width, proj), row, row,
+              (inner, width), (inner,), (width, inner), row, row, row)
+    table = []
+    for tensors in layers:
+        for t, shape in zip(tensors, shapes):
+            if not _bf16_operand(t, shape, index):
+                return None
+            table.append(t.data_ptr())
+    m_len = 0
+    if mems is not None:
+        if (type(mems) is not torch.Tensor or mems.dtype is not torch.bfloat16
+                or mems.dim() != 4 or mems.get_device() != index
+                or mems.shape[0] != len(layers) or mems.shape[2:] != (batch, width)):
+            return None
+        m_len = mems.shape[1]
+        if m_len and (mems.stride()[1:] != (batch * width, width, 1) or mems.stride(0) % 8
+                      or mems.data_ptr() & 15):
+            return None
+    dims = _TxlDims(len(layers), heads, inner, q_len, m_len, batch, eps)
+    handle = lib()
+    size = handle.orion_txl_workspace_bytes(ctypes.byref(dims))
+    if not size:
+        return None
+    table = (ctypes.c_void_p * len(table))(*table)
+    with torch.cuda.device(index):
+        hidden = torch.empty_like(x)
+        work = torch.empty(size, dtype=torch.uint8, device=x.device)
+        new, new_at, new_stride, from_x = None, None, 0, 0
+        if keep:
+            keep = min(keep, m_len + q_len)
+            from_x = min(keep, q_len)
+            new = torch.empty((len(layers), keep, batch, width), dtype=x.dtype, device=x.device)
+            if keep > q_len:
+                new[:, :keep - q_len].copy_(mems[:, m_len - (keep - q_len):])
+            new_at, new_stride = new[0, keep - from_x].data_ptr(), new.stride(0)
+        rc = handle.orion_txl_hidden(
+            ctypes.byref(dims), table, u.data_ptr(), v.data_ptr(), x.data_ptr(),
+            mems.data_ptr() if m_len else None, mems.stride(0) if m_len else 0,
+            new_at, new_stride, from_x, hidden.data_ptr(), work.data_ptr(), size,
+            _stream_ptr(None))
+    if rc != 0:
+        raise KernelError("orion_txl_hidden", rc)
+    return hidden, new
+
+
+def adaptive_nll(hidden, target, weight, bias, tail_weight, tail_bias, edges):
+    """Losses [n] of ``target`` [n] under an adaptive softmax over ``hidden``
+    [n, 512]; None where the kernels do not take these tensors."""
+    index = hidden.get_device()
+    tails = len(edges) - 2
+    if index < 0 or hidden.dim() != 2 or not 0 <= tails <= TXL_TAILS or not edges[-1] < 1 << 31:
+        return None
+    n, width = hidden.shape
+    if width != TXL_WIDTH or not n or any(lo >= hi for lo, hi in zip(edges, edges[1:])):
+        return None
+    for t, shape in ((hidden, (n, width)), (weight, (edges[-1], width)), (bias, (edges[-1],)),
+                     (tail_weight, (tails, width)), (tail_bias, (tails,))):
+        if not _bf16_operand(t, shape, index):
+            return None
+    if (type(target) is not torch.Tensor or target.dtype is not torch.int64
+            or target.shape != (n,) or target.get_device() != index
+            or not target.is_contiguous()):
+        return None
+    args = _Nll(hidden.data_ptr(), weight.data_ptr(), bias.data_ptr(), tail_weight.data_ptr(),
+                tail_bias.data_ptr(), target.data_ptr(), n, tails,
+                (ctypes.c_int * 9)(*edges))
+    handle = lib()
+    size = handle.orion_nll_workspace_bytes(ctypes.byref(args))
+    if not size:
+        return None
+    with torch.cuda.device(index):
+        nll = torch.empty(n, dtype=hidden.dtype, device=hidden.device)
+        work = torch.empty(size, dtype=torch.uint8, device=hidden.device)
+        rc = handle.orion_nll_bf16(ctypes.byref(args), nll.data_ptr(), work.data_ptr(), size,
+                                   _stream_ptr(None))
+    if rc != 0:
+        raise KernelError("orion_nll_bf16", rc)
+    return nll
