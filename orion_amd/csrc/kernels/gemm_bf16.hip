@@ -34,8 +34,16 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "mfma_tile.h"
 
 namespace {
+
+using mfma_tile::bf16x2;
+using mfma_tile::bf16x8;
+using mfma_tile::f32x2;
+using mfma_tile::f32x4;
+using mfma_tile::u32x2;
+using mfma_tile::u32x4;
 
 constexpr int BM = 256;
 constexpr int BN = 256;
@@ -45,20 +53,12 @@ constexpr int kStages = 2;
 constexpr int kMatBytes = BM * BK * 2;      // 32 KiB per operand and stage
 constexpr int kStageBytes = 2 * kMatBytes;  // A then B
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
 // c += a * b on the matrix core; c lives in accumulator registers and is
 // updated in place (as a builtin call the register allocator shuffles the 256
 // accumulators between register files in every iteration).
 __device__ __forceinline__ void mfma_16x16x32(f32x4& c, const bf16x8& a, const bf16x8& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // Four consecutive elements of a row of C from one accumulator tile.
 __device__ __forceinline__ void store_quad(float* p, const f32x4& v) {
@@ -286,6 +286,161 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_nt_kernel(
   }
 }
 
+// Smaller tiles, for products whose 256 x 256 tiles would leave compute units
+// idle: mfma_tile.h's pipeline (four stages), GROUPS groups of four waves that take
+// every GROUPS-th k-tile (their sums meet in LDS).  Bound by the latency of a
+// k-tile's way to the MFMAs, 0.12 to 0.42 us by tile against 0.06 to 0.22 of matrix
+// core time.  Measured, before (256 x 256) and now, us:
+//   256 x 512 x 256      8.9 ->  3.6      3072 x 1024 x 1024   20.9 -> 10.5
+//   1024 x 1024 x 1024  20.7 ->  6.0      3072 x 1024 x 4096   65.6 -> 26.8
+//   512 x 512 x 8192     121 -> 17.5      2304 x 2304 x 2048   37.4 -> 31.6
+__device__ __forceinline__ void small_tile_of_block(int bid, int tiles_m, int tiles_n, int* tm,
+                                                    int* tn) {
+  // a contiguous range of tiles per XCD, bands of kGroupM tile rows
+  const int total = tiles_m * tiles_n, per = total / kXcds, extra = total % kXcds;
+  const int xcd = bid % kXcds;
+  const int lid = xcd * per + (xcd < extra ? xcd : extra) + bid / kXcds;
+  const int band = kGroupM * tiles_n;
+  const int first_m = lid / band * kGroupM;
+  const int rows = tiles_m - first_m < kGroupM ? tiles_m - first_m : kGroupM;
+  const int in_band = lid % band;
+  *tm = first_m + in_band % rows;
+  *tn = in_band / rows;
+}
+
+template <int TM, int TN, int NS, int GROUPS, typename OutT>
+__global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                              OutT* __restrict__ C, int M, int N, int K) {
+  using namespace mfma_tile;
+  constexpr int kGroupLds = NS * (Rows<TM>::kBytes + Rows<TN>::kBytes);
+  constexpr int kSumLds = (GROUPS - 1) * TM * TN * 4;
+  constexpr int kWaveRows = TM / 2, kWaveCols = TN / 2;
+  constexpr int kRowB = kWaveCols * (int)sizeof(OutT);
+  constexpr int kOutLds = 4 * kWaveRows * kRowB;
+  constexpr int kLds = GROUPS * kGroupLds > kSumLds
+                           ? (GROUPS * kGroupLds > kOutLds ? GROUPS * kGroupLds : kOutLds)
+                           : (kSumLds > kOutLds ? kSumLds : kOutLds);
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave_all & 3, group = wave_all >> 2;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int l16 = lane & 15, lq = lane >> 4;
+  int tm, tn;
+  small_tile_of_block(blockIdx.x, M / TM, N / TN, &tm, &tn);
+  const size_t row0 = (size_t)tm * TM, col0 = (size_t)tn * TN;
+  Rows<TM> a;
+  Rows<TN> b;
+  a.init(wave, lane, [&](int r) { return A + (row0 + r) * K + group * kTileK; });
+  b.init(wave, lane, [&](int r) { return B + (col0 + r) * K + group * kTileK; });
+  f32x4 acc[TM / 32][TN / 32];
+  clear(acc);
+  stream_product<TM, TN, NS>(acc, lds + group * kGroupLds, K / (GROUPS * kTileK),
+                             GROUPS * kTileK, a, b, wm, wn, lane);
+  block_sync();                        // the stages are free
+  if (GROUPS > 1) {
+    f32x4* other = reinterpret_cast<f32x4*>(lds) + wave * 64 + lane;
+    if (group == 1) {
+#pragma unroll
+      for (int i = 0; i < TM / 32; ++i)
+#pragma unroll
+        for (int j = 0; j < TN / 32; ++j) other[(i * (TN / 32) + j) * 256] = acc[i][j];
+    }
+    block_sync();
+    if (group == 0) {
+#pragma unroll
+      for (int i = 0; i < TM / 32; ++i)
+#pragma unroll
+        for (int j = 0; j < TN / 32; ++j) acc[i][j] += other[(i * (TN / 32) + j) * 256];
+    }
+    block_sync();
+    if (group == 1) return;
+  }
+  // whole rows of the wave's block leave as 16-byte pieces, as in the large kernel
+  constexpr int kSlots = kRowB / 16;
+  static_assert(kSlots <= 16, "the swizzle below takes a row's low four bits");
+  constexpr int kRowsPerStore = 64 / kSlots;
+  unsigned char* ep = lds + wave * kWaveRows * kRowB;
+#pragma unroll
+  for (int i = 0; i < TM / 32; ++i)
+#pragma unroll
+    for (int j = 0; j < TN / 32; ++j) {
+      const int byte = (j * 16 + lq * 4) * (int)sizeof(OutT);
+      store_quad(reinterpret_cast<OutT*>(ep + (i * 16 + l16) * kRowB +
+                                         (((byte >> 4) ^ (l16 & (kSlots - 1))) << 4) + (byte & 15)),
+                 acc[i][j]);
+    }
+  OutT* block = C + (row0 + wm * kWaveRows) * N + col0 + wn * kWaveCols;
+#pragma unroll
+  for (int it = 0; it < kWaveRows / kRowsPerStore; ++it) {
+    const int R = it * kRowsPerStore + lane / kSlots, slot = lane % kSlots;
+    const u32x4 v =
+        *reinterpret_cast<const u32x4*>(ep + R * kRowB + ((slot ^ (R & (kSlots - 1))) << 4));
+    *(reinterpret_cast<u32x4*>(block + (size_t)R * N) + slot) = v;
+  }
+}
+
+// What a launch of each tile takes, us: 1.5 + rounds of 256 workgroups * (fixed +
+// per_tile * k-tiles), fitted to products from 256 x 256 x 64 to 4096^3.  The fit is
+// within 20 %; the large tile's estimate counts 0.9 because a round of it keeps the
+// whole chip busy where one of the others waits (8192 x 2560 x 1024: 47 us by 256 x
+// 256 tiles, 54 by 128 x 128, both estimated at 46).
+struct TileCost {
+  int tm, tn, k;          // k: what the depth has to be a multiple of
+  double fixed, per_tile;
+};
+constexpr TileCost kTiles[] = {
+    {256, 256, 64, 4.0, 1.10},
+    {128, 128, 64, 2.0, 0.42},
+    {128, 64, 64, 1.7, 0.28},
+    {64, 64, 64, 1.5, 0.19},
+    {32, 64, 128, 1.5, 0.125},   // two groups of waves
+};
+
+int tile_for(int M, int N, int K) {
+  int best = 0;
+  double best_us = 0.0;
+  for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
+    const TileCost& t = kTiles[i];
+    if (K % t.k != 0) continue;
+    const long long blocks = (long long)(M / t.tm) * (N / t.tn);
+    const double us = 1.5 + (double)((blocks + 255) / 256) * (t.fixed + t.per_tile * (K / BK));
+    if (i == 0 || us < best_us) {
+      best = i;
+      best_us = i == 0 ? 0.9 * us : us;
+    }
+  }
+  return best;
+}
+
+template <typename OutT>
+void launch_gemm(const uint16_t* A, const uint16_t* B, OutT* C, int M, int N, int K,
+                 hipStream_t stream) {
+  const int tile = tile_for(M, N, K);
+  const dim3 grid((unsigned)((M / kTiles[tile].tm) * (N / kTiles[tile].tn)));
+  switch (tile) {
+    case 1:
+      hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<128, 128, 4, 1, OutT>), grid, dim3(256), 0,
+                         stream, A, B, C, M, N, K);
+      break;
+    case 2:
+      hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<128, 64, 4, 1, OutT>), grid, dim3(256), 0,
+                         stream, A, B, C, M, N, K);
+      break;
+    case 3:
+      hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<64, 64, 4, 1, OutT>), grid, dim3(256), 0,
+                         stream, A, B, C, M, N, K);
+      break;
+    case 4:
+      hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<32, 64, 4, 2, OutT>), grid, dim3(512), 0,
+                         stream, A, B, C, M, N, K);
+      break;
+    default:
+      hipLaunchKernelGGL(gemm_bf16_nt_kernel<OutT>, grid, dim3(kThreads), 0, stream, A, B, C, M,
+                         N, K);
+  }
+}
+
 }  // namespace
 
 extern "C" int orion_gemm_bf16_nt(const void* A, const void* B, void* C, int M,
@@ -298,15 +453,10 @@ extern "C" int orion_gemm_bf16_nt(const void* A, const void* B, void* C, int M,
     return ORION_ERR_ALIGN;
   const long long tiles = (long long)(M / BM) * (N / BN);
   if (tiles > 0x7fffffffLL) return ORION_ERR_SHAPE;
-  dim3 grid((unsigned)tiles), block(kThreads);
-  if (out_is_f32) {
-    hipLaunchKernelGGL(gemm_bf16_nt_kernel<float>, grid, block, 0,
-                       (hipStream_t)stream, (const uint16_t*)A,
-                       (const uint16_t*)B, (float*)C, M, N, K);
-  } else {
-    hipLaunchKernelGGL(gemm_bf16_nt_kernel<uint16_t>, grid, block, 0,
-                       (hipStream_t)stream, (const uint16_t*)A,
-                       (const uint16_t*)B, (uint16_t*)C, M, N, K);
-  }
+  if (out_is_f32)
+    launch_gemm((const uint16_t*)A, (const uint16_t*)B, (float*)C, M, N, K, (hipStream_t)stream);
+  else
+    launch_gemm((const uint16_t*)A, (const uint16_t*)B, (uint16_t*)C, M, N, K,
+                (hipStream_t)stream);
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
 }

@@ -5,12 +5,13 @@
 // A k-tile is 64 elements: one 128-byte line of every operand row.  In LDS the
 // 16-byte chunk c of row r sits at position c ^ (r & 7), so the fragment reads of
 // eight consecutive lanes (eight rows, one logical chunk) cover all banks once.
-// Operands go global -> LDS directly; NS stages keep NS - 1 k-tiles in flight and
-// one barrier a k-tile is enough: the stage a wave fills after the barrier is the
-// one that all waves had finished reading before it.
+// Operands go global -> LDS directly, NS k-tiles ahead of the one in work, with one
+// barrier a k-tile.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 namespace mfma_tile {
 
@@ -52,6 +53,18 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// The same in place and opaque to the compiler, which shuffles larger sets of
+// accumulators between registers in every k-tile when it allocates them itself
+// (128 x 128 tiles, 8192 deep: 55 us against 48).  At least three other MFMAs have
+// to lie between two that use the same accumulators, and `settle` between the last
+// one and what reads them.
+__device__ __forceinline__ void mfma_in_place(const bf16x8& a, const bf16x8& b, f32x4& c) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}// the second operand in accumulator registers too, for one that stays
+__device__ __forceinline__ void mfma_in_place_kept(const bf16x8& a, const bf16x8& b, f32x4& c) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "a"(b));
+}
+
 // Two floats to bf16, nearest even, in one register.
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   const f32x2 v = {lo, hi};
@@ -82,37 +95,85 @@ struct Rows {
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) p[i] = row_at((i * 4 + wave) * 8 + (lane >> 3)) + chunk * 8;
   }
+  __device__ __forceinline__ void issue_one(int i, int k, unsigned char* stage) const {
+    load_to_lds(p[i] + k, stage + (i * 4 + wave) * 1024);
+  }
   __device__ __forceinline__ void issue(int k, unsigned char* stage) const {
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) load_to_lds(p[i] + k, stage + (i * 4 + wave) * 1024);
+    for (int i = 0; i < kLoads; ++i) issue_one(i, k, stage);
   }
 };
 
-// acc += A tile * B tile over one k-tile in LDS.  Wave (wm, wn) of 2 x 2 owns rows
-// wm * BM / 2, columns wn * BN / 2.  The B fragment is the first operand, so a
-// lane's four accumulators of tile (i, j) are four consecutive columns of one row:
-// row i * 16 + lane % 16, columns j * 16 + lane / 16 * 4 .. + 3.
+// The fragments of one k-tile that wave (wm, wn) of 2 x 2 needs; it owns rows
+// wm * BM / 2, columns wn * BN / 2.  The B fragment is the MFMA's first operand, so
+// a lane's four accumulators of tile (i, j) are four consecutive columns of one
+// row: row i * 16 + lane % 16, columns j * 16 + lane / 16 * 4 .. + 3.
 template <int BM, int BN>
-__device__ __forceinline__ void tile_step(f32x4 (&acc)[BM / 32][BN / 32], const unsigned char* a,
-                                          const unsigned char* b, int wm, int wn, int lane) {
-  const int l16 = lane & 15, lq = lane >> 4;
-  const unsigned char* pa = a + (wm * (BM / 2) + l16) * kRowBytes;
-  const unsigned char* pb = b + (wn * (BN / 2) + l16) * kRowBytes;
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const int at = ((ks * 4 + lq) ^ (l16 & 7)) << 4;
-    bf16x8 fa[BM / 32], fb[BN / 32];
-#pragma unroll
-    for (int i = 0; i < BM / 32; ++i)
-      fa[i] = *reinterpret_cast<const bf16x8*>(pa + i * 16 * kRowBytes + at);
-#pragma unroll
-    for (int j = 0; j < BN / 32; ++j)
-      fb[j] = *reinterpret_cast<const bf16x8*>(pb + j * 16 * kRowBytes + at);
-#pragma unroll
-    for (int i = 0; i < BM / 32; ++i)
-#pragma unroll
-      for (int j = 0; j < BN / 32; ++j) acc[i][j] = mfma(fb[j], fa[i], acc[i][j]);
+struct Fragments {
+  static constexpr int kI = BM / 32, kJ = BN / 32;
+  static constexpr int kReads = 2 * (kI + kJ);
+  bf16x8 a[2][kI], b[2][kJ];
+  __device__ __forceinline__ void read_one(int r, const unsigned char* ta, const unsigned char* tb,
+                                           int wm, int wn, int lane) {
+    const int ks = r / (kI + kJ), x = r % (kI + kJ);
+    const int l16 = lane & 15;
+    const int at = ((ks * 4 + (lane >> 4)) ^ (l16 & 7)) << 4;
+    if (x < kJ)
+      b[ks][x] = *reinterpret_cast<const bf16x8*>(tb + (wn * (BN / 2) + x * 16 + l16) * kRowBytes +
+                                                  at);
+    else
+      a[ks][x - kJ] = *reinterpret_cast<const bf16x8*>(
+          ta + (wm * (BM / 2) + (x - kJ) * 16 + l16) * kRowBytes + at);
   }
+  __device__ __forceinline__ void read(const unsigned char* ta, const unsigned char* tb, int wm,
+                                       int wn, int lane) {
+#pragma unroll
+    for (int r = 0; r < kReads; ++r) read_one(r, ta, tb, wm, wn, lane);
+  }
+};
+
+// acc += the fragments' product.  `kReads` reads and `kLoads` loads of what comes
+// next are issued one by one between the MFMAs, the reads in the first three
+// quarters: a wave that issues them in a row leaves its matrix core idle meanwhile
+// (128 x 128 tiles, 8192 deep, one workgroup a compute unit: 68 us; the loads alone
+// 40, everything else 49).
+template <int BM, int BN, int kReads, int kLoads, typename Read, typename Load>
+__device__ __forceinline__ void multiply(f32x4 (&acc)[BM / 32][BN / 32],
+                                         const Fragments<BM, BN>& f, Read read, Load load) {
+  constexpr int kI = BM / 32, kJ = BN / 32, kM = 2 * kI * kJ;
+  constexpr int kSpan = kM * 3 / 4 > 0 ? kM * 3 / 4 : 1;
+#pragma unroll
+  for (int m = 0; m < kM; ++m) {
+    const int ks = m / (kI * kJ), i = m / kJ % kI, j = m % kJ;
+    if (kI * kJ >= 4) mfma_in_place(f.b[ks][j], f.a[ks][i], acc[i][j]);
+    else acc[i][j] = mfma(f.b[ks][j], f.a[ks][i], acc[i][j]);
+#pragma unroll
+    for (int r = 0; r < kReads; ++r)
+      if (r * kSpan / (kReads ? kReads : 1) == m) read(r);
+#pragma unroll
+    for (int l = 0; l < kLoads; ++l)
+      if (l * kM / (kLoads ? kLoads : 1) == m) load(l);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+template <int BM, int BN>
+__device__ __forceinline__ void multiply(f32x4 (&acc)[BM / 32][BN / 32],
+                                         const Fragments<BM, BN>& f) {
+  multiply<BM, BN, 0, 0>(acc, f, [](int) {}, [](int) {});
+}
+
+// Whatever wrote the accumulators is done with them, and what follows comes after.
+template <int I, int J>
+__device__ __forceinline__ void settle(f32x4 (&acc)[I][J]) {
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) asm volatile("" : "+a"(acc[i][j]));
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) asm volatile("" : "+a"(acc[i][j]));
 }
 
 template <int I, int J>
@@ -121,10 +182,13 @@ __device__ __forceinline__ void clear(f32x4 (&acc)[I][J]) {
   for (int i = 0; i < I; ++i)
 #pragma unroll
     for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  settle(acc);
 }
 
 // acc += A * B^T over KT >= 1 k-tiles that lie k_step elements apart, both operands
-// staged through NS stages at `lds`.
+// staged through NS stages at `lds`.  The fragments of a whole k-tile are read
+// while the one before it is multiplied: behind the barrier the next tile has
+// landed, and every wave has this one in registers, so its stage is filled again.
 template <int BM, int BN, int NS>
 __device__ __forceinline__ void stream_product(f32x4 (&acc)[BM / 32][BN / 32],
                                                unsigned char* lds, int KT, int k_step,
@@ -132,26 +196,62 @@ __device__ __forceinline__ void stream_product(f32x4 (&acc)[BM / 32][BN / 32],
                                                int wn, int lane) {
   constexpr int kStage = Rows<BM>::kBytes + Rows<BN>::kBytes;
   constexpr int kLoads = Rows<BM>::kLoads + Rows<BN>::kLoads;
-  auto issue = [&](int kt, int stage) {
-    unsigned char* s = lds + stage * kStage;
+  auto issue = [&](int kt, unsigned char* s) {
     a.issue(kt * k_step, s);
     b.issue(kt * k_step, s + Rows<BM>::kBytes);
   };
+  auto read = [&](Fragments<BM, BN>& f, unsigned char* s) {
+    f.read(s, s + Rows<BM>::kBytes, wm, wn, lane);
+  };
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s)
-    if (s < KT) issue(s, s);
-  int cur = 0, fill = NS - 1;
-  for (int kt = 0; kt < KT; ++kt) {
-    // the loads of the k-tiles after this one may still be in flight
-    if (KT - 1 - kt >= NS - 2) wait_vm<kLoads*(NS - 2)>();
+  for (int s = 0; s < NS; ++s)
+    if (s < KT) issue(s, lds + s * kStage);
+  if (KT >= NS) wait_vm<kLoads*(NS - 1)>();
+  else wait_vm<0>();
+  block_sync();
+  Fragments<BM, BN> even, odd;
+  read(even, lds);
+  unsigned char* cur = lds;
+  // kMore: there is a tile to load into the freed stage
+  auto step = [&](const Fragments<BM, BN>& now, Fragments<BM, BN>& next, int kt, auto more) {
+    constexpr bool kMore = decltype(more)::value;
+    // the loads of the tiles after the next one may still be in flight
+    if (kMore || KT - kt >= NS) wait_vm<kLoads*(NS - 2)>();
     else wait_vm<0>();
     block_sync();
-    if (kt + NS - 1 < KT) issue(kt + NS - 1, fill);
-    const unsigned char* s = lds + cur * kStage;
-    tile_step<BM, BN>(acc, s, s + Rows<BM>::kBytes, wm, wn, lane);
-    cur = cur + 1 == NS ? 0 : cur + 1;
-    fill = fill + 1 == NS ? 0 : fill + 1;
+    unsigned char* freed = cur;
+    cur = cur + kStage == lds + NS * kStage ? lds : cur + kStage;
+    if (!kMore && kt + NS < KT) issue(kt + NS, freed);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply<BM, BN, Fragments<BM, BN>::kReads, kMore ? kLoads : 0>(
+        acc, now,
+        [&](int r) { next.read_one(r, cur, cur + Rows<BM>::kBytes, wm, wn, lane); },
+        [&](int l) {
+          if (l < Rows<BM>::kLoads) a.issue_one(l, (kt + NS) * k_step, freed);
+          else b.issue_one(l - Rows<BM>::kLoads, (kt + NS) * k_step, freed + Rows<BM>::kBytes);
+        });
+  };
+  // between these parts the compiler may move accumulators and fragments
+  int kt = 0;
+  for (; kt + 1 + NS < KT; kt += 2) {
+    step(even, odd, kt, std::true_type{});
+    step(odd, even, kt + 1, std::true_type{});
   }
+  settle(acc);
+  for (; kt + 2 < KT; kt += 2) {
+    step(even, odd, kt, std::false_type{});
+    step(odd, even, kt + 1, std::false_type{});
+  }
+  settle(acc);
+  if (kt + 1 < KT) {
+    step(even, odd, kt, std::false_type{});
+    settle(acc);
+    block_sync();                      // odd has arrived
+    even = odd;
+  }
+  settle(acc);
+  multiply(acc, even);
+  settle(acc);
 }
 
 }  // namespace mfma_tile

@@ -41,6 +41,7 @@ using namespace mfma_tile;
 constexpr int kD = 512;               // model width: the length of a norm's row
 constexpr int kHead = 64;             // head width
 constexpr int kPanelTiles = kD / kTileK;
+static_assert(kPanelTiles == 8, "panel_gemm's steps");
 constexpr int kMaxJobs = 64;
 constexpr int kThreads = 256;
 
@@ -150,7 +151,7 @@ __device__ __forceinline__ void panel_gemm(unsigned char* lds, const void* A, co
     for (int kt = 0; kt < kPanelTiles; ++kt) a.issue(kt * kTileK, lds + kt * Rows<BM>::kBytes);
   }
 #pragma unroll
-  for (int s = 0; s < NS - 1; ++s) b.issue(s * kTileK, stages + s * Rows<BN>::kBytes);
+  for (int s = 0; s < NS; ++s) b.issue(s * kTileK, stages + s * Rows<BN>::kBytes);
   if (kNorm) {
     const int cl = lane & 15;
 #pragma unroll
@@ -170,16 +171,35 @@ __device__ __forceinline__ void panel_gemm(unsigned char* lds, const void* A, co
   }
   f32x4 acc[BM / 32][BN / 32];
   clear(acc);
-#pragma unroll
-  for (int kt = 0; kt < kPanelTiles; ++kt) {
-    if (kt + NS - 2 < kPanelTiles) wait_vm<Rows<BN>::kLoads*(NS - 2)>();
-    else wait_vm<0>();
+  Fragments<BM, BN> f[2];
+  wait_vm<Rows<BN>::kLoads*(NS - 1)>();
+  block_sync();
+  f[0].read(lds, stages, wm, wn, lane);
+  auto step = [&](auto tile) {                     // as in stream_product
+    constexpr int kt = decltype(tile)::value;
+    constexpr bool kMore = kt + NS < kPanelTiles;
+    wait_vm<kPanelTiles - kt >= NS ? Rows<BN>::kLoads*(NS - 2) : 0>();
     block_sync();
-    if (kt + NS - 1 < kPanelTiles)
-      b.issue((kt + NS - 1) * kTileK, stages + (kt + NS - 1) % NS * Rows<BN>::kBytes);
-    tile_step<BM, BN>(acc, lds + kt * Rows<BM>::kBytes, stages + kt % NS * Rows<BN>::kBytes, wm,
-                      wn, lane);
-  }
+    __builtin_amdgcn_sched_barrier(0);
+    multiply<BM, BN, Fragments<BM, BN>::kReads, kMore ? Rows<BN>::kLoads : 0>(
+        acc, f[kt & 1],
+        [&](int r) {
+          f[(kt + 1) & 1].read_one(r, lds + (kt + 1) * Rows<BM>::kBytes,
+                                   stages + (kt + 1) % NS * Rows<BN>::kBytes, wm, wn, lane);
+        },
+        [&](int l) {
+          b.issue_one(l, (kt + NS) * kTileK, stages + kt % NS * Rows<BN>::kBytes);
+        });
+  };
+  step(std::integral_constant<int, 0>{});
+  step(std::integral_constant<int, 1>{});
+  step(std::integral_constant<int, 2>{});
+  step(std::integral_constant<int, 3>{});
+  step(std::integral_constant<int, 4>{});
+  step(std::integral_constant<int, 5>{});
+  step(std::integral_constant<int, 6>{});
+  multiply(acc, f[1]);
+  settle(acc);
   if (!kNorm && tn == 0 && (out.x || out.mem)) {
     for (int i = threadIdx.x; i < BM * (kD / 8); i += kThreads) {
       const int r = i / (kD / 8), chunk = i % (kD / 8);
@@ -565,12 +585,15 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Adaptive softmax losses.  The logits (n x 267,738 at the client's vocabulary)
-// never reach memory: a workgroup turns its 128 x 128 tile into one (maximum, sum
-// of exponentials) pair a row, and the last kernel joins a row's pairs.
+// Adaptive softmax losses.  The logits (n x 267,735 at the client's vocabulary)
+// never reach memory: a workgroup takes 128 rows and up to kCritChunk tiles of 128
+// columns of one cluster and leaves one (maximum, sum of exponentials) pair a row;
+// the last kernel joins a row's pairs and computes the target's own logits and the
+// head's entries for the tails as plain dot products.
 
 constexpr int kMaxTails = 7;
-constexpr int kCritM = 128, kCritN = 128, kCritStages = 2;
+constexpr int kCritM = 128, kCritN = 128, kCritStages = 8;
+constexpr int kCritChunk = 16;
 constexpr int kGroupThreads = 1024;
 
 struct Crit {
@@ -580,15 +603,14 @@ struct Crit {
   const int64_t* target;
   int n, tails;
   int edge[kMaxTails + 2];         // 0, cutoffs, n_token
-  int tiles[kMaxTails + 1];        // column tiles of the head and of each tail
+  int chunks[kMaxTails + 1];       // of column tiles, of the head and of each tail
   uint32_t first_block[kMaxTails + 2];
   int row_tiles;                   // of n rows: what every cluster's grid is made for
   // workspace
   int* count;                      // [tails] rows of each tail
   int* place;                      // [n] a row's place within its tail
   int* rows;                       // [tails][n] the rows, in order
-  float* logit;                    // [2][n] the target's logit in the head, in its tail
-  float2* pairs[kMaxTails + 1];    // [rows][tiles]
+  float2* pairs[kMaxTails + 1];    // [rows][chunks]
 };
 
 // Tail of a target (0: in the head or outside the vocabulary).
@@ -639,113 +661,168 @@ __global__ __launch_bounds__(kGroupThreads) void crit_group_kernel(Crit c) {
       if (k < c.tails) c.count[k] = seen[k];
 }
 
-__global__ __launch_bounds__(kThreads, 2) void crit_logits_kernel(Crit c) {
-  __shared__ __attribute__((aligned(16))) unsigned char
-      lds[kCritStages * (Rows<kCritM>::kBytes + Rows<kCritN>::kBytes)];
+// Wave w owns rows 32 w .. + 31, whose 512 elements stay in registers, and all 128
+// columns of a tile; only the weights go through LDS, eight k-tiles ahead and from
+// one column tile straight on to the next, so that a tile's epilogue runs while the
+// next ones' weights arrive.  (As independent 128 x 128 tiles through two or four
+// stages the kernel took 226 and 309 us of a batch-4 request: at eight k-tiles a
+// tile its first loads and its epilogue cost as much as its products.)
+__global__ __launch_bounds__(kThreads, 1) void crit_logits_kernel(Crit c) {
+  constexpr int NS = kCritStages, kStage = Rows<kCritN>::kBytes, kLoads = Rows<kCritN>::kLoads;
+  constexpr int kJ = kCritN / 16;
+  static_assert(NS == kPanelTiles, "the waits below");
+  // the stages, and a tile's biases for each wave (one array: with two the compiler
+  // waits for the loads in flight before every read)
+  __shared__ __attribute__((aligned(16))) unsigned char lds[NS * kStage + 4 * kCritN * 2];
   int k = 0;
   while (k < c.tails && blockIdx.x >= c.first_block[k + 1]) ++k;
-  // eight columns of tiles, then the next row of tiles: an XCD takes the row tiles
-  // of one column of tiles one after the other and reads those weights once
+  // eight chunks, then the next row of tiles: an XCD takes the row tiles of one
+  // chunk one after the other and reads those weights once
   const int local = blockIdx.x - c.first_block[k];
   const int per = 8 * c.row_tiles;
-  const int ct = local / per * 8 + local % 8;
-  const int rt = local % per / 8;
+  const int chunk = local / per * 8 + local % 8;
+  const int row0 = local % per / 8 * kCritM;
   const int rows = k == 0 ? c.n : c.count[k - 1];
-  if (ct >= c.tiles[k] || rt * kCritM >= rows) return;
+  if (chunk >= c.chunks[k] || row0 >= rows) return;
   const int* list = k == 0 ? nullptr : c.rows + (size_t)(k - 1) * c.n;
-  const int lo = c.edge[k];
-  const int plain = c.edge[k + 1] - lo;            // columns of the vocabulary
-  const int cols = k == 0 ? plain + c.tails : plain;
+  const int lo = c.edge[k] + chunk * kCritChunk * kCritN;    // this chunk's tokens
+  const int hi = c.edge[k + 1];
+  const int n_token = c.edge[c.tails + 1];
+  const int all = (hi - lo + kCritN - 1) / kCritN;
+  const int tiles = all < kCritChunk ? all : kCritChunk;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, lq = lane >> 4;
-  const int row0 = rt * kCritM, col0 = ct * kCritN;
-  auto row_of = [&](int at) {
-    at = at < rows ? at : rows - 1;
-    return list ? list[at] : at;
+  // a tile may reach past its cluster (masked below) but not past the vocabulary
+  auto issue_one = [&](int i, int tile, int kt) {
+    int token = lo + tile * kCritN + (i * 4 + wave) * 8 + (lane >> 3);
+    token = token < n_token ? token : n_token - 1;
+    load_to_lds(c.weight + (size_t)token * kD + kt * kTileK + ((lane & 7) ^ (lane >> 3)) * 8,
+                lds + kt * kStage + (i * 4 + wave) * 1024);
   };
-  Rows<kCritM> a;
-  Rows<kCritN> b;
-  a.init(wave, lane, [&](int r) { return c.hidden + (size_t)row_of(row0 + r) * kD; });
-  b.init(wave, lane, [&](int r) {
-    const int col = col0 + r < cols ? col0 + r : cols - 1;
-    return col < plain ? c.weight + (size_t)(lo + col) * kD
-                       : c.tail_weight + (size_t)(col - plain) * kD;
-  });
-  // what the epilogue needs, asked for ahead of the product
-  float bias[kCritN / 32][4];
 #pragma unroll
-  for (int j = 0; j < kCritN / 32; ++j)
+  for (int kt = 0; kt < NS; ++kt)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      int col = col0 + wn * (kCritN / 2) + j * 16 + lq * 4 + e;
-      col = col < cols ? col : cols - 1;
-      const uint16_t* p = col < plain ? c.bias + lo + col : c.tail_bias + (col - plain);
-      bias[j][e] = __builtin_bit_cast(float, (uint32_t)*p << 16);
-    }
-  int row[kCritM / 32], want[kCritM / 32];         // the target's column, if it has one here
+    for (int i = 0; i < kLoads; ++i) issue_one(i, 0, kt);
+  bf16x8 fa[2][2 * kPanelTiles];
 #pragma unroll
-  for (int i = 0; i < kCritM / 32; ++i) {
-    const int at = row0 + wm * (kCritM / 2) + i * 16 + l16;
-    row[i] = row_of(at);
-    const int64_t t = c.target[row[i]];
-    if (at >= rows || t < 0 || t >= c.edge[c.tails + 1]) {
-      want[i] = -1;
-    } else if (k == 0) {
-      const int tail = tail_of(c, t);
-      want[i] = tail ? plain + tail - 1 : (int)t;
-    } else {
-      want[i] = (int)t - lo;
-    }
+  for (int i = 0; i < 2; ++i) {
+    int at = row0 + wave * 32 + i * 16 + l16;
+    at = at < rows ? at : rows - 1;
+    const uint16_t* p = c.hidden + (size_t)(list ? list[at] : at) * kD + lq * 8;
+#pragma unroll
+    for (int ks = 0; ks < 2 * kPanelTiles; ++ks)
+      fa[i][ks] = *reinterpret_cast<const bf16x8*>(p + ks * 32);
   }
-  f32x4 acc[kCritM / 32][kCritN / 32];
-  clear(acc);
-  stream_product<kCritM, kCritN, kCritStages>(acc, lds, kPanelTiles, kTileK, a, b, wm, wn, lane);
+  bf16x8 fb[2][2 * kJ];                             // [even, odd k-tile][k-step, columns]
+  auto read_one = [&](auto odd, int r, int kt) {
+    const int at = ((r / kJ * 4 + lq) ^ (l16 & 7)) << 4;
+    fb[decltype(odd)::value][r] = *reinterpret_cast<const bf16x8*>(
+        lds + kt * kStage + (r % kJ * 16 + l16) * kRowBytes + at);
+  };
 
+  float top[2] = {-__builtin_inff(), -__builtin_inff()}, sum[2] = {0.0f, 0.0f};
+  wait_vm<0>();
   block_sync();
-  float2* half_pairs = reinterpret_cast<float2*>(lds);   // [2][kCritM]
 #pragma unroll
-  for (int i = 0; i < kCritM / 32; ++i) {
-    const int r = wm * (kCritM / 2) + i * 16 + l16;
-    float top = -__builtin_inff();
-#pragma unroll
-    for (int j = 0; j < kCritN / 32; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int col = col0 + wn * (kCritN / 2) + j * 16 + lq * 4 + e;
-        const float v = acc[i][j][e] + bias[j][e];
-        if (col == want[i]) c.logit[(size_t)(k != 0) * c.n + row[i]] = v;
-        acc[i][j][e] = col < cols ? v : -__builtin_inff();
-        top = __builtin_fmaxf(top, acc[i][j][e]);
+  for (int r = 0; r < 2 * kJ; ++r) read_one(std::integral_constant<int, 0>{}, r, 0);
+
+  auto tile = [&](int t, auto last) {
+    constexpr bool kLast = decltype(last)::value;
+    f32x4 acc[2][kJ];
+    clear(acc);
+    // of columns 2 * lane and the next; joined only in the epilogue, or the wait for
+    // them would empty the pipeline
+    uint16_t bias_lo = 0, bias_hi = 0;
+    auto step = [&](auto tile_c) {
+      constexpr int kt = decltype(tile_c)::value;
+      constexpr bool kRead = !kLast || kt + 1 < kPanelTiles;
+      if constexpr (kRead) {
+        // the next k-tile has landed; those after it may still be in flight
+        wait_vm<kLast ? kLoads * (kPanelTiles - 2 - kt) : kLoads * (NS - 2)>();
+        block_sync();
+        __builtin_amdgcn_sched_barrier(0);
+      } else {
+        block_sync();
       }
-    top = __builtin_fmaxf(top, __shfl_xor(top, 16));
-    top = __builtin_fmaxf(top, __shfl_xor(top, 32));
-    const float base = top == -__builtin_inff() ? 0.0f : top;
-    float sum = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kCritN / 32; ++j)
+      for (int m = 0; m < 4 * kJ; ++m) {
+        const int ks = m / (2 * kJ), i = m / kJ % 2, j = m % kJ;
+        mfma_in_place_kept(fb[kt & 1][ks * kJ + j], fa[i][kt * 2 + ks], acc[i][j]);
+        // reads of the next k-tile in the first three quarters, loads of the next
+        // column tile's into the stage that this one has left
+        if (kRead && m % 3 != 2 && m * 2 / 3 < 2 * kJ) {
+          constexpr int kNext = (kt + 1) % kPanelTiles;
+          read_one(std::integral_constant<int, (kt + 1) & 1>{}, (m * 2 + 2) / 3, kNext);
+        }
+        if (!kLast && m % 8 == 2) issue_one(m / 8, t + 1, kt);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    step(std::integral_constant<int, 0>{});
+    {
+      const int token = lo + t * kCritN + lane * 2;
+      bias_lo = c.bias[token < n_token ? token : n_token - 1];
+      bias_hi = c.bias[token + 1 < n_token ? token + 1 : n_token - 1];
+    }
+    step(std::integral_constant<int, 1>{});
+    step(std::integral_constant<int, 2>{});
+    step(std::integral_constant<int, 3>{});
+    step(std::integral_constant<int, 4>{});
+    step(std::integral_constant<int, 5>{});
+    step(std::integral_constant<int, 6>{});
+    step(std::integral_constant<int, 7>{});
+    settle(acc);
+    unsigned char* bias_lds = lds + NS * kStage + wave * kCritN * 2;
+    *reinterpret_cast<uint32_t*>(bias_lds + lane * 4) = bias_lo | (uint32_t)bias_hi << 16;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    // a lane's own columns only; lanes meet at the end
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sum += __expf(acc[i][j][e] - base);
-    sum += __shfl_xor(sum, 16);
-    sum += __shfl_xor(sum, 32);
-    if (lq == 0) half_pairs[wn * kCritM + r] = make_float2(top, sum);
-  }
-  block_sync();
-  const int r = threadIdx.x;
-  if (r < kCritM && row0 + r < rows) {
-    const float2 x = half_pairs[r], y = half_pairs[kCritM + r];
-    const float top = __builtin_fmaxf(x.x, y.x);
-    const float fx = x.x == top ? 1.0f : __expf(x.x - top);
-    const float fy = y.x == top ? 1.0f : __expf(y.x - top);
-    c.pairs[k][(size_t)(row0 + r) * c.tiles[k] + ct] = make_float2(top, x.y * fx + y.y * fy);
+    for (int i = 0; i < 2; ++i) {
+      float m = top[i];
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) {
+        const u32x2 two = *reinterpret_cast<const u32x2*>(bias_lds + (j * 16 + lq * 4) * 2);
+        const f32x4 bj = {bf16_lo(two[0]), bf16_hi(two[0]), bf16_lo(two[1]), bf16_hi(two[1])};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int token = lo + t * kCritN + j * 16 + lq * 4 + e;
+          const float v = acc[i][j][e] + bj[e];
+          acc[i][j][e] = !kLast || token < hi ? v : -__builtin_inff();
+          m = __builtin_fmaxf(m, acc[i][j][e]);
+        }
+      }
+      const float base = m == -__builtin_inff() ? 0.0f : m;
+      float s = sum[i] * __expf(top[i] - base);
+#pragma unroll
+      for (int j = 0; j < kJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += __expf(acc[i][j][e] - base);
+      top[i] = m;
+      sum[i] = s;
+    }
+  };
+  for (int t = 0; t + 1 < tiles; ++t) tile(t, std::false_type{});
+  tile(tiles - 1, std::true_type{});
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float m = top[i], s = sum[i];
+#pragma unroll
+    for (int d = 16; d < 64; d <<= 1) {
+      const float om = __shfl_xor(m, d), os = __shfl_xor(s, d);
+      const float t = __builtin_fmaxf(m, om);
+      s = s * (m == t ? 1.0f : __expf(m - t)) + os * (om == t ? 1.0f : __expf(om - t));
+      m = t;
+    }
+    const int at = row0 + wave * 32 + i * 16 + l16;
+    if (lq == 0 && at < rows) c.pairs[k][(size_t)at * c.chunks[k] + chunk] = make_float2(m, s);
   }
 }
 
-// log of a row's sum of exponentials from its pairs, by one wave.
-__device__ __forceinline__ float join_pairs(const float2* pairs, int count, int lane) {
-  float top = -__builtin_inff(), sum = 0.0f;
+// The pair of a row's pairs, by one wave; (maximum, sum) of the lanes' own to start.
+__device__ __forceinline__ float join_pairs(const float2* pairs, int count, int lane, float top,
+                                            float sum) {
   for (int i = lane; i < count; i += 64) {
     const float2 p = pairs[i];
     const float t = __builtin_fmaxf(top, p.x);
@@ -762,18 +839,52 @@ __device__ __forceinline__ float join_pairs(const float2* pairs, int count, int 
   return top + logf(sum);
 }
 
+// weight . x + bias by one wave, eight elements of the row a lane.
+__device__ __forceinline__ float logit_of(const uint16_t* weight, const uint16_t* bias,
+                                          const u32x4& x, int lane) {
+  const u32x4 w = *reinterpret_cast<const u32x4*>(weight + lane * 8);
+  float s = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    s = __builtin_fmaf(bf16_lo(w[e]), bf16_lo(x[e]), s);
+    s = __builtin_fmaf(bf16_hi(w[e]), bf16_hi(x[e]), s);
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) s += __shfl_xor(s, d);
+  return s + __builtin_bit_cast(float, (uint32_t)*bias << 16);
+}
+
 __global__ __launch_bounds__(kThreads) void crit_losses_kernel(Crit c, uint16_t* nll) {
+  static_assert(kD == 64 * 8, "logit_of's row");
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
   if (row >= c.n) return;
   const int64_t t = c.target[row];
   float loss = 0.0f;                               // a target outside the vocabulary: 0
   if (t >= 0 && t < c.edge[c.tails + 1]) {
-    loss = join_pairs(c.pairs[0] + (size_t)row * c.tiles[0], c.tiles[0], lane) - c.logit[row];
+    const u32x4 x = *reinterpret_cast<const u32x4*>(c.hidden + (size_t)row * kD + lane * 8);
     const int k = tail_of(c, t);
+    const float own = logit_of(c.weight + (size_t)t * kD, c.bias + t, x, lane);
+    // the head's entries for the tails: lane j starts from the j-th
+    float head = own, top = -__builtin_inff(), sum = 0.0f;
+    for (int j = 0; j < c.tails; ++j) {
+      const float v = logit_of(c.tail_weight + (size_t)j * kD, c.tail_bias + j, x, lane);
+      if (lane == j) {
+        top = v;
+        sum = v == -__builtin_inff() ? 0.0f : 1.0f;
+      }
+      if (j == k - 1) head = v;
+    }
+    // a NaN among them has to reach the sum: its maximum does not carry it
+    if (top != top) {
+      top = -__builtin_inff();
+      sum = __builtin_nanf("");
+    }
+    loss = join_pairs(c.pairs[0] + (size_t)row * c.chunks[0], c.chunks[0], lane, top, sum) - head;
     if (k)
-      loss += join_pairs(c.pairs[k] + (size_t)c.place[row] * c.tiles[k], c.tiles[k], lane) -
-              c.logit[(size_t)c.n + row];
+      loss += join_pairs(c.pairs[k] + (size_t)c.place[row] * c.chunks[k], c.chunks[k], lane,
+                         -__builtin_inff(), 0.0f) -
+              own;
   }
   if (lane == 0) nll[row] = (uint16_t)pack_bf16(loss, 0.0f);
 }
@@ -845,12 +956,11 @@ bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
   c->count = p.take<int>(kMaxTails);
   c->place = p.take<int>(a->rows);
   c->rows = p.take<int>((size_t)a->tails * a->rows);
-  c->logit = p.take<float>((size_t)2 * a->rows);
   for (int k = 0; k <= a->tails; ++k) {
     c->first_block[k] = (uint32_t)blocks;
-    c->tiles[k] = (int)tiles((size_t)c->edge[k + 1] - c->edge[k] + (k == 0 ? a->tails : 0), kCritN);
-    c->pairs[k] = p.take<float2>((size_t)a->rows * c->tiles[k]);
-    blocks += tiles(c->tiles[k], 8) * 8 * c->row_tiles;
+    c->chunks[k] = (int)tiles((size_t)c->edge[k + 1] - c->edge[k], kCritN * kCritChunk);
+    c->pairs[k] = p.take<float2>((size_t)a->rows * c->chunks[k]);
+    blocks += tiles(c->chunks[k], 8) * 8 * c->row_tiles;
     if (blocks > 0x7fffffffu) return false;
   }
   c->first_block[a->tails + 1] = (uint32_t)blocks;

@@ -151,3 +151,23 @@ def test_gemm_rejects_bad_shapes_without_launching():
     assert e.value.code == 2
     with pytest.raises(ValueError):
         kernels.gemm_bf16_nt(torch.zeros(256, 64, device=DEV), b)
+
+
+@pytest.mark.parametrize("shape", [
+    # one shape for each tile of the kernel at odd, smallest and pipeline-edge depths
+    (256, 256, 320), (256, 256, 384), (512, 512, 704), (1024, 1024, 192), (1024, 1024, 448),
+    (1024, 2048, 64), (1024, 2048, 576), (2048, 2048, 128), (2048, 2048, 320),
+    (2304, 2304, 1088), (2816, 3328, 192), (4096, 4096, 256)])
+def test_gemm_every_tile_exact_on_small_integers(shape):
+    # integers and depths at which every partial sum is exact in fp32: any order of
+    # the sums gives the same bits, and a fragment out of place does not
+    m, n, k = shape
+    g = torch.Generator(device=DEV).manual_seed(sum(shape))
+    ta, tb = (torch.randint(-4, 5, (rows, k), device=DEV, generator=g).to(torch.bfloat16)
+              for rows in (m, n))
+    want = (ta.float() @ tb.float().t())
+    for dtype in (torch.float32, torch.bfloat16):
+        out = torch.full((m, n), float("nan"), device=DEV, dtype=dtype)
+        for _ in range(3):
+            kernels.gemm_bf16_nt(ta, tb, out=out)
+            assert torch.equal(out, want.to(dtype))
