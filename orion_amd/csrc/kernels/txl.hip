@@ -20,9 +20,10 @@
 //   after       hidden = LN(y)
 //
 // The layer norm rides in the product that reads it: a workgroup's A panel is 64
-// whole rows of 512, so it normalises them itself on the way into LDS (every
-// workgroup of a row panel repeats that; the first column of workgroups also
-// writes the rows, for the residual and the memory).  y stays fp32.
+// whole rows of 512, so it normalises them itself on the way into LDS, from means
+// and squares that the product before left for every 32 columns (every workgroup
+// of a row panel repeats that; the first column of workgroups also writes the rows,
+// for the residual and the memory).  y stays fp32.
 //
 // Sums are fp32 throughout; activations are rounded to bf16 where the model's
 // own operations rounded them, less y, the two query biases (added in fp32) and
@@ -30,6 +31,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "kernels.h"
 #include "mfma_tile.h"
@@ -41,7 +44,6 @@ using namespace mfma_tile;
 constexpr int kD = 512;               // model width: the length of a norm's row
 constexpr int kHead = 64;             // head width
 constexpr int kPanelTiles = kD / kTileK;
-static_assert(kPanelTiles == 8, "panel_gemm's steps");
 constexpr int kMaxJobs = 64;
 constexpr int kThreads = 256;
 
@@ -52,62 +54,88 @@ __device__ __forceinline__ void store_bf16x4(uint16_t* p, const f32x4& v) {
   *reinterpret_cast<u32x2*>(p) = packed;
 }
 
-__device__ __forceinline__ f32x4 load_bf16x4(const uint16_t* p) {
-  const u32x2 v = *reinterpret_cast<const u32x2*>(p);
+__device__ __forceinline__ f32x4 unpack_bf16x4(const u32x2& v) {
   return f32x4{bf16_lo(v[0]), bf16_hi(v[0]), bf16_lo(v[1]), bf16_hi(v[1])};
 }
 
+// Sum over the sixteen lanes of a row of lanes, by rotations within it.
 __device__ __forceinline__ float sum16(float v) {
-#pragma unroll
-  for (int d = 1; d < 16; d <<= 1) v += __shfl_xor(v, d);
+  auto rotated = [](float x, auto by) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                           0x120 + decltype(by)::value, 0xf, 0xf, true));
+  };
+  v += rotated(v, std::integral_constant<int, 8>{});
+  v += rotated(v, std::integral_constant<int, 4>{});
+  v += rotated(v, std::integral_constant<int, 2>{});
+  v += rotated(v, std::integral_constant<int, 1>{});
   return v;
 }
 
 struct Norm {
   const uint16_t* w;
   const uint16_t* b;
+  const float2* parts;
   float eps;
 };
 
-// Layer norm of four rows of 512 by one wave, sixteen lanes a row; lane l % 16
-// gets the 16-byte bf16 chunks l % 16 + 16 * j of its row.  Mean first, then the
-// squared distances from it.
-__device__ __forceinline__ void norm_row(const float* y, const Norm& norm, int cl,
-                                         u32x4 (&out)[4]) {
+// A row's layer norm starts from the mean and the sum of squared distances from it
+// of each of its sixteen parts of 32 elements, left by the product that made the row.
+constexpr int kParts = 16, kPartLen = kD / kParts;
+
+// A row of 512 for layer norm, sixteen lanes a row: lane l % 16 holds the elements
+// of the 16-byte bf16 chunks l % 16 + 16 * j, and one of the parts.
+struct NormRow {
   f32x4 v[4][2];
+  float2 part;
+  __device__ __forceinline__ void load(const float* y, const Norm& norm, int row, int cl) {
+    part = norm.parts[(size_t)row * kParts + cl];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float* p = y + (cl + 16 * j) * 8;
-    v[j][0] = *reinterpret_cast<const f32x4*>(p);
-    v[j][1] = *reinterpret_cast<const f32x4*>(p + 4);
-  }
-  float s = 0.0f;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s += v[j][e >> 2][e & 3];
-  const float mean = sum16(s) * (1.0f / kD);
-  float q = 0.0f;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float d = v[j][e >> 2][e & 3] - mean;
-      q = __builtin_fmaf(d, d, q);
+    for (int j = 0; j < 4; ++j) {
+      const float* p = y + (size_t)row * kD + (cl + 16 * j) * 8;
+      v[j][0] = *reinterpret_cast<const f32x4*>(p);
+      v[j][1] = *reinterpret_cast<const f32x4*>(p + 4);
     }
-  const float rstd = 1.0f / __builtin_sqrtf(sum16(q) * (1.0f / kD) + norm.eps);
+  }
+};
+
+struct NormWeights {
+  float w[4][8], b[4][8];
+  __device__ __forceinline__ void load(const Norm& norm, int cl) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const u32x4 w = *reinterpret_cast<const u32x4*>(norm.w + (cl + 16 * j) * 8);
-    const u32x4 b = *reinterpret_cast<const u32x4*>(norm.b + (cl + 16 * j) * 8);
+    for (int j = 0; j < 4; ++j) {
+      const u32x4 pw = *reinterpret_cast<const u32x4*>(norm.w + (cl + 16 * j) * 8);
+      const u32x4 pb = *reinterpret_cast<const u32x4*>(norm.b + (cl + 16 * j) * 8);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        w[j][2 * e] = bf16_lo(pw[e]);
+        w[j][2 * e + 1] = bf16_hi(pw[e]);
+        b[j][2 * e] = bf16_lo(pb[e]);
+        b[j][2 * e + 1] = bf16_hi(pb[e]);
+      }
+    }
+  }
+};
+
+__device__ __forceinline__ void norm_row(const NormRow& row, const NormWeights& weights,
+                                         float eps, u32x4 (&out)[4]) {
+  const float mean = sum16(row.part.x) * (1.0f / kParts);
+  const float d = row.part.x - mean;
+  const float squares = sum16(__builtin_fmaf((float)kPartLen * d, d, row.part.y));
+  const float rstd = 1.0f / __builtin_sqrtf(squares * (1.0f / kD) + eps);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float lo = (v[j][e >> 1][(e & 1) * 2] - mean) * rstd;
-      const float hi = (v[j][e >> 1][(e & 1) * 2 + 1] - mean) * rstd;
-      out[j][e] = pack_bf16(__builtin_fmaf(lo, bf16_lo(w[e]), bf16_lo(b[e])),
-                            __builtin_fmaf(hi, bf16_hi(w[e]), bf16_hi(b[e])));
+      float x[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int at = e * 2 + h;
+        x[h] = __builtin_fmaf((row.v[j][at >> 2][at & 3] - mean) * rstd, weights.w[j][at],
+                              weights.b[j][at]);
+      }
+      out[j][e] = pack_bf16(x[0], x[1]);
     }
-  }
 }
 
 // Rows of the normalised (or given) input that later launches and the caller read.
@@ -124,106 +152,160 @@ __device__ __forceinline__ void put_row(const RowsOut& out, int row, int chunk, 
 }
 
 // C[M, N] = A[M, 512] * W[N, 512]^T with the whole A panel of a workgroup in LDS:
-// normalised on the way from fp32 (kNorm) or loaded as it is.  W streams through
-// four stages.  N is a multiple of BN; rows past M are computed from the last row
-// and not written.
+// normalised on the way from fp32 (kNorm) or loaded as it is.  Two groups of four
+// waves take the even and the odd k-tiles, W streaming through kPanelStages stages
+// each, and their sums meet in LDS.  With four waves and eight k-tiles in a row the
+// norm took 7,000 cycles of a product's 16,000 and the loop 5,000: one wave a SIMD
+// waits for every latency alone.  N is a multiple of BN; rows past M are computed
+// from the last row and not written.
+constexpr int kPanelThreads = 2 * kThreads;
+constexpr int kPanelStages = 3;
+
+template <int BM, int BN>
+constexpr int panel_lds() {
+  return BM * kD * 2 + 2 * kPanelStages * Rows<BN>::kBytes;
+}
+
 template <int BM, int BN, bool kNorm, typename Epi>
 __device__ __forceinline__ void panel_gemm(unsigned char* lds, const void* A, const uint16_t* W,
-                                           int M, int tm, int tn, const Norm& norm,
+                                           int M, int tm, int tn, int tiles_n, const Norm& norm,
                                            const RowsOut& out, const Epi& epi) {
-  constexpr int NS = 4;
-  constexpr int kPanel = BM * kD * 2;
+  constexpr int NS = kPanelStages, kSteps = kPanelTiles / 2;
+  constexpr int kI = BM / 32, kJ = BN / 32;
+  static_assert(kI == 2, "each group of waves finishes one of two row tiles");
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave8 & 3, group = wave8 >> 2;
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, lq = lane >> 4;
   const int row0 = tm * BM;
-  unsigned char* stages = lds + kPanel;
+  unsigned char* stages = lds + BM * kD * 2 + group * NS * Rows<BN>::kBytes;
+  // k-tile 2 * step + group
+  unsigned char* panel = lds + group * Rows<BM>::kBytes;
+  auto k_of = [&](int step) { return (2 * step + group) * kTileK; };
   Rows<BN> b;
   b.init(wave, lane, [&](int r) { return W + (size_t)(tn * BN + r) * kD; });
-  if (!kNorm) {
+  // the rows are written by one column of workgroups each
+  const int writers = tiles_n < 16 ? tiles_n : 16;
+
+  if constexpr (kNorm) {
+    constexpr int kRows = BM / 32;        // times four rows, a wave
+    const int cl = lane & 15;
+    NormRow rows[kRows];
+    NormWeights weights;
+#pragma unroll
+    for (int it = 0; it < kRows; ++it) {
+      const int row = row0 + wave8 * (BM / 8) + it * 4 + (lane >> 4);
+      rows[it].load(static_cast<const float*>(A), norm, row < M ? row : M - 1, cl);
+    }
+    weights.load(norm, cl);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) b.issue(k_of(s), stages + s * Rows<BN>::kBytes);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int it = 0; it < kRows; ++it) {
+      const int r = wave8 * (BM / 8) + it * 4 + (lane >> 4);
+      const bool put = (wave8 * kRows + it) % writers == tn && row0 + r < M;
+      u32x4 v[4];
+      norm_row(rows[it], weights, norm.eps, v);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int chunk = cl + 16 * j;
+        *reinterpret_cast<u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes + r * kRowBytes +
+                                  (((chunk & 7) ^ (r & 7)) << 4)) = v[j];
+        if (put) put_row(out, row0 + r, chunk, v[j]);
+      }
+    }
+  } else {
     Rows<BM> a;
     a.init(wave, lane, [&](int r) {
       const int row = row0 + r < M ? row0 + r : M - 1;
       return static_cast<const uint16_t*>(A) + (size_t)row * kD;
     });
 #pragma unroll
-    for (int kt = 0; kt < kPanelTiles; ++kt) a.issue(kt * kTileK, lds + kt * Rows<BM>::kBytes);
+    for (int s = 0; s < kSteps; ++s) a.issue(k_of(s), panel + s * 2 * Rows<BM>::kBytes);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) b.issue(k_of(s), stages + s * Rows<BN>::kBytes);
   }
+  const int col0 = tn * BN + wn * (BN / 2) + lq * 4;
+  typename Epi::Ahead ahead[kJ];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) b.issue(s * kTileK, stages + s * Rows<BN>::kBytes);
-  if (kNorm) {
-    const int cl = lane & 15;
-#pragma unroll
-    for (int it = 0; it < BM / 16; ++it) {
-      const int r = wave * (BM / 4) + it * 4 + (lane >> 4);
-      const int row = row0 + r < M ? row0 + r : M - 1;
-      u32x4 v[4];
-      norm_row(static_cast<const float*>(A) + (size_t)row * kD, norm, cl, v);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int chunk = cl + 16 * j;
-        *reinterpret_cast<u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes + r * kRowBytes +
-                                  (((chunk & 7) ^ (r & 7)) << 4)) = v[j];
-        if (tn == 0 && row0 + r < M) put_row(out, row0 + r, chunk, v[j]);
-      }
-    }
-  }
-  f32x4 acc[BM / 32][BN / 32];
+  for (int j = 0; j < kJ; ++j) ahead[j] = epi.ahead(col0 + j * 16);
+
+  f32x4 acc[kI][kJ];
   clear(acc);
   Fragments<BM, BN> f[2];
   wait_vm<Rows<BN>::kLoads*(NS - 1)>();
   block_sync();
-  f[0].read(lds, stages, wm, wn, lane);
-  auto step = [&](auto tile) {                     // as in stream_product
-    constexpr int kt = decltype(tile)::value;
-    constexpr bool kMore = kt + NS < kPanelTiles;
-    wait_vm<kPanelTiles - kt >= NS ? Rows<BN>::kLoads*(NS - 2) : 0>();
+  f[0].read(panel, stages, wm, wn, lane);
+  auto step = [&](auto step_c) {                   // as in stream_product
+    constexpr int st = decltype(step_c)::value;
+    constexpr bool kMore = st + NS < kSteps;
+    wait_vm<kSteps - st >= NS ? Rows<BN>::kLoads*(NS - 2) : 0>();
     block_sync();
     __builtin_amdgcn_sched_barrier(0);
     multiply<BM, BN, Fragments<BM, BN>::kReads, kMore ? Rows<BN>::kLoads : 0>(
-        acc, f[kt & 1],
+        acc, f[st & 1],
         [&](int r) {
-          f[(kt + 1) & 1].read_one(r, lds + (kt + 1) * Rows<BM>::kBytes,
-                                   stages + (kt + 1) % NS * Rows<BN>::kBytes, wm, wn, lane);
+          f[(st + 1) & 1].read_one(r, panel + (st + 1) * 2 * Rows<BM>::kBytes,
+                                   stages + (st + 1) % NS * Rows<BN>::kBytes, wm, wn, lane);
         },
-        [&](int l) {
-          b.issue_one(l, (kt + NS) * kTileK, stages + kt % NS * Rows<BN>::kBytes);
-        });
+        [&](int l) { b.issue_one(l, k_of(st + NS), stages + st % NS * Rows<BN>::kBytes); });
   };
+  static_assert(kSteps == 4, "the steps");
   step(std::integral_constant<int, 0>{});
   step(std::integral_constant<int, 1>{});
   step(std::integral_constant<int, 2>{});
-  step(std::integral_constant<int, 3>{});
-  step(std::integral_constant<int, 4>{});
-  step(std::integral_constant<int, 5>{});
-  step(std::integral_constant<int, 6>{});
   multiply(acc, f[1]);
   settle(acc);
-  if (!kNorm && tn == 0 && (out.x || out.mem)) {
-    for (int i = threadIdx.x; i < BM * (kD / 8); i += kThreads) {
-      const int r = i / (kD / 8), chunk = i % (kD / 8);
-      if (row0 + r < M)
-        put_row(out, row0 + r, chunk,
-                *reinterpret_cast<const u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes +
-                                                r * kRowBytes + (((chunk & 7) ^ (r & 7)) << 4)));
+
+  if constexpr (!kNorm) {
+    if (out.x || out.mem) {               // sixteen lanes a row, as above
+#pragma unroll
+      for (int it = 0; it < BM / 32; ++it) {
+        const int r = wave8 * (BM / 8) + it * 4 + (lane >> 4);
+        if ((wave8 * (BM / 32) + it) % writers != tn || row0 + r >= M) continue;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int chunk = l16 + 16 * j;
+          put_row(out, row0 + r, chunk,
+                  *reinterpret_cast<const u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes +
+                                                  r * kRowBytes +
+                                                  (((chunk & 7) ^ (r & 7)) << 4)));
+        }
+      }
     }
   }
+  block_sync();                           // the panel and the stages have been read
+  // group g finishes row tile g of its waves' two
+  f32x4* meet = reinterpret_cast<f32x4*>(lds) + wave * 64 + lane;
+  if (group == 0) {
 #pragma unroll
-  for (int i = 0; i < BM / 32; ++i) {
-    const int row = row0 + wm * (BM / 2) + i * 16 + l16;
-    if (row >= M) continue;
+    for (int j = 0; j < kJ; ++j) meet[(kJ + j) * 256] = acc[1][j];
+  } else {
 #pragma unroll
-    for (int j = 0; j < BN / 32; ++j)
-      epi(row, tn * BN + wn * (BN / 2) + j * 16 + lq * 4, acc[i][j]);
+    for (int j = 0; j < kJ; ++j) meet[j * 256] = acc[0][j];
+  }
+  block_sync();
+  const int row = row0 + wm * (BM / 2) + group * 16 + l16;
+  if (row >= M) return;
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) {
+    const f32x4 mine = group == 0 ? acc[0][j] : acc[1][j];
+    epi(row, col0 + j * 16, mine + meet[(group * kJ + j) * 256], ahead[j]);
   }
 }
+
+// What is done with four columns of a row of C; `ahead` is what that needs from
+// memory, asked for before the product.
 
 // bf16 store of a plain product.
 struct StoreEpi {
   uint16_t* out;
   int ld;
-  __device__ __forceinline__ void operator()(int row, int col, const f32x4& v) const {
+  struct Ahead {};
+  __device__ __forceinline__ Ahead ahead(int) const { return {}; }
+  __device__ __forceinline__ void operator()(int row, int col, const f32x4& v, Ahead) const {
     store_bf16x4(out + (size_t)row * ld + col, v);
   }
 };
@@ -233,12 +315,19 @@ struct QkvEpi {
   uint16_t *qu, *qv, *kv;
   const uint16_t *u, *v;
   int proj;
-  __device__ __forceinline__ void operator()(int row, int col, const f32x4& x) const {
+  struct Ahead {
+    u32x2 u, v;
+  };
+  __device__ __forceinline__ Ahead ahead(int col) const {
+    const int at = col < proj ? col : 0;
+    return {*reinterpret_cast<const u32x2*>(u + at), *reinterpret_cast<const u32x2*>(v + at)};
+  }
+  __device__ __forceinline__ void operator()(int row, int col, const f32x4& x, Ahead a) const {
     if (col >= proj) {
       store_bf16x4(kv + (size_t)row * (2 * proj) + (col - proj), x);
     } else {
-      store_bf16x4(qu + (size_t)row * proj + col, x + load_bf16x4(u + col));
-      store_bf16x4(qv + (size_t)row * proj + col, x + load_bf16x4(v + col));
+      store_bf16x4(qu + (size_t)row * proj + col, x + unpack_bf16x4(a.u));
+      store_bf16x4(qv + (size_t)row * proj + col, x + unpack_bf16x4(a.v));
     }
   }
 };
@@ -248,28 +337,26 @@ struct ReluEpi {
   uint16_t* out;
   const uint16_t* bias;
   int ld;
-  __device__ __forceinline__ void operator()(int row, int col, const f32x4& x) const {
-    f32x4 v = x + load_bf16x4(bias + col);
+  typedef u32x2 Ahead;
+  __device__ __forceinline__ Ahead ahead(int col) const {
+    return *reinterpret_cast<const u32x2*>(bias + col);
+  }
+  __device__ __forceinline__ void operator()(int row, int col, const f32x4& x, Ahead a) const {
+    f32x4 v = x + unpack_bf16x4(a);
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = v[e] < 0.0f ? 0.0f : v[e];
     store_bf16x4(out + (size_t)row * ld + col, v);
   }
 };
 
-template <int BM, int BN>
-constexpr int panel_lds() {
-  return BM * kD * 2 + 4 * Rows<BN>::kBytes;
-}
-
 // Column of tiles first: with a multiple of eight of them every XCD reads its own
 // share of W and no more.
 template <int BM, int BN, bool kNorm, typename Epi>
-__global__ __launch_bounds__(kThreads, 1) void txl_ln_gemm_kernel(const void* A, const uint16_t* W,
-                                                                  int M, int tiles_n, Norm norm,
-                                                                  RowsOut out, Epi epi) {
+__global__ __launch_bounds__(kPanelThreads, 1) void txl_ln_gemm_kernel(
+    const void* A, const uint16_t* W, int M, int tiles_n, Norm norm, RowsOut out, Epi epi) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[panel_lds<BM, BN>()];
-  panel_gemm<BM, BN, kNorm>(lds, A, W, M, blockIdx.x / tiles_n, blockIdx.x % tiles_n, norm, out,
-                            epi);
+  panel_gemm<BM, BN, kNorm>(lds, A, W, M, blockIdx.x / tiles_n, blockIdx.x % tiles_n, tiles_n,
+                            norm, out, epi);
 }
 
 // Independent products with the same inner length, one launch: workgroups
@@ -286,7 +373,7 @@ struct Jobs {
 };
 constexpr int kJobM = 64, kJobN = 128;
 
-__global__ __launch_bounds__(kThreads, 1) void txl_jobs_kernel(Jobs jobs) {
+__global__ __launch_bounds__(kPanelThreads, 1) void txl_jobs_kernel(Jobs jobs) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[panel_lds<kJobM, kJobN>()];
   const int lane = threadIdx.x & 63;
   const bool before = lane < jobs.count && jobs.first_block[lane] <= blockIdx.x;
@@ -294,7 +381,7 @@ __global__ __launch_bounds__(kThreads, 1) void txl_jobs_kernel(Jobs jobs) {
   const Job job = jobs.job[i];
   const int local = blockIdx.x - jobs.first_block[i];
   panel_gemm<kJobM, kJobN, false>(lds, job.A, job.W, job.M, local / job.tiles_n,
-                                  local % job.tiles_n, Norm{}, RowsOut{},
+                                  local % job.tiles_n, job.tiles_n, Norm{}, RowsOut{},
                                   StoreEpi{job.out, job.ld});
 }
 
@@ -302,12 +389,12 @@ __global__ __launch_bounds__(kThreads, 1) void txl_jobs_kernel(Jobs jobs) {
 // four take the even and the odd k-tiles, which halves the chain of barriers (2048
 // deep: 16 steps instead of 32), and their sums meet in LDS.  32 x 64 tiles give
 // 192 workgroups at 768 rows.  K is a multiple of 128.
-constexpr int kResM = 32, kResN = 64, kResStages = 4;
+constexpr int kResM = 32, kResN = 64, kResStages = 6;
 
 __global__ __launch_bounds__(2 * kThreads, 1) void txl_residual_gemm_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ W, int K,
     const uint16_t* __restrict__ bias, const uint16_t* __restrict__ x, float* __restrict__ y,
-    int M) {
+    float2* __restrict__ parts, int M) {
   constexpr int kGroup = kResStages * (Rows<kResM>::kBytes + Rows<kResN>::kBytes);
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kGroup];
   const int lane = threadIdx.x & 63;
@@ -323,6 +410,15 @@ __global__ __launch_bounds__(2 * kThreads, 1) void txl_residual_gemm_kernel(
     return A + (size_t)row * K + group * kTileK;
   });
   b.init(wave, lane, [&](int r) { return W + (size_t)(col0 + r) * K + group * kTileK; });
+  const int row = row0 + wm * 16 + (lane & 15);
+  const int at = row < M ? row : M - 1;
+  u32x2 add_x[kResN / 32], add_b[kResN / 32];      // for the end, asked for ahead
+#pragma unroll
+  for (int j = 0; j < kResN / 32; ++j) {
+    const int col = col0 + wn * (kResN / 2) + j * 16 + (lane >> 4) * 4;
+    add_x[j] = *reinterpret_cast<const u32x2*>(x + (size_t)at * kD + col);
+    add_b[j] = bias ? *reinterpret_cast<const u32x2*>(bias + col) : u32x2{0, 0};
+  }
   f32x4 acc[kResM / 32][kResN / 32];
   clear(acc);
   stream_product<kResM, kResN, kResStages>(acc, lds + group * kGroup, K / (2 * kTileK),
@@ -334,16 +430,32 @@ __global__ __launch_bounds__(2 * kThreads, 1) void txl_residual_gemm_kernel(
     for (int j = 0; j < kResN / 32; ++j) other[j * 256] = acc[0][j];
   }
   block_sync();
-  const int row = row0 + wm * 16 + (lane & 15);
-  if (group == 1 || row >= M) return;
+  if (group == 1) return;
+  f32x4 v[kResN / 32];
+  float sum = 0.0f, squares = 0.0f;
 #pragma unroll
   for (int j = 0; j < kResN / 32; ++j) {
     const int col = col0 + wn * (kResN / 2) + j * 16 + (lane >> 4) * 4;
-    f32x4 v = acc[0][j] + other[j * 256];
-    if (bias) v += load_bf16x4(bias + col);
-    v += load_bf16x4(x + (size_t)row * kD + col);
-    *reinterpret_cast<f32x4*>(y + (size_t)row * kD + col) = v;
+    v[j] = acc[0][j] + other[j * 256] + unpack_bf16x4(add_b[j]) + unpack_bf16x4(add_x[j]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum += v[j][e];
+    if (row < M) *reinterpret_cast<f32x4*>(y + (size_t)row * kD + col) = v[j];
   }
+  // the wave's 32 columns of a row lie in four lanes
+  static_assert(kResN / 2 == kPartLen, "a wave's columns are a part");
+  sum += __shfl_xor(sum, 16);
+  sum += __shfl_xor(sum, 32);
+  const float mean = sum * (1.0f / kPartLen);
+#pragma unroll
+  for (int j = 0; j < kResN / 32; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float d = v[j][e] - mean;
+      squares = __builtin_fmaf(d, d, squares);
+    }
+  squares += __shfl_xor(squares, 16);
+  squares += __shfl_xor(squares, 32);
+  if (lane < 16 && row < M) parts[(size_t)row * kParts + tn * 2 + wn] = make_float2(mean, squares);
 }
 
 // hidden = LN(y), one wave for four rows.
@@ -351,8 +463,12 @@ __global__ __launch_bounds__(kThreads) void txl_norm_kernel(const float* y, Norm
                                                             uint16_t* hidden, int M) {
   const int row = blockIdx.x * (kThreads / 16) + (threadIdx.x >> 4);
   const int at = row < M ? row : M - 1;
+  NormRow in;
+  NormWeights weights;
   u32x4 v[4];
-  norm_row(y + (size_t)at * kD, norm, threadIdx.x & 15, v);
+  in.load(y, norm, at, threadIdx.x & 15);
+  weights.load(norm, threadIdx.x & 15);
+  norm_row(in, weights, norm.eps, v);
   if (row >= M) return;
 #pragma unroll
   for (int j = 0; j < 4; ++j)
@@ -593,7 +709,7 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
 
 constexpr int kMaxTails = 7;
 constexpr int kCritM = 128, kCritN = 128, kCritStages = 8;
-constexpr int kCritChunk = 16;
+constexpr int kCritChunk = 8;
 constexpr int kGroupThreads = 1024;
 
 struct Crit {
@@ -904,6 +1020,7 @@ struct Pieces {
 struct Buffers {
   uint16_t *x, *x2, *qu, *qv, *att, *h, *kv_x, *kv_mem, *table, *r;
   float* y;
+  float2* parts;
   size_t bytes;
 };
 
@@ -913,6 +1030,7 @@ Buffers buffers_of(const orion_txl_dims& d, void* base) {
   Pieces p{(char*)base};
   Buffers b;
   b.y = p.take<float>(rows * kD);
+  b.parts = p.take<float2>(rows * kParts);
   b.x = p.take<uint16_t>(rows * kD);
   b.x2 = p.take<uint16_t>(rows * kD);
   b.qu = p.take<uint16_t>(rows * proj);
@@ -1010,7 +1128,7 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
   auto flush = [&]() {
     if (jobs.count == 0) return;
     for (int i = jobs.count; i <= kMaxJobs; ++i) jobs.first_block[i] = (uint32_t)blocks;
-    hipLaunchKernelGGL(txl_jobs_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, jobs);
+    hipLaunchKernelGGL(txl_jobs_kernel, dim3((unsigned)blocks), dim3(kPanelThreads), 0, s, jobs);
     jobs.count = 0;
     blocks = 0;
   };
@@ -1043,13 +1161,13 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
     In x = (In)x0;
     if (i == 0) {
       hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 96, false, QkvEpi>), dim3(row_tiles * qkv_tiles),
-                         dim3(kThreads), 0, s, x0, (In)p.qkv, rows, (int)qkv_tiles, Norm{}, out,
+                         dim3(kPanelThreads), 0, s, x0, (In)p.qkv, rows, (int)qkv_tiles, Norm{}, out,
                          qkv);
     } else {
       x = out.x = w.x;
-      const Norm norm = {(In)layers[i - 1].norm2_w, (In)layers[i - 1].norm2_b, d.eps};
+      const Norm norm = {(In)layers[i - 1].norm2_w, (In)layers[i - 1].norm2_b, w.parts, d.eps};
       hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 96, true, QkvEpi>), dim3(row_tiles * qkv_tiles),
-                         dim3(kThreads), 0, s, (const void*)w.y, (In)p.qkv, rows, (int)qkv_tiles,
+                         dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.qkv, rows, (int)qkv_tiles,
                          norm, out, qkv);
     }
     hipLaunchKernelGGL(txl_attention_kernel, dim3(d.heads * d.batch, (unsigned)tiles(d.q_len, kQ)),
@@ -1058,19 +1176,19 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
                        (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
                        d.heads);
     hipLaunchKernelGGL(txl_residual_gemm_kernel, res_grid, dim3(2 * kThreads), 0, s, (In)w.att,
-                       (In)p.out, proj, (In) nullptr, x, w.y, rows);
-    const Norm norm = {(In)p.norm1_w, (In)p.norm1_b, d.eps};
+                       (In)p.out, proj, (In) nullptr, x, w.y, w.parts, rows);
+    const Norm norm = {(In)p.norm1_w, (In)p.norm1_b, w.parts, d.eps};
     RowsOut out2 = {};
     out2.x = w.x2;
     hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 128, true, ReluEpi>), dim3(row_tiles * ff_tiles),
-                       dim3(kThreads), 0, s, (const void*)w.y, (In)p.ff1_w, rows, (int)ff_tiles,
+                       dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.ff1_w, rows, (int)ff_tiles,
                        norm, out2, ReluEpi{w.h, (In)p.ff1_b, d.inner});
     hipLaunchKernelGGL(txl_residual_gemm_kernel, res_grid, dim3(2 * kThreads), 0, s, (In)w.h,
-                       (In)p.ff2_w, d.inner, (In)p.ff2_b, (In)w.x2, w.y, rows);
+                       (In)p.ff2_w, d.inner, (In)p.ff2_b, (In)w.x2, w.y, w.parts, rows);
   }
   const orion_txl_layer& last = layers[d.layers - 1];
   hipLaunchKernelGGL(txl_norm_kernel, dim3((unsigned)tiles(rows, kThreads / 16)), dim3(kThreads), 0,
-                     s, (const float*)w.y, (Norm{(In)last.norm2_w, (In)last.norm2_b, d.eps}),
+                     s, (const float*)w.y, (Norm{(In)last.norm2_w, (In)last.norm2_b, w.parts, d.eps}),
                      (uint16_t*)hidden, rows);
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
 }
