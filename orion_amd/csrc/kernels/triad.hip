@@ -11,8 +11,8 @@
 // short-lived waves (measured over 3 x 1 GiB: 6.72 TB/s; 6.43 TB/s with four
 // waves per workgroup, 6.4 with two accesses per lane, 4.6 for a 2048-workgroup
 // grid-stride loop with four accesses in flight per lane).  A caller-chosen
-// smaller grid walks block-contiguous chunks instead, so any number of compute
-// units (a CU-masked stream may expose a fraction of the 256) drains it.
+// smaller grid loops instead, so any number of compute units (a CU-masked stream
+// may expose a fraction of the 256) drains it.
 //
 // The reference system has no device code of its own; this kernel stands in for
 // the memory-bound half of its toy co-location pair
@@ -25,9 +25,9 @@
 
 namespace {
 
-constexpr int kTriadThreads = 256;  // chunked variant
+constexpr int kTriadThreads = 256;  // looping variants
 constexpr int kOneShotThreads = 64; // one-shot variant: one wavefront per workgroup
-// float4 accesses in flight per lane and per array in the chunked variant.
+// float4 accesses in flight per lane and per array over ranges.
 constexpr int kTriadUnroll = 4;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -63,8 +63,58 @@ __global__ __launch_bounds__(kOneShotThreads) void triad_f32_kernel(
   triad_tail(a, b, c, s, n_vec4, n);
 }
 
-// Caller-chosen grid: workgroup g owns the contiguous range
-// [g * per_block, (g + 1) * per_block) of 16-byte elements.
+// Caller-chosen grid of fewer workgroups than that, two ways.
+//
+// Strided: workgroup g takes tiles g, g + grid, ... of kTile 16-byte elements, so
+// that what is in flight at any moment is one window of each array.  Bound by HBM
+// and, below about 256 workgroups or on a masked stream, by what the waves have in
+// flight.  A range of its own for each workgroup touches as many places of each
+// array as there are workgroups; in us, ranges and strided:
+//   64 Mi elements, 1024 workgroups, 64 compute units   271 -> 256
+//   the same, whole GPU                                 142 -> 131
+//   the same, 200 workgroups                            171 -> 129
+//   256 Mi, 3000 workgroups                             670 -> 568
+//   128 Mi, 300 workgroups, 32 compute units           1146 -> 977
+//   4 Mi, 64 workgroups (caches)                       19.6 -> 14.1
+// Four accesses instead of eight are 1 to 2 % faster on the whole GPU and 2 to 4 %
+// slower on 64 compute units; 512 threads a workgroup lose 16 % on the whole GPU.
+constexpr int kStridedUnroll = 8;
+constexpr size_t kTile = (size_t)kTriadThreads * kStridedUnroll;
+// Where tiles would not go round evenly, ranges.  Below eight tiles a workgroup the
+// last round can be an eighth of the work and more (us, ranges and strided: 1.7 M
+// elements, 65 workgroups, 3.2 tiles each, 7.9 and 9.1; 4.0 M, 116 workgroups, 64
+// compute units, 4.2 tiles, 17.6 and 19.2; 9.3 M, 66 workgroups, 32 compute units,
+// 17 tiles, 95.9 and 91.0).  A thousand workgroups and more take turns on the
+// compute units, which evens it out from two tiles on (42.5 M, 2762 workgroups, 1.9
+// tiles, 81 and 84; 64 Mi, 3000 workgroups, 2.7 tiles, 153 and 132).
+constexpr int kManyGroups = 1024;
+
+__global__ __launch_bounds__(kTriadThreads) void triad_f32_strided_kernel(
+    float* __restrict__ a, const float* __restrict__ b,
+    const float* __restrict__ c, float s, size_t n_vec4, size_t n) {
+  const f32x4* __restrict__ b4 = reinterpret_cast<const f32x4*>(b);
+  const f32x4* __restrict__ c4 = reinterpret_cast<const f32x4*>(c);
+  f32x4* __restrict__ a4 = reinterpret_cast<f32x4*>(a);
+  size_t base = (size_t)blockIdx.x * kTile;
+  for (; base + kTile <= n_vec4; base += (size_t)gridDim.x * kTile) {
+    const size_t i = base + threadIdx.x;
+    f32x4 vb[kStridedUnroll], vc[kStridedUnroll];
+#pragma unroll
+    for (int u = 0; u < kStridedUnroll; ++u) {
+      vb[u] = __builtin_nontemporal_load(&b4[i + u * kTriadThreads]);
+      vc[u] = __builtin_nontemporal_load(&c4[i + u * kTriadThreads]);
+    }
+#pragma unroll
+    for (int u = 0; u < kStridedUnroll; ++u)
+      __builtin_nontemporal_store(triad4(vb[u], vc[u], s), &a4[i + u * kTriadThreads]);
+  }
+  // the last, partial tile; workgroups past it have nothing left
+  for (size_t i = base + threadIdx.x; i < n_vec4; i += kTriadThreads)
+    a4[i] = triad4(b4[i], c4[i], s);
+  triad_tail(a, b, c, s, n_vec4, n);
+}
+
+// Ranges: workgroup g owns elements [g * per_block, (g + 1) * per_block).
 __global__ __launch_bounds__(kTriadThreads) void triad_f32_chunked_kernel(
     float* __restrict__ a, const float* __restrict__ b,
     const float* __restrict__ c, float s, size_t n_vec4, size_t n) {
@@ -108,6 +158,9 @@ extern "C" int orion_triad_f32(float* a, const float* b, const float* c,
   if (grid_blocks <= 0 || (size_t)grid_blocks >= one_shot) {
     hipLaunchKernelGGL(triad_f32_kernel, dim3((unsigned)one_shot), dim3(kOneShotThreads), 0,
                        (hipStream_t)stream, a, b, c, s, n_vec4, n);
+  } else if (n_vec4 >= (grid_blocks < kManyGroups ? 8 : 2) * kTile * (size_t)grid_blocks) {
+    hipLaunchKernelGGL(triad_f32_strided_kernel, dim3((unsigned)grid_blocks),
+                       dim3(kTriadThreads), 0, (hipStream_t)stream, a, b, c, s, n_vec4, n);
   } else {
     hipLaunchKernelGGL(triad_f32_chunked_kernel, dim3((unsigned)grid_blocks),
                        dim3(kTriadThreads), 0, (hipStream_t)stream, a, b, c, s, n_vec4, n);

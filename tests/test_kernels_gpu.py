@@ -41,6 +41,24 @@ def test_triad_any_grid_gives_the_same_bits(grid):
     assert np.array_equal(a.cpu().numpy(), ko.triad(b, c, -0.3))
 
 
+# The loop over a caller's grid changes at eight tiles of 2048 16-byte accesses a
+# workgroup (two from 1024 workgroups on); last tiles whole, partial and of one
+# access; 0 to 3 elements past the last 16 bytes.
+@pytest.mark.parametrize("grid", [1, 3, 64, 1024])
+@pytest.mark.parametrize("half_tiles, more", [(3, 7), (4, -4), (4, 0), (4, 5), (5, 4093),
+                                              (16, -4), (16, 0), (16, 1), (17, 1026)])
+def test_triad_loops_at_the_edges_of_tiles(grid, half_tiles, more):
+    n = half_tiles * grid * 4096 + more
+    rng = np.random.default_rng(n)
+    b, c = (rng.standard_normal(n).astype(np.float32) for _ in range(2))
+    a = torch.full((n + 64,), 7.0, device=DEV)
+    kernels.triad(a[:n], torch.from_numpy(b).to(DEV), torch.from_numpy(c).to(DEV), 0.9,
+                  grid_blocks=grid)
+    assert np.array_equal(a[:n].cpu().numpy().view(np.uint32),
+                          ko.triad(b, c, 0.9).view(np.uint32))
+    assert (a[n:] == 7.0).all()
+
+
 def test_triad_special_values_and_in_place():
     b = np.array([0.0, -0.0, np.inf, 1.0, np.nan, 1e38, -1e38, 1e-45], dtype=np.float32)
     c = np.array([0.0, 0.0, 1.0, np.inf, 1.0, 1e38, 1e38, 1e-45], dtype=np.float32)
