@@ -59,8 +59,12 @@ __device__ __forceinline__ bool aligned16(const orion_lamb_tensor& t) {
   return ((((uintptr_t)t.w | (uintptr_t)t.g | (uintptr_t)t.m | (uintptr_t)t.v) & 15u) == 0);
 }
 
+// Without decay the weight is not in the update at all: 0 * w would be a NaN for an
+// infinite weight, and through the norm for its whole tensor.
+template <bool kDecay>
 __device__ __forceinline__ float update_of(float w, float m, float v, const Coefs& c) {
-  return __builtin_fmaf(c.decay, w, m / (__builtin_sqrtf(v) + c.eps));
+  const float u = m / (__builtin_sqrtf(v) + c.eps);
+  return kDecay ? __builtin_fmaf(c.decay, w, u) : u;
 }
 
 __device__ __forceinline__ void moments(float g, float& m, float& v, const Coefs& c) {
@@ -68,6 +72,7 @@ __device__ __forceinline__ void moments(float g, float& m, float& v, const Coefs
   v = __builtin_fmaf(c.b2c * g, g, c.b2 * v);
 }
 
+template <bool kDecay>
 __global__ __launch_bounds__(kThreads) void lamb_moments_kernel(Group g, Coefs c,
                                                                 float2* partials) {
   const uint32_t block = blockIdx.x;
@@ -95,7 +100,7 @@ __global__ __launch_bounds__(kThreads) void lamb_moments_kernel(Group g, Coefs c
         moments(vg[u][e], m, v, c);
         vm[u][e] = m;
         vv[u][e] = v;
-        const float w = vw[u][e], up = update_of(w, m, v, c);
+        const float w = vw[u][e], up = update_of<kDecay>(w, m, v, c);
         sw = __builtin_fmaf(w, w, sw);
         su = __builtin_fmaf(up, up, su);
       }
@@ -109,7 +114,7 @@ __global__ __launch_bounds__(kThreads) void lamb_moments_kernel(Group g, Coefs c
       moments(t.g[i], m, v, c);
       t.m[i] = m;
       t.v[i] = v;
-      const float w = t.w[i], up = update_of(w, m, v, c);
+      const float w = t.w[i], up = update_of<kDecay>(w, m, v, c);
       sw = __builtin_fmaf(w, w, sw);
       su = __builtin_fmaf(up, up, su);
     }
@@ -176,6 +181,7 @@ __global__ __launch_bounds__(kReduceThreads) void lamb_ratio_kernel(
   }
 }
 
+template <bool kDecay>
 __global__ __launch_bounds__(kThreads) void lamb_update_kernel(Group g, Coefs c,
                                                                const float* __restrict__ factor) {
   const uint32_t block = gridDim.x - 1 - blockIdx.x;   // the first pass's last data first
@@ -197,13 +203,13 @@ __global__ __launch_bounds__(kThreads) void lamb_update_kernel(Group g, Coefs c,
       const uint64_t i = base + (u * kThreads + threadIdx.x) * 4;
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        vw[u][e] = __builtin_fmaf(f, update_of(vw[u][e], vm[u][e], vv[u][e], c), vw[u][e]);
+        vw[u][e] = __builtin_fmaf(f, update_of<kDecay>(vw[u][e], vm[u][e], vv[u][e], c), vw[u][e]);
       __builtin_nontemporal_store(vw[u], reinterpret_cast<f32x4*>(t.w + i));
     }
   } else {
     const uint64_t end = base + kChunk < t.n ? base + kChunk : t.n;
     for (uint64_t i = base + threadIdx.x; i < end; i += kThreads)
-      t.w[i] = __builtin_fmaf(f, update_of(t.w[i], t.m[i], t.v[i], c), t.w[i]);
+      t.w[i] = __builtin_fmaf(f, update_of<kDecay>(t.w[i], t.m[i], t.v[i], c), t.w[i]);
   }
 }
 
@@ -256,12 +262,12 @@ extern "C" int orion_lamb_step(const orion_lamb_tensor* tensors, int count, doub
     }
     if (g.count == 0) break;
     for (int i = g.count; i <= kMaxTensors; ++i) g.first_block[i] = (uint32_t)blocks;
-    hipLaunchKernelGGL(lamb_moments_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, g, c,
-                       partials);
+    hipLaunchKernelGGL(decay != 0.0 ? lamb_moments_kernel<true> : lamb_moments_kernel<false>,
+                       dim3((unsigned)blocks), dim3(kThreads), 0, s, g, c, partials);
     hipLaunchKernelGGL(lamb_ratio_kernel, dim3((unsigned)g.count), dim3(kReduceThreads), 0, s, g,
                        (const float2*)partials, factor, lr, eps);
-    hipLaunchKernelGGL(lamb_update_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, s, g, c,
-                       (const float*)factor);
+    hipLaunchKernelGGL(decay != 0.0 ? lamb_update_kernel<true> : lamb_update_kernel<false>,
+                       dim3((unsigned)blocks), dim3(kThreads), 0, s, g, c, (const float*)factor);
   }
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
 }

@@ -85,6 +85,28 @@ def test_infinite_and_nan_gradients_reach_the_weights_as_before():
         assert all(torch.equal(a, b) for a, b in zip(*results))
 
 
+@pytest.mark.parametrize("bad", [float("inf"), -float("inf"), float("nan")])
+@pytest.mark.parametrize("decay", [0.0, 0.01])
+def test_infinite_and_nan_weights_give_what_the_operations_give(decay, bad):
+    results = []
+    for dense in (True, False):
+        opt, params = _optimizer((8, 64, 5000), 0, decay, seed=6)
+        params[0].data[3] = bad             # a workgroup's part of a chunk
+        params[2].data[100] = bad           # a whole one
+        if not dense:          # the element-wise way
+            opt.param_groups[0]["lr"] = torch.tensor(0.1, device=DEV)
+        opt.step()
+        results.append([p.detach().clone() for p in params])
+    for got, want in zip(*results):
+        # a dozen fp32 roundings of 6e-8 each on either side
+        finite = want[want.isfinite()]
+        top = float(finite.abs().max()) if finite.numel() else 0.0
+        assert torch.allclose(got, want, rtol=2e-6, atol=2e-6 * top, equal_nan=True)
+    if decay == 0.0 and bad == bad:
+        # without decay an infinite weight is in no update: it stays, the others move
+        assert [int((~p.isfinite()).sum()) for p in results[0]] == [1, 0, 1]
+
+
 def test_lists_that_take_the_elementwise_way():
     base = torch.ones(8, 6, device=DEV)
     ok = [torch.ones(8, 6, device=DEV)]
