@@ -8,6 +8,7 @@ import atexit
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -170,8 +171,10 @@ def gemm_bf16_nt(a, b, out=None, out_dtype=torch.bfloat16, stream=None):
 
 def plain_eager():
     """False while something has to see every operation: a transform or a mode
-    that rewrites them, or a tracer."""
-    return (torch._C._functorch.peek_interpreter_stack() is None
+    that rewrites them, a tracer, or forward-mode derivatives, which ``no_grad``
+    leaves on and whose dual tensors have no type of their own."""
+    return (forward_ad._current_level < 0
+            and torch._C._functorch.peek_interpreter_stack() is None
             and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._len_torch_function_stack() == 0
             and not torch.jit.is_tracing()

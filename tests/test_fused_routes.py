@@ -1,0 +1,65 @@
+"""Which calls of the Transformer-XL model and of LAMB may take the kernels: whatever
+has to see the operations, or would get another answer from the kernels, keeps them.
+The kernels' entry points are replaced by recorders, so this runs without a GPU."""
+
+import pytest
+import torch
+from torch.autograd import forward_ad
+from torch.nn.attention import SDPBackend, sdpa_kernel
+
+from orion_amd import kernels
+from orion_amd.benchmark_suite import transformer_xl as txl
+
+CONFIG = dict(n_token=100, n_layer=3, n_head=2, d_model=128, d_head=64, d_inner=128,
+              dropout=0.1, tgt_len=8, mem_len=8, cutoffs=[20, 50])
+
+
+@pytest.fixture
+def model():
+    torch.manual_seed(0)
+    return txl.MemTransformerLM(**CONFIG).eval().to(torch.bfloat16)
+
+
+@pytest.fixture
+def routes(monkeypatch):
+    """Names of the entry points called, with their arguments; each declines."""
+    calls = []
+    for name in ("txl_hidden", "adaptive_nll"):
+        monkeypatch.setattr(kernels, name,
+                            lambda *args, name=name: calls.append((name, args)))
+    return calls
+
+
+def _inputs():
+    g = torch.Generator().manual_seed(1)
+    data, target = (torch.randint(0, CONFIG["n_token"], (8, 2), generator=g) for _ in range(2))
+    return data, target
+
+
+def _names(routes):
+    return [name for name, _ in routes]
+
+
+def test_plain_inference_asks_the_kernels(model, routes):
+    with torch.no_grad():
+        model(*_inputs())
+    assert _names(routes) == ["txl_hidden", "adaptive_nll"]
+
+
+def test_forward_mode_derivatives_keep_the_operations(model, routes):
+    # no_grad does not switch forward mode off, and a dual tensor is a plain Tensor
+    hidden = torch.randn(5, CONFIG["d_model"]).to(torch.bfloat16)
+    target = torch.randint(0, CONFIG["n_token"], (5,))
+    with torch.no_grad(), forward_ad.dual_level():
+        assert not kernels.plain_eager()
+        dual = forward_ad.make_dual(hidden, torch.ones_like(hidden))
+        assert forward_ad.unpack_dual(model.crit(dual, target)).tangent is not None
+        # a tangent that enters with a weight
+        weight = model.word_emb.weight
+        del model.word_emb.weight
+        model.word_emb.weight = forward_ad.make_dual(weight.detach(), torch.ones_like(weight))
+        with sdpa_kernel(SDPBackend.MATH):       # the one with a forward-mode formula
+            states, _ = model.hidden_states(_inputs()[0], None)
+        assert forward_ad.unpack_dual(states).tangent is not None
+    assert not routes
+    assert kernels.plain_eager()
