@@ -118,7 +118,7 @@ class AdaptiveLogSoftmax(nn.Module):
     def forward(self, hidden, target):
         """hidden [n, d], target [n] -> nll [n] (in the order of the rows)."""
         if (type(self) is AdaptiveLogSoftmax and hidden.dtype is torch.bfloat16
-                and kernels.inference_only()):
+                and self.n_clusters == len(self.edges) - 2 and kernels.inference_only()):
             nll = kernels.adaptive_nll(hidden, target, self.weight, self.bias,
                                        self.cluster_weight, self.cluster_bias, self.edges)
             if nll is not None:
@@ -235,7 +235,8 @@ class MemTransformerLM(nn.Module):
     def _fused_hidden_states(self, x, mems):
         """The layers through ``kernels.txl_hidden``; None unless every module it
         passes by is the plain one, in its inference form, with nothing attached."""
-        if (type(self) is not MemTransformerLM or not self.n_layer or _global_hooks()
+        if (type(self) is not MemTransformerLM or not self.n_layer
+                or not len(self.attn) == len(self.ff) == self.n_layer or _global_hooks()
                 or not _plain(self.drop)):
             return None
         layers, eps, inner = [], self.attn[0].norm.eps, self.ff[0].net[0].out_features

@@ -63,3 +63,25 @@ def test_forward_mode_derivatives_keep_the_operations(model, routes):
         assert forward_ad.unpack_dual(states).tangent is not None
     assert not routes
     assert kernels.plain_eager()
+
+
+def _expect_operations(model, routes, allowed=()):
+    with torch.no_grad():
+        model(*_inputs())
+    assert _names(routes) == list(allowed)
+    routes.clear()
+
+
+def test_sizes_that_the_operations_read_are_the_modules_own(model, routes):
+    # the operations run the first n_layer blocks and the first n_clusters tails
+    model.n_layer = 2
+    _expect_operations(model, routes, ["adaptive_nll"])
+    model.n_layer = 3
+    block = model.ff.pop(2)
+    model.n_layer = 2
+    _expect_operations(model, routes, ["adaptive_nll"])
+    model.n_layer = 3
+    model.ff.append(block)
+    _expect_operations(model, routes, ["txl_hidden", "adaptive_nll"])
+    model.crit.n_clusters = 1
+    _expect_operations(model, routes, ["txl_hidden"])
