@@ -166,6 +166,8 @@ def _plain(module):
                 or type(module) is nn.Dropout and module.training and module.p)
 
 
+_ATTN_ORDER = ("qkv", "pos", "out", "drop", "norm")
+_ATTN_PARTS, _FF_PARTS = set(_ATTN_ORDER), {"net", "norm"}
 _PLAIN_TYPES = {RelativeAttention, FeedForward, nn.Sequential, nn.Linear, nn.LayerNorm,
                 nn.Dropout, nn.ReLU}
 
@@ -244,16 +246,16 @@ class MemTransformerLM(nn.Module):
             if type(attn) is not RelativeAttention or type(ff) is not FeedForward:
                 return None
             a, f = attn._modules, ff._modules
-            net = f["net"]
-            parts = [*a.values(), *f.values(), attn, ff]
-            if type(net) is not nn.Sequential or len(a) != 5 or len(f) != 2 or len(net) != 5:
+            if a.keys() != _ATTN_PARTS or f.keys() != _FF_PARTS:
                 return None         # not the modules their constructors make
-            parts += net._modules.values()
+            qkv, pos, out, drop, norm1 = (a[name] for name in _ATTN_ORDER)
+            net, norm2 = f["net"], f["norm"]
+            if type(net) is not nn.Sequential or len(net) != 5:
+                return None
+            parts = [*a.values(), *f.values(), attn, ff, *net._modules.values()]
             if not all(map(_plain, parts)):
                 return None
-            qkv, pos, out, drop, norm1 = a.values()
             ff1, relu, drop1, ff2, drop2 = net._modules.values()
-            norm2 = f["norm"]
             if not (type(qkv) is type(pos) is type(out) is type(ff1) is type(ff2) is nn.Linear
                     and type(norm1) is type(norm2) is nn.LayerNorm and type(relu) is nn.ReLU
                     and type(drop) is type(drop1) is type(drop2) is nn.Dropout

@@ -85,3 +85,18 @@ def test_sizes_that_the_operations_read_are_the_modules_own(model, routes):
     _expect_operations(model, routes, ["txl_hidden", "adaptive_nll"])
     model.crit.n_clusters = 1
     _expect_operations(model, routes, ["txl_hidden"])
+
+
+def test_modules_are_told_by_name_not_by_order_of_registration(model, routes):
+    # here pos and out are of one shape: only their names tell them apart
+    attn = model.attn[0]
+    parts = {name: attn._modules.pop(name) for name in list(attn._modules)}
+    for name in ("qkv", "out", "pos", "drop", "norm"):
+        setattr(attn, name, parts[name])
+    with torch.no_grad():
+        model(*_inputs())
+    (_, args), _ = routes
+    assert args[4][0][:3] == (attn.qkv.weight, attn.pos.weight, attn.out.weight)
+    routes.clear()
+    attn.extra = torch.nn.Identity()
+    _expect_operations(model, routes, ["adaptive_nll"])
