@@ -182,12 +182,12 @@ def plain_eager():
 
 
 def plain_tensors(tensors, dtype, device):
-    """Whether these are ordinary contiguous tensors of the device: what a kernel
-    that takes addresses can work on."""
+    """Whether these are ordinary contiguous tensors of the device, their values as
+    they lie in memory: what a kernel that takes addresses can work on."""
     for t in tensors:
         if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype is not dtype
                 or t.device != device or t.layout is not torch.strided
-                or not t.is_contiguous()):
+                or t.is_neg() or not t.is_contiguous()):
             return False
     return True
 
@@ -233,7 +233,7 @@ def _bf16_operand(t, shape, index):
     ``index`` and 16-byte aligned."""
     return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype is torch.bfloat16
             and t.shape == shape and t.get_device() == index and t.layout is torch.strided
-            and t.is_contiguous() and not t.data_ptr() & 15)
+            and not t.is_neg() and t.is_contiguous() and not t.data_ptr() & 15)
 
 
 def inference_only():
@@ -269,7 +269,7 @@ def txl_hidden(x, mems, u, v, layers, inner, eps, keep):
     m_len = 0
     if mems is not None:
         if (type(mems) is not torch.Tensor or mems.dtype is not torch.bfloat16
-                or mems.dim() != 4 or mems.get_device() != index
+                or mems.dim() != 4 or mems.get_device() != index or mems.is_neg()
                 or mems.shape[0] != len(layers) or mems.shape[2:] != (batch, width)):
             return None
         m_len = mems.shape[1]
@@ -318,7 +318,7 @@ def adaptive_nll(hidden, target, weight, bias, tail_weight, tail_bias, edges):
         if not _bf16_operand(t, shape, index):
             return None
     if (type(target) is not torch.Tensor or target.dtype is not torch.int64
-            or target.shape != (n,) or target.get_device() != index
+            or target.shape != (n,) or target.get_device() != index or target.is_neg()
             or not target.is_contiguous()):
         return None
     args = _Nll(hidden.data_ptr(), weight.data_ptr(), bias.data_ptr(), tail_weight.data_ptr(),

@@ -100,3 +100,15 @@ def test_modules_are_told_by_name_not_by_order_of_registration(model, routes):
     routes.clear()
     attn.extra = torch.nn.Identity()
     _expect_operations(model, routes, ["adaptive_nll"])
+
+
+def test_lazily_negated_tensors_keep_the_operations():
+    # contiguous and of type Tensor, but their memory holds the other sign
+    ok = torch.ones(4, 4)
+    negated = torch._neg_view(ok)
+    assert kernels.plain_tensors([ok, ok], torch.float32, ok.device)
+    assert not kernels.plain_tensors([ok, negated], torch.float32, ok.device)
+    ok = torch.ones(4, 8, dtype=torch.bfloat16)
+    index = ok.get_device()
+    for t, plain in ((ok, True), (torch._neg_view(ok), False)):
+        assert kernels._bf16_operand(t, (4, 8), index) is plain
