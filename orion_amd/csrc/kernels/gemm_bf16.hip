@@ -380,11 +380,12 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(cons
   }
 }
 
-// What a launch of each tile takes, us: 1.5 + rounds of 256 workgroups * (fixed +
-// per_tile * k-tiles), fitted to products from 256 x 256 x 64 to 4096^3.  The fit is
-// within 20 %; the large tile's estimate counts 0.9 because a round of it keeps the
-// whole chip busy where one of the others waits (8192 x 2560 x 1024: 47 us by 256 x
-// 256 tiles, 54 by 128 x 128, both estimated at 46).
+// What a launch of each tile takes, us: 1.5 + rounds of as many workgroups as the
+// stream has compute units * (fixed + per_tile * k-tiles), fitted to products from
+// 256 x 256 x 64 to 4096^3 on the whole GPU.  The fit is within 20 %; the large
+// tile's estimate counts 0.9 because a round of it keeps the whole chip busy where one
+// of the others waits (8192 x 2560 x 1024: 47 us by 256 x 256 tiles, 54 by 128 x 128,
+// both estimated at 46).
 struct TileCost {
   int tm, tn, k;          // k: what the depth has to be a multiple of
   double fixed, per_tile;
@@ -396,15 +397,16 @@ constexpr TileCost kTiles[] = {
     {64, 64, 64, 1.5, 0.19},
     {32, 64, 128, 1.5, 0.125},   // two groups of waves
 };
+constexpr int kWholeGpu = 256;   // compute units
 
-int tile_for(int M, int N, int K) {
+int tile_for(int M, int N, int K, int cus) {
   int best = 0;
   double best_us = 0.0;
   for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
     const TileCost& t = kTiles[i];
     if (K % t.k != 0) continue;
     const long long blocks = (long long)(M / t.tm) * (N / t.tn);
-    const double us = 1.5 + (double)((blocks + 255) / 256) * (t.fixed + t.per_tile * (K / BK));
+    const double us = 1.5 + (double)((blocks + cus - 1) / cus) * (t.fixed + t.per_tile * (K / BK));
     if (i == 0 || us < best_us) {
       best = i;
       best_us = i == 0 ? 0.9 * us : us;
@@ -413,10 +415,34 @@ int tile_for(int M, int N, int K) {
   return best;
 }
 
+// Compute units that a stream may use; the whole GPU where that cannot be told.
+int compute_units_of(hipStream_t stream) {
+  uint32_t mask[16] = {0};
+  if (hipExtStreamGetCUMask(stream, 16, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return kWholeGpu;
+  }
+  int cus = 0;
+  for (uint32_t word : mask) cus += __builtin_popcount(word);
+  return cus > 0 && cus < kWholeGpu ? cus : kWholeGpu;
+}
+
+// The tile for a stream.  On some of the compute units the smaller tiles' workgroups
+// only take turns (64 of them, us by 256 x 256 and by the whole GPU's choice: 2048^3
+// 36.8 and 51.4; 1024 x 4096 x 512 13.7 and 23.5), so where the whole GPU's choice is
+// a smaller one the stream is asked for its mask (0.2 us) and the rounds are counted
+// with that.
+int tile_for_stream(int M, int N, int K, hipStream_t stream) {
+  const int tile = tile_for(M, N, K, kWholeGpu);
+  if (tile == 0 || stream == nullptr) return tile;
+  const int cus = compute_units_of(stream);
+  return cus == kWholeGpu ? tile : tile_for(M, N, K, cus);
+}
+
 template <typename OutT>
 void launch_gemm(const uint16_t* A, const uint16_t* B, OutT* C, int M, int N, int K,
                  hipStream_t stream) {
-  const int tile = tile_for(M, N, K);
+  const int tile = tile_for_stream(M, N, K, stream);
   const dim3 grid((unsigned)((M / kTiles[tile].tm) * (N / kTiles[tile].tn)));
   switch (tile) {
     case 1:

@@ -121,7 +121,7 @@ def _shutdown():
 def _stream_ptr(stream):
     if stream is None:
         stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    return stream.cuda_stream
 
 
 def _check_device(*tensors):

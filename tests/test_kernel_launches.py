@@ -1,0 +1,97 @@
+"""What the kernel library launches, without a GPU: its host code runs in a child
+process behind a recorder of the HIP runtime's launches (tests/native/launch_log.cpp),
+with addresses that nothing reads."""
+
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+from orion_amd import _lib
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+CHILD = """
+import ctypes, json, sys
+log = ctypes.CDLL(sys.argv[1])
+lib = ctypes.CDLL(sys.argv[2])
+log.launch_log_name.restype = log.launch_log_kernel.restype = ctypes.c_char_p
+P, Z, D = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_double
+lib.orion_gemm_bf16_nt.argtypes = [P, P, P] + [ctypes.c_int] * 4 + [P]
+lib.orion_lamb_workspace_bytes.argtypes = [P, ctypes.c_int]
+lib.orion_lamb_workspace_bytes.restype = Z
+lib.orion_lamb_step.argtypes = [P, ctypes.c_int, D, D, D, D, D, P, Z, P]
+AT = 1 << 40                      # an aligned address that nothing reads
+
+def taken():
+    out = [(log.launch_log_name(i).decode(), log.launch_log_grid(i), log.launch_log_block(i))
+           for i in range(log.launch_log_size())]
+    log.launch_log_clear()
+    return out
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    if not os.path.exists(_lib.KERNELS_LIB):
+        pytest.fail("liborion_kernels.so is not built")
+    shim = str(tmp_path_factory.mktemp("launch_log") / "liblaunchlog.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-Wall",
+                    os.path.join(ROOT, "tests", "native", "launch_log.cpp"), "-o", shim],
+                   check=True)
+
+    def child(body, *args):
+        env = dict(os.environ, LD_PRELOAD=shim)
+        out = subprocess.run([sys.executable, "-c", CHILD + body, shim, _lib.KERNELS_LIB,
+                              json.dumps(args)], env=env, check=True, capture_output=True,
+                             text=True, timeout=120)
+        return json.loads(out.stdout)
+    return child
+
+
+GEMM = """
+out = []
+for m, n, k, cus, stream in json.loads(sys.argv[3])[0]:
+    log.launch_log_set_compute_units(cus)
+    rc = lib.orion_gemm_bf16_nt(AT, AT, AT, m, n, k, 0, stream and AT)
+    queries = log.launch_log_queries()
+    out.append((rc, taken(), queries))
+print(json.dumps(out))
+"""
+
+# Workgroups of the tile that measured fastest, by size and compute units of the stream.
+GEMM_TILES = [
+    # the whole GPU
+    (256, 512, 256, 256, 64), (1024, 1024, 1024, 256, 256), (3072, 1024, 1024, 256, 192),
+    (2816, 3328, 1856, 256, 143),
+    # streams limited to some compute units: 256 x 256 tiles where smaller ones would
+    # only take turns (us, 256 x 256 and what the whole GPU's rule takes: 36.8 and 51.4;
+    # 13.7 and 23.5; 23.4 and 34.3; 38.3 and 46.6; 8.5 and 20.5; 8.6 and 12.6)
+    (2048, 2048, 2048, 64, 64), (1024, 4096, 512, 64, 64), (4096, 2048, 1024, 128, 128),
+    (3072, 1024, 1024, 32, 48), (1792, 1024, 192, 32, 28), (2560, 1024, 192, 64, 40),
+    # and smaller ones where they still pay (256 x 256 tiles and these: 121 and 31, 121
+    # and 23, 60 and 44)
+    (512, 512, 8192, 32, 32), (512, 512, 8192, 64, 64), (1792, 768, 3648, 64, 84),
+]
+
+
+def test_gemm_tiles_follow_the_streams_compute_units(run):
+    got = run(GEMM, [(m, n, k, cus, True) for m, n, k, cus, _ in GEMM_TILES])
+    bad = []
+    for case, (rc, launches, _) in zip(GEMM_TILES, got):
+        assert rc == 0 and len(launches) == 1
+        if launches[0][1] != case[-1]:
+            bad.append((case, launches))
+    assert not bad
+
+
+def test_gemm_asks_for_the_compute_units_only_where_they_decide(run):
+    (rc, whole, queries), (_, null, null_queries), (rc_unknown, unknown, _) = run(GEMM, [
+        (8192, 8192, 8192, 64, True),       # 256 x 256 tiles on any stream
+        (2048, 2048, 2048, 64, False),      # the null stream spans the GPU
+        (2048, 2048, 2048, 0, True)])       # a failing query: the whole GPU, and no error left
+    assert rc == rc_unknown == 0
+    assert queries == 0 and whole[0][1] == 1024
+    assert null_queries == 0 and null[0][1] == unknown[0][1] == 256
