@@ -161,13 +161,13 @@ def _global_hooks():
 
 def _plain(module):
     """Calling the module is its class's forward and nothing else, in inference."""
-    attrs = module.__dict__
-    return type(module) in _PLAIN_TYPES and not (attrs["_forward_hooks"] or attrs["_forward_pre_hooks"] or "forward" in attrs
-                or type(module) is nn.Dropout and module.training and module.p)
+    kind, attrs = type(module), module.__dict__
+    return kind in _PLAIN_TYPES and not (
+        attrs["_forward_hooks"] or attrs["_forward_pre_hooks"] or "forward" in attrs
+        or kind is nn.Dropout and module.training and module.p)
 
 
-_ATTN_ORDER = ("qkv", "pos", "out", "drop", "norm")
-_ATTN_PARTS, _FF_PARTS = set(_ATTN_ORDER), {"net", "norm"}
+_ATTN_PARTS, _FF_PARTS = {"qkv", "pos", "out", "drop", "norm"}, {"net", "norm"}
 _PLAIN_TYPES = {RelativeAttention, FeedForward, nn.Sequential, nn.Linear, nn.LayerNorm,
                 nn.Dropout, nn.ReLU}
 
@@ -248,14 +248,13 @@ class MemTransformerLM(nn.Module):
             a, f = attn._modules, ff._modules
             if a.keys() != _ATTN_PARTS or f.keys() != _FF_PARTS:
                 return None         # not the modules their constructors make
-            qkv, pos, out, drop, norm1 = (a[name] for name in _ATTN_ORDER)
+            qkv, pos, out, drop, norm1 = a["qkv"], a["pos"], a["out"], a["drop"], a["norm"]
             net, norm2 = f["net"], f["norm"]
             if type(net) is not nn.Sequential or len(net) != 5:
                 return None
-            parts = [*a.values(), *f.values(), attn, ff, *net._modules.values()]
-            if not all(map(_plain, parts)):
+            ff1, relu, drop1, ff2, drop2 = inside = net._modules.values()
+            if not all(map(_plain, [*a.values(), net, norm2, attn, ff, *inside])):
                 return None
-            ff1, relu, drop1, ff2, drop2 = net._modules.values()
             if not (type(qkv) is type(pos) is type(out) is type(ff1) is type(ff2) is nn.Linear
                     and type(norm1) is type(norm2) is nn.LayerNorm and type(relu) is nn.ReLU
                     and type(drop) is type(drop1) is type(drop2) is nn.Dropout

@@ -181,13 +181,16 @@ def plain_eager():
             and not torch.compiler.is_compiling())
 
 
-def plain_tensors(tensors, dtype, device):
-    """Whether these are ordinary contiguous tensors of the device, their values as
-    they lie in memory: what a kernel that takes addresses can work on."""
+_TENSOR_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+def plain_tensors(tensors, dtype, index):
+    """Whether these are ordinary contiguous tensors of GPU ``index`` (-1: of the CPU),
+    their values as they lie in memory: what a kernel that takes addresses can work on."""
+    types, strided = _TENSOR_TYPES, torch.strided    # looked up once: lists are long
     for t in tensors:
-        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype is not dtype
-                or t.device != device or t.layout is not torch.strided
-                or t.is_neg() or not t.is_contiguous()):
+        if (type(t) not in types or t.dtype is not dtype or t.get_device() != index
+                or t.layout is not strided or t.is_neg() or not t.is_contiguous()):
             return False
     return True
 
@@ -195,10 +198,10 @@ def plain_tensors(tensors, dtype, device):
 def lamb_takes(params, grads, ms, vs):
     """Whether ``lamb_step`` takes these lists: contiguous fp32 tensors of one
     GPU, of equal shapes item by item."""
-    device = params[0].device
-    if device.type != "cuda" or not plain_eager():
+    if not params[0].is_cuda or not plain_eager():
         return False
-    if not all(plain_tensors(ts, torch.float32, device) for ts in (params, grads, ms, vs)):
+    index = params[0].get_device()
+    if not all(plain_tensors(ts, torch.float32, index) for ts in (params, grads, ms, vs)):
         return False
     return all(p.shape == g.shape == m.shape == v.shape
                for p, g, m, v in zip(params, grads, ms, vs))
@@ -231,7 +234,7 @@ TXL_WIDTH, TXL_HEAD, TXL_TAILS = 512, 64, 7     # what the Transformer-XL kernel
 def _bf16_operand(t, shape, index):
     """Whether a tensor is what the bf16 kernels read: plain, contiguous, on GPU
     ``index`` and 16-byte aligned."""
-    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype is torch.bfloat16
+    return (type(t) in _TENSOR_TYPES and t.dtype is torch.bfloat16
             and t.shape == shape and t.get_device() == index and t.layout is torch.strided
             and not t.is_neg() and t.is_contiguous() and not t.data_ptr() & 15)
 

@@ -106,8 +106,8 @@ def test_lazily_negated_tensors_keep_the_operations():
     # contiguous and of type Tensor, but their memory holds the other sign
     ok = torch.ones(4, 4)
     negated = torch._neg_view(ok)
-    assert kernels.plain_tensors([ok, ok], torch.float32, ok.device)
-    assert not kernels.plain_tensors([ok, negated], torch.float32, ok.device)
+    assert kernels.plain_tensors([ok, ok], torch.float32, ok.get_device())
+    assert not kernels.plain_tensors([ok, negated], torch.float32, ok.get_device())
     ok = torch.ones(4, 8, dtype=torch.bfloat16)
     index = ok.get_device()
     for t, plain in ((ok, True), (torch._neg_view(ok), False)):
