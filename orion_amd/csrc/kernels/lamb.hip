@@ -11,18 +11,20 @@
 // all stayed on chip would move; as separate element-wise operations it is 100.
 //
 // Measured on the 16-layer, 267,735-token Transformer-XL (188 M parameters, 182
-// tensors): 1.26 ms a step, 6.0 TB/s over the 40 bytes, against 5.2 ms for the
+// tensors): 1.30 ms a step, 5.8 TB/s over the 40 bytes, against 5.2 ms for the
 // element-wise operations.  Four 16-byte accesses per lane and array in
-// workgroups of 256 lanes; two per lane take 1.31 ms, eight 1.37, 512 lanes 1.35.
+// workgroups of 256 lanes; two per lane are 4 % slower, eight 9 %, 512 lanes 7 %.
 // Taking the tensors in groups small enough for the memory-side cache gains
-// nothing over the launches it adds (16 M elements a group: 1.28 ms, 4 M: 1.48),
-// so a launch takes as many tensors as its arguments hold.
+// nothing over the launches it adds, so a group is as many tensors as the arguments
+// hold, and its launches are cut by time only (kMomentsBlocks).
 //
 // The sums run in a fixed order (thread, wavefront, workgroup in fp32 over 4096
 // elements, then fp64 over the workgroups), so a step gives the same bits twice.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "kernels.h"
 
@@ -33,10 +35,16 @@ constexpr int kUnroll = 4;                            // 16-byte accesses per la
 constexpr int kChunk = kThreads * 4 * kUnroll;        // elements per workgroup
 constexpr int kMaxTensors = 64;                       // one lane of a wavefront each
 constexpr int kReduceThreads = 1024;
+// Workgroups of one launch of each pass.  A launch cannot be held back once it has
+// begun, and best-effort kernels run on budgets of 100 us and more, so none takes longer
+// than that: 5120 (21 M elements) are 89 us of the first pass, 8192 (34 M) 87 us of the
+// second.  The step on the 188 M parameters: 1.286 ms in as few launches as the
+// arguments allow (0.54 ms the longest), 1.305 so, 1.343 with 4096 in both passes.
+constexpr uint64_t kMomentsBlocks = 5120, kUpdateBlocks = 8192;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// One launch's tensors, by value in the kernel's arguments (3.1 KiB): nothing to
+// One launch's tensors, by value in the kernel's arguments (2.8 KiB): nothing to
 // upload, nothing that has to outlive the call.
 struct Group {
   orion_lamb_tensor t[kMaxTensors];
@@ -73,9 +81,9 @@ __device__ __forceinline__ void moments(float g, float& m, float& v, const Coefs
 }
 
 template <bool kDecay>
-__global__ __launch_bounds__(kThreads) void lamb_moments_kernel(Group g, Coefs c,
+__global__ __launch_bounds__(kThreads) void lamb_moments_kernel(Group g, Coefs c, uint32_t first,
                                                                 float2* partials) {
-  const uint32_t block = blockIdx.x;
+  const uint32_t block = first + blockIdx.x;
   const int ti = tensor_of_block(g, block);
   const orion_lamb_tensor t = g.t[ti];
   const uint64_t base = (uint64_t)(block - g.first_block[ti]) * kChunk;
@@ -182,9 +190,10 @@ __global__ __launch_bounds__(kReduceThreads) void lamb_ratio_kernel(
 }
 
 template <bool kDecay>
-__global__ __launch_bounds__(kThreads) void lamb_update_kernel(Group g, Coefs c,
+__global__ __launch_bounds__(kThreads) void lamb_update_kernel(Group g, Coefs c, uint32_t first,
                                                                const float* __restrict__ factor) {
-  const uint32_t block = gridDim.x - 1 - blockIdx.x;   // the first pass's last data first
+  // the first pass's last data first
+  const uint32_t block = g.first_block[kMaxTensors] - 1 - (first + blockIdx.x);
   const int ti = tensor_of_block(g, block);
   const orion_lamb_tensor t = g.t[ti];
   const uint64_t base = (uint64_t)(block - g.first_block[ti]) * kChunk;
@@ -262,12 +271,16 @@ extern "C" int orion_lamb_step(const orion_lamb_tensor* tensors, int count, doub
     }
     if (g.count == 0) break;
     for (int i = g.count; i <= kMaxTensors; ++i) g.first_block[i] = (uint32_t)blocks;
-    hipLaunchKernelGGL(decay != 0.0 ? lamb_moments_kernel<true> : lamb_moments_kernel<false>,
-                       dim3((unsigned)blocks), dim3(kThreads), 0, s, g, c, partials);
+    for (uint64_t at = 0; at < blocks; at += kMomentsBlocks)
+      hipLaunchKernelGGL(decay != 0.0 ? lamb_moments_kernel<true> : lamb_moments_kernel<false>,
+                         dim3((unsigned)std::min(kMomentsBlocks, blocks - at)), dim3(kThreads), 0, s,
+                         g, c, (uint32_t)at, partials);
     hipLaunchKernelGGL(lamb_ratio_kernel, dim3((unsigned)g.count), dim3(kReduceThreads), 0, s, g,
                        (const float2*)partials, factor, lr, eps);
-    hipLaunchKernelGGL(decay != 0.0 ? lamb_update_kernel<true> : lamb_update_kernel<false>,
-                       dim3((unsigned)blocks), dim3(kThreads), 0, s, g, c, (const float*)factor);
+    for (uint64_t at = 0; at < blocks; at += kUpdateBlocks)
+      hipLaunchKernelGGL(decay != 0.0 ? lamb_update_kernel<true> : lamb_update_kernel<false>,
+                         dim3((unsigned)std::min(kUpdateBlocks, blocks - at)), dim3(kThreads), 0, s,
+                         g, c, (uint32_t)at, (const float*)factor);
   }
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
 }

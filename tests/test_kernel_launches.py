@@ -95,3 +95,31 @@ def test_gemm_asks_for_the_compute_units_only_where_they_decide(run):
     assert rc == rc_unknown == 0
     assert queries == 0 and whole[0][1] == 1024
     assert null_queries == 0 and null[0][1] == unknown[0][1] == 256
+
+
+LAMB = """
+counts = json.loads(sys.argv[3])[0]
+table = (ctypes.c_uint64 * (5 * len(counts)))()
+for i, n in enumerate(counts):
+    table[5 * i:5 * i + 5] = [AT] * 4 + [n]
+size = lib.orion_lamb_workspace_bytes(table, len(counts))
+rc = lib.orion_lamb_step(table, len(counts), 0.1, 0.9, 0.999, 1e-6, 0.0, AT, size, None)
+print(json.dumps((rc, taken())))
+"""
+
+
+@pytest.mark.parametrize("counts", [
+    # the Transformer-XL client's: an embedding of 137 M elements, its bias, one layer's
+    [267735 * 512, 267735, 3 * 512 * 512, 512 * 512, 512 * 512, 512, 512, 2048 * 512, 2048,
+     2048 * 512, 512, 512, 512],
+    [5120 * 4096 - 1, 1], [5120 * 4096], [8192 * 4096 + 1], [3] * 130, [5, 0, 70001]])
+def test_no_launch_of_a_lamb_step_is_long(run, counts):
+    # a launch once begun cannot be held back: best-effort training has to leave gaps
+    rc, launches = run(LAMB, counts)
+    assert rc == 0
+    for kernel, most in (("lamb_moments", 5120), ("lamb_update", 8192)):
+        grids = [grid for name, grid, _ in launches if kernel in name]
+        assert max(grids) <= most
+        assert sum(grids) == sum(-(-n // 4096) for n in counts)
+    ratios = [grid for name, grid, _ in launches if "lamb_ratio" in name]
+    assert sum(ratios) == sum(n > 0 for n in counts)
