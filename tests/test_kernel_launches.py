@@ -123,3 +123,24 @@ def test_no_launch_of_a_lamb_step_is_long(run, counts):
         assert sum(grids) == sum(-(-n // 4096) for n in counts)
     ratios = [grid for name, grid, _ in launches if "lamb_ratio" in name]
     assert sum(ratios) == sum(n > 0 for n in counts)
+
+
+KERNELS = """
+print(json.dumps([log.launch_log_kernel(i).decode() for i in range(log.launch_log_kernels())]))
+"""
+
+
+def test_the_scheduler_knows_the_classes_of_the_clients_kernels(run):
+    # by the counters: none of these names tells what bounds its kernel, and a kernel of
+    # unknown class passes beside anything
+    from orion_amd.profiling import cu_need, rocprof
+    names = subprocess.run(["c++filt"], input="\n".join(run(KERNELS)), capture_output=True,
+                           check=True, text=True).stdout.split("\n")
+    names = {rocprof.short_name(n) for n in names}
+    own = {n for n in names if "lamb_" in n or "txl_" in n or "crit_" in n}
+    assert len(own) == 12
+    assert {n for n in own if cu_need.classify_source(n)[1] != "counters"} == set()
+    # a LAMB step reaches 70 and 79 % of the HBM rate in its passes
+    assert cu_need.classify("void lamb_moments_kernel") == 0
+    assert cu_need.classify("void lamb_update_kernel") == 0
+    assert cu_need.classify("crit_logits_kernel") == 1
