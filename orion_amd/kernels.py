@@ -231,12 +231,26 @@ def lamb_step(params, grads, ms, vs, lr, betas, eps, weight_decay):
 TXL_WIDTH, TXL_HEAD, TXL_TAILS = 512, 64, 7     # what the Transformer-XL kernels are built for
 
 
+def _bf16_addresses(tensors, shapes, index):
+    """Addresses of tensors that are what the bf16 kernels read: plain, contiguous, of
+    these shapes, on GPU ``index`` and 16-byte aligned; None if one is not.  (Lazily
+    negated tensors are imaginary parts of conjugates: of no 16-bit brain float.)"""
+    types, bf16, strided = _TENSOR_TYPES, torch.bfloat16, torch.strided
+    out = []
+    for t, shape in zip(tensors, shapes):
+        if (type(t) not in types or t.dtype is not bf16 or t.shape != shape
+                or t.get_device() != index or t.layout is not strided
+                or not t.is_contiguous()):
+            return None
+        at = t.data_ptr()
+        if at & 15:
+            return None
+        out.append(at)
+    return out
+
+
 def _bf16_operand(t, shape, index):
-    """Whether a tensor is what the bf16 kernels read: plain, contiguous, on GPU
-    ``index`` and 16-byte aligned."""
-    return (type(t) in _TENSOR_TYPES and t.dtype is torch.bfloat16
-            and t.shape == shape and t.get_device() == index and t.layout is torch.strided
-            and not t.is_neg() and t.is_contiguous() and not t.data_ptr() & 15)
+    return _bf16_addresses((t,), (shape,), index) is not None
 
 
 def inference_only():
@@ -265,14 +279,14 @@ def txl_hidden(x, mems, u, v, layers, inner, eps, keep):
               (inner, width), (inner,), (width, inner), row, row, row)
     table = []
     for tensors in layers:
-        for t, shape in zip(tensors, shapes):
-            if not _bf16_operand(t, shape, index):
-                return None
-            table.append(t.data_ptr())
+        addresses = _bf16_addresses(tensors, shapes, index)
+        if addresses is None:
+            return None
+        table += addresses
     m_len = 0
     if mems is not None:
         if (type(mems) is not torch.Tensor or mems.dtype is not torch.bfloat16
-                or mems.dim() != 4 or mems.get_device() != index or mems.is_neg()
+                or mems.dim() != 4 or mems.get_device() != index
                 or mems.shape[0] != len(layers) or mems.shape[2:] != (batch, width)):
             return None
         m_len = mems.shape[1]
@@ -321,7 +335,7 @@ def adaptive_nll(hidden, target, weight, bias, tail_weight, tail_bias, edges):
         if not _bf16_operand(t, shape, index):
             return None
     if (type(target) is not torch.Tensor or target.dtype is not torch.int64
-            or target.shape != (n,) or target.get_device() != index or target.is_neg()
+            or target.shape != (n,) or target.get_device() != index
             or not target.is_contiguous()):
         return None
     args = _Nll(hidden.data_ptr(), weight.data_ptr(), bias.data_ptr(), tail_weight.data_ptr(),
