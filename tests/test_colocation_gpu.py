@@ -410,3 +410,48 @@ def test_high_priority_training_client(tmp_path):
     dec = _check_replay(co_dir)
     # every high-priority record was handed to the scheduler thread's own stream
     assert sum(1 for l in dec.splitlines() if l.startswith("D 1 1 k")) >= 45 * hp_kernels - hp_kernels
+
+
+@pytest.mark.parametrize("best_effort", [False, True])
+def test_transformer_xl_bf16_inference_client(tmp_path, best_effort):
+    """The client's bf16 request, which runs through the package's own kernels, in
+    either role: the last request's losses are those of the same steps without the
+    interception library, bit for bit."""
+    from orion_amd.benchmark_suite import client_common as cc
+    from orion_amd.benchmark_suite import transformer_trainer as tt
+    n_req, small = 12, {"n_layer": 4}
+    client = {"arch": "transformer", "kernel_file": "", "num_kernels": 0, "num_iters": n_req,
+              "args": {"batchsize": 2, "rps": 0, "uniform": False, "dummy_data": True,
+                       "train": False, "dtype": "bf16", "model_config": small}}
+    if best_effort:
+        other = {"arch": "gemm_bf16", "kernel_file": "", "num_kernels": 0, "num_iters": 4000,
+                 "args": {"batchsize": 1024, "rps": 0, "uniform": False, "dummy_data": True,
+                          "train": False}}
+        job, mine = [client, other], 0
+    else:
+        other = {"arch": "triad_f32", "kernel_file": "", "num_kernels": 0,
+                 "num_iters": 1_000_000,
+                 "args": {"batchsize": 1 << 22, "rps": 0, "uniform": False,
+                          "dummy_data": True, "train": True}}
+        job, mine = [other, client], 1
+    filled, co, _, _, co_dir = _run_iso_and_co(str(tmp_path), job)
+    assert co[mine]["iterations"] == n_req
+    # the request did run through the kernels, and the scheduler knows their classes
+    with open(filled[mine]["kernel_file"]) as f:
+        rows = [line.split(",") for line in f.read().splitlines()[1:]]
+    own = [r for r in rows if "txl_" in r[0] or "crit_" in r[0]]
+    assert len(own) == 2 + 5 * small["n_layer"] + 1 + 3
+    assert {int(r[1]) for r in own if "txl_" in r[0] and "positions" not in r[0]} <= {0, 1}
+
+    with cc.MODEL_INIT_LOCK:
+        cc.seed_everything(42)
+        model = tt.MemTransformerLM(**dict(tt.MODEL_CONFIG, **small)).eval()
+    model = model.to("cuda:0").to(torch.bfloat16)
+    data, target = (t.to("cuda:0") for t in tt.DummyDataLoader(2, 42).batch())
+    mems = None
+    with torch.no_grad():
+        for _ in range(cc.UNCAPTURED_STEPS + n_req):
+            want, mems = model(data, target, mems)
+    out = torch.load(os.path.join(co_dir, f"client_{mine}_output.pt"), weights_only=True)
+    assert torch.equal(out, want.float().cpu())
+    _check_replay(co_dir)
