@@ -189,3 +189,27 @@ def test_gemm_every_tile_exact_on_small_integers(shape):
         for _ in range(3):
             kernels.gemm_bf16_nt(ta, tb, out=out)
             assert torch.equal(out, want.to(dtype))
+
+
+@pytest.mark.parametrize("cus", [0, 32, 64])
+def test_gemm_on_a_limited_stream_and_captured(cus):
+    # the tile depends on the compute units that the stream may use, which are asked for
+    # while the stream is being captured too
+    m, n, k = 1024, 1024, 192
+    g = torch.Generator(device=DEV).manual_seed(cus)
+    ta, tb = (torch.randint(-4, 5, (rows, k), device=DEV, generator=g).to(torch.bfloat16)
+              for rows in (m, n))
+    out = torch.empty((m, n), device=DEV)
+    stream = kernels.cu_masked_stream(cus)
+    torch.cuda.synchronize()
+    kernels.gemm_bf16_nt(ta, tb, out=out, stream=stream)
+    stream.synchronize()
+    assert torch.equal(out, ta.float() @ tb.float().t())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        kernels.gemm_bf16_nt(ta, tb, out=out)
+    for _ in range(3):
+        ta.copy_(torch.randint(-4, 5, (m, k), device=DEV, generator=g))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ta.float() @ tb.float().t())

@@ -173,3 +173,59 @@ def test_captured_request_replays():
         torch.cuda.synchronize()
         want_nll, want_new = _fused(model, *fresh)
         assert torch.equal(nll, want_nll) and torch.equal(new, want_new)
+
+
+@pytest.mark.parametrize("n_head,d_inner,q_len,m_len,batch", [
+    # the inference client's own widths
+    (8, 2048, 192, 192, 4), (8, 2048, 101, 192, 3),
+    # k-tiles of the residual products about their six stages, for each of the two groups
+    # of waves: 5, 6, 7, 8, 9 and 10 behind the feed-forward layer; 6 and 9 behind attention
+    (4, 640, 64, 0, 1), (4, 768, 33, 7, 1), (4, 896, 64, 0, 1), (4, 1024, 64, 0, 1),
+    (12, 1152, 40, 30, 2), (18, 1280, 64, 0, 1)])
+def test_client_widths_no_further_from_64_bits_than_the_operations(n_head, d_inner, q_len, m_len,
+                                                                   batch):
+    changes = dict(n_layer=2, n_head=n_head, d_inner=d_inner)
+    model = _model(**changes)
+    inputs = _inputs(model, q_len, m_len, batch)
+    with torch.no_grad():
+        x = model.word_emb(inputs[0]) * 512 ** 0.5
+        assert model._fused_hidden_states(x, inputs[2]) is not None
+    nll, new = _fused(model, *inputs)
+    old_nll, old_new = _operations(model, *inputs)
+    double = txl.MemTransformerLM(**dict(CONFIG, **changes))
+    double.load_state_dict(model.state_dict())
+    double = double.eval().to(DEV, torch.float64)
+    with torch.no_grad():
+        want_nll, want_new = double(*inputs[:2], None if m_len == 0 else inputs[2].double())
+    for got, old, want in ((nll, old_nll, want_nll), (new, old_new, want_new)):
+        # two bf16 computations in another order are off by as much, within their noise
+        assert _off(got, want) <= 1.25 * _off(old, want) + 1e-4
+
+
+def test_losses_over_clusters_of_many_chunks():
+    # a workgroup takes 1024 columns: a head of three chunks with a ragged last one, a tail
+    # of one token, one of exactly a chunk, one of 66 chunks (more than a wave joins at a
+    # time) whose last holds one token; rows of each tail past one tile of 128
+    tails = [2900, 2901, 3925]
+    n_token = 3925 + 65 * 1024 + 1
+    g = torch.Generator(device=DEV).manual_seed(5)
+    crit = txl.AdaptiveLogSoftmax(n_token, 512, tails).to(DEV)
+    for p in crit.parameters():
+        # logits of some +-30, so that the chunks' maxima differ
+        p.data.normal_(0.0, 0.3 if p.dim() == 2 else 1.0, generator=g)
+    crit = crit.to(torch.bfloat16)
+    rows = 700
+    hidden = torch.randn(rows, 512, device=DEV, generator=g).to(torch.bfloat16)
+    cluster = torch.randint(0, 4, (rows,), device=DEV, generator=g)
+    low = torch.tensor([0] + tails, device=DEV)[cluster]
+    size = torch.tensor([2900, 1, 1024, n_token - 3925], device=DEV)[cluster]
+    target = low + (torch.rand(rows, device=DEV, generator=g) * size).long()
+    target[:8] = torch.tensor([0, 1023, 1024, 2047, 2048, 2899, n_token - 2, n_token - 1],
+                              device=DEV)
+    with torch.no_grad():
+        got = kernels.adaptive_nll(hidden, target, crit.weight, crit.bias, crit.cluster_weight,
+                                   crit.cluster_bias, crit.edges)
+        full = crit.double().full_logprob(hidden.double())
+    want = -full.gather(1, target[:, None]).squeeze(1)
+    # one rounding to bf16 of an fp32 result
+    assert torch.allclose(got.double(), want, rtol=2 ** -8, atol=1e-4)
