@@ -15,10 +15,13 @@ Shapes follow the reference: token ids and targets are time-major
 ``[tgt_len, batch]``; ``forward(data, target, mems)`` returns the per-token
 negative log-likelihood ``[tgt_len, batch]`` and the new memory.
 
-Attention runs through ``scaled_dot_product_attention``: the content term
-(q + u)·k is the fused kernel's own product and the position term (q + v)·r,
-shifted to relative offsets, goes in as its additive bias together with the
-causal mask.
+As operations, attention runs through ``scaled_dot_product_attention``: the
+content term (q + u)·k is the fused kernel's own product and the position term
+(q + v)·r, shifted to relative offsets, goes in as its additive bias together with
+the causal mask.  Inference in bf16 (no gradients, hooks, autocast or tracing, model
+width 512, heads 64 wide) runs through the package's own kernels instead
+(``kernels.txl_hidden``, ``kernels.adaptive_nll``), and so does a LAMB step over
+contiguous fp32 tensors of one GPU (``kernels.lamb_step``).
 """
 
 import math

@@ -309,8 +309,9 @@ __device__ __forceinline__ void small_tile_of_block(int bid, int tiles_m, int ti
 }
 
 template <int TM, int TN, int NS, int GROUPS, typename OutT>
-__global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
-                              OutT* __restrict__ C, int M, int N, int K) {
+__global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, OutT* __restrict__ C, int M,
+    int N, int K) {
   using namespace mfma_tile;
   constexpr int kGroupLds = NS * (Rows<TM>::kBytes + Rows<TN>::kBytes);
   constexpr int kSumLds = (GROUPS - 1) * TM * TN * 4;

@@ -273,14 +273,14 @@ extern "C" int orion_lamb_step(const orion_lamb_tensor* tensors, int count, doub
     for (int i = g.count; i <= kMaxTensors; ++i) g.first_block[i] = (uint32_t)blocks;
     for (uint64_t at = 0; at < blocks; at += kMomentsBlocks)
       hipLaunchKernelGGL(decay != 0.0 ? lamb_moments_kernel<true> : lamb_moments_kernel<false>,
-                         dim3((unsigned)std::min(kMomentsBlocks, blocks - at)), dim3(kThreads), 0, s,
-                         g, c, (uint32_t)at, partials);
+                         dim3((unsigned)std::min(kMomentsBlocks, blocks - at)), dim3(kThreads), 0,
+                         s, g, c, (uint32_t)at, partials);
     hipLaunchKernelGGL(lamb_ratio_kernel, dim3((unsigned)g.count), dim3(kReduceThreads), 0, s, g,
                        (const float2*)partials, factor, lr, eps);
     for (uint64_t at = 0; at < blocks; at += kUpdateBlocks)
       hipLaunchKernelGGL(decay != 0.0 ? lamb_update_kernel<true> : lamb_update_kernel<false>,
-                         dim3((unsigned)std::min(kUpdateBlocks, blocks - at)), dim3(kThreads), 0, s,
-                         g, c, (uint32_t)at, (const float*)factor);
+                         dim3((unsigned)std::min(kUpdateBlocks, blocks - at)), dim3(kThreads), 0,
+                         s, g, c, (uint32_t)at, (const float*)factor);
   }
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
 }

@@ -60,7 +60,9 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
 // one and what reads them.
 __device__ __forceinline__ void mfma_in_place(const bf16x8& a, const bf16x8& b, f32x4& c) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
-}// the second operand in accumulator registers too, for one that stays
+}
+
+// the second operand in accumulator registers too, for one that stays
 __device__ __forceinline__ void mfma_in_place_kept(const bf16x8& a, const bf16x8& b, f32x4& c) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "a"(b));
 }

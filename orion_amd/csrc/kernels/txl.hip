@@ -4,7 +4,7 @@
 // same model as framework operations
 // (benchmarking/benchmark_suite/transformer_trainer.py:63-86, :144).
 //
-// A request is small (768 token rows at batch 4: 0.2 TFLOP, a third of it in the
+// A request is small (768 token rows at batch 4: 0.2 TFLOP, half of it in the
 // vocabulary) and a chain of 16 layers, so what bounds it is the number of
 // dependent launches and the latency inside each, not a rate.  Five launches a
 // layer; whatever does not depend on the chain runs before it, for all layers at
@@ -21,9 +21,9 @@
 //
 // The layer norm rides in the product that reads it: a workgroup's A panel is 64
 // whole rows of 512, so it normalises them itself on the way into LDS, from means
-// and squares that the product before left for every 32 columns (every workgroup
-// of a row panel repeats that; the first column of workgroups also writes the rows,
-// for the residual and the memory).  y stays fp32.
+// and squares that the product before left for every 32 columns (every workgroup of
+// a row panel repeats that; up to sixteen of them write a share of the rows each, for
+// the residual and the memory).  y stays fp32.
 //
 // Sums are fp32 throughout; activations are rounded to bf16 where the model's
 // own operations rounded them, less y, the two query biases (added in fp32) and
@@ -154,9 +154,10 @@ __device__ __forceinline__ void put_row(const RowsOut& out, int row, int chunk, 
 // C[M, N] = A[M, 512] * W[N, 512]^T with the whole A panel of a workgroup in LDS:
 // normalised on the way from fp32 (kNorm) or loaded as it is.  Two groups of four
 // waves take the even and the odd k-tiles, W streaming through kPanelStages stages
-// each, and their sums meet in LDS.  With four waves and eight k-tiles in a row the
-// norm took 7,000 cycles of a product's 16,000 and the loop 5,000: one wave a SIMD
-// waits for every latency alone.  N is a multiple of BN; rows past M are computed
+// each, and their sums meet in LDS: with four waves and eight k-tiles in a row, one
+// wave a SIMD, every latency of the norm and of the loop is waited for alone (11.5 us
+// a launch then, 8.3 so and with the rows' statistics from the product before, at 768
+// rows).  N is a multiple of BN; rows past M are computed
 // from the last row and not written.
 constexpr int kPanelThreads = 2 * kThreads;
 constexpr int kPanelStages = 3;
@@ -503,7 +504,7 @@ __global__ __launch_bounds__(kD / 2) void txl_positions_kernel(uint16_t* table) 
 // distances from the workgroup's first query to the stage's last key on.
 //
 // Bound by latency: at batch 4 (96 workgroups, 384 keys, 3 stages) the matrix
-// cores have some 150 MFMAs a wave.  The next stage's rows travel through
+// cores have at most 78 MFMAs a wave, 26 a stage.  The next stage's rows travel through
 // registers while this one is worked on.
 constexpr int kAttnThreads = 512;
 constexpr int kQ = 64, kKeys = 128;
@@ -1161,14 +1162,14 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
     In x = (In)x0;
     if (i == 0) {
       hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 96, false, QkvEpi>), dim3(row_tiles * qkv_tiles),
-                         dim3(kPanelThreads), 0, s, x0, (In)p.qkv, rows, (int)qkv_tiles, Norm{}, out,
-                         qkv);
+                         dim3(kPanelThreads), 0, s, x0, (In)p.qkv, rows, (int)qkv_tiles, Norm{},
+                         out, qkv);
     } else {
       x = out.x = w.x;
       const Norm norm = {(In)layers[i - 1].norm2_w, (In)layers[i - 1].norm2_b, w.parts, d.eps};
       hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 96, true, QkvEpi>), dim3(row_tiles * qkv_tiles),
-                         dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.qkv, rows, (int)qkv_tiles,
-                         norm, out, qkv);
+                         dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.qkv, rows,
+                         (int)qkv_tiles, norm, out, qkv);
     }
     hipLaunchKernelGGL(txl_attention_kernel, dim3(d.heads * d.batch, (unsigned)tiles(d.q_len, kQ)),
                        dim3(kAttnThreads), 0, s, (In)w.qu, (In)w.qv,
@@ -1181,14 +1182,15 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
     RowsOut out2 = {};
     out2.x = w.x2;
     hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 128, true, ReluEpi>), dim3(row_tiles * ff_tiles),
-                       dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.ff1_w, rows, (int)ff_tiles,
-                       norm, out2, ReluEpi{w.h, (In)p.ff1_b, d.inner});
+                       dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.ff1_w, rows,
+                       (int)ff_tiles, norm, out2, ReluEpi{w.h, (In)p.ff1_b, d.inner});
     hipLaunchKernelGGL(txl_residual_gemm_kernel, res_grid, dim3(2 * kThreads), 0, s, (In)w.h,
                        (In)p.ff2_w, d.inner, (In)p.ff2_b, (In)w.x2, w.y, w.parts, rows);
   }
   const orion_txl_layer& last = layers[d.layers - 1];
   hipLaunchKernelGGL(txl_norm_kernel, dim3((unsigned)tiles(rows, kThreads / 16)), dim3(kThreads), 0,
-                     s, (const float*)w.y, (Norm{(In)last.norm2_w, (In)last.norm2_b, w.parts, d.eps}),
+                     s, (const float*)w.y,
+                     (Norm{(In)last.norm2_w, (In)last.norm2_b, w.parts, d.eps}),
                      (uint16_t*)hidden, rows);
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
 }

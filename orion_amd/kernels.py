@@ -1,7 +1,9 @@
 """ctypes bindings of liborion_kernels.so (the hand-written gfx950 kernels).
 
 torch is used only as the owner of device memory and streams; the arithmetic
-runs in the HIP kernels behind the C ABI declared in ``include/orion_kernels.h``.
+runs in the HIP kernels behind the C ABI declared in ``include/orion_kernels.h``
+(the co-location kernels) and ``include/orion_model_kernels.h`` (the kernels of the
+Transformer-XL client: ``transformer_xl.py`` asks here which calls they take).
 """
 
 import atexit
