@@ -160,8 +160,11 @@ def gemm_bf16_nt(a, b, out=None, out_dtype=torch.bfloat16, stream=None):
     n = b.shape[0]
     if out is None:
         out = torch.empty((m, n), dtype=out_dtype, device=a.device)
-    _check_device(out)
-    if out.shape != (m, n) or out.dtype not in (torch.bfloat16, torch.float32):
+        fits = True
+    else:
+        _check_device(out)
+        fits = out.shape == (m, n)
+    if not fits or out.dtype not in (torch.bfloat16, torch.float32):
         raise ValueError("gemm_bf16_nt output must be [M,N] bf16 or fp32")
     rc = lib().orion_gemm_bf16_nt(a.data_ptr(), b.data_ptr(), out.data_ptr(),
                                   m, n, k, int(out.dtype == torch.float32),
