@@ -213,3 +213,15 @@ def test_gemm_on_a_limited_stream_and_captured(cus):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, ta.float() @ tb.float().t())
+
+
+# the 32 x 64 tile's two groups of waves: 1 to 8 and 64 k-tiles each, about its four stages
+@pytest.mark.parametrize("k", [128, 256, 384, 512, 640, 768, 896, 1024, 8192])
+def test_gemm_two_wave_groups_exact_on_small_integers(k):
+    # as above: every partial sum is exact in fp32
+    g = torch.Generator(device=DEV).manual_seed(k)
+    ta, tb = (torch.randint(-4, 5, (rows, k), device=DEV, generator=g).to(torch.bfloat16)
+              for rows in (256, 512))
+    want = (ta.float() @ tb.float().t())
+    for dtype in (torch.float32, torch.bfloat16):
+        assert torch.equal(kernels.gemm_bf16_nt(ta, tb, out_dtype=dtype), want.to(dtype))
