@@ -432,10 +432,13 @@ int compute_units_of(hipStream_t stream) {
 // only take turns (64 of them, us by 256 x 256 and by the whole GPU's choice: 2048^3
 // 36.8 and 51.4; 1024 x 4096 x 512 13.7 and 23.5), so where the whole GPU's choice is
 // a smaller one the stream is asked for its mask (0.2 us) and the rounds are counted
-// with that.
+// with that.  The runtime's own streams (null, legacy, per thread) have none, and their
+// handles are constants that only launches are sure to take.
 int tile_for_stream(int M, int N, int K, hipStream_t stream) {
   const int tile = tile_for(M, N, K, kWholeGpu);
-  if (tile == 0 || stream == nullptr) return tile;
+  if (tile == 0 || stream == nullptr || stream == hipStreamLegacy ||
+      stream == hipStreamPerThread)
+    return tile;
   const int cus = compute_units_of(stream);
   return cus == kWholeGpu ? tile : tile_for(M, N, K, cus);
 }

@@ -55,7 +55,7 @@ GEMM = """
 out = []
 for m, n, k, cus, stream in json.loads(sys.argv[3])[0]:
     log.launch_log_set_compute_units(cus)
-    rc = lib.orion_gemm_bf16_nt(AT, AT, AT, m, n, k, 0, stream and AT)
+    rc = lib.orion_gemm_bf16_nt(AT, AT, AT, m, n, k, 0, AT if stream is True else stream)
     queries = log.launch_log_queries()
     out.append((rc, taken(), queries))
 print(json.dumps(out))
@@ -88,13 +88,17 @@ def test_gemm_tiles_follow_the_streams_compute_units(run):
 
 
 def test_gemm_asks_for_the_compute_units_only_where_they_decide(run):
-    (rc, whole, queries), (_, null, null_queries), (rc_unknown, unknown, _) = run(GEMM, [
+    (rc, whole, queries), *runtimes_own, (rc_unknown, unknown, _) = run(GEMM, [
         (8192, 8192, 8192, 64, True),       # 256 x 256 tiles on any stream
-        (2048, 2048, 2048, 64, False),      # the null stream spans the GPU
+        (2048, 2048, 2048, 64, None),       # the null, legacy and per-thread streams span
+        (2048, 2048, 2048, 64, 1),          # the GPU, and are no handles to ask about
+        (2048, 2048, 2048, 64, 2),
         (2048, 2048, 2048, 0, True)])       # a failing query: the whole GPU, and no error left
     assert rc == rc_unknown == 0
     assert queries == 0 and whole[0][1] == 1024
-    assert null_queries == 0 and null[0][1] == unknown[0][1] == 256
+    for status, launches, asked in runtimes_own:
+        assert status == 0 and asked == 0 and launches[0][1] == 256
+    assert unknown[0][1] == 256
 
 
 LAMB = """
