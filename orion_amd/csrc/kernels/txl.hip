@@ -300,17 +300,6 @@ __device__ __forceinline__ void panel_gemm(unsigned char* lds, const void* A, co
 // What is done with four columns of a row of C; `ahead` is what that needs from
 // memory, asked for before the product.
 
-// bf16 store of a plain product.
-struct StoreEpi {
-  uint16_t* out;
-  int ld;
-  struct Ahead {};
-  __device__ __forceinline__ Ahead ahead(int) const { return {}; }
-  __device__ __forceinline__ void operator()(int row, int col, const f32x4& v, Ahead) const {
-    store_bf16x4(out + (size_t)row * ld + col, v);
-  }
-};
-
 // [q k v]: the query leaves twice, with each of the two learned biases.
 struct QkvEpi {
   uint16_t *qu, *qv, *kv;
@@ -361,29 +350,161 @@ __global__ __launch_bounds__(kPanelThreads, 1) void txl_ln_gemm_kernel(
 }
 
 // Independent products with the same inner length, one launch: workgroups
-// first_block[i] .. first_block[i + 1] of the grid are job i's.
+// first_block[i] .. first_block[i + 1] of the grid are job i's.  A workgroup takes 256
+// columns, 32 a wave, whose weights stay in registers as the MFMA's fragments over
+// kJobPanels panels of 32 rows, which come to LDS four panels ahead.  N is a multiple
+// of 32.  As 64 x 128 tiles that each brought their own weights the launch took 50 us of
+// a batch-4 request, bound by a workgroup's start (2 us of 6, in 7.5 rounds); so 30, a
+// panel bound by the LDS reads of its rows, which every wave needs whole (256 KiB).  The
+// weights come by whole lines through LDS: loaded as fragments, where lanes side by side
+// are different rows, they take the address unit four times as long (32 us).
 struct Job {
   const uint16_t *A, *W;
   uint16_t* out;
-  int M, tiles_n, ld;
+  int M, N;
 };
 struct Jobs {
   Job job[kMaxJobs];
   uint32_t first_block[kMaxJobs + 1];
   int count;
 };
-constexpr int kJobM = 64, kJobN = 128;
+constexpr int kJobThreads = 512, kJobM = 32, kJobN = 256, kJobPanels = 8;
+constexpr int kJobPanelBytes = kJobM * kD * 2;
+constexpr int kJobWaveN = kJobN / 8;
+constexpr int kJobPassTiles = kPanelTiles / 2;     // k-tiles of weights in LDS at a time
+constexpr int kJobPassBytes = kJobPassTiles * kJobWaveN * kRowBytes;   // of a wave
+constexpr int kJobRing = 5;                        // panels; the weights lie in the last four
+constexpr int kJobLds = kJobRing * kJobPanelBytes;
+static_assert(8 * kJobPassBytes == 4 * kJobPanelBytes, "the weights' place");
 
-__global__ __launch_bounds__(kPanelThreads, 1) void txl_jobs_kernel(Jobs jobs) {
-  __shared__ __attribute__((aligned(16))) unsigned char lds[panel_lds<kJobM, kJobN>()];
+__global__ __launch_bounds__(kJobThreads, 1) void txl_jobs_kernel(Jobs jobs) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kJobLds];
   const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
   const bool before = lane < jobs.count && jobs.first_block[lane] <= blockIdx.x;
   const int i = __builtin_amdgcn_readfirstlane(__popcll(__ballot(before)) - 1);
   const Job job = jobs.job[i];
   const int local = blockIdx.x - jobs.first_block[i];
-  panel_gemm<kJobM, kJobN, false>(lds, job.A, job.W, job.M, local / job.tiles_n,
-                                  local % job.tiles_n, job.tiles_n, Norm{}, RowsOut{},
-                                  StoreEpi{job.out, job.ld});
+  const int tiles_n = (job.N + kJobN - 1) / kJobN;
+  const int tn = local % tiles_n, row0 = local / tiles_n * (kJobPanels * kJobM);
+  const int want = tn * kJobN + wave * kJobWaveN;
+  const int col0 = want < job.N ? want : job.N - kJobWaveN;
+  const int chunk = ((lane & 7) ^ (lane >> 3)) * 8;
+  unsigned char* mine = lds + kJobPanelBytes + wave * kJobPassBytes;
+  const uint16_t* weights = job.W + (size_t)(col0 + (lane >> 3)) * kD + chunk;
+  // wave w brings the w-th k-tile of the rows, eight rows an instruction; past the last
+  // row that one again
+  auto fetch = [&](int panel) {
+#pragma unroll
+    for (int b = 0; b < kJobM / 8; ++b) {
+      int row = row0 + panel * kJobM + b * 8 + (lane >> 3);
+      row = row < job.M ? row : job.M - 1;
+      load_to_lds(job.A + (size_t)row * kD + wave * kTileK + chunk,
+                  lds + panel % kJobRing * kJobPanelBytes + (wave * kJobM + b * 8) * kRowBytes);
+    }
+  };
+  auto fragment = [&](const unsigned char* base, int row, int ks) {
+    return *reinterpret_cast<const bf16x8*>(base + row * kRowBytes +
+                                            (((ks * 4 + lq) ^ (row & 7)) << 4));
+  };
+  // the first half of the weights straight to LDS, the other through registers, so that
+  // both are on their way at once
+  constexpr int kBlocks = kJobWaveN / 8;
+  u32x4 later[kJobPassTiles][kBlocks];
+#pragma unroll
+  for (int t = 0; t < kJobPassTiles; ++t)
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+      load_to_lds(weights + (size_t)b * 8 * kD + t * kTileK,
+                  mine + (t * kJobWaveN + b * 8) * kRowBytes);
+#pragma unroll
+  for (int t = 0; t < kJobPassTiles; ++t)
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+      later[t][b] = *reinterpret_cast<const u32x4*>(weights + (size_t)b * 8 * kD +
+                                                    (kJobPassTiles + t) * kTileK);
+  fetch(0);
+  bf16x8 w[2 * kPanelTiles][2];                    // [k-step][columns]
+  auto read_weights = [&](int first) {
+#pragma unroll
+    for (int t = 0; t < kJobPassTiles; ++t)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          w[(first + t) * 2 + ks][j] = fragment(mine + t * kJobWaveN * kRowBytes, j * 16 + l16, ks);
+    __builtin_amdgcn_s_waitcnt(0xc07f);            // read before anything overwrites it
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  wait_vm<0>();
+  read_weights(0);
+#pragma unroll
+  for (int t = 0; t < kJobPassTiles; ++t)
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+      *reinterpret_cast<u32x4*>(mine + (t * kJobWaveN + b * 8) * kRowBytes + lane * 16) =
+          later[t][b];
+  __builtin_amdgcn_s_waitcnt(0xc07f);
+  __builtin_amdgcn_sched_barrier(0);
+  read_weights(kJobPassTiles);
+  const int left = (job.M - row0 + kJobM - 1) / kJobM;
+  const int panels = left < kJobPanels ? left : kJobPanels;
+  // every panel leaves four stores a wave behind
+  const bool whole = want < job.N && row0 + panels * kJobM <= job.M;
+  for (int p = 0; p < panels; ++p) {
+    // A panel's four loads are followed by at least twelve more and four stores (the
+    // loads of the three panels after it, the stores of one) when its turn comes.
+    if (whole && p > 0) wait_vm<16>();
+    else wait_vm<0>();
+    block_sync();                      // this panel is whole, the one before has been read
+    if (p == 0)
+      for (int n = 1; n < kJobRing - 1; ++n) fetch(n);
+    fetch(p + kJobRing - 1);
+    f32x4 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // the next four k-steps' rows on their way while four are multiplied
+    constexpr int kAhead = 4, kGroups = 2 * kPanelTiles / kAhead;
+    bf16x8 a[2][kAhead][2];
+    auto read = [&](int g) {
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int ks = g * kAhead + s;
+          a[g & 1][s][i] =
+              fragment(lds + p % kJobRing * kJobPanelBytes + (ks >> 1) * kJobM * kRowBytes,
+                       i * 16 + l16, ks & 1);
+        }
+    };
+    read(0);
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+      if (g + 1 < kGroups) read(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            acc[i][j] = mfma(w[g * kAhead + s][j], a[g & 1][s][i], acc[i][j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (want >= job.N) continue;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = row0 + p * kJobM + i * 16 + l16;
+      if (row >= job.M) continue;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        store_bf16x4(job.out + (size_t)row * job.N + col0 + j * 16 + lq * 4, acc[i][j]);
+    }
+  }
+  wait_vm<0>();                        // nothing lands in LDS that is no longer ours
 }
 
 // y[M, 512] = x + bias + A[M, K] * W[512, K]^T in fp32.  Eight waves: two groups of
@@ -1129,15 +1250,15 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
   auto flush = [&]() {
     if (jobs.count == 0) return;
     for (int i = jobs.count; i <= kMaxJobs; ++i) jobs.first_block[i] = (uint32_t)blocks;
-    hipLaunchKernelGGL(txl_jobs_kernel, dim3((unsigned)blocks), dim3(kPanelThreads), 0, s, jobs);
+    hipLaunchKernelGGL(txl_jobs_kernel, dim3((unsigned)blocks), dim3(kJobThreads), 0, s, jobs);
     jobs.count = 0;
     blocks = 0;
   };
   auto add = [&](In A, In W, uint16_t* out, int M, int N) {
     if (M == 0) return;
-    jobs.job[jobs.count] = Job{A, W, out, M, N / kJobN, N};
+    jobs.job[jobs.count] = Job{A, W, out, M, N};
     jobs.first_block[jobs.count++] = (uint32_t)blocks;
-    blocks += tiles(M, kJobM) * (N / kJobN);
+    blocks += tiles(M, kJobM * kJobPanels) * tiles(N, kJobN);
     if (jobs.count == kMaxJobs) flush();
   };
   for (int i = 0; i < d.layers; ++i) {
