@@ -72,6 +72,25 @@ __device__ __forceinline__ float sum16(float v) {
   return v;
 }
 
+// The values of lanes l, l ^ 16, l ^ 32, l ^ 48 joined: v_permlane*_swap of a register with
+// a copy of itself leaves a pair's two halves in the two registers, which takes a few
+// cycles where a shuffle goes through LDS.  (In assembly: the builtins' second result came
+// out as the first one here.  What was just written needs two cycles before the swap.)
+template <typename Join>
+__device__ __forceinline__ float over_rows(float v, Join join) {
+  float other = v;
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(v), "+v"(other));
+  v = other = join(v, other);
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(v), "+v"(other));
+  return join(v, other);
+}
+__device__ __forceinline__ float max_over_rows(float v) {
+  return over_rows(v, [](float a, float b) { return __builtin_fmaxf(a, b); });
+}
+__device__ __forceinline__ float sum_over_rows(float v) {
+  return over_rows(v, [](float a, float b) { return a + b; });
+}
+
 struct Norm {
   const uint16_t* w;
   const uint16_t* b;
@@ -607,35 +626,39 @@ __global__ __launch_bounds__(kD / 2) void txl_positions_kernel(uint16_t* table) 
   table[(size_t)blockIdx.x * kD + kD / 2 + c] = (uint16_t)(v >> 16);
 }
 
-// Relative attention of 64 queries of one head of one sequence.
+// Relative attention of 32 queries of one head of one sequence.
 //
 //   score(i, j) = ((q_i + u) k_j + (q_i + v) r_(m + i - j)) / 8,   j <= m + i
 //
 // with m rows of memory in front of the segment.  Eight waves: wave w takes
-// queries 16 (w % 4) .. + 15 and the first or second half of each stage of 128
-// keys (online softmax; the halves meet in LDS at the end).  K and R are the first
+// queries 16 (w % 2) .. + 15 and one quarter of each stage of 128 keys (online
+// softmax; the quarters meet in LDS at the end).  K and R are the first
 // MFMA operand, so a lane's values belong to ONE query (lane % 16) and to four
 // consecutive keys or distances: the softmax needs two shuffles a maximum, and the
 // probabilities are already where the second product wants its operand, given V
 // transposed and its keys taken in the same order.
 //
-// The shift by relative distance is a shear: the wave computes the 80 distances
-// that its 16 x 64 block of pairs touches, keeps them in LDS as fp32 and each lane
-// picks entry (query - key + 63) of its row.  A stage's R rows are the 192
+// The shift by relative distance is a shear: the wave computes the 48 distances
+// that its 16 x 32 block of pairs touches, keeps them in LDS as fp32 and each lane
+// picks entry (query - key + 31) of its row.  A stage's R rows are the 160
 // distances from the workgroup's first query to the stage's last key on.
 //
-// Bound by latency: at batch 4 (96 workgroups, 384 keys, 3 stages) the matrix
-// cores have at most 78 MFMAs a wave, 26 a stage.  The next stage's rows travel through
-// registers while this one is worked on.
+// Bound by LDS and by the softmax's arithmetic, of two waves a SIMD: at batch 4 (192
+// workgroups, 384 keys, 3 stages) a stage takes 1.6 us of every wave and a
+// launch 8.2; with 64 queries a workgroup, 96 of them, 2.1 and 10.1.  The next stage's rows
+// travel through registers while this one is worked on.
 constexpr int kAttnThreads = 512;
-constexpr int kQ = 64, kKeys = 128;
+constexpr int kQ = 32, kKeys = 128;
+constexpr int kParts4 = 4, kPartKeys = kKeys / kParts4;
 constexpr int kDistances = kQ + kKeys;         // a stage's R rows
 constexpr int kVtRow = (kKeys / 2 + 2) * 4;    // bytes of a row of V transposed
-constexpr int kShearRow = 84;                  // floats of a row of position scores
+constexpr int kShearRow = 52;                  // floats of a row of position scores
 constexpr int kAttnR = kKeys * kRowBytes;
 constexpr int kAttnV = kAttnR + kDistances * kRowBytes;
 constexpr int kAttnShear = kAttnV + kHead * kVtRow;
 constexpr int kAttnLds = kAttnShear + 8 * 16 * kShearRow * 4;
+constexpr int kMeetRow = 20;                   // floats a lane leaves at the end
+static_assert(8 * 64 * kMeetRow * 4 <= kAttnLds, "in place of the stage");
 
 __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
     const uint16_t* __restrict__ qu, const uint16_t* __restrict__ qv,
@@ -646,16 +669,18 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
-  const int head = blockIdx.x % heads, b = blockIdx.x / heads;
-  const int q0 = blockIdx.y * kQ;
+  const int head = blockIdx.x % heads, b = blockIdx.x / heads % batch;
+  const int q0 = blockIdx.x / heads / batch * kQ;
   const int klen = mlen + qlen;
   const int proj = heads * kHead;
-  const int w4 = wave & 3, half = wave >> 2;
+  const int qt = wave & 1, part = wave >> 1;
 
+  const size_t key_step = (size_t)batch * (2 * proj);
+  const uint16_t* in_mem = kv_mem + (size_t)b * (2 * proj) + head * kHead;
+  const uint16_t* in_x = kv_x + (size_t)b * (2 * proj) + head * kHead;
   auto key_row = [&](int j) {
     j = j < klen ? j : klen - 1;
-    return (j < mlen ? kv_mem + ((size_t)j * batch + b) * (2 * proj)
-                     : kv_x + ((size_t)(j - mlen) * batch + b) * (2 * proj)) + head * kHead;
+    return j < mlen ? in_mem + (unsigned)j * key_step : in_x + (unsigned)(j - mlen) * key_step;
   };
   // this thread's share of a stage
   u32x4 nk[2], nr[3], nv[2];
@@ -668,6 +693,7 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       const int u = i * kAttnThreads + threadIdx.x;
+      if (u >= kDistances * 8) break;
       int d = mlen + q0 - (j0 + kKeys - 1) + (u >> 3);
       d = d < 0 ? 0 : d < klen ? d : klen - 1;
       nr[i] = *reinterpret_cast<const u32x4*>(r + (size_t)d * proj + head * kHead + (u & 7) * 8);
@@ -686,6 +712,7 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       const int u = i * kAttnThreads + threadIdx.x, row = u >> 3;
+      if (u >= kDistances * 8) break;
       *reinterpret_cast<u32x4*>(lds + kAttnR + row * kRowBytes + (((u & 7) ^ (row & 7)) << 4)) =
           nr[i];
     }
@@ -700,7 +727,7 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
     }
   };
 
-  const int qi = q0 + w4 * 16 + l16;            // this lane's query
+  const int qi = q0 + qt * 16 + l16;            // this lane's query
   bf16x8 fqu[2], fqv[2];
   {
     const int q = qi < qlen ? qi : qlen - 1;
@@ -730,39 +757,58 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
     put();
     block_sync();
     if (st + 1 < stages) fetch(j0 + kKeys);
-    const int jw = j0 + 64 * half;              // this wave's first key
-    if (jw > mlen + q0 + w4 * 16 + 15) continue;   // all of them in the future
+    const int jw = j0 + kPartKeys * part;       // this wave's first key
+    if (jw > mlen + q0 + qt * 16 + 15) continue;   // all of them in the future
 
-    f32x4 s[4];
+    // Everything this wave takes from the stage, in one go: read one by one between the
+    // MFMAs, each waits for LDS by itself (a stage took 1.5 us of which 0.1 are products).
+    bf16x8 fr[3][2], fk[2][2];
+    u32x2 fv[4][2];
 #pragma unroll
-    for (int t = 0; t < 5; ++t) {
-      f32x4 g = zero;
+    for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        g = mfma(fragment(kAttnR, 16 * w4 + 64 - 64 * half + 16 * t + l16, ks), fqv[ks], g);
-      *reinterpret_cast<f32x4*>(shear + 16 * t + lq * 4) = g;
+      for (int t = 0; t < 3; ++t)
+        fr[t][ks] = fragment(kAttnR, 16 * qt + 96 - kPartKeys * part + 16 * t + l16, ks);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) fk[t][ks] = fragment(0, kPartKeys * part + 16 * t + l16, ks);
     }
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      s[t] = zero;
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        s[t] = mfma(fragment(0, 64 * half + 16 * t + l16, ks), fqu[ks], s[t]);
+    for (int d = 0; d < 4; ++d) {
+      const unsigned char* vt =
+          lds + kAttnV + (16 * d + l16) * kVtRow + (kPartKeys * part + lq * 4) * 2;
+      fv[d][0] = *reinterpret_cast<const u32x2*>(vt);
+      fv[d][1] = *reinterpret_cast<const u32x2*>(vt + 32);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 g[3] = {zero, zero, zero}, s[2] = {zero, zero};
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int t = 0; t < 3; ++t) g[t] = mfma(fr[t][ks], fqv[ks], g[t]);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) s[t] = mfma(fk[t][ks], fqu[ks], s[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < 3; ++t) *reinterpret_cast<f32x4*>(shear + 16 * t + lq * 4) = g[t];
     // the rows of position scores cross lanes of this wave only
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    float by_distance[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) by_distance[t][e] = shear[l16 + 31 - (16 * t + lq * 4 + e)];
+    __builtin_amdgcn_sched_barrier(0);
+    const int last = mlen + qi - jw - lq * 4;     // of this lane's keys, counted from its first
     float top = -__builtin_inff();
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int k = 16 * t + lq * 4 + e;
-        const float v = s[t][e] + shear[l16 + 63 - k];
-        s[t][e] = jw + k <= mlen + qi ? v : -__builtin_inff();
+        const float v = s[t][e] + by_distance[t][e];
+        s[t][e] = 16 * t + e <= last ? v : -__builtin_inff();
         top = __builtin_fmaxf(top, s[t][e]);
       }
-    top = __builtin_fmaxf(top, __shfl_xor(top, 16));
-    top = __builtin_fmaxf(top, __shfl_xor(top, 32));
+    top = max_over_rows(top);
     const float m_new = __builtin_fmaxf(m, top);
     const float base = m_new == -__builtin_inff() ? 0.0f : m_new;
     const float scale = __builtin_amdgcn_exp2f((m - base) * kExp);
@@ -770,56 +816,54 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
     l *= scale;
 #pragma unroll
     for (int d = 0; d < 4; ++d) o[d] *= scale;
-    uint32_t p[4][2];
+    u32x4 p;
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
+    for (int t = 0; t < 2; ++t) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         s[t][e] = __builtin_amdgcn_exp2f((s[t][e] - base) * kExp);
         l += s[t][e];
       }
-      p[t][0] = pack_bf16(s[t][0], s[t][1]);
-      p[t][1] = pack_bf16(s[t][2], s[t][3]);
+      p[2 * t] = pack_bf16(s[t][0], s[t][1]);
+      p[2 * t + 1] = pack_bf16(s[t][2], s[t][3]);
     }
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const u32x4 pg = {p[2 * g][0], p[2 * g][1], p[2 * g + 1][0], p[2 * g + 1][1]};
-      const bf16x8 fp = __builtin_bit_cast(bf16x8, pg);
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const unsigned char* vt =
-            lds + kAttnV + (16 * d + l16) * kVtRow + (64 * half + 32 * g + lq * 4) * 2;
-        const u32x2 lo = *reinterpret_cast<const u32x2*>(vt);
-        const u32x2 hi = *reinterpret_cast<const u32x2*>(vt + 32);
-        const u32x4 fv = {lo[0], lo[1], hi[0], hi[1]};
-        o[d] = mfma(__builtin_bit_cast(bf16x8, fv), fp, o[d]);
-      }
+    for (int d = 0; d < 4; ++d) {
+      const u32x4 f = {fv[d][0][0], fv[d][0][1], fv[d][1][0], fv[d][1][1]};
+      o[d] = mfma(__builtin_bit_cast(bf16x8, f), __builtin_bit_cast(bf16x8, p), o[d]);
     }
   }
   // l holds this lane's keys only
-  l += __shfl_xor(l, 16);
-  l += __shfl_xor(l, 32);
+  l = sum_over_rows(l);
   block_sync();
-  float* meet = reinterpret_cast<float*>(lds) + (w4 * 64 + lane) * 20;
-  if (half == 1) {
-    meet[0] = m;
-    meet[1] = l;
+  // the quarters meet: wave (qt, part) finishes head columns 16 * part .. + 15
+  float* meet = reinterpret_cast<float*>(lds);
+  {
+    float* mine = meet + (wave * 64 + lane) * kMeetRow;
+    mine[0] = m;
+    mine[1] = l;
 #pragma unroll
-    for (int d = 0; d < 4; ++d) *reinterpret_cast<f32x4*>(meet + 4 + d * 4) = o[d];
+    for (int d = 0; d < 4; ++d) *reinterpret_cast<f32x4*>(mine + 4 + d * 4) = o[d];
   }
   block_sync();
-  if (half == 1 || qi >= qlen) return;
-  const float m1 = meet[0];
-  const float top = __builtin_fmaxf(m, m1);
-  const float a0 = m == top ? 1.0f : __builtin_amdgcn_exp2f((m - top) * kExp);
-  const float a1 = m1 == top ? 1.0f : __builtin_amdgcn_exp2f((m1 - top) * kExp);
-  const float inv = 1.0f / (l * a0 + meet[1] * a1);
-  uint16_t* dst = out + ((size_t)qi * batch + b) * proj + head * kHead;
+  if (qi >= qlen) return;
+  float ms[kParts4], top = -__builtin_inff();
 #pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    const f32x4 o1 = *reinterpret_cast<const f32x4*>(meet + 4 + d * 4);
-    store_bf16x4(dst + 16 * d + lq * 4, (o[d] * a0 + o1 * a1) * inv);
+  for (int p = 0; p < kParts4; ++p) {
+    ms[p] = meet[((p * 2 + qt) * 64 + lane) * kMeetRow];
+    top = __builtin_fmaxf(top, ms[p]);
   }
+  float all = 0.0f;
+  f32x4 sum = zero;
+#pragma unroll
+  for (int p = 0; p < kParts4; ++p) {
+    const float* of = meet + ((p * 2 + qt) * 64 + lane) * kMeetRow;
+    const float a = ms[p] == top ? 1.0f : __builtin_amdgcn_exp2f((ms[p] - top) * kExp);
+    all = __builtin_fmaf(of[1], a, all);
+    sum += *reinterpret_cast<const f32x4*>(of + 4 + part * 4) * a;
+  }
+  store_bf16x4(out + ((size_t)qi * batch + b) * proj + head * kHead + 16 * part + lq * 4,
+               sum * (1.0f / all));
 }
 
 // ---------------------------------------------------------------------------
@@ -1171,7 +1215,7 @@ bool dims_fit(const orion_txl_dims& d) {
   return d.q_len > 0 && d.m_len >= 0 && d.batch > 0 && d.layers > 0 && d.heads > 0 &&
          d.heads % 2 == 0 && d.heads <= 1024 && d.inner > 0 && d.inner % 128 == 0 &&
          d.inner <= (1 << 20) && ((int64_t)d.q_len + d.m_len) * d.batch < (1 << 24) &&
-         d.q_len <= 65535 * kQ;
+         d.q_len <= 65535 * 64;
 }
 
 size_t tiles(size_t n, int tile) { return (n + tile - 1) / tile; }
@@ -1292,7 +1336,7 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
                          dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.qkv, rows,
                          (int)qkv_tiles, norm, out, qkv);
     }
-    hipLaunchKernelGGL(txl_attention_kernel, dim3(d.heads * d.batch, (unsigned)tiles(d.q_len, kQ)),
+    hipLaunchKernelGGL(txl_attention_kernel, dim3((unsigned)(d.heads * d.batch * tiles(d.q_len, kQ))),
                        dim3(kAttnThreads), 0, s, (In)w.qu, (In)w.qv,
                        (In)(w.kv_mem + (size_t)i * mem_rows * 2 * proj), (In)w.kv_x,
                        (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
