@@ -868,15 +868,26 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
 
 // ---------------------------------------------------------------------------
 // Adaptive softmax losses.  The logits (n x 267,735 at the client's vocabulary)
-// never reach memory: a workgroup takes 128 rows and up to kCritChunk tiles of 128
-// columns of one cluster and leaves one (maximum, sum of exponentials) pair a row;
-// the last kernel joins a row's pairs and computes the target's own logits and the
-// head's entries for the tails as plain dot products.
+// never reach memory: a workgroup takes 256 rows and a chunk of a cluster's columns, in
+// tiles of 64, and leaves one (reference, sum of exponentials) pair a row; the last
+// kernel joins a row's pairs and computes the target's own logits and the head's entries
+// for the tails as plain dot products.
 
 constexpr int kMaxTails = 7;
-constexpr int kCritM = 128, kCritN = 128, kCritStages = 8;
-constexpr int kCritChunk = 8;
+constexpr int kCritM = 256, kCritN = 64, kCritStages = 16;
+constexpr int kCritWaveM = kCritM / 4;
+constexpr int kCritLeast = 4, kCritMost = 64;    // tiles of a chunk
+constexpr int kCritBlocks = 256;                 // one a compute unit
 constexpr int kGroupThreads = 1024;
+
+// The work as it turns out on the device: every cluster's columns in chunks of the same
+// number of tiles, an item for each chunk and 256 rows.
+struct CritPlan {
+  int chunk;                       // tiles
+  int chunks[kMaxTails + 1];       // of the head and of each tail
+  int row_tiles[kMaxTails + 1];
+  int first_item[kMaxTails + 2];
+};
 
 struct Crit {
   const uint16_t* hidden;          // [n, 512]
@@ -885,14 +896,14 @@ struct Crit {
   const int64_t* target;
   int n, tails;
   int edge[kMaxTails + 2];         // 0, cutoffs, n_token
-  int chunks[kMaxTails + 1];       // of column tiles, of the head and of each tail
-  uint32_t first_block[kMaxTails + 2];
-  int row_tiles;                   // of n rows: what every cluster's grid is made for
+  int least;                       // tiles of a chunk, at least
+  int stride[kMaxTails + 1];       // chunks that a row's pairs have room for
   // workspace
+  CritPlan* plan;
   int* count;                      // [tails] rows of each tail
   int* place;                      // [n] a row's place within its tail
   int* rows;                       // [tails][n] the rows, in order
-  float2* pairs[kMaxTails + 1];    // [rows][chunks]
+  float2* pairs[kMaxTails + 1];    // [rows][stride]
 };
 
 // Tail of a target (0: in the head or outside the vocabulary).
@@ -903,7 +914,9 @@ __device__ __forceinline__ int tail_of(const Crit& c, int64_t t) {
   return tail;
 }
 
-// One workgroup: the rows of every tail, in their order.
+// One workgroup: the rows of every tail, in their order, and the plan: chunks of the fewest
+// tiles that leave no more items than compute units (an item starts with its rows, 7 us,
+// and a second round of a few takes as long as the first).
 __global__ __launch_bounds__(kGroupThreads) void crit_group_kernel(Crit c) {
   constexpr int kWaves = kGroupThreads / 64;
   __shared__ int wave_count[kMaxTails][kWaves];
@@ -937,159 +950,336 @@ __global__ __launch_bounds__(kGroupThreads) void crit_group_kernel(Crit c) {
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0)
+  if (threadIdx.x >= 64) return;
+  int row_tiles[kMaxTails + 1], cols[kMaxTails + 1];
+  int64_t all = 0;
+  const int mine = c.least + lane;                 // tiles: every lane tries another number
+  static_assert(kCritMost - kCritLeast < 64, "a lane for each");
 #pragma unroll
-    for (int k = 0; k < kMaxTails; ++k)
-      if (k < c.tails) c.count[k] = seen[k];
+  for (int k = 0; k <= kMaxTails; ++k) {
+    const int rows = k == 0 ? c.n : k <= c.tails ? seen[k > 0 ? k - 1 : 0] : 0;
+    if (k > 0 && k <= c.tails && lane == 0) c.count[k - 1] = rows;
+    row_tiles[k] = (rows + kCritM - 1) / kCritM;
+    cols[k] = k <= c.tails ? (c.edge[k + 1] - c.edge[k] + kCritN - 1) / kCritN : 0;
+    all += (int64_t)row_tiles[k] * ((cols[k] + mine - 1) / mine);
+  }
+  const uint64_t enough = __ballot(all <= kCritBlocks || mine >= kCritMost);
+  const int chunk = c.least + __builtin_ctzll(enough);   // the last lane's is past kCritMost
+  if (lane != 0) return;
+  CritPlan& plan = *c.plan;
+  plan.chunk = chunk;
+  int items = 0;
+#pragma unroll
+  for (int k = 0; k <= kMaxTails; ++k) {
+    plan.chunks[k] = (cols[k] + chunk - 1) / chunk;
+    plan.row_tiles[k] = row_tiles[k];
+    plan.first_item[k] = items;
+    items += row_tiles[k] * ((cols[k] + chunk - 1) / chunk);
+  }
+  plan.first_item[kMaxTails + 1] = items;
 }
 
-// Wave w owns rows 32 w .. + 31, whose 512 elements stay in registers, and all 128
-// columns of a tile; only the weights go through LDS, eight k-tiles ahead and from
-// one column tile straight on to the next, so that a tile's epilogue runs while the
-// next ones' weights arrive.  (As independent 128 x 128 tiles through two or four
-// stages the kernel took 226 and 309 us of a batch-4 request: at eight k-tiles a
-// tile its first loads and its epilogue cost as much as its products.)
-__global__ __launch_bounds__(kThreads, 1) void crit_logits_kernel(Crit c) {
+// Wave w owns rows 64 w .. + 63, whose 512 elements stay in registers (all 256 accumulator
+// ones), and all 64 columns of a tile; only the weights go through LDS, sixteen k-tiles
+// ahead and from one column tile straight on to the next.  Bound by the matrix cores: a
+// wave reads one fragment for four products (with 32 rows a wave, two, LDS reads alone
+// took as long as the products), a barrier stands between two k-tiles of sixty-four, and
+// the epilogue is six instructions an element: the accumulators start from the bias, and
+// the exponentials are taken against the lane's first tile's maximum, which is only
+// replaced when a sum gets out of hand.  A batch-4 request's logits
+// take 103 us, at 1.9 GHz and 72 % of what the matrix cores can issue; 155 with 128 rows
+// a workgroup, tiles of 128 columns one after the other and chunks of eight.
+__device__ __forceinline__ void mfma_by_kept(const bf16x8& a, const bf16x8& kept, f32x4& c) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(kept));
+}
+
+template <int I, int J>
+__device__ __forceinline__ void settle_vector(f32x4 (&acc)[I][J]) {   // mfma_tile.h's settle
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) asm volatile("" : "+v"(acc[i][j]));
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < I; ++i)
+#pragma unroll
+    for (int j = 0; j < J; ++j) asm volatile("" : "+v"(acc[i][j]));
+}
+
+__device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int k, int chunk,
+                                          int row0, int rows, int width) {
   constexpr int NS = kCritStages, kStage = Rows<kCritN>::kBytes, kLoads = Rows<kCritN>::kLoads;
-  constexpr int kJ = kCritN / 16;
-  static_assert(NS == kPanelTiles, "the waits below");
-  // the stages, and a tile's biases for each wave (one array: with two the compiler
-  // waits for the loads in flight before every read)
-  __shared__ __attribute__((aligned(16))) unsigned char lds[NS * kStage + 4 * kCritN * 2];
-  int k = 0;
-  while (k < c.tails && blockIdx.x >= c.first_block[k + 1]) ++k;
-  // eight chunks, then the next row of tiles: an XCD takes the row tiles of one
-  // chunk one after the other and reads those weights once
-  const int local = blockIdx.x - c.first_block[k];
-  const int per = 8 * c.row_tiles;
-  const int chunk = local / per * 8 + local % 8;
-  const int row0 = local % per / 8 * kCritM;
-  const int rows = k == 0 ? c.n : c.count[k - 1];
-  if (chunk >= c.chunks[k] || row0 >= rows) return;
+  constexpr int kI = kCritWaveM / 16, kJ = kCritN / 16;
+  static_assert(NS == 2 * kPanelTiles && kPanelTiles % 2 == 0, "the order of the loads");
+  static_assert((kCritMost + 1) * kCritN * 2 <= 4 * kCritWaveM * kRowBytes, "the biases' place");
   const int* list = k == 0 ? nullptr : c.rows + (size_t)(k - 1) * c.n;
-  const int lo = c.edge[k] + chunk * kCritChunk * kCritN;    // this chunk's tokens
-  const int hi = c.edge[k + 1];
-  const int n_token = c.edge[c.tails + 1];
-  const int all = (hi - lo + kCritN - 1) / kCritN;
-  const int tiles = all < kCritChunk ? all : kCritChunk;
+  const int lo = c.edge[k] + chunk * width;                  // this chunk's tokens
+  const int left = c.edge[k + 1] - lo;
+  const int tokens = left < width ? left : width;
+  const int tiles = (tokens + kCritN - 1) / kCritN;
+  const int last_token = lo + tokens - 1;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
-  // a tile may reach past its cluster (masked below) but not past the vocabulary
-  auto issue_one = [&](int i, int tile, int kt) {
-    int token = lo + tile * kCritN + (i * 4 + wave) * 8 + (lane >> 3);
-    token = token < n_token ? token : n_token - 1;
-    load_to_lds(c.weight + (size_t)token * kD + kt * kTileK + ((lane & 7) ^ (lane >> 3)) * 8,
-                lds + kt * kStage + (i * 4 + wave) * 1024);
+  // rows of weights past the chunk are its last one again (masked below)
+  struct Source {
+    const uint16_t* p[kLoads];
   };
+  auto source = [&](int tile) {
+    Source s;
 #pragma unroll
-  for (int kt = 0; kt < NS; ++kt)
+    for (int i = 0; i < kLoads; ++i) {
+      int token = lo + tile * kCritN + (i * 4 + wave) * 8 + (lane >> 3);
+      token = token < last_token ? token : last_token;
+      s.p[i] = c.weight + (size_t)token * kD + ((lane & 7) ^ (lane >> 3)) * 8;
+    }
+    return s;
+  };
+  auto issue_one = [&](const Source& s, int i, int kt, int stage) {
+    load_to_lds(s.p[i] + kt * kTileK, lds + stage * kStage + (i * 4 + wave) * 1024);
+  };
+  {
+    const Source s0 = source(0), s1 = source(1);
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) issue_one(i, 0, kt);
-  bf16x8 fa[2][2 * kPanelTiles];
+    for (int q = 0; q < NS - 1; ++q)
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    int at = row0 + wave * 32 + i * 16 + l16;
-    at = at < rows ? at : rows - 1;
-    const uint16_t* p = c.hidden + (size_t)(list ? list[at] : at) * kD + lq * 8;
-#pragma unroll
-    for (int ks = 0; ks < 2 * kPanelTiles; ++ks)
-      fa[i][ks] = *reinterpret_cast<const bf16x8*>(p + ks * 32);
+      for (int i = 0; i < kLoads; ++i)
+        issue_one(q < kPanelTiles ? s0 : s1, i, q % kPanelTiles, q);
+    __builtin_amdgcn_sched_barrier(0);
   }
-  bf16x8 fb[2][2 * kJ];                             // [even, odd k-tile][k-step, columns]
-  auto read_one = [&](auto odd, int r, int kt) {
-    const int at = ((r / kJ * 4 + lq) ^ (l16 & 7)) << 4;
-    fb[decltype(odd)::value][r] = *reinterpret_cast<const bf16x8*>(
-        lds + kt * kStage + (r % kJ * 16 + l16) * kRowBytes + at);
-  };
+  // the chunk's biases: loads of them in the loop would be waited for together with every
+  // other load in flight
+  constexpr int kBiasLoads = kCritMost * kCritN / kThreads;
+  uint16_t bias_line[kBiasLoads];
 
-  float top[2] = {-__builtin_inff(), -__builtin_inff()}, sum[2] = {0.0f, 0.0f};
+  // The wave's rows, by whole lines, and through LDS into the fragments' order.
+  unsigned char* own = lds + NS * kStage + wave * kCritWaveM * kRowBytes;
+  bf16x8 fa[kI][2 * kPanelTiles];
+  {
+    int from[kCritWaveM / 8];
+#pragma unroll
+    for (int g = 0; g < kCritWaveM / 8; ++g) {
+      const int at = row0 + wave * kCritWaveM + g * 8 + (lane >> 3);
+      from[g] = at < rows ? at : rows - 1;
+    }
+    if (list) {
+#pragma unroll
+      for (int g = 0; g < kCritWaveM / 8; ++g) from[g] = list[from[g]];
+    }
+    constexpr int kHalf = kPanelTiles / 2, kLines = kCritWaveM / 8;
+    u32x4 line[kHalf][kLines];                      // half of the k-tiles at a time
+    auto load = [&](int kt, int g) {
+      line[kt % kHalf][g] = *reinterpret_cast<const u32x4*>(
+          c.hidden + (size_t)from[g] * kD + ((lane & 7) ^ (lane >> 3)) * 8 + kt * kTileK);
+    };
+#pragma unroll
+    for (int g = 0; g < kLines; ++g) {
+#pragma unroll
+      for (int kt = 0; kt < kHalf; ++kt) load(kt, g);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int b = 0; b < kBiasLoads; ++b) {
+      const int token = lo + b * kThreads + threadIdx.x;
+      bias_line[b] = c.bias[token < last_token ? token : last_token];
+    }
+#pragma unroll
+    for (int kt = 0; kt < kPanelTiles; ++kt) {
+#pragma unroll
+      for (int g = 0; g < kLines; ++g)
+        *reinterpret_cast<u32x4*>(own + g * 8 * kRowBytes + lane * 16) = line[kt % kHalf][g];
+#pragma unroll
+      for (int i = 0; i < kI; ++i)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+          fa[i][kt * 2 + ks] = *reinterpret_cast<const bf16x8*>(
+              own + (i * 16 + l16) * kRowBytes + (((ks * 4 + lq) ^ (l16 & 7)) << 4));
+      if (kt == kHalf - 1) {
+#pragma unroll
+        for (int next = kHalf; next < kPanelTiles; ++next)
+#pragma unroll
+          for (int g = 0; g < kLines; ++g) load(next, g);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  block_sync();
+  uint16_t* biases = reinterpret_cast<uint16_t*>(lds + NS * kStage);   // in the rows' place
+#pragma unroll
+  for (int b = 0; b < kBiasLoads; ++b) biases[b * kThreads + threadIdx.x] = bias_line[b];
+  bf16x8 fb[2][2 * kJ];                             // [even, odd k-tile][k-step, columns]
+  // from here on a read is an offset from one of four addresses
+  const unsigned char* place[2][2];
+#pragma unroll
+  for (int half = 0; half < 2; ++half)
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      place[half][ks] = lds + half * kPanelTiles * kStage + l16 * kRowBytes +
+                        (((ks * 4 + lq) ^ (l16 & 7)) << 4);
+  auto read_one = [&](auto odd, int r, int stage) {
+    fb[decltype(odd)::value][r] = *reinterpret_cast<const bf16x8*>(
+        place[stage / kPanelTiles][r / kJ] + stage % kPanelTiles * kStage +
+        r % kJ * 16 * kRowBytes);
+  };
   wait_vm<0>();
   block_sync();
 #pragma unroll
   for (int r = 0; r < 2 * kJ; ++r) read_one(std::integral_constant<int, 0>{}, r, 0);
 
-  auto tile = [&](int t, auto last) {
-    constexpr bool kLast = decltype(last)::value;
-    f32x4 acc[2][kJ];
-    clear(acc);
-    // of columns 2 * lane and the next; joined only in the epilogue, or the wait for
-    // them would empty the pipeline
-    uint16_t bias_lo = 0, bias_hi = 0;
-    auto step = [&](auto tile_c) {
-      constexpr int kt = decltype(tile_c)::value;
-      constexpr bool kRead = !kLast || kt + 1 < kPanelTiles;
-      if constexpr (kRead) {
-        // the next k-tile has landed; those after it may still be in flight
-        wait_vm<kLast ? kLoads * (kPanelTiles - 2 - kt) : kLoads * (NS - 2)>();
-        block_sync();
-        __builtin_amdgcn_sched_barrier(0);
-      } else {
-        block_sync();
-      }
+  constexpr float kLog2e = 1.44269504088896340736f;
+  const float kNone = -__builtin_inff();
+  float ref[kI], sum[kI];
 #pragma unroll
-      for (int m = 0; m < 4 * kJ; ++m) {
-        const int ks = m / (2 * kJ), i = m / kJ % 2, j = m % kJ;
-        mfma_in_place_kept(fb[kt & 1][ks * kJ + j], fa[i][kt * 2 + ks], acc[i][j]);
-        // reads of the next k-tile in the first three quarters, loads of the next
-        // column tile's into the stage that this one has left
-        if (kRead && m % 3 != 2 && m * 2 / 3 < 2 * kJ) {
-          constexpr int kNext = (kt + 1) % kPanelTiles;
-          read_one(std::integral_constant<int, (kt + 1) & 1>{}, (m * 2 + 2) / 3, kNext);
+  for (int i = 0; i < kI; ++i) {
+    ref[i] = kNone;
+    sum[i] = 0.0f;
+  }
+  // The bias is one more product, by a row of ones: only the first of a fragment's 32
+  // elements counts, lane group 0's first.
+  const u32x4 one = {lq == 0 ? 0x3f80u : 0u, 0, 0, 0};
+  const uint32_t first = lq == 0 ? 0xffffu : 0u;
+  uint32_t bias[kJ];
+  auto read_bias = [&](int tile) {
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) bias[j] = biases[tile * kCritN + j * 16 + l16];
+  };
+  read_bias(0);
+  float base[kI] = {0.0f, 0.0f, 0.0f, 0.0f};        // the reference, or 0 without one
+  auto term = [&](float v, int i) { return __builtin_amdgcn_exp2f((v - base[i]) * kLog2e); };
+  // a tile's exponentials `part` (a lane's own columns; lanes meet at the end) to the sums;
+  // without a reference, or with one so far below that the sum might overflow, they are
+  // taken again against a new one
+  auto take = [&](const f32x4 (&acc)[kI][kJ], float (&part)[kI]) {
+#pragma unroll
+    for (int i = 0; i < kI; ++i) {
+      if (__any(ref[i] == kNone || part[i] > 0x1p60f)) {
+        float m = ref[i];
+#pragma unroll
+        for (int j = 0; j < kJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) m = __builtin_fmaxf(m, acc[i][j][e]);
+        base[i] = m == kNone ? 0.0f : m;
+        sum[i] *= term(ref[i], i);
+        ref[i] = m;
+        part[i] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < kJ; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part[i] += term(acc[i][j][e], i);
+      }
+      sum[i] += part[i];
+    }
+  };
+  Source next = source(1);
+  // Tile t's products, between them the exponentials of the tile before.
+  auto tile = [&](int t, auto parity, f32x4 (&acc)[kI][kJ], f32x4 (&old)[kI][kJ]) {
+    constexpr int half = decltype(parity)::value ? kPanelTiles : 0;   // this tile's first stage
+    const Source after = source(t + 2);
+    float part[kI] = {0.0f, 0.0f, 0.0f, 0.0f}, one_term = 0.0f;
+    static_assert(kI == 4, "part and base");
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) {
+      const u32x4 b = {bias[j] & first, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < kI; ++i)
+        asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0"
+                     : "=v"(acc[i][j]) : "v"(b), "v"(one));
+    }
+    // by now the products before those have written the old tile
+#pragma unroll
+    for (int i = 0; i < kI; ++i)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) asm volatile("" : "+v"(old[i][j]));
+    // k-tiles 2 * pair and the next.  Behind the barrier every wave has read the first of
+    // them and the two after it have landed, so the stage before them and the first one's
+    // are filled again; twelve k-tiles may be in flight.
+    auto step = [&](auto pair_c) {
+      constexpr int kFirst = decltype(pair_c)::value * 2;
+      wait_vm<kLoads*(NS - 4)>();
+      block_sync();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int kt = kFirst + h;
+#pragma unroll
+        for (int m = 0; m < 2 * kI * kJ; ++m) {
+          const int ks = m / (kI * kJ), i = m / kJ % kI, j = m % kJ;
+          mfma_by_kept(fb[h][ks * kJ + j], fa[i][kt * 2 + ks], acc[i][j]);
+          if (m % 3 == 1 && m / 3 < 2 * kJ) {       // the next k-tile's fragments
+            const int stage = kt + 1 < kPanelTiles ? half + kt + 1 : kPanelTiles - half;
+            if (h == 0) read_one(std::integral_constant<int, 1>{}, m / 3, stage);
+            else read_one(std::integral_constant<int, 0>{}, m / 3, stage);
+          }
+          if (h == 0 && m % 8 == 2) {
+            const int x = m / 8;                    // two loads for each stage
+            if (x < kLoads) {
+              if (kFirst == 0) issue_one(next, x, kPanelTiles - 1, 2 * kPanelTiles - half - 1);
+              else issue_one(after, x, kFirst - 1, half + kFirst - 1);
+            } else {
+              issue_one(after, x - kLoads, kFirst, half + kFirst);
+            }
+          }
+          // an element of the old tile every four products, one instruction behind each of
+          // them: in a row they would wait for each other
+          const int at = kt * 2 * kI * kJ + m;
+          static_assert(kPanelTiles * 2 == 4 * 4, "four products an element");
+          const int x = at / 4, oi = x / (kJ * 4);
+          if (at % 4 == 0) one_term = old[oi][x / 4 % kJ][x % 4] - base[oi];
+          else if (at % 4 == 1) one_term *= kLog2e;
+          else if (at % 4 == 2) one_term = __builtin_amdgcn_exp2f(one_term);
+          else part[oi] += one_term;
+          if (at % 4 < 3) asm volatile("" : "+v"(one_term));
+          else asm volatile("" : "+v"(part[oi]));
+          __builtin_amdgcn_sched_barrier(0);
         }
-        if (!kLast && m % 8 == 2) issue_one(m / 8, t + 1, kt);
-        __builtin_amdgcn_sched_barrier(0);
       }
     };
     step(std::integral_constant<int, 0>{});
-    {
-      const int token = lo + t * kCritN + lane * 2;
-      bias_lo = c.bias[token < n_token ? token : n_token - 1];
-      bias_hi = c.bias[token + 1 < n_token ? token + 1 : n_token - 1];
-    }
+    read_bias(t + 1);
     step(std::integral_constant<int, 1>{});
     step(std::integral_constant<int, 2>{});
     step(std::integral_constant<int, 3>{});
-    step(std::integral_constant<int, 4>{});
-    step(std::integral_constant<int, 5>{});
-    step(std::integral_constant<int, 6>{});
-    step(std::integral_constant<int, 7>{});
-    settle(acc);
-    unsigned char* bias_lds = lds + NS * kStage + wave * kCritN * 2;
-    *reinterpret_cast<uint32_t*>(bias_lds + lane * 4) = bias_lo | (uint32_t)bias_hi << 16;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-    // a lane's own columns only; lanes meet at the end
+    next = after;
+    take(old, part);
+  };
+  auto last_tile = [&](f32x4 (&acc)[kI][kJ]) {
+    settle_vector(acc);
+    float part[kI];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float m = top[i];
-#pragma unroll
-      for (int j = 0; j < kJ; ++j) {
-        const u32x2 two = *reinterpret_cast<const u32x2*>(bias_lds + (j * 16 + lq * 4) * 2);
-        const f32x4 bj = {bf16_lo(two[0]), bf16_hi(two[0]), bf16_lo(two[1]), bf16_hi(two[1])};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int token = lo + t * kCritN + j * 16 + lq * 4 + e;
-          const float v = acc[i][j][e] + bj[e];
-          acc[i][j][e] = !kLast || token < hi ? v : -__builtin_inff();
-          m = __builtin_fmaxf(m, acc[i][j][e]);
-        }
-      }
-      const float base = m == -__builtin_inff() ? 0.0f : m;
-      float s = sum[i] * __expf(top[i] - base);
+    for (int i = 0; i < kI; ++i) {
+      part[i] = 0.0f;
 #pragma unroll
       for (int j = 0; j < kJ; ++j)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s += __expf(acc[i][j][e] - base);
-      top[i] = m;
-      sum[i] = s;
+        for (int e = 0; e < 4; ++e) {
+          const int token = lo + (tiles - 1) * kCritN + j * 16 + lq * 4 + e;
+          if (token > last_token) acc[i][j][e] = kNone;
+          part[i] += term(acc[i][j][e], i);
+        }
     }
+    take(acc, part);
   };
-  for (int t = 0; t + 1 < tiles; ++t) tile(t, std::false_type{});
-  tile(tiles - 1, std::true_type{});
+  f32x4 even[kI][kJ], odd[kI][kJ];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    float m = top[i], s = sum[i];
+  for (int i = 0; i < kI; ++i)
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) odd[i][j] = f32x4{kNone, kNone, kNone, kNone};   // before the first
+  int t = 0;
+  for (; t + 1 < tiles; t += 2) {
+    tile(t, std::integral_constant<int, 0>{}, even, odd);
+    tile(t + 1, std::integral_constant<int, 1>{}, odd, even);
+  }
+  if (t < tiles) {
+    tile(t, std::integral_constant<int, 0>{}, even, odd);
+    last_tile(even);
+  } else {
+    last_tile(odd);
+  }
+  wait_vm<0>();                        // nothing lands in LDS that is no longer ours
+#pragma unroll
+  for (int i = 0; i < kI; ++i) {
+    float m = ref[i], s = sum[i];
 #pragma unroll
     for (int d = 16; d < 64; d <<= 1) {
       const float om = __shfl_xor(m, d), os = __shfl_xor(s, d);
@@ -1097,8 +1287,32 @@ __global__ __launch_bounds__(kThreads, 1) void crit_logits_kernel(Crit c) {
       s = s * (m == t ? 1.0f : __expf(m - t)) + os * (om == t ? 1.0f : __expf(om - t));
       m = t;
     }
-    const int at = row0 + wave * 32 + i * 16 + l16;
-    if (lq == 0 && at < rows) c.pairs[k][(size_t)at * c.chunks[k] + chunk] = make_float2(m, s);
+    const int at = row0 + wave * kCritWaveM + i * 16 + l16;
+    if (lq == 0 && at < rows) c.pairs[k][(size_t)at * c.stride[k] + chunk] = make_float2(m, s);
+  }
+}
+
+__global__ __launch_bounds__(kThreads, 1) void crit_logits_kernel(Crit c) {
+  // the stages, and 8 KiB for each wave's rows on their way to registers (one array: with
+  // two the compiler waits for the loads in flight before every read)
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kCritStages * Rows<kCritN>::kBytes + 4 * kCritWaveM * kRowBytes];
+  auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  const CritPlan& plan = *c.plan;
+  const int items = uniform(plan.first_item[kMaxTails + 1]);
+  for (int item = blockIdx.x; item < items; item += kCritBlocks) {
+    int k = 0;
+    while (k < c.tails && item >= uniform(plan.first_item[k + 1])) ++k;
+    // eight chunks, then their next rows: an XCD (of eight, in turn) takes all the rows of a
+    // chunk and brings its weights once
+    const int local = item - uniform(plan.first_item[k]);
+    const int row_tiles = uniform(plan.row_tiles[k]), width = uniform(plan.chunk) * kCritN;
+    const int group = local / (8 * row_tiles), in_group = local % (8 * row_tiles);
+    const int others = uniform(plan.chunks[k]) - group * 8, abreast = others < 8 ? others : 8;
+    const int chunk = group * 8 + in_group % abreast;
+    const int row0 = in_group / abreast * kCritM;
+    const int rows = k == 0 ? c.n : uniform(c.count[k - 1]);
+    crit_item(c, lds, k, chunk, row0, rows, width);
+    block_sync();                      // the next item's loads land where this one's were read
   }
 }
 
@@ -1162,9 +1376,10 @@ __global__ __launch_bounds__(kThreads) void crit_losses_kernel(Crit c, uint16_t*
       top = -__builtin_inff();
       sum = __builtin_nanf("");
     }
-    loss = join_pairs(c.pairs[0] + (size_t)row * c.chunks[0], c.chunks[0], lane, top, sum) - head;
+    loss = join_pairs(c.pairs[0] + (size_t)row * c.stride[0], c.plan->chunks[0], lane, top, sum) -
+           head;
     if (k)
-      loss += join_pairs(c.pairs[k] + (size_t)c.place[row] * c.chunks[k], c.chunks[k], lane,
+      loss += join_pairs(c.pairs[k] + (size_t)c.place[row] * c.stride[k], c.plan->chunks[k], lane,
                          -__builtin_inff(), 0.0f) -
               own;
   }
@@ -1218,7 +1433,7 @@ bool dims_fit(const orion_txl_dims& d) {
          d.q_len <= 65535 * 64;
 }
 
-size_t tiles(size_t n, int tile) { return (n + tile - 1) / tile; }
+size_t tiles(size_t n, size_t tile) { return (n + tile - 1) / tile; }
 
 bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
   if (a->rows <= 0 || a->rows >= (1 << 24) || a->tails < 0 || a->tails > kMaxTails) return false;
@@ -1230,24 +1445,23 @@ bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
   c->target = (const int64_t*)a->target;
   c->n = a->rows;
   c->tails = a->tails;
-  c->row_tiles = (int)tiles(a->rows, kCritM);
-  uint64_t blocks = 0;
   for (int k = 0; k <= a->tails + 1; ++k) {
     c->edge[k] = a->edges[k];
     if (k == 0 ? a->edges[0] != 0 : a->edges[k] <= a->edges[k - 1]) return false;
   }
+  // every row is one of the head's, so chunks are at least as many tiles as its items ask for
+  const size_t head = tiles(a->rows, kCritM) * tiles(a->edges[1], kCritN);
+  const size_t least = tiles(head, kCritBlocks);
+  c->least = (int)(least < kCritLeast ? kCritLeast : least > kCritMost ? kCritMost : least);
   Pieces p{(char*)base};
+  c->plan = p.take<CritPlan>(1);
   c->count = p.take<int>(kMaxTails);
   c->place = p.take<int>(a->rows);
   c->rows = p.take<int>((size_t)a->tails * a->rows);
   for (int k = 0; k <= a->tails; ++k) {
-    c->first_block[k] = (uint32_t)blocks;
-    c->chunks[k] = (int)tiles((size_t)c->edge[k + 1] - c->edge[k], kCritN * kCritChunk);
-    c->pairs[k] = p.take<float2>((size_t)a->rows * c->chunks[k]);
-    blocks += tiles(c->chunks[k], 8) * 8 * c->row_tiles;
-    if (blocks > 0x7fffffffu) return false;
+    c->stride[k] = (int)tiles((size_t)c->edge[k + 1] - c->edge[k], kCritN * c->least);
+    c->pairs[k] = p.take<float2>((size_t)a->rows * c->stride[k]);
   }
-  c->first_block[a->tails + 1] = (uint32_t)blocks;
   *bytes = p.used;
   return true;
 }
@@ -1380,8 +1594,7 @@ extern "C" int orion_nll_bf16(const orion_nll* args, void* nll, void* workspace,
     return ORION_ERR_ALIGN;
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(crit_group_kernel, dim3(1), dim3(kGroupThreads), 0, s, c);
-  hipLaunchKernelGGL(crit_logits_kernel, dim3(c.first_block[c.tails + 1]), dim3(kThreads), 0, s,
-                     c);
+  hipLaunchKernelGGL(crit_logits_kernel, dim3(kCritBlocks), dim3(kThreads), 0, s, c);
   hipLaunchKernelGGL(crit_losses_kernel, dim3((unsigned)tiles(c.n, kThreads / 64)), dim3(kThreads),
                      0, s, c, (uint16_t*)nll);
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;

@@ -229,3 +229,63 @@ def test_losses_over_clusters_of_many_chunks():
     want = -full.gather(1, target[:, None]).squeeze(1)
     # one rounding to bf16 of an fp32 result
     assert torch.allclose(got.double(), want, rtol=2 ** -8, atol=1e-4)
+
+
+@pytest.mark.parametrize("q_len,m_len,batch", [(31, 97, 1), (32, 225, 1), (33, 31, 2), (97, 1, 3),
+                                               (5, 64, 4), (3, 257, 1), (2, 171, 3)])
+def test_edges_of_query_blocks_and_of_the_kept_weights_rows(q_len, m_len, batch):
+    """32 queries a workgroup, 32 keys a wave; the memory's rows in panels of 32, eight
+    panels a workgroup (256, 257 and 513 rows)."""
+    model = _model()
+    inputs = _inputs(model, q_len, m_len, batch)
+    nll, new = _fused(model, *inputs)
+    old_nll, old_new = _operations(model, *inputs)
+    want_nll, want_new = _in_64_bits(model, *inputs)
+    # bf16 computations in another order, within their noise of each other
+    assert _off(nll, want_nll) <= 1.25 * _off(old_nll, want_nll) + 1e-4
+    assert _off(new, want_new) <= 1.25 * _off(old_new, want_new) + 1e-4
+
+
+def _losses_in_64_bits(hidden, target, weight, bias, tail_weight, tail_bias, edges):
+    hidden, weight, bias, tail_weight, tail_bias = (
+        t.double() for t in (hidden, weight, bias, tail_weight, tail_bias))
+    head = torch.cat([hidden @ weight[:edges[1]].t() + bias[:edges[1]],
+                      hidden @ tail_weight.t() + tail_bias], 1).log_softmax(1)
+    loss = -head.gather(1, target.clamp(max=edges[1] - 1)[:, None]).squeeze(1)
+    for c, (lo, hi) in enumerate(zip(edges[1:], edges[2:])):
+        at = ((target >= lo) & (target < hi)).nonzero().squeeze(1)
+        tail = (hidden[at] @ weight[lo:hi].t() + bias[lo:hi]).log_softmax(1)
+        loss[at] = -(head[at, edges[1] + c] + tail.gather(1, (target[at] - lo)[:, None]).squeeze(1))
+    return loss
+
+
+@pytest.mark.parametrize("rows,edges", [
+    (1, [0, 1]), (3, [0, 64, 65]), (255, [0, 63, 127, 700]), (257, [0, 1000, 5000]),
+    (600, [0, 300, 20000, 60000]), (1500, [0, 257, 513, 4610])])
+@pytest.mark.parametrize("biases", ["plain", "lowest", "infinite", "steps", "peaks"])
+def test_losses_whatever_a_tile_starts_with(rows, edges, biases):
+    """Tiles of 64 columns, items of 256 rows, and a sum's reference taken from a lane's
+    first columns: the lowest finite bias there, none at all, or one far below or above
+    what follows."""
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    tokens, tails = edges[-1], len(edges) - 2
+    hidden = torch.randn(rows, 512, device=DEV, generator=g).bfloat16()
+    weight = (torch.randn(tokens, 512, device=DEV, generator=g) * 0.05).bfloat16()
+    tail_weight = (torch.randn(tails, 512, device=DEV, generator=g) * 0.05).bfloat16()
+    tail_bias = torch.randn(tails, device=DEV, generator=g).bfloat16()
+    bias = torch.randn(tokens, device=DEV, generator=g)
+    at = torch.arange(tokens, device=DEV)
+    bias = {"plain": lambda: bias,
+            "lowest": lambda: torch.where(at % 64 < 40, -3.3e38, bias),
+            "infinite": lambda: torch.where(at // 64 % 3 == 0, -float("inf"), bias - 300),
+            "steps": lambda: bias + at // 64 % 7 * 70 - 400,
+            "peaks": lambda: bias + (at % 1000 == 999) * 5000.0}[biases]().bfloat16()
+    target = torch.randint(0, tokens, (rows,), device=DEV, generator=g)
+    args = (hidden, target, weight, bias, tail_weight, tail_bias, edges)
+    got, want = kernels.adaptive_nll(*args).double(), _losses_in_64_bits(*args)
+    plain = want.abs() < 1e30
+    # a bf16 result: half a unit in the last place, 2 ** -9, of a loss of one or more;
+    # below, sums of logits of some hundreds in fp32, 1e-3
+    assert bool(((got - want).abs() <= 2 ** -8 * want.abs().clamp(min=1.0))[plain].all())
+    rest = want[~plain].bfloat16().double()
+    assert bool(((got[~plain] == rest) | (got[~plain].isnan() & rest.isnan())).all())
