@@ -286,14 +286,18 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_nt_kernel(
   }
 }
 
-// Smaller tiles, for products whose 256 x 256 tiles would leave compute units
-// idle: mfma_tile.h's pipeline (four stages), GROUPS groups of four waves that take
-// every GROUPS-th k-tile (their sums meet in LDS).  Bound by the latency of a
-// k-tile's way to the MFMAs, 0.12 to 0.42 us by tile against 0.06 to 0.22 of matrix
-// core time.  Measured, before (256 x 256) and now, us:
-//   256 x 512 x 256      8.9 ->  3.6      3072 x 1024 x 1024   20.9 -> 10.5
-//   1024 x 1024 x 1024  20.7 ->  6.0      3072 x 1024 x 4096   65.6 -> 26.8
-//   512 x 512 x 8192     121 -> 17.5      2304 x 2304 x 2048   37.4 -> 31.6
+// Other tiles, for products that 256 x 256 tiles would spread badly over the compute units:
+// mfma_tile.h's pipeline (HALVES: the one by k-steps, where two k-tiles' fragments would
+// fill the registers), GROUPS groups of four waves that take every GROUPS-th k-tile (their
+// sums meet in LDS).  Tiles that do not divide 256 reach past the last row and column.
+// Small products are bound by the latency of a k-tile's way to the MFMAs, 0.12 to 0.34 us
+// by tile against 0.06 to 0.22 of matrix core time; those that fill the chip by its clock
+// (1.9 instead of 2.4 GHz) and by LDS.  Measured, by 256 x 256, by 128 x 128 and smaller
+// ones only, and now, us:
+//   256 x 512 x 256      8.9   3.6   3.6      2304 x 2304 x 2048  38.5  31.0  23.6
+//   1024 x 1024 x 1024  19.7   5.8   5.8      2560 x 2560 x 4096  68.0  56.6  49.3
+//   3072 x 1024 x 1024  20.1  10.2   9.2      2816 x 3328 x 1920  39.0  45.4  35.0
+//   3072 x 1024 x 4096  65.7  26.9  26.6      4864 x 1792 x 3072  55.9  69.3  53.1
 __device__ __forceinline__ void small_tile_of_block(int bid, int tiles_m, int tiles_n, int* tm,
                                                     int* tn) {
   // a contiguous range of tiles per XCD, bands of kGroupM tile rows
@@ -308,16 +312,20 @@ __device__ __forceinline__ void small_tile_of_block(int bid, int tiles_m, int ti
   *tn = in_band / rows;
 }
 
-template <int TM, int TN, int NS, int GROUPS, typename OutT>
+template <int TM, int TN, int NS, int GROUPS, bool HALVES, typename OutT>
 __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
     const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, OutT* __restrict__ C, int M,
     int N, int K) {
   using namespace mfma_tile;
+  constexpr int kI = TM / 32, kJ = TN / 32;
   constexpr int kGroupLds = NS * (Rows<TM>::kBytes + Rows<TN>::kBytes);
   constexpr int kSumLds = (GROUPS - 1) * TM * TN * 4;
   constexpr int kWaveRows = TM / 2, kWaveCols = TN / 2;
-  constexpr int kRowB = kWaveCols * (int)sizeof(OutT);
-  constexpr int kOutLds = 4 * kWaveRows * kRowB;
+  // rows of a wave's block on their way out, 16 bytes apart so that the sixteen rows that
+  // one instruction writes keep to banks of their own
+  constexpr int kRowB = kWaveCols * (int)sizeof(OutT), kRowLds = kRowB + 16;
+  constexpr int kPassI = kI < 3 ? kI : 3, kPassRows = kPassI * 16;
+  constexpr int kOutLds = 4 * kPassRows * kRowLds;
   constexpr int kLds = GROUPS * kGroupLds > kSumLds
                            ? (GROUPS * kGroupLds > kOutLds ? GROUPS * kGroupLds : kOutLds)
                            : (kSumLds > kOutLds ? kSumLds : kOutLds);
@@ -328,72 +336,90 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
   const int wm = wave >> 1, wn = wave & 1;
   const int l16 = lane & 15, lq = lane >> 4;
   int tm, tn;
-  small_tile_of_block(blockIdx.x, M / TM, N / TN, &tm, &tn);
-  const size_t row0 = (size_t)tm * TM, col0 = (size_t)tn * TN;
+  small_tile_of_block(blockIdx.x, (M + TM - 1) / TM, (N + TN - 1) / TN, &tm, &tn);
+  // a tile may reach past the last row or column, which it then reads again
+  const int row0 = tm * TM, col0 = tn * TN;
   Rows<TM> a;
   Rows<TN> b;
-  a.init(wave, lane, [&](int r) { return A + (row0 + r) * K + group * kTileK; });
-  b.init(wave, lane, [&](int r) { return B + (col0 + r) * K + group * kTileK; });
-  f32x4 acc[TM / 32][TN / 32];
+  a.init(wave, lane, [&](int r) {
+    return A + (size_t)(256 % TM == 0 || row0 + r < M ? row0 + r : M - 1) * K + group * kTileK;
+  });
+  b.init(wave, lane, [&](int r) {
+    return B + (size_t)(256 % TN == 0 || col0 + r < N ? col0 + r : N - 1) * K + group * kTileK;
+  });
+  f32x4 acc[kI][kJ];
   clear(acc);
-  stream_product<TM, TN, NS>(acc, lds + group * kGroupLds, K / (GROUPS * kTileK),
-                             GROUPS * kTileK, a, b, wm, wn, lane);
+  if constexpr (HALVES)
+    stream_product_halves<TM, TN, NS>(acc, lds, K / kTileK, a, b, wm, wn, lane);
+  else
+    stream_product<TM, TN, NS>(acc, lds + group * kGroupLds, K / (GROUPS * kTileK),
+                               GROUPS * kTileK, a, b, wm, wn, lane);
   block_sync();                        // the stages are free
   if (GROUPS > 1) {
     f32x4* other = reinterpret_cast<f32x4*>(lds) + wave * 64 + lane;
     if (group == 1) {
 #pragma unroll
-      for (int i = 0; i < TM / 32; ++i)
+      for (int i = 0; i < kI; ++i)
 #pragma unroll
-        for (int j = 0; j < TN / 32; ++j) other[(i * (TN / 32) + j) * 256] = acc[i][j];
+        for (int j = 0; j < kJ; ++j) other[(i * kJ + j) * 256] = acc[i][j];
     }
     block_sync();
     if (group == 0) {
 #pragma unroll
-      for (int i = 0; i < TM / 32; ++i)
+      for (int i = 0; i < kI; ++i)
 #pragma unroll
-        for (int j = 0; j < TN / 32; ++j) acc[i][j] += other[(i * (TN / 32) + j) * 256];
+        for (int j = 0; j < kJ; ++j) acc[i][j] += other[(i * kJ + j) * 256];
     }
     block_sync();
     if (group == 1) return;
   }
-  // whole rows of the wave's block leave as 16-byte pieces, as in the large kernel
-  constexpr int kSlots = kRowB / 16;
-  static_assert(kSlots <= 16, "the swizzle below takes a row's low four bits");
-  constexpr int kRowsPerStore = 64 / kSlots;
-  unsigned char* ep = lds + wave * kWaveRows * kRowB;
+  // whole rows of the wave's block leave as 16-byte pieces, three rows of fragments at a time
+  constexpr int kSlots = kRowB / 16, kPerSlot = 16 / (int)sizeof(OutT);
+  unsigned char* ep = lds + wave * kPassRows * kRowLds;
+  const int row_w = row0 + wm * kWaveRows, col_w = col0 + wn * kWaveCols;
 #pragma unroll
-  for (int i = 0; i < TM / 32; ++i)
+  for (int i0 = 0; i0 < kI; i0 += kPassI) {
+    constexpr int kAll = kPassRows * kSlots;
+    const int rows = (kI - i0 < kPassI ? kI - i0 : kPassI) * 16;
 #pragma unroll
-    for (int j = 0; j < TN / 32; ++j) {
-      const int byte = (j * 16 + lq * 4) * (int)sizeof(OutT);
-      store_quad(reinterpret_cast<OutT*>(ep + (i * 16 + l16) * kRowB +
-                                         (((byte >> 4) ^ (l16 & (kSlots - 1))) << 4) + (byte & 15)),
-                 acc[i][j]);
+    for (int i = i0; i < i0 + kPassI && i < kI; ++i)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j)
+        store_quad(reinterpret_cast<OutT*>(ep + ((i - i0) * 16 + l16) * kRowLds) + j * 16 + lq * 4,
+                   acc[i][j]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+#pragma unroll
+    for (int first = 0; first < kAll; first += 64) {
+      const int at = first + lane, R = at / kSlots, slot = at % kSlots;
+      if (first >= rows * kSlots) break;
+      if (kAll % 64 != 0 && R >= rows) continue;
+      const int row = row_w + i0 * 16 + R, col = col_w + slot * kPerSlot;
+      if ((256 % TM != 0 && row >= M) || (256 % TN != 0 && col >= N)) continue;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(ep + R * kRowLds + slot * 16);
+      *reinterpret_cast<u32x4*>(C + (size_t)row * N + col) = v;
     }
-  OutT* block = C + (row0 + wm * kWaveRows) * N + col0 + wn * kWaveCols;
-#pragma unroll
-  for (int it = 0; it < kWaveRows / kRowsPerStore; ++it) {
-    const int R = it * kRowsPerStore + lane / kSlots, slot = lane % kSlots;
-    const u32x4 v =
-        *reinterpret_cast<const u32x4*>(ep + R * kRowB + ((slot ^ (R & (kSlots - 1))) << 4));
-    *(reinterpret_cast<u32x4*>(block + (size_t)R * N) + slot) = v;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
   }
 }
 
-// What a launch of each tile takes, us: 1.5 + rounds of as many workgroups as the
-// stream has compute units * (fixed + per_tile * k-tiles), fitted to products from
-// 256 x 256 x 64 to 4096^3 on the whole GPU.  The fit is within 20 %; the large
-// tile's estimate counts 0.9 because a round of it keeps the whole chip busy where one
-// of the others waits (8192 x 2560 x 1024: 47 us by 256 x 256 tiles, 54 by 128 x 128,
-// both estimated at 46).
+// What a launch of each tile takes, us: 1.5 + rounds of as many workgroups as the stream
+// has compute units * (fixed + per_tile * k-tiles), fitted to 150 products drawn from
+// 256 x 256 x 64 to 8192 x 8192 x 8192 on the whole GPU (the last three to products that
+// they win).  The fit is within 20 %; the large tile's estimate counts 0.9 because a round
+// of it keeps the whole chip busy where one of the others waits (8192 x 2560 x 1024: 47 us
+// by 256 x 256 tiles, 54 by 128 x 128, both estimated at 46).  Over the drawn products the
+// choice takes 1 % longer than the best of these tiles each time would.
 struct TileCost {
   int tm, tn, k;          // k: what the depth has to be a multiple of
   double fixed, per_tile;
 };
 constexpr TileCost kTiles[] = {
-    {256, 256, 64, 4.0, 1.10},
-    {128, 128, 64, 2.0, 0.42},
+    {256, 256, 64, 4.65, 0.958},
+    {256, 128, 64, 3.44, 0.584},
+    {192, 224, 64, 6.25, 0.733},
+    {192, 128, 64, 3.92, 0.470},
+    {128, 128, 64, 2.80, 0.336},
+    {96, 128, 64, 2.96, 0.301},
     {128, 64, 64, 1.7, 0.28},
     {64, 64, 64, 1.5, 0.19},
     {32, 64, 128, 1.5, 0.125},   // two groups of waves
@@ -406,7 +432,7 @@ int tile_for(int M, int N, int K, int cus) {
   for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
     const TileCost& t = kTiles[i];
     if (K % t.k != 0) continue;
-    const long long blocks = (long long)(M / t.tm) * (N / t.tn);
+    const long long blocks = (long long)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
     const double us = 1.5 + (double)((blocks + cus - 1) / cus) * (t.fixed + t.per_tile * (K / BK));
     if (i == 0 || us < best_us) {
       best = i;
@@ -443,31 +469,29 @@ int tile_for_stream(int M, int N, int K, hipStream_t stream) {
   return cus == kWholeGpu ? tile : tile_for(M, N, K, cus);
 }
 
+template <int TM, int TN, int NS, int GROUPS, bool HALVES, typename OutT>
+void launch_tiles(const uint16_t* A, const uint16_t* B, OutT* C, int M, int N, int K,
+                  hipStream_t stream) {
+  const dim3 grid((unsigned)((M + TM - 1) / TM * ((N + TN - 1) / TN)));
+  hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<TM, TN, NS, GROUPS, HALVES, OutT>), grid,
+                     dim3(GROUPS * 256), 0, stream, A, B, C, M, N, K);
+}
+
 template <typename OutT>
 void launch_gemm(const uint16_t* A, const uint16_t* B, OutT* C, int M, int N, int K,
                  hipStream_t stream) {
-  const int tile = tile_for_stream(M, N, K, stream);
-  const dim3 grid((unsigned)((M / kTiles[tile].tm) * (N / kTiles[tile].tn)));
-  switch (tile) {
-    case 1:
-      hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<128, 128, 4, 1, OutT>), grid, dim3(256), 0,
-                         stream, A, B, C, M, N, K);
-      break;
-    case 2:
-      hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<128, 64, 4, 1, OutT>), grid, dim3(256), 0,
-                         stream, A, B, C, M, N, K);
-      break;
-    case 3:
-      hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<64, 64, 4, 1, OutT>), grid, dim3(256), 0,
-                         stream, A, B, C, M, N, K);
-      break;
-    case 4:
-      hipLaunchKernelGGL((gemm_bf16_nt_tile_kernel<32, 64, 4, 2, OutT>), grid, dim3(512), 0,
-                         stream, A, B, C, M, N, K);
-      break;
+  switch (tile_for_stream(M, N, K, stream)) {
+    case 1: return launch_tiles<256, 128, 3, 1, true>(A, B, C, M, N, K, stream);
+    case 2: return launch_tiles<192, 224, 3, 1, true>(A, B, C, M, N, K, stream);
+    case 3: return launch_tiles<192, 128, 4, 1, true>(A, B, C, M, N, K, stream);
+    case 4: return launch_tiles<128, 128, 4, 1, true>(A, B, C, M, N, K, stream);
+    case 5: return launch_tiles<96, 128, 4, 1, false>(A, B, C, M, N, K, stream);
+    case 6: return launch_tiles<128, 64, 4, 1, false>(A, B, C, M, N, K, stream);
+    case 7: return launch_tiles<64, 64, 4, 1, false>(A, B, C, M, N, K, stream);
+    case 8: return launch_tiles<32, 64, 4, 2, false>(A, B, C, M, N, K, stream);
     default:
-      hipLaunchKernelGGL(gemm_bf16_nt_kernel<OutT>, grid, dim3(kThreads), 0, stream, A, B, C, M,
-                         N, K);
+      hipLaunchKernelGGL(gemm_bf16_nt_kernel<OutT>, dim3((unsigned)((M / BM) * (N / BN))),
+                         dim3(kThreads), 0, stream, A, B, C, M, N, K);
   }
 }
 

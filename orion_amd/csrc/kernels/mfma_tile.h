@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #include <type_traits>
+#include <utility>
 
 namespace mfma_tile {
 
@@ -139,24 +140,35 @@ struct Fragments {
 // quarters: a wave that issues them in a row leaves its matrix core idle meanwhile
 // (128 x 128 tiles, 8192 deep, one workgroup a compute unit: 68 us; the loads alone
 // 40, everything else 49).
+// (Each product is a template of its own: loops of this size are not unrolled any more, and
+// operands picked at run time go through memory.)
+template <int BM, int BN, int kReads, int kLoads, typename Read, typename Load, int... kAt>
+__device__ __forceinline__ void multiply(f32x4 (&acc)[BM / 32][BN / 32],
+                                         const Fragments<BM, BN>& f, Read read, Load load,
+                                         std::integer_sequence<int, kAt...>) {
+  constexpr int kI = BM / 32, kJ = BN / 32, kM = 2 * kI * kJ;
+  constexpr int kSpan = kM * 3 / 4 > 0 ? kM * 3 / 4 : 1;
+  auto product = [&](auto at) {
+    constexpr int m = decltype(at)::value;
+    constexpr int ks = m / (kI * kJ), i = m / kJ % kI, j = m % kJ;
+    if constexpr (kI * kJ >= 4) mfma_in_place(f.b[ks][j], f.a[ks][i], acc[i][j]);
+    else acc[i][j] = mfma(f.b[ks][j], f.a[ks][i], acc[i][j]);
+    constexpr int kRead = (m * kReads + kSpan - 1) / kSpan;
+    constexpr int kReadEnd = ((m + 1) * kReads + kSpan - 1) / kSpan;
+#pragma unroll
+    for (int x = kRead; x < (kReadEnd < kReads ? kReadEnd : kReads); ++x) read(x);
+    constexpr int kLoad = (m * kLoads + kM - 1) / kM, kLoadEnd = ((m + 1) * kLoads + kM - 1) / kM;
+#pragma unroll
+    for (int x = kLoad; x < (kLoadEnd < kLoads ? kLoadEnd : kLoads); ++x) load(x);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  (product(std::integral_constant<int, kAt>{}), ...);
+}
 template <int BM, int BN, int kReads, int kLoads, typename Read, typename Load>
 __device__ __forceinline__ void multiply(f32x4 (&acc)[BM / 32][BN / 32],
                                          const Fragments<BM, BN>& f, Read read, Load load) {
-  constexpr int kI = BM / 32, kJ = BN / 32, kM = 2 * kI * kJ;
-  constexpr int kSpan = kM * 3 / 4 > 0 ? kM * 3 / 4 : 1;
-#pragma unroll
-  for (int m = 0; m < kM; ++m) {
-    const int ks = m / (kI * kJ), i = m / kJ % kI, j = m % kJ;
-    if (kI * kJ >= 4) mfma_in_place(f.b[ks][j], f.a[ks][i], acc[i][j]);
-    else acc[i][j] = mfma(f.b[ks][j], f.a[ks][i], acc[i][j]);
-#pragma unroll
-    for (int r = 0; r < kReads; ++r)
-      if (r * kSpan / (kReads ? kReads : 1) == m) read(r);
-#pragma unroll
-    for (int l = 0; l < kLoads; ++l)
-      if (l * kM / (kLoads ? kLoads : 1) == m) load(l);
-    __builtin_amdgcn_sched_barrier(0);
-  }
+  multiply<BM, BN, kReads, kLoads>(
+      acc, f, read, load, std::make_integer_sequence<int, 2 * (BM / 32) * (BN / 32)>{});
 }
 template <int BM, int BN>
 __device__ __forceinline__ void multiply(f32x4 (&acc)[BM / 32][BN / 32],
@@ -253,6 +265,109 @@ __device__ __forceinline__ void stream_product(f32x4 (&acc)[BM / 32][BN / 32],
   }
   settle(acc);
   multiply(acc, even);
+  settle(acc);
+}
+
+// The same for tiles whose fragments of two whole k-tiles do not fit the registers: two
+// sets of one k-step (half a k-tile) each.  While the first k-step is multiplied the second
+// is read; behind the barrier every wave has all of this tile in registers and the next
+// one has landed; while the second k-step is multiplied the next tile's first is read and
+// this one's stage is filled again.
+template <int BM, int BN>
+struct HalfFragments {
+  static constexpr int kI = BM / 32, kJ = BN / 32, kReads = kI + kJ;
+  bf16x8 a[kI], b[kJ];
+  // B first: every row of products needs all of it
+  template <int kStep>
+  __device__ __forceinline__ void read_one(int r, const unsigned char* ta, const unsigned char* tb,
+                                           int wm, int wn, int lane) {
+    const int l16 = lane & 15;
+    const int at = ((kStep * 4 + (lane >> 4)) ^ (l16 & 7)) << 4;
+    if (r < kJ)
+      b[r] = *reinterpret_cast<const bf16x8*>(tb + (wn * (BN / 2) + r * 16 + l16) * kRowBytes + at);
+    else
+      a[r - kJ] = *reinterpret_cast<const bf16x8*>(
+          ta + (wm * (BM / 2) + (r - kJ) * 16 + l16) * kRowBytes + at);
+  }
+};
+
+template <int BM, int BN, int kReads, int kLoads, typename Read, typename Load, int... kAt>
+__device__ __forceinline__ void multiply_half(f32x4 (&acc)[BM / 32][BN / 32],
+                                              const HalfFragments<BM, BN>& f, Read read, Load load,
+                                              std::integer_sequence<int, kAt...>) {
+  constexpr int kJ = BN / 32, kM = (BM / 32) * kJ, kSpan = kM * 3 / 4;
+  auto product = [&](auto at) {
+    constexpr int m = decltype(at)::value;
+    mfma_in_place(f.b[m % kJ], f.a[m / kJ], acc[m / kJ][m % kJ]);
+    constexpr int kRead = (m * kReads + kSpan - 1) / kSpan;
+    constexpr int kReadEnd = ((m + 1) * kReads + kSpan - 1) / kSpan;
+#pragma unroll
+    for (int x = kRead; x < (kReadEnd < kReads ? kReadEnd : kReads); ++x) read(x);
+    constexpr int kLoad = (m * kLoads + kM - 1) / kM, kLoadEnd = ((m + 1) * kLoads + kM - 1) / kM;
+#pragma unroll
+    for (int x = kLoad; x < (kLoadEnd < kLoads ? kLoadEnd : kLoads); ++x) load(x);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  (product(std::integral_constant<int, kAt>{}), ...);
+}
+
+template <int BM, int BN, int NS>
+__device__ __forceinline__ void stream_product_halves(f32x4 (&acc)[BM / 32][BN / 32],
+                                                      unsigned char* lds, int KT,
+                                                      const Rows<BM>& a, const Rows<BN>& b, int wm,
+                                                      int wn, int lane) {
+  constexpr int kStage = Rows<BM>::kBytes + Rows<BN>::kBytes;
+  constexpr int kLoads = Rows<BM>::kLoads + Rows<BN>::kLoads;
+  constexpr int kReads = HalfFragments<BM, BN>::kReads;
+  constexpr std::make_integer_sequence<int, (BM / 32) * (BN / 32)> kProducts{};
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    if (s < KT) {
+      a.issue(s * kTileK, lds + s * kStage);
+      b.issue(s * kTileK, lds + s * kStage + Rows<BM>::kBytes);
+    }
+  if (KT >= NS) wait_vm<kLoads*(NS - 1)>();
+  else wait_vm<0>();
+  block_sync();
+  HalfFragments<BM, BN> first, second;
+#pragma unroll
+  for (int r = 0; r < kReads; ++r)
+    first.template read_one<0>(r, lds, lds + Rows<BM>::kBytes, wm, wn, lane);
+  unsigned char* cur = lds;
+  // kMore: there is a tile to load into the freed stage; kNext: one to read from
+  auto step = [&](int kt, auto more, auto next) {
+    constexpr bool kMore = decltype(more)::value, kNext = decltype(next)::value;
+    multiply_half<BM, BN, kReads, 0>(
+        acc, first,
+        [&](int r) {
+          second.template read_one<1>(r, cur, cur + Rows<BM>::kBytes, wm, wn, lane);
+        },
+        [](int) {}, kProducts);
+    unsigned char* freed = cur;
+    if constexpr (kNext) {
+      if (kMore || KT - kt >= NS) wait_vm<kLoads*(NS - 2)>();
+      else wait_vm<0>();
+      block_sync();
+      cur = cur + kStage == lds + NS * kStage ? lds : cur + kStage;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    multiply_half<BM, BN, kNext ? kReads : 0, kMore ? kLoads : 0>(
+        acc, second,
+        [&](int r) {
+          first.template read_one<0>(r, cur, cur + Rows<BM>::kBytes, wm, wn, lane);
+        },
+        [&](int l) {
+          if (l < Rows<BM>::kLoads) a.issue_one(l, (kt + NS) * kTileK, freed);
+          else b.issue_one(l - Rows<BM>::kLoads, (kt + NS) * kTileK, freed + Rows<BM>::kBytes);
+        },
+        kProducts);
+  };
+  int kt = 0;
+  for (; kt + NS < KT; ++kt) step(kt, std::true_type{}, std::true_type{});
+  settle(acc);
+  for (; kt + 1 < KT; ++kt) step(kt, std::false_type{}, std::true_type{});
+  settle(acc);
+  step(kt, std::false_type{}, std::false_type{});
   settle(acc);
 }
 

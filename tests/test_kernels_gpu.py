@@ -225,3 +225,32 @@ def test_gemm_two_wave_groups_exact_on_small_integers(k):
     want = (ta.float() @ tb.float().t())
     for dtype in (torch.float32, torch.bfloat16):
         assert torch.equal(kernels.gemm_bf16_nt(ta, tb, out_dtype=dtype), want.to(dtype))
+
+
+@pytest.mark.parametrize("tile,shape,cus", [
+    ("256x128", (1280, 3328, 64), 0), ("256x128", (256, 2304, 128), 32),
+    ("256x128", (256, 2304, 192), 32), ("256x128", (256, 2304, 320), 32),
+    ("192x224", (2560, 7168, 1088), 0), ("192x224", (1280, 6656, 1856), 0),
+    ("192x128", (768, 768, 320), 32), ("192x128", (768, 768, 384), 32),
+    ("192x128", (1280, 3328, 576), 0),
+    ("128x128", (768, 2816, 64), 0), ("128x128", (256, 1280, 128), 32),
+    ("128x128", (256, 1280, 256), 32), ("128x128", (256, 1536, 320), 32),
+    ("96x128", (768, 2816, 320), 0), ("96x128", (256, 1280, 384), 32)])
+def test_gemm_tiles_past_the_edges_exact_on_small_integers(tile, shape, cus):
+    """Tiles that do not divide 256 and tiles by k-steps, at depths around their stages and
+    on as many compute units as make the rule take them; as above, every partial sum is
+    exact in fp32.  A row past the last one would land in the guard behind the result."""
+    m, n, k = shape
+    g = torch.Generator(device=DEV).manual_seed(sum(shape))
+    ta, tb = (torch.randint(-4, 5, (rows, k), device=DEV, generator=g).to(torch.bfloat16)
+              for rows in (m, n))
+    want = ta.float() @ tb.float().t()
+    stream = kernels.cu_masked_stream(cus) if cus else torch.cuda.current_stream()
+    for dtype in (torch.float32, torch.bfloat16):
+        guarded = torch.full((m + 256, n), 7.0, device=DEV, dtype=dtype)
+        out = guarded[:m]
+        torch.cuda.synchronize()
+        kernels.gemm_bf16_nt(ta, tb, out=out, stream=stream)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want.to(dtype))
+        assert bool((guarded[m:] == 7.0).all())
