@@ -685,12 +685,45 @@ constexpr int kAttnLds = kAttnShear + 8 * 16 * kShearRow * 4;
 constexpr int kMeetRow = 20;                   // floats a lane leaves at the end
 static_assert(8 * 64 * kMeetRow * 4 <= kAttnLds, "in place of the stage");
 
+// Weights of the launches that follow, read by workgroups of their own on compute units
+// that attention leaves idle, so that they come from the memory-side cache then: a
+// request's vocabulary has pushed them out since they were last used (a batch-4 request
+// takes 845 us so, 904 without; batch 1, 16 tokens 706 and 792).
+constexpr int kTouchBlocks = 32;
+struct Coming {
+  const uint16_t* p[4];
+  uint32_t bytes[4];                   // multiples of 16
+  uint32_t first_block;
+};
+__device__ __forceinline__ void touch(const Coming& coming) {
+  constexpr uint32_t kEach = kAttnThreads * 16, kUnroll = 4;
+  const uint32_t mine = (blockIdx.x - coming.first_block) * kEach + threadIdx.x * 16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const char* p = reinterpret_cast<const char*>(coming.p[i]);
+    for (uint32_t at = mine; at < coming.bytes[i]; at += kUnroll * kTouchBlocks * kEach) {
+      u32x4 v[kUnroll];
+#pragma unroll
+      for (uint32_t u = 0; u < kUnroll; ++u) {
+        const uint32_t to = at + u * kTouchBlocks * kEach;
+        v[u] = *reinterpret_cast<const u32x4*>(p + (to < coming.bytes[i] ? to : at));
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < kUnroll; ++u) asm volatile("" ::"v"(v[u]));
+    }
+  }
+}
+
 __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
     const uint16_t* __restrict__ qu, const uint16_t* __restrict__ qv,
     const uint16_t* __restrict__ kv_mem, const uint16_t* __restrict__ kv_x,
     const uint16_t* __restrict__ r, uint16_t* __restrict__ out, int qlen, int mlen, int batch,
-    int heads) {
+    int heads, Coming coming) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[kAttnLds];
+  if (blockIdx.x >= coming.first_block) {
+    touch(coming);
+    return;
+  }
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
@@ -1458,6 +1491,8 @@ bool dims_fit(const orion_txl_dims& d) {
          d.q_len <= 65535 * 64;
 }
 
+constexpr size_t kComputeUnits = 256;
+
 size_t tiles(size_t n, size_t tile) { return (n + tile - 1) / tile; }
 
 bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
@@ -1575,12 +1610,19 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
                          dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.qkv, rows,
                          qkv_map, norm, out, qkv);
     }
+    const size_t attn_blocks = d.heads * d.batch * tiles(d.q_len, kQ);
+    const bool idle = attn_blocks + kTouchBlocks <= kComputeUnits;
+    const uint32_t of_proj = (uint32_t)proj * kD * 2, of_inner = (uint32_t)d.inner * kD * 2;
+    const Coming coming = {
+        {(In)p.out, (In)p.ff1_w, (In)p.ff2_w, i + 1 < d.layers ? (In)layers[i + 1].qkv : (In)p.out},
+        {of_proj, of_inner, of_inner, i + 1 < d.layers ? 3 * of_proj : 0},
+        (uint32_t)attn_blocks};
     hipLaunchKernelGGL(txl_attention_kernel,
-                       dim3((unsigned)(d.heads * d.batch * tiles(d.q_len, kQ))),
+                       dim3((unsigned)(attn_blocks + (idle ? kTouchBlocks : 0))),
                        dim3(kAttnThreads), 0, s, (In)w.qu, (In)w.qv,
                        (In)(w.kv_mem + (size_t)i * mem_rows * 2 * proj), (In)w.kv_x,
                        (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
-                       d.heads);
+                       d.heads, coming);
     hipLaunchKernelGGL(txl_residual_gemm_kernel, dim3(res_map.blocks()), dim3(2 * kThreads), 0, s, (In)w.att,
                        (In)p.out, proj, (In) nullptr, x, w.y, w.parts, rows, res_map);
     const Norm norm = {(In)p.norm1_w, (In)p.norm1_b, w.parts, d.eps};
