@@ -296,7 +296,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_nt_kernel(
 // ones only, and now, us:
 //   256 x 512 x 256      8.9   3.6   3.6      2304 x 2304 x 2048  38.5  31.0  23.6
 //   1024 x 1024 x 1024  19.7   5.8   5.8      2560 x 2560 x 4096  68.0  56.6  49.3
-//   3072 x 1024 x 1024  20.1  10.2   9.2      2816 x 3328 x 1920  39.0  45.4  35.0
+//   3072 x 1024 x 1024  20.1  10.2   9.7      2816 x 3328 x 1920  39.0  45.4  35.0
 //   3072 x 1024 x 4096  65.7  26.9  26.6      4864 x 1792 x 3072  55.9  69.3  53.1
 __device__ __forceinline__ void small_tile_of_block(int bid, int tiles_m, int tiles_n, int* tm,
                                                     int* tn) {
@@ -405,7 +405,8 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
 // What a launch of each tile takes, us: 1.5 + rounds of as many workgroups as the stream
 // has compute units * (fixed + per_tile * k-tiles), fitted to 150 products drawn from
 // 256 x 256 x 64 to 8192 x 8192 x 8192 on the whole GPU (the last three to products that
-// they win).  The fit is within 20 %; the large tile's estimate counts 0.9 because a round
+// they win, 96 x 128 with operands out of the caches: 3072 x 1024, 16 k-tiles 11.2 us
+// against 10.1 by 128 x 128, 64 k-tiles 34.0 against 38.0).  The fit is within 20 %; the large tile's estimate counts 0.9 because a round
 // of it keeps the whole chip busy where one of the others waits (8192 x 2560 x 1024: 47 us
 // by 256 x 256 tiles, 54 by 128 x 128, both estimated at 46).  Over the drawn products the
 // choice takes 1 % longer than the best of these tiles each time would.
@@ -419,7 +420,7 @@ constexpr TileCost kTiles[] = {
     {192, 224, 64, 6.25, 0.733},
     {192, 128, 64, 3.92, 0.470},
     {128, 128, 64, 2.80, 0.336},
-    {96, 128, 64, 2.96, 0.301},
+    {96, 128, 64, 3.8, 0.305},
     {128, 64, 64, 1.7, 0.28},
     {64, 64, 64, 1.5, 0.19},
     {32, 64, 128, 1.5, 0.125},   // two groups of waves

@@ -235,7 +235,8 @@ def test_gemm_two_wave_groups_exact_on_small_integers(k):
     ("192x128", (1280, 3328, 576), 0),
     ("128x128", (768, 2816, 64), 0), ("128x128", (256, 1280, 128), 32),
     ("128x128", (256, 1280, 256), 32), ("128x128", (256, 1536, 320), 32),
-    ("96x128", (768, 2816, 320), 0), ("96x128", (256, 1280, 384), 32)])
+    ("96x128", (3072, 1024, 2560), 0), ("96x128", (256, 1280, 2112), 32),
+    ("96x128", (256, 1280, 2176), 32)])
 def test_gemm_tiles_past_the_edges_exact_on_small_integers(tile, shape, cus):
     """Tiles that do not divide 256 and tiles by k-steps, at depths around their stages and
     on as many compute units as make the rule take them; as above, every partial sum is
