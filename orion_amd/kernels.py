@@ -120,9 +120,16 @@ def _shutdown():
         _lib.unload(_lib.KERNELS_LIB)
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream_ptr(stream):
+    """The handle of ``stream``, or of the current device's current stream.  Callers hold
+    device tensors, so the runtime is up; a ``torch.cuda.Stream`` made only to be asked
+    for its handle costs more than half as much as the launch itself."""
     if stream is None:
-        stream = torch.cuda.current_stream()
+        return _raw_stream(_current_device())
     return stream.cuda_stream
 
 
@@ -134,15 +141,19 @@ def _check_device(*tensors):
             raise ValueError("orion_amd kernels take contiguous tensors only")
 
 
+_TENSOR_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
 def triad(a, b, c, s, grid_blocks=0, stream=None):
     """a = b + s * c (fp32, one FMA per element), in place into ``a``."""
     _check_device(a, b, c)
     if not (a.dtype == b.dtype == c.dtype == torch.float32):
         raise ValueError("triad is fp32")
-    if not (a.numel() == b.numel() == c.numel()):
+    n = a.numel()
+    if not n == b.numel() == c.numel():
         raise ValueError("triad operands differ in length")
     rc = lib().orion_triad_f32(a.data_ptr(), b.data_ptr(), c.data_ptr(),
-                               ctypes.c_float(s), a.numel(), grid_blocks,
+                               ctypes.c_float(s), n, grid_blocks,
                                _stream_ptr(stream))
     if rc != 0:
         raise KernelError("orion_triad_f32", rc)
@@ -159,7 +170,10 @@ def gemm_bf16_nt(a, b, out=None, out_dtype=torch.bfloat16, stream=None):
     m, k = a.shape
     n = b.shape[0]
     if out is None:
-        out = torch.empty((m, n), dtype=out_dtype, device=a.device)
+        # the same tensor either way; parsing a device takes as long as the kernel of a
+        # small product
+        out = (a.new_empty((m, n), dtype=out_dtype) if type(a) in _TENSOR_TYPES
+               else torch.empty((m, n), dtype=out_dtype, device=a.device))
         fits = True
     else:
         _check_device(out)
@@ -184,9 +198,6 @@ def plain_eager():
             and torch._C._len_torch_function_stack() == 0
             and not torch.jit.is_tracing()
             and not torch.compiler.is_compiling())
-
-
-_TENSOR_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 
 def plain_tensors(tensors, dtype, index):
