@@ -35,6 +35,7 @@
 
 #include "kernels.h"
 #include "mfma_tile.h"
+#include "stream_units.h"
 
 namespace {
 
@@ -296,8 +297,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_nt_kernel(
 // ones only, and now, us:
 //   256 x 512 x 256      8.9   3.6   3.6      2304 x 2304 x 2048  38.5  31.0  23.6
 //   1024 x 1024 x 1024  19.7   5.8   5.8      2560 x 2560 x 4096  68.0  56.6  49.3
-//   3072 x 1024 x 1024  20.1  10.2   9.7      2816 x 3328 x 1920  39.0  45.4  35.0
-//   3072 x 1024 x 4096  65.7  26.9  26.6      4864 x 1792 x 3072  55.9  69.3  53.1
+//   3072 x 1024 x 1024  20.1  10.2   9.7
+//   3072 x 1024 x 4096  65.7  26.9  26.6
 __device__ __forceinline__ void small_tile_of_block(int bid, int tiles_m, int tiles_n, int* tm,
                                                     int* tn) {
   // a contiguous range of tiles per XCD, bands of kGroupM tile rows
@@ -410,29 +411,29 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
 // of it keeps the whole chip busy where one of the others waits (8192 x 2560 x 1024: 47 us
 // by 256 x 256 tiles, 54 by 128 x 128, both estimated at 46).  Over the drawn products the
 // choice takes 1 % longer than the best of these tiles each time would.
+// On a stream limited to some compute units only the tiles that were measured there count.
 struct TileCost {
   int tm, tn, k;          // k: what the depth has to be a multiple of
+  bool limited;           // measured on limited streams too
   double fixed, per_tile;
 };
 constexpr TileCost kTiles[] = {
-    {256, 256, 64, 4.65, 0.958},
-    {256, 128, 64, 3.44, 0.584},
-    {192, 224, 64, 6.25, 0.733},
-    {192, 128, 64, 3.92, 0.470},
-    {128, 128, 64, 2.80, 0.336},
-    {96, 128, 64, 3.8, 0.305},
-    {128, 64, 64, 1.7, 0.28},
-    {64, 64, 64, 1.5, 0.19},
-    {32, 64, 128, 1.5, 0.125},   // two groups of waves
+    {256, 256, 64, true, 4.65, 0.958},
+    {256, 128, 64, false, 3.44, 0.584},
+    {192, 128, 64, false, 3.92, 0.470},
+    {128, 128, 64, true, 2.80, 0.336},
+    {96, 128, 64, false, 3.8, 0.305},
+    {128, 64, 64, true, 1.7, 0.28},
+    {64, 64, 64, true, 1.5, 0.19},
+    {32, 64, 128, true, 1.5, 0.125},   // two groups of waves
 };
-constexpr int kWholeGpu = 256;   // compute units
 
 int tile_for(int M, int N, int K, int cus) {
   int best = 0;
   double best_us = 0.0;
   for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
     const TileCost& t = kTiles[i];
-    if (K % t.k != 0) continue;
+    if (K % t.k != 0 || (cus != stream_units::kWholeGpu && !t.limited)) continue;
     const long long blocks = (long long)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
     const double us = 1.5 + (double)((blocks + cus - 1) / cus) * (t.fixed + t.per_tile * (K / BK));
     if (i == 0 || us < best_us) {
@@ -443,30 +444,15 @@ int tile_for(int M, int N, int K, int cus) {
   return best;
 }
 
-// Compute units that a stream may use; the whole GPU where that cannot be told.
-int compute_units_of(hipStream_t stream) {
-  uint32_t mask[16] = {0};
-  if (hipExtStreamGetCUMask(stream, 16, mask) != hipSuccess) {
-    (void)hipGetLastError();
-    return kWholeGpu;
-  }
-  int cus = 0;
-  for (uint32_t word : mask) cus += __builtin_popcount(word);
-  return cus > 0 && cus < kWholeGpu ? cus : kWholeGpu;
-}
-
 // The tile for a stream.  On some of the compute units the smaller tiles' workgroups
 // only take turns (64 of them, us by 256 x 256 and by the whole GPU's choice: 2048^3
 // 36.8 and 51.4; 1024 x 4096 x 512 13.7 and 23.5), so where the whole GPU's choice is
-// a smaller one the stream is asked for its mask (0.2 us) and the rounds are counted
-// with that.  The runtime's own streams (null, legacy, per thread) have none, and their
-// handles are constants that only launches are sure to take.
+// a smaller one the stream is asked for its mask and the rounds are counted with that.
 int tile_for_stream(int M, int N, int K, hipStream_t stream) {
+  using stream_units::kWholeGpu;
   const int tile = tile_for(M, N, K, kWholeGpu);
-  if (tile == 0 || stream == nullptr || stream == hipStreamLegacy ||
-      stream == hipStreamPerThread)
-    return tile;
-  const int cus = compute_units_of(stream);
+  if (tile == 0) return tile;
+  const int cus = stream_units::compute_units_of(stream);
   return cus == kWholeGpu ? tile : tile_for(M, N, K, cus);
 }
 
@@ -483,13 +469,12 @@ void launch_gemm(const uint16_t* A, const uint16_t* B, OutT* C, int M, int N, in
                  hipStream_t stream) {
   switch (tile_for_stream(M, N, K, stream)) {
     case 1: return launch_tiles<256, 128, 3, 1, true>(A, B, C, M, N, K, stream);
-    case 2: return launch_tiles<192, 224, 3, 1, true>(A, B, C, M, N, K, stream);
-    case 3: return launch_tiles<192, 128, 4, 1, true>(A, B, C, M, N, K, stream);
-    case 4: return launch_tiles<128, 128, 4, 1, true>(A, B, C, M, N, K, stream);
-    case 5: return launch_tiles<96, 128, 4, 1, false>(A, B, C, M, N, K, stream);
-    case 6: return launch_tiles<128, 64, 4, 1, false>(A, B, C, M, N, K, stream);
-    case 7: return launch_tiles<64, 64, 4, 1, false>(A, B, C, M, N, K, stream);
-    case 8: return launch_tiles<32, 64, 4, 2, false>(A, B, C, M, N, K, stream);
+    case 2: return launch_tiles<192, 128, 4, 1, true>(A, B, C, M, N, K, stream);
+    case 3: return launch_tiles<128, 128, 4, 1, true>(A, B, C, M, N, K, stream);
+    case 4: return launch_tiles<96, 128, 4, 1, false>(A, B, C, M, N, K, stream);
+    case 5: return launch_tiles<128, 64, 4, 1, false>(A, B, C, M, N, K, stream);
+    case 6: return launch_tiles<64, 64, 4, 1, false>(A, B, C, M, N, K, stream);
+    case 7: return launch_tiles<32, 64, 4, 2, false>(A, B, C, M, N, K, stream);
     default:
       hipLaunchKernelGGL(gemm_bf16_nt_kernel<OutT>, dim3((unsigned)((M / BM) * (N / BN))),
                          dim3(kThreads), 0, stream, A, B, C, M, N, K);

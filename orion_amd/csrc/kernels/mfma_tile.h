@@ -272,7 +272,9 @@ __device__ __forceinline__ void stream_product(f32x4 (&acc)[BM / 32][BN / 32],
 // sets of one k-step (half a k-tile) each.  While the first k-step is multiplied the second
 // is read; behind the barrier every wave has all of this tile in registers and the next
 // one has landed; while the second k-step is multiplied the next tile's first is read and
-// this one's stage is filled again.
+// this one's stage is filled again.  Bound as above, with LDS busy most of the time; by
+// 128 x 128 tiles 3072 x 1024 x 1024 takes 9.7 us so and 10.2 with whole k-tiles, 2560 x
+// 2560 x 4096 57.4 and 56.6.
 template <int BM, int BN>
 struct HalfFragments {
   static constexpr int kI = BM / 32, kJ = BN / 32, kReads = kI + kJ;

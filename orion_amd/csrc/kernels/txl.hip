@@ -36,6 +36,7 @@
 
 #include "kernels.h"
 #include "mfma_tile.h"
+#include "stream_units.h"
 
 namespace {
 
@@ -1491,8 +1492,6 @@ bool dims_fit(const orion_txl_dims& d) {
          d.q_len <= 65535 * 64;
 }
 
-constexpr size_t kComputeUnits = 256;
-
 size_t tiles(size_t n, size_t tile) { return (n + tile - 1) / tile; }
 
 bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
@@ -1589,6 +1588,7 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
   const int row_tiles = (int)tiles(rows, 64);
   const TileMap qkv_map(row_tiles, 3 * proj / 96, 1), ff_map(row_tiles, d.inner / 128, 1);
   const TileMap res_map((int)tiles(rows, kResM), kD / kResN, 64 / kResM);
+  const size_t units = stream_units::compute_units_of(s);
   for (int i = 0; i < d.layers; ++i) {
     const orion_txl_layer& p = layers[i];
     // x_i also goes into the memory's last rows
@@ -1611,7 +1611,7 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
                          qkv_map, norm, out, qkv);
     }
     const size_t attn_blocks = d.heads * d.batch * tiles(d.q_len, kQ);
-    const bool idle = attn_blocks + kTouchBlocks <= kComputeUnits;
+    const bool idle = attn_blocks + kTouchBlocks <= units;
     const uint32_t of_proj = (uint32_t)proj * kD * 2, of_inner = (uint32_t)d.inner * kD * 2;
     const Coming coming = {
         {(In)p.out, (In)p.ff1_w, (In)p.ff2_w, i + 1 < d.layers ? (In)layers[i + 1].qkv : (In)p.out},

@@ -227,31 +227,27 @@ def test_gemm_two_wave_groups_exact_on_small_integers(k):
         assert torch.equal(kernels.gemm_bf16_nt(ta, tb, out_dtype=dtype), want.to(dtype))
 
 
-@pytest.mark.parametrize("tile,shape,cus", [
-    ("256x128", (1280, 3328, 64), 0), ("256x128", (256, 2304, 128), 32),
-    ("256x128", (256, 2304, 192), 32), ("256x128", (256, 2304, 320), 32),
-    ("192x224", (2560, 7168, 1088), 0), ("192x224", (1280, 6656, 1856), 0),
-    ("192x128", (768, 768, 320), 32), ("192x128", (768, 768, 384), 32),
-    ("192x128", (1280, 3328, 576), 0),
-    ("128x128", (768, 2816, 64), 0), ("128x128", (256, 1280, 128), 32),
-    ("128x128", (256, 1280, 256), 32), ("128x128", (256, 1536, 320), 32),
-    ("96x128", (3072, 1024, 2560), 0), ("96x128", (256, 1280, 2112), 32),
-    ("96x128", (256, 1280, 2176), 32)])
-def test_gemm_tiles_past_the_edges_exact_on_small_integers(tile, shape, cus):
-    """Tiles that do not divide 256 and tiles by k-steps, at depths around their stages and
-    on as many compute units as make the rule take them; as above, every partial sum is
-    exact in fp32.  A row past the last one would land in the guard behind the result."""
+@pytest.mark.parametrize("tile,shape", [
+    ("256x128", (1280, 3328, 64)), ("256x128", (1280, 3328, 128)), ("256x128", (1280, 3328, 192)),
+    ("256x128", (1280, 3328, 256)), ("256x128", (1024, 5632, 576)),
+    ("192x128", (1280, 3328, 320)), ("192x128", (1280, 3328, 448)), ("192x128", (1280, 3328, 576)),
+    ("128x128", (768, 2816, 64)), ("128x128", (768, 2816, 128)), ("128x128", (768, 2816, 192)),
+    ("128x128", (768, 2816, 256)), ("128x128", (512, 5632, 320)),
+    ("96x128", (3072, 1024, 2560)), ("96x128", (3072, 1024, 2624))])
+def test_gemm_tiles_past_the_edges_exact_on_small_integers(tile, shape):
+    """Tiles that do not divide 256 and tiles by k-steps, at depths around their stages; as
+    above, every partial sum is exact in fp32.  A row past the last one would land in the
+    guard behind the result."""
     m, n, k = shape
     g = torch.Generator(device=DEV).manual_seed(sum(shape))
     ta, tb = (torch.randint(-4, 5, (rows, k), device=DEV, generator=g).to(torch.bfloat16)
               for rows in (m, n))
     want = ta.float() @ tb.float().t()
-    stream = kernels.cu_masked_stream(cus) if cus else torch.cuda.current_stream()
     for dtype in (torch.float32, torch.bfloat16):
         guarded = torch.full((m + 256, n), 7.0, device=DEV, dtype=dtype)
         out = guarded[:m]
         torch.cuda.synchronize()
-        kernels.gemm_bf16_nt(ta, tb, out=out, stream=stream)
+        kernels.gemm_bf16_nt(ta, tb, out=out)
         torch.cuda.synchronize()
         assert torch.equal(out, want.to(dtype))
         assert bool((guarded[m:] == 7.0).all())
