@@ -1043,13 +1043,17 @@ __global__ __launch_bounds__(kGroupThreads) void crit_group_kernel(Crit c) {
 // ahead and from one column tile straight on to the next.  Bound by the matrix cores: a
 // wave reads one fragment for four products (with 32 rows a wave, two, LDS reads alone
 // took as long as the products), a barrier stands between two k-tiles of sixty-four, and
-// the epilogue is six instructions an element: the accumulators start from the bias, and
-// the exponentials are taken against the lane's first tile's maximum, which is only
-// replaced when a sum gets out of hand.  A batch-4 request's logits
+// the epilogue is six instructions an element: the bias is one more product behind the
+// others (in front of them every partial sum would be rounded at its magnitude), and the
+// exponentials are taken against the lane's first tile's maximum, which is only replaced
+// when a sum gets out of hand.  A batch-4 request's logits
 // take 103 us, at 1.9 GHz and 72 % of what the matrix cores can issue; 155 with 128 rows
 // a workgroup, tiles of 128 columns one after the other and chunks of eight.
 __device__ __forceinline__ void mfma_by_kept(const bf16x8& a, const bf16x8& kept, f32x4& c) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(kept));
+}
+__device__ __forceinline__ void first_by_kept(const bf16x8& a, const bf16x8& kept, f32x4& c) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "a"(kept));
 }
 
 template <int I, int J>
@@ -1070,7 +1074,7 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
   constexpr int NS = kCritStages, kStage = Rows<kCritN>::kBytes, kLoads = Rows<kCritN>::kLoads;
   constexpr int kI = kCritWaveM / 16, kJ = kCritN / 16;
   static_assert(NS == 2 * kPanelTiles && kPanelTiles % 2 == 0, "the order of the loads");
-  static_assert((kCritMost + 1) * kCritN * 2 <= 4 * kCritWaveM * kRowBytes, "the biases' place");
+  static_assert(kCritMost * kCritN * 2 <= 4 * kCritWaveM * kRowBytes, "the biases' place");
   const int* list = k == 0 ? nullptr : c.rows + (size_t)(k - 1) * c.n;
   const int lo = c.edge[k] + chunk * width;                  // this chunk's tokens
   const int left = c.edge[k + 1] - lo;
@@ -1194,8 +1198,8 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
     ref[i] = kNone;
     sum[i] = 0.0f;
   }
-  // The bias is one more product, by a row of ones: only the first of a fragment's 32
-  // elements counts, lane group 0's first.
+  // The bias is a product by a row of ones: only the first of a fragment's 32 elements
+  // counts, lane group 0's first.
   const u32x4 one = {lq == 0 ? 0x3f80u : 0u, 0, 0, 0};
   const uint32_t first = lq == 0 ? 0xffffu : 0u;
   uint32_t bias[kJ];
@@ -1203,7 +1207,6 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
 #pragma unroll
     for (int j = 0; j < kJ; ++j) bias[j] = biases[tile * kCritN + j * 16 + l16];
   };
-  read_bias(0);
   float base[kI] = {0.0f, 0.0f, 0.0f, 0.0f};        // the reference, or 0 without one
   auto term = [&](float v, int i) { return __builtin_amdgcn_exp2f((v - base[i]) * kLog2e); };
   // a tile's exponentials `part` (a lane's own columns; lanes meet at the end) to the sums;
@@ -1237,19 +1240,6 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
     const Source after = source(t + 2);
     float part[kI] = {0.0f, 0.0f, 0.0f, 0.0f}, one_term = 0.0f;
     static_assert(kI == 4, "part and base");
-#pragma unroll
-    for (int j = 0; j < kJ; ++j) {
-      const u32x4 b = {bias[j] & first, 0, 0, 0};
-#pragma unroll
-      for (int i = 0; i < kI; ++i)
-        asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, 0"
-                     : "=v"(acc[i][j]) : "v"(b), "v"(one));
-    }
-    // by now the products before those have written the old tile
-#pragma unroll
-    for (int i = 0; i < kI; ++i)
-#pragma unroll
-      for (int j = 0; j < kJ; ++j) asm volatile("" : "+v"(old[i][j]));
     // k-tiles 2 * pair and the next.  Behind the barrier every wave has read the first of
     // them and the two after it have landed, so the stage before them and the first one's
     // are filled again; twelve k-tiles may be in flight.
@@ -1264,7 +1254,8 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
 #pragma unroll
         for (int m = 0; m < 2 * kI * kJ; ++m) {
           const int ks = m / (kI * kJ), i = m / kJ % kI, j = m % kJ;
-          mfma_by_kept(fb[h][ks * kJ + j], fa[i][kt * 2 + ks], acc[i][j]);
+          if (kt == 0 && ks == 0) first_by_kept(fb[h][j], fa[i][0], acc[i][j]);
+          else mfma_by_kept(fb[h][ks * kJ + j], fa[i][kt * 2 + ks], acc[i][j]);
           if (m % 3 == 1 && m / 3 < 2 * kJ) {       // the next k-tile's fragments
             const int stage = kt + 1 < kPanelTiles ? half + kt + 1 : kPanelTiles - half;
             if (h == 0) read_one(std::integral_constant<int, 1>{}, m / 3, stage);
@@ -1295,12 +1286,26 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
       }
     };
     step(std::integral_constant<int, 0>{});
-    read_bias(t + 1);
+    read_bias(t);
     step(std::integral_constant<int, 1>{});
     step(std::integral_constant<int, 2>{});
     step(std::integral_constant<int, 3>{});
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) {
+      const u32x4 b = {bias[j] & first, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < kI; ++i)
+        asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                     : "+v"(acc[i][j]) : "v"(b), "v"(one));
+    }
     next = after;
     take(old, part);
+    // written before anything reads them: their exponentials start behind the next product
+    asm volatile("s_nop 15" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < kI; ++i)
+#pragma unroll
+      for (int j = 0; j < kJ; ++j) asm volatile("" : "+v"(acc[i][j]));
   };
   auto last_tile = [&](f32x4 (&acc)[kI][kJ]) {
     settle_vector(acc);

@@ -289,3 +289,28 @@ def test_losses_whatever_a_tile_starts_with(rows, edges, biases):
     assert bool(((got - want).abs() <= 2 ** -8 * want.abs().clamp(min=1.0))[plain].all())
     rest = want[~plain].bfloat16().double()
     assert bool(((got[~plain] == rest) | (got[~plain].isnan() & rest.isnan())).all())
+
+
+@pytest.mark.parametrize("edges", [[0, 700], [0, 700, 2000]])
+def test_losses_are_rounded_at_the_biases_once(edges):
+    """Biases far above the logits' own sums and a target that takes nearly all: a loss
+    near zero is the difference of two sums at the biases' magnitude."""
+    g = torch.Generator(device=DEV).manual_seed(7)
+    rows, tokens, tails, level = 1024, edges[-1], len(edges) - 2, 16384.0
+    weight = (torch.randn(tokens, 512, device=DEV, generator=g) * 0.05).bfloat16()
+    target = torch.randint(0, tokens, (rows,), device=DEV, generator=g)
+    hidden = (0.3 * torch.randn(rows, 512, device=DEV, generator=g)
+              + 10 * weight[target].float()).bfloat16()
+    bias = torch.full((tokens,), level, device=DEV).bfloat16()
+    tail_weight = (torch.randn(tails, 512, device=DEV, generator=g) * 0.05).bfloat16()
+    tail_bias = torch.full((tails,), level, device=DEV).bfloat16()
+    args = (hidden, target, weight, bias, tail_weight, tail_bias, edges)
+    got, want = kernels.adaptive_nll(*args).double(), _losses_in_64_bits(*args)
+    # Logits lie between the level and twice it, where fp32 has steps of level / 2 ** 23.
+    # Half a step each: the logits under the sum of exponentials, that sum's logarithm with
+    # its reference, the target's own logit; a tail's target has the head's three too.  1e-4
+    # for products of 512 terms; the result is a bf16.
+    half = level * 2 ** -24
+    bound = torch.where(target < edges[1], 3.0, 6.0) * half + 1e-4 + 2 ** -8 * want
+    assert bool((want[target < edges[1]] < 0.1).any())
+    assert bool(((got - want).abs() <= bound).all())
