@@ -1038,8 +1038,8 @@ __global__ __launch_bounds__(kGroupThreads) void crit_group_kernel(Crit c) {
   plan.first_item[kMaxTails + 1] = items;
 }
 
-// Wave w owns rows 64 w .. + 63, whose 512 elements stay in registers (all 256 accumulator
-// ones), and all 64 columns of a tile; only the weights go through LDS, sixteen k-tiles
+// Wave w owns rows 64 w .. + 63 (or 32 w .. + 31 of an item of up to 128 rows), whose 512
+// elements stay in registers (all 256 accumulator ones), and all 64 columns of a tile; only the weights go through LDS, sixteen k-tiles
 // ahead and from one column tile straight on to the next.  Bound by the matrix cores: a
 // wave reads one fragment for four products (with 32 rows a wave, two, LDS reads alone
 // took as long as the products), a barrier stands between two k-tiles of sixty-four, and
@@ -1069,12 +1069,13 @@ __device__ __forceinline__ void settle_vector(f32x4 (&acc)[I][J]) {   // mfma_ti
     for (int j = 0; j < J; ++j) asm volatile("" : "+v"(acc[i][j]));
 }
 
+template <int kWaveM>
 __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int k, int chunk,
                                           int row0, int rows, int width) {
   constexpr int NS = kCritStages, kStage = Rows<kCritN>::kBytes, kLoads = Rows<kCritN>::kLoads;
-  constexpr int kI = kCritWaveM / 16, kJ = kCritN / 16;
+  constexpr int kI = kWaveM / 16, kJ = kCritN / 16, kM = 2 * kI * kJ;   // products a k-tile
   static_assert(NS == 2 * kPanelTiles && kPanelTiles % 2 == 0, "the order of the loads");
-  static_assert(kCritMost * kCritN * 2 <= 4 * kCritWaveM * kRowBytes, "the biases' place");
+  static_assert(kCritMost * kCritN * 2 <= 4 * kWaveM * kRowBytes, "the biases' place");
   const int* list = k == 0 ? nullptr : c.rows + (size_t)(k - 1) * c.n;
   const int lo = c.edge[k] + chunk * width;                  // this chunk's tokens
   const int left = c.edge[k + 1] - lo;
@@ -1117,20 +1118,20 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
   uint16_t bias_line[kBiasLoads];
 
   // The wave's rows, by whole lines, and through LDS into the fragments' order.
-  unsigned char* own = lds + NS * kStage + wave * kCritWaveM * kRowBytes;
+  unsigned char* own = lds + NS * kStage + wave * kWaveM * kRowBytes;
   bf16x8 fa[kI][2 * kPanelTiles];
   {
-    int from[kCritWaveM / 8];
+    int from[kWaveM / 8];
 #pragma unroll
-    for (int g = 0; g < kCritWaveM / 8; ++g) {
-      const int at = row0 + wave * kCritWaveM + g * 8 + (lane >> 3);
+    for (int g = 0; g < kWaveM / 8; ++g) {
+      const int at = row0 + wave * kWaveM + g * 8 + (lane >> 3);
       from[g] = at < rows ? at : rows - 1;
     }
     if (list) {
 #pragma unroll
-      for (int g = 0; g < kCritWaveM / 8; ++g) from[g] = list[from[g]];
+      for (int g = 0; g < kWaveM / 8; ++g) from[g] = list[from[g]];
     }
-    constexpr int kHalf = kPanelTiles / 2, kLines = kCritWaveM / 8;
+    constexpr int kHalf = kPanelTiles / 2, kLines = kWaveM / 8;
     u32x4 line[kHalf][kLines];                      // half of the k-tiles at a time
     auto load = [&](int kt, int g) {
       line[kt % kHalf][g] = *reinterpret_cast<const u32x4*>(
@@ -1193,10 +1194,11 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
   constexpr float kLog2e = 1.44269504088896340736f;
   const float kNone = -__builtin_inff();
   float ref[kI], sum[kI];
+  float base[kI];                                   // the reference, or 0 without one
 #pragma unroll
   for (int i = 0; i < kI; ++i) {
     ref[i] = kNone;
-    sum[i] = 0.0f;
+    sum[i] = base[i] = 0.0f;
   }
   // The bias is a product by a row of ones: only the first of a fragment's 32 elements
   // counts, lane group 0's first.
@@ -1207,7 +1209,6 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
 #pragma unroll
     for (int j = 0; j < kJ; ++j) bias[j] = biases[tile * kCritN + j * 16 + l16];
   };
-  float base[kI] = {0.0f, 0.0f, 0.0f, 0.0f};        // the reference, or 0 without one
   auto term = [&](float v, int i) { return __builtin_amdgcn_exp2f((v - base[i]) * kLog2e); };
   // a tile's exponentials `part` (a lane's own columns; lanes meet at the end) to the sums;
   // without a reference, or with one so far below that the sum might overflow, they are
@@ -1238,8 +1239,9 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
   auto tile = [&](int t, auto parity, f32x4 (&acc)[kI][kJ], f32x4 (&old)[kI][kJ]) {
     constexpr int half = decltype(parity)::value ? kPanelTiles : 0;   // this tile's first stage
     const Source after = source(t + 2);
-    float part[kI] = {0.0f, 0.0f, 0.0f, 0.0f}, one_term = 0.0f;
-    static_assert(kI == 4, "part and base");
+    float part[kI], one_term = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kI; ++i) part[i] = 0.0f;
     // k-tiles 2 * pair and the next.  Behind the barrier every wave has read the first of
     // them and the two after it have landed, so the stage before them and the first one's
     // are filled again; twelve k-tiles may be in flight.
@@ -1252,17 +1254,20 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
       for (int h = 0; h < 2; ++h) {
         const int kt = kFirst + h;
 #pragma unroll
-        for (int m = 0; m < 2 * kI * kJ; ++m) {
+        for (int m = 0; m < kM; ++m) {
           const int ks = m / (kI * kJ), i = m / kJ % kI, j = m % kJ;
           if (kt == 0 && ks == 0) first_by_kept(fb[h][j], fa[i][0], acc[i][j]);
           else mfma_by_kept(fb[h][ks * kJ + j], fa[i][kt * 2 + ks], acc[i][j]);
-          if (m % 3 == 1 && m / 3 < 2 * kJ) {       // the next k-tile's fragments
+          // the next k-tile's fragments, in the first three quarters
+          const bool reads = kI == 4 ? m % 3 == 1 : m % 3 != 1;
+          const int r = kI == 4 ? m / 3 : m - (m + 2) / 3;
+          if (reads && r < 2 * kJ) {
             const int stage = kt + 1 < kPanelTiles ? half + kt + 1 : kPanelTiles - half;
-            if (h == 0) read_one(std::integral_constant<int, 1>{}, m / 3, stage);
-            else read_one(std::integral_constant<int, 0>{}, m / 3, stage);
+            if (h == 0) read_one(std::integral_constant<int, 1>{}, r, stage);
+            else read_one(std::integral_constant<int, 0>{}, r, stage);
           }
-          if (h == 0 && m % 8 == 2) {
-            const int x = m / 8;                    // two loads for each stage
+          if (h == 0 && m % (kM / 4) == kI / 2) {
+            const int x = m / (kM / 4);             // two loads for each stage
             if (x < kLoads) {
               if (kFirst == 0) issue_one(next, x, kPanelTiles - 1, 2 * kPanelTiles - half - 1);
               else issue_one(after, x, kFirst - 1, half + kFirst - 1);
@@ -1272,7 +1277,7 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
           }
           // an element of the old tile every four products, one instruction behind each of
           // them: in a row they would wait for each other
-          const int at = kt * 2 * kI * kJ + m;
+          const int at = kt * kM + m;
           static_assert(kPanelTiles * 2 == 4 * 4, "four products an element");
           const int x = at / 4, oi = x / (kJ * 4);
           if (at % 4 == 0) one_term = old[oi][x / 4 % kJ][x % 4] - base[oi];
@@ -1351,7 +1356,7 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
       s = s * (m == t ? 1.0f : __expf(m - t)) + os * (om == t ? 1.0f : __expf(om - t));
       m = t;
     }
-    const int at = row0 + wave * kCritWaveM + i * 16 + l16;
+    const int at = row0 + wave * kWaveM + i * 16 + l16;
     if (lq == 0 && at < rows) c.pairs[k][(size_t)at * c.stride[k] + chunk] = make_float2(m, s);
   }
 }
@@ -1359,7 +1364,8 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
 __global__ __launch_bounds__(kThreads, 1) void crit_logits_kernel(Crit c) {
   // the stages, and 8 KiB for each wave's rows on their way to registers (one array: with
   // two the compiler waits for the loads in flight before every read)
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kCritStages * Rows<kCritN>::kBytes + 4 * kCritWaveM * kRowBytes];
+  constexpr int kLds = kCritStages * Rows<kCritN>::kBytes + 4 * kCritWaveM * kRowBytes;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kLds];
   auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   const CritPlan& plan = *c.plan;
   const int items = uniform(plan.first_item[kMaxTails + 1]);
@@ -1375,7 +1381,13 @@ __global__ __launch_bounds__(kThreads, 1) void crit_logits_kernel(Crit c) {
     const int chunk = group * 8 + in_group % abreast;
     const int row0 = in_group / abreast * kCritM;
     const int rows = k == 0 ? c.n : uniform(c.count[k - 1]);
-    crit_item(c, lds, k, chunk, row0, rows, width);
+    // Rows that fit 128 are multiplied by 32 a wave.  By 64, half of them for nothing, a
+    // request on a stream of few compute units waits for the products: 16 rows of the
+    // client's vocabulary on 32 units 402 us, so 244; 64 units 209 and 131, 256 units 76 and
+    // 57.  Rows that do not fit keep 64 a wave: by 32 their weights would come twice (256
+    // rows on 32 units 589 with items of 128, 387 so).
+    if (rows - row0 <= kCritM / 2) crit_item<kCritWaveM / 2>(c, lds, k, chunk, row0, rows, width);
+    else crit_item<kCritWaveM>(c, lds, k, chunk, row0, rows, width);
     block_sync();                      // the next item's loads land where this one's were read
   }
 }

@@ -314,3 +314,25 @@ def test_losses_are_rounded_at_the_biases_once(edges):
     bound = torch.where(target < edges[1], 3.0, 6.0) * half + 1e-4 + 2 ** -8 * want
     assert bool((want[target < edges[1]] < 0.1).any())
     assert bool(((got - want).abs() <= bound).all())
+
+
+def _some_losses(rows, edges, seed=0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    tokens, tails = edges[-1], len(edges) - 2
+    hidden = torch.randn(rows, 512, device=DEV, generator=g).bfloat16()
+    weight, tail_weight = ((torch.randn(n, 512, device=DEV, generator=g) * 0.05).bfloat16()
+                           for n in (tokens, tails))
+    bias, tail_bias = (torch.randn(n, device=DEV, generator=g).bfloat16()
+                       for n in (tokens, tails))
+    target = torch.randint(0, tokens, (rows,), device=DEV, generator=g)
+    return hidden, target, weight, bias, tail_weight, tail_bias, edges
+
+
+@pytest.mark.parametrize("rows", [31, 32, 33, 127, 128, 129, 256, 383, 384, 385])
+def test_losses_by_items_of_128_and_of_256_rows(rows):
+    """An item whose rows fit 128 keeps 32 of them a wave, any other 64."""
+    for edges in ([0, 130], [0, 65, 2000, 2100]):
+        args = _some_losses(rows, edges, rows)
+        got, want = kernels.adaptive_nll(*args).double(), _losses_in_64_bits(*args)
+        # a bf16 result and fp32 sums of logits of some units
+        assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + 1e-4).all())
