@@ -171,28 +171,24 @@ __device__ __forceinline__ void put_row(const RowsOut& out, int row, int chunk, 
     *reinterpret_cast<u32x4*>(out.mem + (size_t)(row - out.mem_from) * kD + chunk * 8) = v;
 }
 
-// Workgroup -> tile.  The eight XCDs, each with an L2 of its own, are given workgroups in
-// turn; every launch of a layer gives the same 64 rows (`unit` tiles) to the same XCD, all
-// of their columns, so that what a launch leaves is in the L2 of the one that reads it
-// next, and no XCD reads another's rows.  A request takes 897 us so and 931 with the
-// columns dealt out instead, where every XCD reads all rows; with every launch's own tiles
-// in turn (32 rows here, 64 there) 916 against 901.  Below eight units the rest of the
-// XCDs share the columns.  Tiles past the edges have nothing to do.
+// Workgroup -> tile of the layers' products.  The eight XCDs, each with an L2 of its own, are
+// given workgroups in turn; each takes an even, contiguous share of the tiles counted along
+// the rows' columns, so that every product of a layer gives (nearly) the same rows to the
+// same XCD, which then finds in its L2 what the one before left.  With the columns dealt
+// out instead, so that every XCD reads all rows, a batch-4 request took 4 % longer.  With
+// whole panels of 64 rows an XCD twelve panels left half of the XCDs half the work of the
+// others: 839 us, 814 so; on streams of 32 and 64 compute units 4709 and 2469, 3913 and
+// 2067 so.
 struct TileMap {
-  int tiles_m, tiles_n, unit, groups, cols, rows;
-  __host__ TileMap(int tiles_m, int tiles_n, int unit)
-      : tiles_m(tiles_m), tiles_n(tiles_n), unit(unit) {
-    const int units = (tiles_m + unit - 1) / unit;
-    groups = units >= 8 ? 8 : units >= 4 ? 4 : units >= 2 ? 2 : 1;
-    cols = (tiles_n + 8 / groups - 1) / (8 / groups);
-    rows = (units + groups - 1) / groups * unit;
-  }
-  __host__ unsigned blocks() const { return 8u * rows * cols; }
-  __device__ __forceinline__ bool tile(int block, int* tm, int* tn) const {
-    const int xcd = block % 8, row = block / 8 / cols;
-    *tm = (row / unit * groups + xcd % groups) * unit + row % unit;
-    *tn = xcd / groups + block / 8 % cols * (8 / groups);
-    return *tm < tiles_m && *tn < tiles_n;
+  unsigned tiles, tiles_n;
+  __host__ TileMap(size_t tiles_m, size_t tiles_n)
+      : tiles((unsigned)(tiles_m * tiles_n)), tiles_n((unsigned)tiles_n) {}
+  __host__ unsigned blocks() const { return tiles; }
+  __device__ __forceinline__ void tile(unsigned block, int* tm, int* tn) const {
+    const unsigned xcd = block % 8, extra = tiles % 8;
+    const unsigned at = xcd * (tiles / 8) + (xcd < extra ? xcd : extra) + block / 8;
+    *tm = at / tiles_n;
+    *tn = at % tiles_n;
   }
 };
 
@@ -389,7 +385,7 @@ __global__ __launch_bounds__(kPanelThreads, 1) void txl_ln_gemm_kernel(
     const void* A, const uint16_t* W, int M, TileMap map, Norm norm, RowsOut out, Epi epi) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[panel_lds<BM, BN>()];
   int tm, tn;
-  if (!map.tile(blockIdx.x, &tm, &tn)) return;
+  map.tile(blockIdx.x, &tm, &tn);
   panel_gemm<BM, BN, kNorm>(lds, A, W, M, tm, tn, map.tiles_n, norm, out, epi);
 }
 
@@ -568,7 +564,7 @@ __global__ __launch_bounds__(2 * kThreads, 1) void txl_residual_gemm_kernel(
   const int wave = wave8 & 3, group = wave8 >> 2;
   const int wm = wave >> 1, wn = wave & 1;
   int tm, tn;
-  if (!map.tile(blockIdx.x, &tm, &tn)) return;
+  map.tile(blockIdx.x, &tm, &tn);
   const int row0 = tm * kResM, col0 = tn * kResN;
   Rows<kResM> a;
   Rows<kResN> b;
@@ -1602,9 +1598,8 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
   }
   flush();
 
-  const int row_tiles = (int)tiles(rows, 64);
-  const TileMap qkv_map(row_tiles, 3 * proj / 96, 1), ff_map(row_tiles, d.inner / 128, 1);
-  const TileMap res_map((int)tiles(rows, kResM), kD / kResN, 64 / kResM);
+  const TileMap qkv_map(tiles(rows, 64), 3 * proj / 96), ff_map(tiles(rows, 64), d.inner / 128);
+  const TileMap res_map(tiles(rows, kResM), kD / kResN);
   const size_t units = stream_units::compute_units_of(s);
   for (int i = 0; i < d.layers; ++i) {
     const orion_txl_layer& p = layers[i];

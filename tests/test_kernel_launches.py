@@ -129,6 +129,40 @@ def test_no_launch_of_a_lamb_step_is_long(run, counts):
     assert sum(ratios) == sum(n > 0 for n in counts)
 
 
+TXL = """
+I = ctypes.c_int
+class Dims(ctypes.Structure):
+    _fields_ = [(n, I) for n in ("layers", "heads", "inner", "q_len", "m_len", "batch")] + [
+        ("eps", ctypes.c_float)]
+lib.orion_txl_workspace_bytes.argtypes = [P]
+lib.orion_txl_workspace_bytes.restype = Z
+lib.orion_txl_hidden.argtypes = [P] * 6 + [Z, P, Z, I, P, P, Z, P]
+out = []
+for layers, heads, inner, q_len, m_len, batch, cus in json.loads(sys.argv[3])[0]:
+    log.launch_log_set_compute_units(cus)
+    dims = Dims(layers, heads, inner, q_len, m_len, batch, 1e-5)
+    size = lib.orion_txl_workspace_bytes(ctypes.byref(dims))
+    stride = m_len * batch * 512
+    rc = lib.orion_txl_hidden(ctypes.byref(dims), (P * (11 * layers))(*[AT] * (11 * layers)),
+                              AT, AT, AT, AT, stride, None, 0, 0, AT, AT, size, AT)
+    out.append((rc, taken()))
+print(json.dumps(out))
+"""
+
+
+@pytest.mark.parametrize("q_len,batch", [(192, 4), (192, 2), (192, 1), (101, 3), (16, 1), (65, 7)])
+def test_no_workgroup_of_a_layers_products_is_empty(run, q_len, batch):
+    # the scheduler reads a launch's need of compute units from its number of workgroups
+    ((rc, launches),) = run(TXL, [(2, 8, 2048, q_len, 192, batch, 256)])
+    assert rc == 0
+    panels, halves = -(-q_len * batch // 64), -(-q_len * batch // 32)
+    grids = {part: {grid for name, grid, _ in launches if part in name}
+             for part in ("ln_gemm_kernelILi64ELi96E", "ln_gemm_kernelILi64ELi128E", "residual_gemm")}
+    assert grids == {"ln_gemm_kernelILi64ELi96E": {panels * 3 * 8 * 64 // 96},
+                     "ln_gemm_kernelILi64ELi128E": {panels * 2048 // 128},
+                     "residual_gemm": {halves * 512 // 64}}
+
+
 KERNELS = """
 print(json.dumps([log.launch_log_kernel(i).decode() for i in range(log.launch_log_kernels())]))
 """
