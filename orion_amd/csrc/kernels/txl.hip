@@ -36,7 +36,6 @@
 
 #include "kernels.h"
 #include "mfma_tile.h"
-#include "stream_units.h"
 
 namespace {
 
@@ -685,8 +684,16 @@ static_assert(8 * 64 * kMeetRow * 4 <= kAttnLds, "in place of the stage");
 // Weights of the launches that follow, read by workgroups of their own on compute units
 // that attention leaves idle, so that they come from the memory-side cache then: a
 // request's vocabulary has pushed them out since they were last used (a batch-4 request
-// takes 845 us so, 904 without; batch 1, 16 tokens 706 and 792).
-constexpr int kTouchBlocks = 32;
+// takes 801 us so, 866 without; batch 1, 16 tokens 630 and 689).  Each of these workgroups
+// reads 192 KiB, about what fits attention's time: 32 of them a layer of the client's, more
+// for wider ones while units are left (all of the weights by 32 workgroups took 830 us
+// instead of 728 at an inner width of 65536, 731 so).  How many follows attention's size
+// alone, not the compute units of the stream: they are the last of the grid, and on streams
+// of 32 to 128 units, where they wait for attention's own, requests take between 10 % less
+// and 0.1 % more time than without.  Beside a GEMM or a triad on another stream (16 pairs)
+// requests take 0 to 11 % less, in one pair 2 % more, and the other's rate changes by -2 to
+// +8 %.
+constexpr uint32_t kTouchBytes = 192 << 10, kUnits = 256;
 struct Coming {
   const uint16_t* p[4];
   uint32_t bytes[4];                   // multiples of 16
@@ -694,15 +701,16 @@ struct Coming {
 };
 __device__ __forceinline__ void touch(const Coming& coming) {
   constexpr uint32_t kEach = kAttnThreads * 16, kUnroll = 4;
+  const uint32_t step = (gridDim.x - coming.first_block) * kEach;
   const uint32_t mine = (blockIdx.x - coming.first_block) * kEach + threadIdx.x * 16;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const char* p = reinterpret_cast<const char*>(coming.p[i]);
-    for (uint32_t at = mine; at < coming.bytes[i]; at += kUnroll * kTouchBlocks * kEach) {
+    for (uint32_t at = mine; at < coming.bytes[i]; at += kUnroll * step) {
       u32x4 v[kUnroll];
 #pragma unroll
       for (uint32_t u = 0; u < kUnroll; ++u) {
-        const uint32_t to = at + u * kTouchBlocks * kEach;
+        const uint32_t to = at + u * step;
         v[u] = *reinterpret_cast<const u32x4*>(p + (to < coming.bytes[i] ? to : at));
       }
 #pragma unroll
@@ -1600,7 +1608,6 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
 
   const TileMap qkv_map(tiles(rows, 64), 3 * proj / 96), ff_map(tiles(rows, 64), d.inner / 128);
   const TileMap res_map(tiles(rows, kResM), kD / kResN);
-  const size_t units = stream_units::compute_units_of(s);
   for (int i = 0; i < d.layers; ++i) {
     const orion_txl_layer& p = layers[i];
     // x_i also goes into the memory's last rows
@@ -1623,14 +1630,22 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
                          qkv_map, norm, out, qkv);
     }
     const size_t attn_blocks = d.heads * d.batch * tiles(d.q_len, kQ);
-    const bool idle = attn_blocks + kTouchBlocks <= units;
-    const uint32_t of_proj = (uint32_t)proj * kD * 2, of_inner = (uint32_t)d.inner * kD * 2;
-    const Coming coming = {
-        {(In)p.out, (In)p.ff1_w, (In)p.ff2_w, i + 1 < d.layers ? (In)layers[i + 1].qkv : (In)p.out},
-        {of_proj, of_inner, of_inner, i + 1 < d.layers ? 3 * of_proj : 0},
-        (uint32_t)attn_blocks};
+    Coming coming = {{}, {}, (uint32_t)attn_blocks};
+    size_t left = attn_blocks < kUnits ? (kUnits - attn_blocks) * kTouchBytes : 0, ahead = 0;
+    int count = 0;
+    auto add_coming = [&](const void* weights, size_t rows) {
+      const size_t bytes = rows * kD * 2 < left ? rows * kD * 2 : left;
+      coming.p[count] = (In)weights;
+      coming.bytes[count++] = (uint32_t)bytes;
+      left -= bytes;
+      ahead += bytes;
+    };
+    add_coming(p.out, proj);
+    add_coming(p.ff1_w, d.inner);
+    add_coming(p.ff2_w, d.inner);
+    if (i + 1 < d.layers) add_coming(layers[i + 1].qkv, 3 * (size_t)proj);
     hipLaunchKernelGGL(txl_attention_kernel,
-                       dim3((unsigned)(attn_blocks + (idle ? kTouchBlocks : 0))),
+                       dim3((unsigned)(attn_blocks + tiles(ahead, kTouchBytes))),
                        dim3(kAttnThreads), 0, s, (In)w.qu, (In)w.qv,
                        (In)(w.kv_mem + (size_t)i * mem_rows * 2 * proj), (In)w.kv_x,
                        (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,

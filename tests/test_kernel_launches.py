@@ -145,7 +145,8 @@ for layers, heads, inner, q_len, m_len, batch, cus in json.loads(sys.argv[3])[0]
     stride = m_len * batch * 512
     rc = lib.orion_txl_hidden(ctypes.byref(dims), (P * (11 * layers))(*[AT] * (11 * layers)),
                               AT, AT, AT, AT, stride, None, 0, 0, AT, AT, size, AT)
-    out.append((rc, taken()))
+    queries = log.launch_log_queries()
+    out.append((rc, taken(), queries))
 print(json.dumps(out))
 """
 
@@ -153,7 +154,7 @@ print(json.dumps(out))
 @pytest.mark.parametrize("q_len,batch", [(192, 4), (192, 2), (192, 1), (101, 3), (16, 1), (65, 7)])
 def test_no_workgroup_of_a_layers_products_is_empty(run, q_len, batch):
     # the scheduler reads a launch's need of compute units from its number of workgroups
-    ((rc, launches),) = run(TXL, [(2, 8, 2048, q_len, 192, batch, 256)])
+    ((rc, launches, _),) = run(TXL, [(2, 8, 2048, q_len, 192, batch, 256)])
     assert rc == 0
     panels, halves = -(-q_len * batch // 64), -(-q_len * batch // 32)
     grids = {part: {grid for name, grid, _ in launches if part in name}
@@ -161,6 +162,22 @@ def test_no_workgroup_of_a_layers_products_is_empty(run, q_len, batch):
     assert grids == {"ln_gemm_kernelILi64ELi96E": {panels * 3 * 8 * 64 // 96},
                      "ln_gemm_kernelILi64ELi128E": {panels * 2048 // 128},
                      "residual_gemm": {halves * 512 // 64}}
+
+
+@pytest.mark.parametrize("inner,q_len,batch,own,ahead", [
+    # 192 KiB of the coming weights a workgroup: 6 MiB of a layer, 4.5 of the last
+    (2048, 192, 4, 192, [32, 24]), (2048, 16, 1, 8, [32, 24]),
+    # as many as attention leaves of 256 compute units
+    (2048, 192, 5, 240, [16, 16]), (2048, 128, 8, 256, [0, 0]), (2048, 192, 8, 384, [0, 0]),
+    (65536, 192, 4, 192, [64, 64]), (65536, 16, 1, 8, [248, 248])])
+def test_weights_read_ahead_follow_attentions_size_on_any_stream(run, inner, q_len, batch, own,
+                                                                 ahead):
+    # a launch may be issued to another stream than the call names, so that one is not asked
+    for rc, launches, queries in run(TXL, [(2, 8, inner, q_len, 192, batch, cus)
+                                           for cus in (32, 64, 128, 256)]):
+        assert rc == 0 and queries == 0
+        assert [grid for name, grid, _ in launches if "attention" in name] == [
+            own + more for more in ahead]
 
 
 KERNELS = """
