@@ -680,6 +680,7 @@ constexpr int kAttnShear = kAttnV + kHead * kVtRow;
 constexpr int kAttnLds = kAttnShear + 8 * 16 * kShearRow * 4;
 constexpr int kMeetRow = 20;                   // floats a lane leaves at the end
 static_assert(8 * 64 * kMeetRow * 4 <= kAttnLds, "in place of the stage");
+constexpr size_t kAttnMost = (1u << 23) - 1024;   // workgroups: a grid has less than 2^32 threads
 
 // Weights of the launches that follow, read by workgroups of their own on compute units
 // that attention leaves idle, so that they come from the memory-side cache then: a
@@ -697,7 +698,7 @@ constexpr uint32_t kTouchBytes = 192 << 10, kUnits = 256;
 struct Coming {
   const uint16_t* p[4];
   uint32_t bytes[4];                   // multiples of 16
-  uint32_t first_block;
+  uint32_t first_block;                // of the launch
 };
 __device__ __forceinline__ void touch(const Coming& coming) {
   constexpr uint32_t kEach = kAttnThreads * 16, kUnroll = 4;
@@ -723,7 +724,7 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
     const uint16_t* __restrict__ qu, const uint16_t* __restrict__ qv,
     const uint16_t* __restrict__ kv_mem, const uint16_t* __restrict__ kv_x,
     const uint16_t* __restrict__ r, uint16_t* __restrict__ out, int qlen, int mlen, int batch,
-    int heads, Coming coming) {
+    int heads, uint32_t first, Coming coming) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[kAttnLds];
   if (blockIdx.x >= coming.first_block) {
     touch(coming);
@@ -732,8 +733,9 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
-  const int head = blockIdx.x % heads, b = blockIdx.x / heads % batch;
-  const int q0 = blockIdx.x / heads / batch * kQ;
+  const uint32_t block = first + blockIdx.x;
+  const int head = block % heads, b = block / heads % batch;
+  const int q0 = block / heads / batch * kQ;
   const int klen = mlen + qlen;
   const int proj = heads * kHead;
   const int qt = wave & 1, part = wave >> 1;
@@ -1506,11 +1508,13 @@ Buffers buffers_of(const orion_txl_dims& d, void* base) {
   return b;
 }
 
+constexpr int kMostQueries = 65535 * 64;         // longer segments keep the operations
+
 bool dims_fit(const orion_txl_dims& d) {
   return d.q_len > 0 && d.m_len >= 0 && d.batch > 0 && d.layers > 0 && d.heads > 0 &&
          d.heads % 2 == 0 && d.heads <= 1024 && d.inner > 0 && d.inner % 128 == 0 &&
          d.inner <= (1 << 20) && ((int64_t)d.q_len + d.m_len) * d.batch < (1 << 24) &&
-         d.q_len <= 65535 * 64;
+         d.q_len <= kMostQueries;
 }
 
 size_t tiles(size_t n, size_t tile) { return (n + tile - 1) / tile; }
@@ -1629,8 +1633,8 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
                          dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.qkv, rows,
                          qkv_map, norm, out, qkv);
     }
-    const size_t attn_blocks = d.heads * d.batch * tiles(d.q_len, kQ);
-    Coming coming = {{}, {}, (uint32_t)attn_blocks};
+    const size_t attn_blocks = (size_t)d.heads * d.batch * tiles(d.q_len, kQ);
+    Coming coming = {};
     size_t left = attn_blocks < kUnits ? (kUnits - attn_blocks) * kTouchBytes : 0, ahead = 0;
     int count = 0;
     auto add_coming = [&](const void* weights, size_t rows) {
@@ -1644,12 +1648,16 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
     add_coming(p.ff1_w, d.inner);
     add_coming(p.ff2_w, d.inner);
     if (i + 1 < d.layers) add_coming(layers[i + 1].qkv, 3 * (size_t)proj);
-    hipLaunchKernelGGL(txl_attention_kernel,
-                       dim3((unsigned)(attn_blocks + tiles(ahead, kTouchBytes))),
-                       dim3(kAttnThreads), 0, s, (In)w.qu, (In)w.qv,
-                       (In)(w.kv_mem + (size_t)i * mem_rows * 2 * proj), (In)w.kv_x,
-                       (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
-                       d.heads, coming);
+    for (size_t first = 0; first < attn_blocks; first += kAttnMost) {
+      const size_t own = attn_blocks - first < kAttnMost ? attn_blocks - first : kAttnMost;
+      coming.first_block = (uint32_t)own;
+      hipLaunchKernelGGL(txl_attention_kernel,
+                         dim3((unsigned)(own + tiles(ahead, kTouchBytes))), dim3(kAttnThreads), 0,
+                         s, (In)w.qu, (In)w.qv,
+                         (In)(w.kv_mem + (size_t)i * mem_rows * 2 * proj), (In)w.kv_x,
+                         (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
+                         d.heads, (uint32_t)first, coming);
+    }
     hipLaunchKernelGGL(txl_residual_gemm_kernel, dim3(res_map.blocks()), dim3(2 * kThreads), 0, s, (In)w.att,
                        (In)p.out, proj, (In) nullptr, x, w.y, w.parts, rows, res_map);
     const Norm norm = {(In)p.norm1_w, (In)p.norm1_b, w.parts, d.eps};

@@ -180,6 +180,15 @@ def test_weights_read_ahead_follow_attentions_size_on_any_stream(run, inner, q_l
             own + more for more in ahead]
 
 
+def test_no_launch_of_attention_has_more_threads_than_a_grid_can_have(run):
+    # many short segments: 2 blocks of queries for each of 6.4 million heads
+    ((rc, launches, _),) = run(TXL, [(1, 32, 256, 33, 0, 200_000, 256)])
+    assert rc == 0
+    attention = [(grid, block) for name, grid, block in launches if "attention" in name]
+    assert sum(grid for grid, _ in attention) == 32 * 200_000 * 2
+    assert all(grid * block < 1 << 32 for grid, block in attention)
+
+
 KERNELS = """
 print(json.dumps([log.launch_log_kernel(i).decode() for i in range(log.launch_log_kernels())]))
 """
