@@ -411,21 +411,29 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
 // of it keeps the whole chip busy where one of the others waits (8192 x 2560 x 1024: 47 us
 // by 256 x 256 tiles, 54 by 128 x 128, both estimated at 46).  Over the drawn products the
 // choice takes 1 % longer than the best of these tiles each time would.
-// On a stream limited to some compute units only the tiles that were measured there count.
-struct TileCost {
-  int tm, tn, k;          // k: what the depth has to be a multiple of
-  bool limited;           // measured on limited streams too
+// Streams limited to some compute units have costs of their own, and only the tiles that
+// were measured there.  With the whole GPU's, 3 % of the products drawn for 32, 64 and 128
+// units went from 128 x 128 to 256 x 256, which takes longer (us, these and the whole GPU's
+// choice: 768 x 2816 x 384 on 128 units 9.9 and 11.2, 6656 x 256 x 448 on 64 units 10.4 and
+// 11.9, 256 x 2816 x 256 on 32 units 8.2 and 9.1; 5 to 18 % at 16 such products, with
+// operands in the caches and out of them).
+struct Cost {
   double fixed, per_tile;
 };
+struct TileCost {
+  int tm, tn, k;          // k: what the depth has to be a multiple of
+  Cost whole, limited;
+};
+constexpr Cost kUnmeasured = {0.0, 0.0};
 constexpr TileCost kTiles[] = {
-    {256, 256, 64, true, 4.65, 0.958},
-    {256, 128, 64, false, 3.44, 0.584},
-    {192, 128, 64, false, 3.92, 0.470},
-    {128, 128, 64, true, 2.80, 0.336},
-    {96, 128, 64, false, 3.8, 0.305},
-    {128, 64, 64, true, 1.7, 0.28},
-    {64, 64, 64, true, 1.5, 0.19},
-    {32, 64, 128, true, 1.5, 0.125},   // two groups of waves
+    {256, 256, 64, {4.65, 0.958}, {4.0, 1.10}},
+    {256, 128, 64, {3.44, 0.584}, kUnmeasured},
+    {192, 128, 64, {3.92, 0.470}, kUnmeasured},
+    {128, 128, 64, {2.80, 0.336}, {2.0, 0.42}},
+    {96, 128, 64, {3.8, 0.305}, kUnmeasured},
+    {128, 64, 64, {1.7, 0.28}, {1.7, 0.28}},
+    {64, 64, 64, {1.5, 0.19}, {1.5, 0.19}},
+    {32, 64, 128, {1.5, 0.125}, {1.5, 0.125}},   // two groups of waves
 };
 
 int tile_for(int M, int N, int K, int cus) {
@@ -433,9 +441,10 @@ int tile_for(int M, int N, int K, int cus) {
   double best_us = 0.0;
   for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
     const TileCost& t = kTiles[i];
-    if (K % t.k != 0 || (cus != stream_units::kWholeGpu && !t.limited)) continue;
+    const Cost& c = cus == stream_units::kWholeGpu ? t.whole : t.limited;
+    if (K % t.k != 0 || c.per_tile == 0.0) continue;
     const long long blocks = (long long)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
-    const double us = 1.5 + (double)((blocks + cus - 1) / cus) * (t.fixed + t.per_tile * (K / BK));
+    const double us = 1.5 + (double)((blocks + cus - 1) / cus) * (c.fixed + c.per_tile * (K / BK));
     if (i == 0 || us < best_us) {
       best = i;
       best_us = i == 0 ? 0.9 * us : us;
