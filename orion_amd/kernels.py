@@ -170,9 +170,10 @@ def gemm_bf16_nt(a, b, out=None, out_dtype=torch.bfloat16, stream=None):
     m, k = a.shape
     n = b.shape[0]
     if out is None:
-        # the same tensor either way; parsing a device takes as long as the kernel of a
-        # small product
-        out = (a.new_empty((m, n), dtype=out_dtype) if type(a) in _TENSOR_TYPES
+        # the same tensor either way (``new_empty`` refuses named dimensions); parsing a
+        # device takes as long as the kernel of a small product
+        out = (a.new_empty((m, n), dtype=out_dtype)
+               if type(a) in _TENSOR_TYPES and not a.has_names()
                else torch.empty((m, n), dtype=out_dtype, device=a.device))
         fits = True
     else:

@@ -251,3 +251,12 @@ def test_gemm_tiles_past_the_edges_exact_on_small_integers(tile, shape):
         torch.cuda.synchronize()
         assert torch.equal(out, want.to(dtype))
         assert bool((guarded[m:] == 7.0).all())
+
+
+@pytest.mark.filterwarnings("ignore:Named tensors")
+def test_gemm_takes_tensors_with_named_dimensions():
+    g = torch.Generator(device=DEV).manual_seed(2)
+    ta, tb = (torch.randint(-4, 5, (256, 128), device=DEV, generator=g).to(torch.bfloat16)
+              for _ in range(2))
+    want = kernels.gemm_bf16_nt(ta, tb)
+    assert torch.equal(kernels.gemm_bf16_nt(ta.rename("m", "k"), tb.rename("n", "k")), want)
