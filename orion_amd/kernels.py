@@ -128,9 +128,11 @@ def _stream_ptr(stream):
     """The handle of ``stream``, or of the current device's current stream.  Callers hold
     device tensors, so the runtime is up; a ``torch.cuda.Stream`` made only to be asked
     for its handle costs more than half as much as the launch itself."""
-    if stream is None:
-        return _raw_stream(_current_device())
-    return stream.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    if _raw_stream is None or _current_device is None:     # private: not in every torch
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def _check_device(*tensors):

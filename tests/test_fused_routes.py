@@ -110,3 +110,13 @@ def test_lazily_negated_tensors_keep_the_operations():
     assert negated.is_neg() and negated.is_contiguous() and type(negated) is torch.Tensor
     assert kernels.plain_tensors([ok, ok], torch.float32, ok.get_device())
     assert not kernels.plain_tensors([ok, negated], torch.float32, ok.get_device())
+
+
+@pytest.mark.parametrize("missing", ["_raw_stream", "_current_device"])
+def test_the_current_streams_handle_without_torchs_private_queries(monkeypatch, missing):
+    monkeypatch.setattr(kernels, "_raw_stream", lambda device: 100 + device)
+    monkeypatch.setattr(kernels, "_current_device", lambda: 3)
+    assert kernels._stream_ptr(None) == 103
+    monkeypatch.setattr(kernels, missing, None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"cuda_stream": 7}))
+    assert kernels._stream_ptr(None) == 7
