@@ -87,6 +87,17 @@ def test_gemm_tiles_follow_the_streams_compute_units(run):
     assert not bad
 
 
+def test_gemm_edge_cases_run_on_the_tiles_that_they_name(run):
+    from tests.test_kernels_gpu import EDGE_TILES
+    got = run(GEMM, [(*shape, 256, True) for _, shape in EDGE_TILES])
+    for (tile, (m, n, k)), (rc, launches, _) in zip(EDGE_TILES, got):
+        rows, cols = map(int, tile.split("x"))
+        ((name, grid, _),) = launches
+        assert rc == 0 and f"tile_kernelILi{rows}ELi{cols}E" in name, (tile, m, n, k, name)
+        assert grid == -(-m // rows) * (n // cols)
+    assert {m % 96 for tile, (m, _, _) in EDGE_TILES if tile == "96x128"} == {0, 32, 64}
+
+
 def test_gemm_on_limited_streams_by_costs_measured_there(run):
     # 128 x 128 tiles 5 to 18 % faster than the 256 x 256 that the whole GPU's costs ask for
     cases = [(768, 2816, 384, 128, 132), (2048, 1792, 448, 128, 224), (512, 4352, 448, 128, 136),

@@ -227,13 +227,21 @@ def test_gemm_two_wave_groups_exact_on_small_integers(k):
         assert torch.equal(kernels.gemm_bf16_nt(ta, tb, out_dtype=dtype), want.to(dtype))
 
 
-@pytest.mark.parametrize("tile,shape", [
+# Depths around the stages of the tiles by k-steps, and partial last tiles of those that do
+# not divide 256; test_kernel_launches.py holds each shape to its tile.
+EDGE_TILES = [
     ("256x128", (1280, 3328, 64)), ("256x128", (1280, 3328, 128)), ("256x128", (1280, 3328, 192)),
     ("256x128", (1280, 3328, 256)), ("256x128", (1024, 5632, 576)),
     ("192x128", (1280, 3328, 320)), ("192x128", (1280, 3328, 448)), ("192x128", (1280, 3328, 576)),
     ("128x128", (768, 2816, 64)), ("128x128", (768, 2816, 128)), ("128x128", (768, 2816, 192)),
     ("128x128", (768, 2816, 256)), ("128x128", (512, 5632, 320)),
-    ("96x128", (3072, 1024, 2560)), ("96x128", (3072, 1024, 2624))])
+    ("96x128", (3072, 1024, 2560)), ("96x128", (3072, 1024, 2624)),
+    # 32 and 64 of the last tile's 96 rows
+    ("96x128", (512, 4352, 2112)), ("96x128", (1280, 1792, 2176)), ("96x128", (1024, 2304, 2176)),
+    ("96x128", (2560, 1024, 2240))]
+
+
+@pytest.mark.parametrize("tile,shape", EDGE_TILES)
 def test_gemm_tiles_past_the_edges_exact_on_small_integers(tile, shape):
     """Tiles that do not divide 256 and tiles by k-steps, at depths around their stages; as
     above, every partial sum is exact in fp32.  A row past the last one would land in the

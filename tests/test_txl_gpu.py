@@ -1,5 +1,5 @@
 """The Transformer-XL kernels against the model's own operations: both against the
-same model in 64 bits, at the edges of the attention's 64-query and 128-key blocks,
+same model in 64 bits, at the edges of the attention's 32-query and 128-key blocks,
 of the products' row tiles and of the vocabulary's column tiles."""
 
 import pytest
@@ -203,9 +203,9 @@ def test_client_widths_no_further_from_64_bits_than_the_operations(n_head, d_inn
 
 
 def test_losses_over_clusters_of_many_chunks():
-    # a workgroup takes 1024 columns: a head of three chunks with a ragged last one, a tail
-    # of one token, one of exactly a chunk, one of 66 chunks (more than a wave joins at a
-    # time) whose last holds one token; rows of each tail past one tile of 128
+    # With this many rows an item takes a chunk of 640 columns: a head of five chunks with a
+    # ragged last one, a tail of one token, one of two chunks, one of 105 chunks (more than a
+    # wave joins at a time) whose last holds one token; rows of each tail past one item's 256.
     tails = [2900, 2901, 3925]
     n_token = 3925 + 65 * 1024 + 1
     g = torch.Generator(device=DEV).manual_seed(5)
@@ -214,7 +214,7 @@ def test_losses_over_clusters_of_many_chunks():
         # logits of some +-30, so that the chunks' maxima differ
         p.data.normal_(0.0, 0.3 if p.dim() == 2 else 1.0, generator=g)
     crit = crit.to(torch.bfloat16)
-    rows = 700
+    rows = 1200
     hidden = torch.randn(rows, 512, device=DEV, generator=g).to(torch.bfloat16)
     cluster = torch.randint(0, 4, (rows,), device=DEV, generator=g)
     low = torch.tensor([0] + tails, device=DEV)[cluster]
@@ -336,3 +336,22 @@ def test_losses_by_items_of_128_and_of_256_rows(rows):
         got, want = kernels.adaptive_nll(*args).double(), _losses_in_64_bits(*args)
         # a bf16 result and fp32 sums of logits of some units
         assert bool(((got - want).abs() <= 2 ** -8 * want.abs() + 1e-4).all())
+
+
+@pytest.mark.parametrize("rows,edges", [
+    # 258 items of the head's 64 columns and 4 of a tail of one token: some workgroups go on
+    # from a full item of the head to one of few rows of the tail
+    (66000, [0, 64, 65]),
+    # chunks of the largest length, 64 tiles: 67 items of rows for each of the head's three
+    # chunks (the last of 29 tiles), then a tail's five (the last of 57)
+    (17000, [0, 10000, 30000])])
+def test_losses_over_more_items_than_workgroups(rows, edges):
+    args = _some_losses(rows, edges)
+    got = kernels.adaptive_nll(*args)
+    hidden, target, *rest = args
+    for at in range(0, rows, 4000):
+        want = _losses_in_64_bits(hidden[at:at + 4000], target[at:at + 4000], *rest)
+        off = (got[at:at + 4000].double() - want).abs()
+        # a bf16 result and fp32 sums of logits of some units
+        assert bool((off <= 2 ** -8 * want.abs() + 1e-4).all())
+    assert torch.equal(got, kernels.adaptive_nll(*args))
