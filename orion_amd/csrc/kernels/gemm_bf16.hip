@@ -404,13 +404,19 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
 }
 
 // What a launch of each tile takes, us: 1.5 + rounds of as many workgroups as the stream
-// has compute units * (fixed + per_tile * k-tiles), fitted to 150 products drawn from
-// 256 x 256 x 64 to 8192 x 8192 x 8192 on the whole GPU (the last three to products that
-// they win, 96 x 128 with operands out of the caches: 3072 x 1024, 16 k-tiles 11.2 us
-// against 10.1 by 128 x 128, 64 k-tiles 34.0 against 38.0).  The fit is within 20 %; the large tile's estimate counts 0.9 because a round
-// of it keeps the whole chip busy where one of the others waits (8192 x 2560 x 1024: 47 us
-// by 256 x 256 tiles, 54 by 128 x 128, both estimated at 46).  Over the drawn products the
-// choice takes 1 % longer than the best of these tiles each time would.
+// has compute units * (fixed + per_tile * k-tiles), fitted on the whole GPU, with operands
+// in the caches, to 150 products drawn from 256 x 256 x 64 to 8192 x 8192 x 8192.  For
+// nine in ten the estimate of the chosen tile is 0.64 to 1.15 of its time, lowest for large
+// products, which take the clock down; what counts is the order: over the drawn products
+// the choice takes 0.9 % longer in the geometric mean than the best of these tiles each time
+// would, and 15 % at most.  The large tile's estimate counts 0.9 because a round of it keeps
+// the whole chip busy where one of the others waits (8192 x 2560 x 1024: 48 us by 256 x 256
+// tiles, 52 by 128 x 128, 61 with operands out of the caches, estimated at 42 and 42).
+// 96 x 128 lies closest to another tile, 128 x 128, so its costs follow a sweep of those two
+// at ten sizes from 512 x 4352 to 5888 x 512, with operands in the caches and out of them:
+// 8 k-tiles 3 % faster to 3 % slower, 16 8 % faster to 2 % slower, 24 10 % faster to 2 %
+// slower, 32 6 to 14 % faster; at 24 sizes of 33 to 128 k-tiles 23 % faster to 2 % slower.
+// They cross at 17 k-tiles.
 // Streams limited to some compute units have costs of their own, and only the tiles that
 // were measured there.  With the whole GPU's, 3 % of the products drawn for 32, 64 and 128
 // units went from 128 x 128 to 256 x 256, which takes longer (us, these and the whole GPU's
@@ -430,7 +436,7 @@ constexpr TileCost kTiles[] = {
     {256, 128, 64, {3.44, 0.584}, kUnmeasured},
     {192, 128, 64, {3.92, 0.470}, kUnmeasured},
     {128, 128, 64, {2.80, 0.336}, {2.0, 0.42}},
-    {96, 128, 64, {3.8, 0.305}, kUnmeasured},
+    {96, 128, 64, {3.33, 0.305}, kUnmeasured},
     {128, 64, 64, {1.7, 0.28}, {1.7, 0.28}},
     {64, 64, 64, {1.5, 0.19}, {1.5, 0.19}},
     {32, 64, 128, {1.5, 0.125}, {1.5, 0.125}},   // two groups of waves

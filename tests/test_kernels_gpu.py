@@ -238,7 +238,10 @@ EDGE_TILES = [
     ("96x128", (3072, 1024, 2560)), ("96x128", (3072, 1024, 2624)),
     # 32 and 64 of the last tile's 96 rows
     ("96x128", (512, 4352, 2112)), ("96x128", (1280, 1792, 2176)), ("96x128", (1024, 2304, 2176)),
-    ("96x128", (2560, 1024, 2240))]
+    ("96x128", (2560, 1024, 2240)),
+    # from 18 k-tiles on
+    ("96x128", (512, 4352, 1152)), ("96x128", (1280, 1792, 1216)), ("96x128", (3072, 1024, 1152)),
+    ("128x128", (512, 4352, 1088)), ("128x128", (3072, 1024, 1024))]
 
 
 @pytest.mark.parametrize("tile,shape", EDGE_TILES)
