@@ -290,7 +290,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_bf16_nt_kernel(
 // Other tiles, for products that 256 x 256 tiles would spread badly over the compute units:
 // mfma_tile.h's pipeline (HALVES: the one by k-steps, where two k-tiles' fragments would
 // fill the registers), GROUPS groups of four waves that take every GROUPS-th k-tile (their
-// sums meet in LDS).  Tiles that do not divide 256 reach past the last row and column.
+// sums meet in LDS).  Tiles whose rows do not divide 256 reach past the last one.
 // Small products are bound by the latency of a k-tile's way to the MFMAs, 0.12 to 0.34 us
 // by tile against 0.06 to 0.22 of matrix core time; those that fill the chip by its clock
 // (1.9 instead of 2.4 GHz) and by LDS.  Measured, by 256 x 256, by 128 x 128 and smaller
@@ -338,16 +338,15 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
   const int l16 = lane & 15, lq = lane >> 4;
   int tm, tn;
   small_tile_of_block(blockIdx.x, (M + TM - 1) / TM, (N + TN - 1) / TN, &tm, &tn);
-  // a tile may reach past the last row or column, which it then reads again
+  static_assert(256 % TN == 0, "no tile reaches past the last column");
+  // a tile may reach past the last row, which it then reads again
   const int row0 = tm * TM, col0 = tn * TN;
   Rows<TM> a;
   Rows<TN> b;
   a.init(wave, lane, [&](int r) {
     return A + (size_t)(256 % TM == 0 || row0 + r < M ? row0 + r : M - 1) * K + group * kTileK;
   });
-  b.init(wave, lane, [&](int r) {
-    return B + (size_t)(256 % TN == 0 || col0 + r < N ? col0 + r : N - 1) * K + group * kTileK;
-  });
+  b.init(wave, lane, [&](int r) { return B + (size_t)(col0 + r) * K + group * kTileK; });
   f32x4 acc[kI][kJ];
   clear(acc);
   if constexpr (HALVES)
@@ -381,6 +380,7 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
 #pragma unroll
   for (int i0 = 0; i0 < kI; i0 += kPassI) {
     constexpr int kAll = kPassRows * kSlots;
+    static_assert(16 * kSlots % 64 == 0, "whole instructions");
     const int rows = (kI - i0 < kPassI ? kI - i0 : kPassI) * 16;
 #pragma unroll
     for (int i = i0; i < i0 + kPassI && i < kI; ++i)
@@ -393,9 +393,8 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
     for (int first = 0; first < kAll; first += 64) {
       const int at = first + lane, R = at / kSlots, slot = at % kSlots;
       if (first >= rows * kSlots) break;
-      if (kAll % 64 != 0 && R >= rows) continue;
       const int row = row_w + i0 * 16 + R, col = col_w + slot * kPerSlot;
-      if ((256 % TM != 0 && row >= M) || (256 % TN != 0 && col >= N)) continue;
+      if (256 % TM != 0 && row >= M) continue;
       const u32x4 v = *reinterpret_cast<const u32x4*>(ep + R * kRowLds + slot * 16);
       *reinterpret_cast<u32x4*>(C + (size_t)row * N + col) = v;
     }

@@ -63,11 +63,6 @@ __device__ __forceinline__ void mfma_in_place(const bf16x8& a, const bf16x8& b, 
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
 
-// the second operand in accumulator registers too, for one that stays
-__device__ __forceinline__ void mfma_in_place_kept(const bf16x8& a, const bf16x8& b, f32x4& c) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "a"(b));
-}
-
 // Two floats to bf16, nearest even, in one register.
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   const f32x2 v = {lo, hi};

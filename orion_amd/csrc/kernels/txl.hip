@@ -655,7 +655,7 @@ __global__ __launch_bounds__(kD / 2) void txl_positions_kernel(uint16_t* table) 
 // queries 16 (w % 2) .. + 15 and one quarter of each stage of 128 keys (online
 // softmax; the quarters meet in LDS at the end).  K and R are the first
 // MFMA operand, so a lane's values belong to ONE query (lane % 16) and to four
-// consecutive keys or distances: the softmax needs two shuffles a maximum, and the
+// consecutive keys or distances: the softmax needs two swaps of lanes a maximum, and the
 // probabilities are already where the second product wants its operand, given V
 // transposed and its keys taken in the same order.
 //
@@ -1045,16 +1045,18 @@ __global__ __launch_bounds__(kGroupThreads) void crit_group_kernel(Crit c) {
 }
 
 // Wave w owns rows 64 w .. + 63 (or 32 w .. + 31 of an item of up to 128 rows), whose 512
-// elements stay in registers (all 256 accumulator ones), and all 64 columns of a tile; only the weights go through LDS, sixteen k-tiles
-// ahead and from one column tile straight on to the next.  Bound by the matrix cores: a
-// wave reads one fragment for four products (with 32 rows a wave, two, LDS reads alone
-// took as long as the products), a barrier stands between two k-tiles of sixty-four, and
-// the epilogue is six instructions an element: the bias is one more product behind the
+// elements stay in registers (all 256 accumulator ones), and all 64 columns of a tile; only
+// the weights go through LDS, sixteen k-tiles ahead and from one column tile straight on to
+// the next.  A wave reads one fragment for four products (with 32 rows a wave, two, LDS reads
+// alone took as long as the products), a barrier stands between two k-tiles of sixty-four,
+// and the epilogue is six instructions an element: the bias is one more product behind the
 // others (in front of them every partial sum would be rounded at its magnitude), and the
 // exponentials are taken against the lane's first tile's maximum, which is only replaced
-// when a sum gets out of hand.  A batch-4 request's logits
-// take 103 us, at 1.9 GHz and 72 % of what the matrix cores can issue; 155 with 128 rows
-// a workgroup, tiles of 128 columns one after the other and chunks of eight.
+// when a sum gets out of hand.  A batch-4 request's logits take 101 us, in which the matrix
+// cores are busy for half of the time and 306 MB are read; 155 with 128 rows a workgroup,
+// tiles of 128 columns one after the other and chunks of eight.  What stays of a lane's
+// values does not fit the registers: eight of them lie in scratch, written once and read at
+// most twice an item, outside the loop over the tiles.
 __device__ __forceinline__ void mfma_by_kept(const bf16x8& a, const bf16x8& kept, f32x4& c) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "a"(kept));
 }
@@ -1339,7 +1341,8 @@ __device__ __forceinline__ void crit_item(const Crit& c, unsigned char* lds, int
 #pragma unroll
   for (int i = 0; i < kI; ++i)
 #pragma unroll
-    for (int j = 0; j < kJ; ++j) odd[i][j] = f32x4{kNone, kNone, kNone, kNone};   // before the first
+    for (int j = 0; j < kJ; ++j)       // before the first
+      odd[i][j] = f32x4{kNone, kNone, kNone, kNone};
   int t = 0;
   for (; t + 1 < tiles; t += 2) {
     tile(t, std::integral_constant<int, 0>{}, even, odd);
@@ -1658,16 +1661,17 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
                          (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
                          d.heads, (uint32_t)first, coming);
     }
-    hipLaunchKernelGGL(txl_residual_gemm_kernel, dim3(res_map.blocks()), dim3(2 * kThreads), 0, s, (In)w.att,
-                       (In)p.out, proj, (In) nullptr, x, w.y, w.parts, rows, res_map);
+    hipLaunchKernelGGL(txl_residual_gemm_kernel, dim3(res_map.blocks()), dim3(2 * kThreads), 0, s,
+                       (In)w.att, (In)p.out, proj, (In) nullptr, x, w.y, w.parts, rows, res_map);
     const Norm norm = {(In)p.norm1_w, (In)p.norm1_b, w.parts, d.eps};
     RowsOut out2 = {};
     out2.x = w.x2;
     hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 128, true, ReluEpi>), dim3(ff_map.blocks()),
                        dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.ff1_w, rows,
                        ff_map, norm, out2, ReluEpi{w.h, (In)p.ff1_b, d.inner});
-    hipLaunchKernelGGL(txl_residual_gemm_kernel, dim3(res_map.blocks()), dim3(2 * kThreads), 0, s, (In)w.h,
-                       (In)p.ff2_w, d.inner, (In)p.ff2_b, (In)w.x2, w.y, w.parts, rows, res_map);
+    hipLaunchKernelGGL(txl_residual_gemm_kernel, dim3(res_map.blocks()), dim3(2 * kThreads), 0, s,
+                       (In)w.h, (In)p.ff2_w, d.inner, (In)p.ff2_b, (In)w.x2, w.y, w.parts, rows,
+                       res_map);
   }
   const orion_txl_layer& last = layers[d.layers - 1];
   hipLaunchKernelGGL(txl_norm_kernel, dim3((unsigned)tiles(rows, kThreads / 16)), dim3(kThreads), 0,
