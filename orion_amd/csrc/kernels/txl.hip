@@ -6,24 +6,24 @@
 //
 // A request is small (768 token rows at batch 4: 0.2 TFLOP, half of it in the
 // vocabulary) and a chain of 16 layers, so what bounds it is the number of
-// dependent launches and the latency inside each, not a rate.  Five launches a
+// dependent steps and the latency inside each, not a rate.  Two launches a
 // layer; whatever does not depend on the chain runs before it, for all layers at
 // once:
 //
 //   before      positions (sinusoids); keys and values of the memory and the
-//               projected positions of every layer
-//   layer i     x_i = LN(y), [q k v] = x_i Wqkv^T          ln_gemm
-//               attention                                   txl_attention
-//               y = x_i + att Wo^T                          residual_gemm
-//               x' = LN(y), h = relu(x' W1^T + b1)          ln_gemm
-//               y = x' + h W2^T + b2                        residual_gemm
+//               projected positions of every layer; [q k v] = x_0 Wqkv^T
+//   layer i     attention                                   txl_attention
+//               y = x_i + att Wo^T                          txl_layer, four products
+//               x' = LN(y), h = relu(x' W1^T + b1)
+//               y = x' + h W2^T + b2
+//               x_i+1 = LN(y), [q k v] = x_i+1 Wqkv^T
 //   after       hidden = LN(y)
 //
-// The layer norm rides in the product that reads it: a workgroup's A panel is 64
-// whole rows of 512, so it normalises them itself on the way into LDS, from means
-// and squares that the product before left for every 32 columns (every workgroup of
-// a row panel repeats that; up to sixteen of them write a share of the rows each, for
-// the residual and the memory).  y stays fp32.
+// The layer norm rides in the product that reads it: a workgroup has 48 whole rows
+// of 512, so it normalises them itself on the way into LDS, from means and squares
+// that the product before left for every 32 columns (every workgroup of a row panel
+// repeats that; each writes a share of the rows, for the residual and the memory).
+// y stays fp32.
 //
 // Sums are fp32 throughout; activations are rounded to bf16 where the model's
 // own operations rounded them, less y, the two query biases (added in fp32) and
@@ -52,6 +52,11 @@ __device__ __forceinline__ void store_bf16x4(uint16_t* p, const f32x4& v) {
   packed[0] = pack_bf16(v[0], v[1]);
   packed[1] = pack_bf16(v[2], v[3]);
   *reinterpret_cast<u32x2*>(p) = packed;
+}
+
+__device__ __forceinline__ u32x4 pack_bf16x8(const f32x4& a, const f32x4& b) {
+  return u32x4{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(b[0], b[1]),
+               pack_bf16(b[2], b[3])};
 }
 
 __device__ __forceinline__ f32x4 unpack_bf16x4(const u32x2& v) {
@@ -102,6 +107,36 @@ struct Norm {
 // of each of its sixteen parts of 32 elements, left by the product that made the row.
 constexpr int kParts = 16, kPartLen = kD / kParts;
 
+// A row's -mean / deviation and 1 / deviation, from a part in each of sixteen lanes.
+__device__ __forceinline__ float2 row_stats(const float2& part, float eps) {
+  const float mean = sum16(part.x) * (1.0f / kParts);
+  const float d = part.x - mean;
+  const float squares = sum16(__builtin_fmaf((float)kPartLen * d, d, part.y));
+  const float variance = squares * (1.0f / kD) + eps;
+  // one step of Newton's from the instruction's value (zero for an infinite variance, where
+  // the step has none): two roundings as a square root and a division have, a tenth of the
+  // instructions
+  const float r = __builtin_amdgcn_rsqf(variance);
+  const float off = __builtin_fmaf(-variance * r, r, 1.0f);
+  const float rstd = r == 0.0f ? r : __builtin_fmaf(0.5f * r, off, r);
+  return make_float2(-mean * rstd, rstd);
+}
+
+// Eight elements of a row, normalised; `shift` is -mean * rstd.
+__device__ __forceinline__ u32x4 norm_chunk(const f32x4 (&v)[2], float shift, float rstd,
+                                            const u32x4& w, const u32x4& b) {
+  u32x4 out;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const f32x4& x = v[e >> 1];
+    out[e] = pack_bf16(
+        __builtin_fmaf(__builtin_fmaf(x[e * 2 & 3], rstd, shift), bf16_lo(w[e]), bf16_lo(b[e])),
+        __builtin_fmaf(__builtin_fmaf(x[(e * 2 + 1) & 3], rstd, shift), bf16_hi(w[e]),
+                       bf16_hi(b[e])));
+  }
+  return out;
+}
+
 // A row of 512 for layer norm, sixteen lanes a row: lane l % 16 holds the elements
 // of the 16-byte bf16 chunks l % 16 + 16 * j, and one of the parts.
 struct NormRow {
@@ -118,43 +153,25 @@ struct NormRow {
   }
 };
 
+// Weights and biases of the chunks first + 64 / J * j.
+template <int J>
 struct NormWeights {
-  float w[4][8], b[4][8];
-  __device__ __forceinline__ void load(const Norm& norm, int cl) {
+  u32x4 w[J], b[J];
+  __device__ __forceinline__ void load(const Norm& norm, int first) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const u32x4 pw = *reinterpret_cast<const u32x4*>(norm.w + (cl + 16 * j) * 8);
-      const u32x4 pb = *reinterpret_cast<const u32x4*>(norm.b + (cl + 16 * j) * 8);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        w[j][2 * e] = bf16_lo(pw[e]);
-        w[j][2 * e + 1] = bf16_hi(pw[e]);
-        b[j][2 * e] = bf16_lo(pb[e]);
-        b[j][2 * e + 1] = bf16_hi(pb[e]);
-      }
+    for (int j = 0; j < J; ++j) {
+      w[j] = *reinterpret_cast<const u32x4*>(norm.w + (first + 64 / J * j) * 8);
+      b[j] = *reinterpret_cast<const u32x4*>(norm.b + (first + 64 / J * j) * 8);
     }
   }
 };
 
-__device__ __forceinline__ void norm_row(const NormRow& row, const NormWeights& weights,
+__device__ __forceinline__ void norm_row(const NormRow& row, const NormWeights<4>& weights,
                                          float eps, u32x4 (&out)[4]) {
-  const float mean = sum16(row.part.x) * (1.0f / kParts);
-  const float d = row.part.x - mean;
-  const float squares = sum16(__builtin_fmaf((float)kPartLen * d, d, row.part.y));
-  const float rstd = 1.0f / __builtin_sqrtf(squares * (1.0f / kD) + eps);
+  const float2 stats = row_stats(row.part, eps);
 #pragma unroll
   for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float x[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int at = e * 2 + h;
-        x[h] = __builtin_fmaf((row.v[j][at >> 2][at & 3] - mean) * rstd, weights.w[j][at],
-                              weights.b[j][at]);
-      }
-      out[j][e] = pack_bf16(x[0], x[1]);
-    }
+    out[j] = norm_chunk(row.v[j], stats.x, stats.y, weights.w[j], weights.b[j]);
 }
 
 // Rows of the normalised (or given) input that later launches and the caller read.
@@ -170,14 +187,9 @@ __device__ __forceinline__ void put_row(const RowsOut& out, int row, int chunk, 
     *reinterpret_cast<u32x4*>(out.mem + (size_t)(row - out.mem_from) * kD + chunk * 8) = v;
 }
 
-// Workgroup -> tile of the layers' products.  The eight XCDs, each with an L2 of its own, are
-// given workgroups in turn; each takes an even, contiguous share of the tiles counted along
-// the rows' columns, so that every product of a layer gives (nearly) the same rows to the
-// same XCD, which then finds in its L2 what the one before left.  With the columns dealt
-// out instead, so that every XCD reads all rows, a batch-4 request took 4 % longer.  With
-// whole panels of 64 rows an XCD twelve panels left half of the XCDs half the work of the
-// others: 839 us, 814 so; on streams of 32 and 64 compute units 4709 and 2469, 3913 and
-// 2067 so.
+// Workgroup -> tile.  The eight XCDs, each with an L2 of its own, are given workgroups in
+// turn; each takes an even, contiguous share of the tiles counted along the rows' columns, so
+// that an XCD reads its own rows only.
 struct TileMap {
   unsigned tiles, tiles_n;
   __host__ TileMap(size_t tiles_m, size_t tiles_n)
@@ -191,13 +203,9 @@ struct TileMap {
   }
 };
 
-// C[M, N] = A[M, 512] * W[N, 512]^T with the whole A panel of a workgroup in LDS:
-// normalised on the way from fp32 (kNorm) or loaded as it is.  Two groups of four
-// waves take the even and the odd k-tiles, W streaming through kPanelStages stages
-// each, and their sums meet in LDS: with four waves and eight k-tiles in a row, one
-// wave a SIMD, every latency of the norm and of the loop is waited for alone (11.5 us
-// a launch then, 8.3 so and with the rows' statistics from the product before, at 768
-// rows).  N is a multiple of BN; rows past M are computed
+// C[M, N] = A[M, 512] * W[N, 512]^T with the whole A panel of a workgroup in LDS.  Two
+// groups of four waves take the even and the odd k-tiles, W streaming through kPanelStages
+// stages each, and their sums meet in LDS.  N is a multiple of BN; rows past M are computed
 // from the last row and not written.
 constexpr int kPanelThreads = 2 * kThreads;
 constexpr int kPanelStages = 3;
@@ -207,9 +215,9 @@ constexpr int panel_lds() {
   return BM * kD * 2 + 2 * kPanelStages * Rows<BN>::kBytes;
 }
 
-template <int BM, int BN, bool kNorm, typename Epi>
-__device__ __forceinline__ void panel_gemm(unsigned char* lds, const void* A, const uint16_t* W,
-                                           int M, int tm, int tn, int tiles_n, const Norm& norm,
+template <int BM, int BN, typename Epi>
+__device__ __forceinline__ void panel_gemm(unsigned char* lds, const uint16_t* A,
+                                           const uint16_t* W, int M, int tm, int tn, int tiles_n,
                                            const RowsOut& out, const Epi& epi) {
   constexpr int NS = kPanelStages, kSteps = kPanelTiles / 2;
   constexpr int kI = BM / 32, kJ = BN / 32;
@@ -229,45 +237,15 @@ __device__ __forceinline__ void panel_gemm(unsigned char* lds, const void* A, co
   // the rows are written by one column of workgroups each
   const int writers = tiles_n < 16 ? tiles_n : 16;
 
-  if constexpr (kNorm) {
-    constexpr int kRows = BM / 32;        // times four rows, a wave
-    const int cl = lane & 15;
-    NormRow rows[kRows];
-    NormWeights weights;
+  Rows<BM> a;
+  a.init(wave, lane, [&](int r) {
+    const int row = row0 + r < M ? row0 + r : M - 1;
+    return A + (size_t)row * kD;
+  });
 #pragma unroll
-    for (int it = 0; it < kRows; ++it) {
-      const int row = row0 + wave8 * (BM / 8) + it * 4 + (lane >> 4);
-      rows[it].load(static_cast<const float*>(A), norm, row < M ? row : M - 1, cl);
-    }
-    weights.load(norm, cl);
+  for (int s = 0; s < kSteps; ++s) a.issue(k_of(s), panel + s * 2 * Rows<BM>::kBytes);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) b.issue(k_of(s), stages + s * Rows<BN>::kBytes);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int it = 0; it < kRows; ++it) {
-      const int r = wave8 * (BM / 8) + it * 4 + (lane >> 4);
-      const bool put = (wave8 * kRows + it) % writers == tn && row0 + r < M;
-      u32x4 v[4];
-      norm_row(rows[it], weights, norm.eps, v);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int chunk = cl + 16 * j;
-        *reinterpret_cast<u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes + r * kRowBytes +
-                                  (((chunk & 7) ^ (r & 7)) << 4)) = v[j];
-        if (put) put_row(out, row0 + r, chunk, v[j]);
-      }
-    }
-  } else {
-    Rows<BM> a;
-    a.init(wave, lane, [&](int r) {
-      const int row = row0 + r < M ? row0 + r : M - 1;
-      return static_cast<const uint16_t*>(A) + (size_t)row * kD;
-    });
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) a.issue(k_of(s), panel + s * 2 * Rows<BM>::kBytes);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) b.issue(k_of(s), stages + s * Rows<BN>::kBytes);
-  }
+  for (int s = 0; s < NS; ++s) b.issue(k_of(s), stages + s * Rows<BN>::kBytes);
   const int col0 = tn * BN + wn * (BN / 2) + lq * 4;
   typename Epi::Ahead ahead[kJ];
 #pragma unroll
@@ -300,20 +278,17 @@ __device__ __forceinline__ void panel_gemm(unsigned char* lds, const void* A, co
   multiply(acc, f[1]);
   settle(acc);
 
-  if constexpr (!kNorm) {
-    if (out.x || out.mem) {               // sixteen lanes a row, as above
+  if (out.mem) {                          // sixteen lanes a row
 #pragma unroll
-      for (int it = 0; it < BM / 32; ++it) {
-        const int r = wave8 * (BM / 8) + it * 4 + (lane >> 4);
-        if ((wave8 * (BM / 32) + it) % writers != tn || row0 + r >= M) continue;
+    for (int it = 0; it < BM / 32; ++it) {
+      const int r = wave8 * (BM / 8) + it * 4 + (lane >> 4);
+      if ((wave8 * (BM / 32) + it) % writers != tn || row0 + r >= M) continue;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int chunk = l16 + 16 * j;
-          put_row(out, row0 + r, chunk,
-                  *reinterpret_cast<const u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes +
-                                                  r * kRowBytes +
-                                                  (((chunk & 7) ^ (r & 7)) << 4)));
-        }
+      for (int j = 0; j < 4; ++j) {
+        const int chunk = l16 + 16 * j;
+        put_row(out, row0 + r, chunk,
+                *reinterpret_cast<const u32x4*>(lds + (chunk >> 3) * Rows<BM>::kBytes +
+                                                r * kRowBytes + (((chunk & 7) ^ (r & 7)) << 4)));
       }
     }
   }
@@ -360,32 +335,37 @@ struct QkvEpi {
       store_bf16x4(qv + (size_t)row * proj + col, x + unpack_bf16x4(a.v));
     }
   }
+  // the same for eight columns
+  struct Needs {
+    u32x4 u, v;
+  };
+  __device__ __forceinline__ Needs needs(int col) const {
+    const int at = col < proj ? col : 0;
+    return {*reinterpret_cast<const u32x4*>(u + at), *reinterpret_cast<const u32x4*>(v + at)};
+  }
+  __device__ __forceinline__ void operator()(int row, int col, const f32x4& left,
+                                             const f32x4& right, const Needs& a) const {
+    auto with = [&](const u32x4& b) {
+      return pack_bf16x8(left + unpack_bf16x4(u32x2{b[0], b[1]}),
+                         right + unpack_bf16x4(u32x2{b[2], b[3]}));
+    };
+    if (col >= proj) {
+      *reinterpret_cast<u32x4*>(kv + (size_t)row * (2 * proj) + (col - proj)) =
+          pack_bf16x8(left, right);
+    } else {
+      *reinterpret_cast<u32x4*>(qu + (size_t)row * proj + col) = with(a.u);
+      *reinterpret_cast<u32x4*>(qv + (size_t)row * proj + col) = with(a.v);
+    }
+  }
 };
 
-// h = relu(v + bias); a NaN stays one.
-struct ReluEpi {
-  uint16_t* out;
-  const uint16_t* bias;
-  int ld;
-  typedef u32x2 Ahead;
-  __device__ __forceinline__ Ahead ahead(int col) const {
-    return *reinterpret_cast<const u32x2*>(bias + col);
-  }
-  __device__ __forceinline__ void operator()(int row, int col, const f32x4& x, Ahead a) const {
-    f32x4 v = x + unpack_bf16x4(a);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = v[e] < 0.0f ? 0.0f : v[e];
-    store_bf16x4(out + (size_t)row * ld + col, v);
-  }
-};
-
-template <int BM, int BN, bool kNorm, typename Epi>
-__global__ __launch_bounds__(kPanelThreads, 1) void txl_ln_gemm_kernel(
-    const void* A, const uint16_t* W, int M, TileMap map, Norm norm, RowsOut out, Epi epi) {
+template <int BM, int BN, typename Epi>
+__global__ __launch_bounds__(kPanelThreads, 1) void txl_panel_gemm_kernel(
+    const uint16_t* A, const uint16_t* W, int M, TileMap map, RowsOut out, Epi epi) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[panel_lds<BM, BN>()];
   int tm, tn;
   map.tile(blockIdx.x, &tm, &tn);
-  panel_gemm<BM, BN, kNorm>(lds, A, W, M, tm, tn, map.tiles_n, norm, out, epi);
+  panel_gemm<BM, BN>(lds, A, W, M, tm, tn, map.tiles_n, out, epi);
 }
 
 // Independent products with the same inner length, one launch: workgroups
@@ -546,78 +526,668 @@ __global__ __launch_bounds__(kJobThreads, 1) void txl_jobs_kernel(Jobs jobs) {
   wait_vm<0>();                        // nothing lands in LDS that is no longer ours
 }
 
-// y[M, 512] = x + bias + A[M, K] * W[512, K]^T in fp32.  Eight waves: two groups of
-// four take the even and the odd k-tiles, which halves the chain of barriers (2048
-// deep: 16 steps instead of 32), and their sums meet in LDS.  32 x 64 tiles give
-// 192 workgroups at 768 rows.  K is a multiple of 128.
-constexpr int kResM = 32, kResN = 64, kResStages = 6;
+// One launch a layer behind attention: attention's projection, the feed-forward layer and
+// the next layer's queries, keys and values.  As launches of their own, with 64 x 96, 64 x
+// 128 and 32 x 64 tiles, the four products took 32 us of a batch-4 request's layer: a launch
+// begins 2 us after the last one ends, waits 2 us for its first data and reads weights only
+// then.  So 24: 4 for the first product, 6.5, 5.5 and 5.5 for the others (a request 694 us
+// instead of 801; batch 1, 16 tokens 555 and 660; batch 16 2050 and 2183).
+//
+// Rows come in panels of up to 48.  The work is a list of tasks, 32 or 128 columns of a
+// product for a panel; a task that reads what others of its panel write waits until a
+// counter says that they are done.  Its weights, 128 KiB, come meanwhile: a compute unit
+// takes in 60 to 100 KiB a us, and as much again of rows.  (16 rows more a panel and half the
+// columns a task than 32 rows and 64 or 256, which need twice the weights: 772 us a request
+// instead of 803.)  Panels are dealt out to up to eight groups of workgroups (with eight one
+// an XCD, which get workgroups in turn), evenly by 16 rows.
+//
+// Every wait ends, on any number of compute units and beside any other kernel: a group's
+// tasks are taken from a counter in the order of the products, a task waits only for tasks
+// of its own group before it, and a task that has been taken is run by a workgroup that is
+// running.  (The first task not finished waits for nothing; a workgroup takes its next task
+// ahead, but that comes after the one that it runs.)
+//
+// What one workgroup writes and another reads within the launch is written through to
+// memory (sc1, agent scope), and a counter is raised when its workgroup's stores have been
+// acknowledged.  Readers may cache it: a line of it holds one panel's values of one product
+// only, no one reads it in this launch before the counter says so, and caches start a launch
+// without lines of the launches before.  So nothing depends on where a workgroup runs.  A
+// stage whose 192 workgroups hand on 32 KiB a panel takes 1.6 us so (2.0 with a panel's
+// workgroups on all XCDs), 4.3 (6.8) with release and acquire fences, 2.5 to 2.9 as a launch.
+constexpr int kLayerThreads = 512;
+constexpr int kGroups = 8, kGroupMost = 32;          // workgroups of a group, one a compute unit
+constexpr int kPanelTiles16 = 3, kPanelRows = 16 * kPanelTiles16;
+constexpr int kRowTileBytes = kPanelRows * kRowBytes;        // a panel's k-tile
+constexpr int kUnits4 = 4, kUnitCols = 32;           // a wave's weights: four k-tiles of 32 columns
+constexpr int kUnitBytes = kUnitCols * kRowBytes, kUnitLoads = kUnitBytes / 1024;
+constexpr int kOwn = 159 * 128;                      // a wave's share of the LDS
+constexpr int kLayerLds = 8 * kOwn;
+constexpr int kResCols = 32, kNormCols = 128;        // of a task
+constexpr int kResTasks = kD / kResCols;
+constexpr int kLine = 32;                            // counters lie a 128-byte line apart
+constexpr int kCoherent = 16;                        // sc1
 
-__global__ __launch_bounds__(2 * kThreads, 1) void txl_residual_gemm_kernel(
-    const uint16_t* __restrict__ A, const uint16_t* __restrict__ W, int K,
-    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ x, float* __restrict__ y,
-    float2* __restrict__ parts, int M, TileMap map) {
-  constexpr int kGroup = kResStages * (Rows<kResM>::kBytes + Rows<kResN>::kBytes);
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2 * kGroup];
-  const int lane = threadIdx.x & 63;
-  const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wave = wave8 & 3, group = wave8 >> 2;
-  const int wm = wave >> 1, wn = wave & 1;
-  int tm, tn;
-  map.tile(blockIdx.x, &tm, &tn);
-  const int row0 = tm * kResM, col0 = tn * kResN;
-  Rows<kResM> a;
-  Rows<kResN> b;
-  a.init(wave, lane, [&](int r) {
-    const int row = row0 + r < M ? row0 + r : M - 1;
-    return A + (size_t)row * K + group * kTileK;
-  });
-  b.init(wave, lane, [&](int r) { return W + (size_t)(col0 + r) * K + group * kTileK; });
-  const int row = row0 + wm * 16 + (lane & 15);
-  const int at = row < M ? row : M - 1;
-  u32x2 add_x[kResN / 32], add_b[kResN / 32];      // for the end, asked for ahead
-#pragma unroll
-  for (int j = 0; j < kResN / 32; ++j) {
-    const int col = col0 + wn * (kResN / 2) + j * 16 + (lane >> 4) * 4;
-    add_x[j] = *reinterpret_cast<const u32x2*>(x + (size_t)at * kD + col);
-    add_b[j] = bias ? *reinterpret_cast<const u32x2*>(bias + col) : u32x2{0, 0};
+// Memory that other workgroups of the launch write or read; offsets in bytes.  What lies
+// past `bytes` reads as zero and is not written.
+struct Shared {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ Shared(const void* p, int bytes)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000)) {}
+  __device__ __forceinline__ u32x4 load16(int at) const {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, at, 0, 0);
   }
-  f32x4 acc[kResM / 32][kResN / 32];
-  clear(acc);
-  stream_product<kResM, kResN, kResStages>(acc, lds + group * kGroup, K / (2 * kTileK),
-                                           2 * kTileK, a, b, wm, wn, lane);
+  __device__ __forceinline__ u32x2 load8(int at) const {
+    return __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, 0);
+  }
+  __device__ __forceinline__ void store16(int at, const u32x4& v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, at, 0, kCoherent);
+  }
+  __device__ __forceinline__ void store8(int at, const u32x2& v) const {
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, at, 0, kCoherent);
+  }
+};
+
+__device__ __forceinline__ bf16x8 panel_fragment(const unsigned char* base, int row, int ks,
+                                                 int lq) {
+  return *reinterpret_cast<const bf16x8*>(base + row * kRowBytes +
+                                          (((ks * 4 + lq) ^ (row & 7)) << 4));
+}
+
+// The weights of a wave's next task: k-tiles of 32 columns that come by whole lines through
+// LDS into registers, as the MFMA's fragments.  Fragment j of a k-tile takes the columns
+// 8 * (i / 4) + 4 * j + i % 4, so that a lane's accumulators of both are eight columns in a row.
+struct Plan {
+  const uint16_t* W;            // 32 columns
+  int even, odd;                // this lane's chunk of rows lane / 8 and 8 + lane / 8, bytes
+  int ld, first, last;          // k-tiles: this wave's first, the last of all (past it that again)
+  int units;                    // of the four that there are
+};
+
+__device__ __forceinline__ void buffer_to_lds(const Shared& from, int lane_at, int at,
+                                              unsigned char* to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      from.r, (__attribute__((address_space(3))) void*)to, 16, lane_at, at, 0, 0);
+}
+
+__device__ __forceinline__ Plan plan_of(const uint16_t* W, int ld, int first, int units,
+                                        int lane) {
+  const int at = (lane >> 3) * ld * 2, chunk = (lane & 7) ^ ((lane >> 3) & 3);
+  return {W,  at + chunk * 16, at + 16 * ld + (chunk ^ 4) * 16, ld, first, ld / kTileK - 1, units};
+}
+
+// Half h (sixteen rows) of unit u.
+__device__ __forceinline__ void issue_half(const Plan& plan, int u, int h, unsigned char* to) {
+  if (u >= plan.units) return;
+  const Shared W(plan.W, kUnitCols * plan.ld * 2);
+  const int tile = plan.first + u < plan.last ? plan.first + u : plan.last;
+  const int at = h * 32 * plan.ld + tile * kRowBytes;
+  buffer_to_lds(W, plan.even, at, to);
+  buffer_to_lds(W, plan.odd, at, to + 8 * kRowBytes);
+}
+__device__ __forceinline__ void issue_unit(const Plan& plan, int u, unsigned char* to) {
+  issue_half(plan, u, 0, to);
+  issue_half(plan, u, 1, to + kUnitBytes / 2);
+}
+
+typedef bf16x8 Weights[kUnits4][2][2];               // [k-tile][k-step][fragment]
+
+// A unit's first sixteen rows lie at `from`, the others 2 KiB or `apart` behind them.
+__device__ __forceinline__ void take_unit(Weights& w, int u, const unsigned char* from, int lane,
+                                          int apart = kUnitBytes / 2) {
+  const int l16 = lane & 15, lq = lane >> 4;
+  from += l16 < 8 ? 0 : apart - kUnitBytes / 2;
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int row = (l16 >> 2) * 8 + j * 4 + (l16 & 3);
+      w[u][ks][j] = *reinterpret_cast<const bf16x8*>(from + row * kRowBytes +
+                                                     (((ks * 4 + lq) ^ (l16 & 7)) << 4));
+    }
+}
+
+// Sum over eight lanes that lie side by side.
+__device__ __forceinline__ float sum8(float v) {
+  auto moved = [](float x, auto how) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(how)::value,
+                                           0xf, 0xf, true));
+  };
+  v += moved(v, std::integral_constant<int, 0xb1>{});     // lane ^ 1
+  v += moved(v, std::integral_constant<int, 0x4e>{});     // lane ^ 2
+  v += moved(v, std::integral_constant<int, 0x141>{});    // 7 - lane
+  return v;
+}
+
+struct Panel {
+  int row0, rows;
+};
+
+// The thread, anew for each task: what is computed from it then belongs to the task (kept
+// over all of them it fills the registers).
+__device__ __forceinline__ int thread_of_task() {
+  int thread = threadIdx.x;
+  asm volatile("" : "+v"(thread));
+  return thread;
+}
+
+constexpr int kSumBytes = 7168;        // of a wave's own: its sums in a residual task
+
+// LDS in a norm task, and where the next task's weights go meanwhile.
+struct NormPlaces {
+  static constexpr int kPanel = kPanelRows * kD * 2;         // bytes of the normalised rows
+  static constexpr int kMeet = 6 * 4 * 1024;                 // and of the halves' sums behind them
+  static constexpr int kFree = (8 * kOwn - kPanel - kMeet) / 8 / 128 * 128;
+  static constexpr int kDead = kPanel / 8;                   // free once the rows have been read
+  static_assert(kFree >= 5 * kUnitBytes / 2 && kDead >= 3 * kUnitBytes / 2, "four units a wave");
+  // units 0 and 1 and half of 3 in the free part, unit 2 and the other half in the rows' place
+  static __device__ __forceinline__ int of(int unit, int wave) {
+    return unit == 2 ? wave * kDead
+                     : kPanel + kMeet + wave * kFree + (unit == 3 ? 2 : unit) * kUnitBytes;
+  }
+  static __device__ __forceinline__ int rest_of_last(int wave) { return wave * kDead + kUnitBytes; }
+};
+
+// Where a task's weights wait for it: as its workgroup's first, or as the task before left them.
+enum class Place { kFirst, kBehindNorm, kBehindSum };
+
+// What a workgroup carries from task to task.
+struct Run {
+  unsigned char* lds;
+  uint32_t* next;               // the group's counter of tasks
+  uint32_t* taken;              // in LDS: what it said last
+  Place place;
+
+  __device__ __forceinline__ uint32_t take() const {
+    return __hip_atomic_fetch_add(next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ int wave() const {
+    return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  }
+  __device__ __forceinline__ unsigned char* own() const { return lds + wave() * kOwn; }
+  // A task's weights, and what it waits for (nothing for a null counter); after it everyone
+  // knows the next task.  loads(): exactly kLoads loads, which are not waited for.
+  template <int kLoads, typename Loads>
+  __device__ __forceinline__ void wait_for(Weights& w, int lane, const uint32_t* counter,
+                                           uint32_t target, Loads loads) {
+    uint32_t seen = target, coming = 0;
+    if (threadIdx.x == 0) {
+      coming = take();
+      if (counter) seen = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    loads();
+    wait_vm<kLoads>();
+    if (place == Place::kBehindNorm) {
+#pragma unroll
+      for (int u = 0; u < kUnits4; ++u)
+        take_unit(w, u, lds + NormPlaces::of(u, wave()), lane,
+                  u < 3 ? kUnitBytes / 2
+                        : NormPlaces::rest_of_last(wave()) - NormPlaces::of(3, wave()));
+    } else {
+      const int at = place == Place::kFirst ? 0 : kSumBytes;
+#pragma unroll
+      for (int u = 0; u < kUnits4; ++u)
+        take_unit(w, u, own() + (u < 3 ? at + u * kUnitBytes : at ? 0 : 3 * kUnitBytes), lane);
+    }
+    if (threadIdx.x == 0) {
+      while ((int)(seen - target) < 0)
+        seen = __hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *taken = coming;
+    }
+    block_sync();
+  }
+};
+
+// y = x + bias + A W^T for 32 columns of a panel, in fp32, with the means and squares of the
+// part that they are.  The eight waves share the depth, KT k-tiles each at a time, and their
+// sums meet in LDS: so a wave's rows and weights pass through LDS once and no wave waits for
+// another before the end.  K is a multiple of 64.  kWait: A and x come from this launch.
+// ahead(step): 0, the next task is known; 1, the stores are on their way and three units of its
+// weights may go to LDS from kSumBytes on.
+template <int KT, bool kWait, typename Ahead, int... kTile>
+__device__ __forceinline__ void residual_task(Run& run, const Plan& plan, const Panel& panel,
+                                              int tn, const uint16_t* A, int K,
+                                              const uint16_t* bias, const uint16_t* x, float* y,
+                                              float2* parts, const uint32_t* counter,
+                                              uint32_t target, Ahead ahead,
+                                              std::integer_sequence<int, kTile...>) {
+  constexpr int kSumRow = kResCols + 4;            // floats
+  constexpr int kI = kPanelTiles16, kJ = kResCols / 16;
+  // rows that need not be waited for lie beside the weights on their way
+  constexpr int kRowsAt = kWait ? 0 : KT * kUnitBytes;
+  constexpr int kFit = (kOwn - kRowsAt) / kRowTileBytes, kAhead = kFit < KT ? kFit : KT;
+  static_assert(kAhead > 0 && (kWait || kAhead == KT), "");
+  static_assert(kPanelRows * kSumRow * 4 <= kSumBytes && kSumBytes + 3 * kUnitBytes <= kOwn, "");
+  const int thread = thread_of_task(), lane = thread & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(thread >> 6);
+  const int l16 = lane & 15, lq = lane >> 4;
+  unsigned char* own = run.lds + wave * kOwn;
+  const int tiles = K / kTileK, col0 = tn * kResCols;
+  // the element that this thread finishes (of the first 384)
+  const int r = thread >> 3, col = col0 + (thread & 7) * 4;
+  const int at = r < panel.rows ? r : panel.rows - 1;
+  const u32x2 add_b = bias ? *reinterpret_cast<const u32x2*>(bias + col) : u32x2{0, 0};
+  u32x2 add_x = {0, 0};
+  if constexpr (!kWait)
+    add_x = *reinterpret_cast<const u32x2*>(x + (size_t)(panel.row0 + at) * kD + col);
+  // rows past the last one are not read
+  const Shared rows(A + (size_t)panel.row0 * K, panel.rows * K * 2);
+  const int rows_at = (lane >> 3) * K * 2 + ((lane & 7) ^ (lane >> 3)) * 16;
+  Weights w;
+  f32x4 acc[kI][kJ];
+#pragma unroll
+  for (int i = 0; i < kI; ++i)
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int base = 0; base < tiles; base += 8 * KT) {
+    const int mine = base + wave * KT;
+    // past the last k-tile that one again, not multiplied
+    auto issue_rows = [&](int kt) {
+      const int tile = mine + kt < tiles ? mine + kt : tiles - 1;
+#pragma unroll
+      for (int b = 0; b < kPanelRows / 8; ++b)
+        buffer_to_lds(rows, rows_at, b * 16 * K + tile * kRowBytes,
+                    own + kRowsAt + kt % kAhead * kRowTileBytes + b * 8 * kRowBytes);
+    };
+    // what need not be waited for is on its way with a first task's weights
+    const bool at_once = !kWait && (base > 0 || run.place == Place::kFirst);
+    if (at_once) {
+#pragma unroll
+      for (int kt = 0; kt < kAhead; ++kt) issue_rows(kt);
+    }
+    if (base == 0) {
+      run.wait_for<0>(w, lane, kWait ? counter : nullptr, target, [] {});
+      if constexpr (kWait)
+        add_x =
+            Shared(x + (size_t)panel.row0 * kD, panel.rows * kD * 2).load8((at * kD + col) * 2);
+    } else {
+      Plan more = plan;
+      more.first = mine;
+#pragma unroll
+      for (int u = 0; u < KT; ++u) issue_unit(more, u, own + u * kUnitBytes);
+      wait_vm<0>();
+#pragma unroll
+      for (int u = 0; u < KT; ++u) take_unit(w, u, own + u * kUnitBytes, lane);
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!at_once) {
+#pragma unroll
+      for (int kt = 0; kt < kAhead; ++kt) issue_rows(kt);
+    }
+    if (base == 0) ahead(0);
+    auto multiply_tile = [&](auto tile) {
+      constexpr int kt = decltype(tile)::value;
+      constexpr int kIssued = kt + kAhead < KT ? kt + kAhead : KT;
+      wait_vm<kWait ? (kIssued - kt - 1) * (kPanelRows / 8) : 0>();
+      bf16x8 a[2][kI];
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < kI; ++i)
+          a[ks][i] = panel_fragment(own + kRowsAt + kt % kAhead * kRowTileBytes, i * 16 + l16, ks,
+                                    lq);
+      if constexpr (kt + kAhead < KT) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);        // read before it is overwritten
+        __builtin_amdgcn_sched_barrier(0);
+        issue_rows(kt + kAhead);
+      }
+      if (mine + kt >= tiles) return;
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int i = 0; i < kI; ++i)
+#pragma unroll
+          for (int j = 0; j < kJ; ++j) acc[i][j] = mfma(w[kt][ks][j], a[ks][i], acc[i][j]);
+    };
+    (multiply_tile(std::integral_constant<int, kTile>{}), ...);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < kI; ++i)
+#pragma unroll
+    for (int j = 0; j < kJ; ++j)
+      *reinterpret_cast<f32x4*>(own + ((i * 16 + l16) * kSumRow + lq * 8 + j * 4) * 4) = acc[i][j];
   block_sync();
-  f32x4* other = reinterpret_cast<f32x4*>(lds) + wave * 64 + lane;
-  if (group == 1) {
+  if (r < kPanelRows) {
+    f32x4 product = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int j = 0; j < kResN / 32; ++j) other[j * 256] = acc[0][j];
-  }
-  block_sync();
-  if (group == 1) return;
-  f32x4 v[kResN / 32];
-  float sum = 0.0f, squares = 0.0f;
-#pragma unroll
-  for (int j = 0; j < kResN / 32; ++j) {
-    const int col = col0 + wn * (kResN / 2) + j * 16 + (lane >> 4) * 4;
-    v[j] = acc[0][j] + other[j * 256] + unpack_bf16x4(add_b[j]) + unpack_bf16x4(add_x[j]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) sum += v[j][e];
-    if (row < M) *reinterpret_cast<f32x4*>(y + (size_t)row * kD + col) = v[j];
-  }
-  // the wave's 32 columns of a row lie in four lanes
-  static_assert(kResN / 2 == kPartLen, "a wave's columns are a part");
-  sum += __shfl_xor(sum, 16);
-  sum += __shfl_xor(sum, 32);
-  const float mean = sum * (1.0f / kPartLen);
-#pragma unroll
-  for (int j = 0; j < kResN / 32; ++j)
+    for (int w = 0; w < 8; ++w)
+      product += *reinterpret_cast<const f32x4*>(run.lds + w * kOwn +
+                                                 (r * kSumRow + (thread & 7) * 4) * 4);
+    const f32x4 v = product + unpack_bf16x4(add_b) + unpack_bf16x4(add_x);
+    Shared(y + (size_t)panel.row0 * kD, panel.rows * kD * 4)
+        .store16((r * kD + col) * 4, __builtin_bit_cast(u32x4, v));
+    // eight threads hold the part
+    static_assert(kResCols == kPartLen, "a task's columns are a part");
+    const float mean = sum8(v[0] + v[1] + v[2] + v[3]) * (1.0f / kPartLen);
+    float squares = 0.0f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float d = v[j][e] - mean;
+      const float d = v[e] - mean;
       squares = __builtin_fmaf(d, d, squares);
     }
-  squares += __shfl_xor(squares, 16);
-  squares += __shfl_xor(squares, 32);
-  if (lane < 16 && row < M) parts[(size_t)row * kParts + tn * 2 + wn] = make_float2(mean, squares);
+    squares = sum8(squares);
+    if ((thread & 7) == 0)
+      Shared(parts + (size_t)panel.row0 * kParts, panel.rows * kParts * 8)
+          .store8((r * kParts + tn) * 8, u32x2{__builtin_bit_cast(uint32_t, mean),
+                                               __builtin_bit_cast(uint32_t, squares)});
+  }
+  ahead(1);
+}
+
+// 128 columns of LN(y) W^T for a panel: wave (c, g) takes 32 of the columns and half of the
+// depth.  put(row, chunk, values): normalised rows, of which each task writes a share;
+// needs(column): what finish(row, column, left, right, needs) wants from memory for eight
+// columns; ahead(step): 0, the next task is known; 1, its weights may go to
+// the free part of NormPlaces, and 2, behind the stores, to the rows' place.
+template <typename PutRow, typename Needs, typename Finish, typename Ahead>
+__device__ __forceinline__ void norm_task(Run& run, const Panel& panel, int tn, int tasks,
+                                          const float* y, const Norm& norm,
+                                          const uint32_t* counter, uint32_t target, PutRow put,
+                                          Needs needs, Finish finish, Ahead ahead) {
+  constexpr int KT = kUnits4, kI = kPanelTiles16, kJ = 2, kPasses = kPanelRows / 16;
+  const int thread = thread_of_task(), lane = thread & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(thread >> 6);
+  const int l16 = lane & 15, lq = lane >> 4, cg = wave & 3, kg = wave >> 2;
+  const int col0 = tn * kNormCols + cg * 32;
+  const int cl = lane & 31;                        // 32 lanes a row, two rows at a time
+  unsigned char* lds = run.lds;
+  NormWeights<2> weights;
+  Weights w;
+  run.wait_for<4>(w, lane, counter, target, [&] { weights.load(norm, cl); });
+  {
+    const Shared rows(y + (size_t)panel.row0 * kD, panel.rows * kD * 4);
+    const Shared sums(norm.parts + (size_t)panel.row0 * kParts, panel.rows * kParts * 8);
+    __builtin_amdgcn_sched_barrier(0);
+    // rows past the last one are zeros
+    constexpr int kRows = 2 * kPasses;             // of a wave
+    const int first = wave * kRows;
+    f32x2 part[2];                                 // of rows 0 to 3, and of 4 and 5
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      part[h] = __builtin_bit_cast(
+          f32x2, sums.load8(((first + (h ? 4 + (lq & 1) : lq)) * kParts + l16) * 8));
+    f32x4 v[kPasses][2][2];
+#pragma unroll
+    for (int it = 0; it < kPasses; ++it)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          v[it][j][h] = __builtin_bit_cast(
+              f32x4, rows.load16(((first + it * 2 + (lane >> 5)) * kD + (cl + 32 * j) * 8 + h * 4) *
+                                 4));
+    ahead(0);
+    float shift[kRows], rstd[kRows];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float2 stats = row_stats(make_float2(part[h][0], part[h][1]), norm.eps);
+#pragma unroll
+      for (int i = 0; i < (h ? 2 : 4); ++i) {
+        shift[h * 4 + i] = __builtin_bit_cast(
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, stats.x), i * 16));
+        rstd[h * 4 + i] = __builtin_bit_cast(
+            float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, stats.y), i * 16));
+      }
+    }
+#pragma unroll
+    for (int it = 0; it < kPasses; ++it)           // the rows are here
+#pragma unroll
+      for (int j = 0; j < 2; ++j) asm volatile("" ::"v"(v[it][j][0]), "v"(v[it][j][1]));
+    ahead(1);
+#pragma unroll
+    for (int it = 0; it < kPasses; ++it) {
+      __builtin_amdgcn_sched_barrier(0);
+      const bool second = lane >= 32;
+      const int r = first + it * 2 + second;
+      const float m = second ? shift[it * 2 + 1] : shift[it * 2];
+      const float s = second ? rstd[it * 2 + 1] : rstd[it * 2];
+      u32x4 out[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int chunk = cl + 32 * j;
+        out[j] = norm_chunk(v[it][j], m, s, weights.w[j], weights.b[j]);
+        *reinterpret_cast<u32x4*>(lds + (chunk >> 3) * kRowTileBytes + r * kRowBytes +
+                                  (((chunk & 7) ^ (r & 7)) << 4)) = out[j];
+      }
+      if ((wave * kPasses + it) % tasks == tn && r < panel.rows) {
+        put(r, cl, out[0]);
+        put(r, cl + 32, out[1]);
+      }
+    }
+  }
+  const auto needed = needs(col0 + lq * 8);
+  block_sync();
+  f32x4 acc[kI][kJ];
+#pragma unroll
+  for (int i = 0; i < kI; ++i)
+#pragma unroll
+    for (int j = 0; j < kJ; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  bf16x8 a[2][2][kI];                  // the next k-tile's while one is multiplied
+  auto read = [&](int kt) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < kI; ++i)
+        a[kt & 1][ks][i] =
+            panel_fragment(lds + (kg * KT + kt) * kRowTileBytes, i * 16 + l16, ks, lq);
+  };
+  read(0);
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    if (kt + 1 < KT) read(kt + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < kI; ++i)
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) acc[i][j] = mfma(w[kt][ks][j], a[kt & 1][ks][i], acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // Half g finishes row tile g, and row tile 2 of every second four waves' columns.
+  f32x4* meet = reinterpret_cast<f32x4*>(lds + NormPlaces::kPanel) + cg * 64 + lane;
+  const bool both = (cg & 1) == kg;                // this wave finishes two row tiles
+#pragma unroll
+  for (int j = 0; j < kJ; ++j) {
+    meet[(kg * 2 + j) * 256] = kg ? acc[0][j] : acc[1][j];
+    if (!both) meet[(4 + j) * 256] = acc[2][j];
+  }
+  block_sync();
+  const f32x4* other = meet + (1 - kg) * 2 * 256;
+  finish(kg * 16 + l16, col0 + lq * 8, (kg ? acc[1][0] : acc[0][0]) + other[0],
+         (kg ? acc[1][1] : acc[0][1]) + other[256], needed);
+  if (both)
+    finish(32 + l16, col0 + lq * 8, acc[2][0] + meet[4 * 256], acc[2][1] + meet[5 * 256], needed);
+  ahead(2);
+}
+
+struct Layer {
+  struct Product {
+    const uint16_t* W;
+    int ld, columns;                      // of a task
+    int tasks;                            // of a panel
+    uint32_t inverse;                     // 2^32 over them
+  } product[4];                           // out, ff1, ff2, the next layer's qkv
+  int products;                           // 4, in the last layer 3
+  const uint16_t *att, *x, *ff1_b, *ff2_b;
+  Norm norm1, norm2;                      // the parts of y1 and y2
+  float *y1, *y2;
+  float2 *parts1, *parts2;
+  uint16_t *x2, *h;
+  RowsOut rows_out;                       // the next layer's input
+  QkvEpi qkv;
+  uint32_t* counters;                     // kLine apart: 8 of tasks, then 3 a panel
+  int layer, rows, inner, proj, groups, panels;   // panels a group has counters for
+};
+
+// The kernel's arguments, read anew where they are needed (from the scalar cache): sixty
+// registers of them do not fit, and the compiler would keep them in lanes of vector ones.
+__device__ __forceinline__ const Layer& arguments() {
+  auto at = (const __attribute__((address_space(4))) Layer*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(at));
+  return *(const Layer*)at;
+}
+
+__global__ __launch_bounds__(kLayerThreads, 1) void txl_layer_kernel(Layer) {
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kLayerLds + 16];
+  const int group = blockIdx.x % arguments().groups;
+  // this group's share of the row tiles, and its panels': even ones
+  int first16, tiles16, panels;
+  int ff1_at, ff2_at, qkv_at, tasks;     // tasks before each product's
+  uint32_t before;                       // taken in the layers before
+  Run run;
+  run.lds = lds;
+  run.taken = reinterpret_cast<uint32_t*>(lds + kLayerLds);
+  run.place = Place::kFirst;
+  {
+    const Layer& a = arguments();
+    run.next = a.counters + group * kLine;
+    if (threadIdx.x == 0) *run.taken = run.take();
+    const int all16 = (a.rows + 15) / 16, each = all16 / a.groups, extra = all16 % a.groups;
+    tiles16 = each + (group < extra ? 1 : 0);
+    first16 = group * each + (group < extra ? group : extra);
+    panels = (tiles16 + kPanelTiles16 - 1) / kPanelTiles16;
+    ff1_at = panels * kResTasks;
+    ff2_at = ff1_at + panels * a.product[1].tasks;
+    qkv_at = ff2_at + ff1_at;
+    const int all = qkv_at + panels * a.product[3].tasks;
+    tasks = a.products == 4 ? all : qkv_at;
+    // every workgroup takes one task more than there are
+    before = (uint32_t)a.layer * (all + gridDim.x / a.groups);
+  }
+  const int share = tiles16 / panels, larger = tiles16 - share * panels;
+  struct Task {
+    int number, stage, panel, tn;
+  };
+  auto task_of = [&](int number, Plan* plan) {
+    const int stage = (number >= ff1_at) + (number >= ff2_at) + (number >= qkv_at);
+    const unsigned at =
+        number - (stage < 2 ? (stage == 0 ? 0 : ff1_at) : stage == 2 ? ff2_at : qkv_at);
+    const Layer::Product& product = arguments().product[stage];
+    unsigned panel = __umulhi(at, product.inverse);    // or one more
+    if (at - panel * product.tasks >= (unsigned)product.tasks) ++panel;
+    const int tn = (int)(at - panel * product.tasks), wave = run.wave();
+    const int col0 = tn * product.columns + (stage & 1 ? (wave & 3) * kUnitCols : 0);
+    // a sum's waves share the depth, a norm's two halves
+    const int first = stage == 0 ? wave : (stage == 2 ? wave : wave >> 2) * kUnits4;
+    *plan = plan_of(product.W + (size_t)col0 * product.ld, product.ld, first,
+                    stage == 0 ? 1 : kUnits4, thread_of_task() & 63);
+    return Task{number, stage, (int)panel, tn};
+  };
+  block_sync();
+  const int number = (int)(__builtin_amdgcn_readfirstlane(*run.taken) - before);
+  if (number >= tasks) return;
+  Plan plan;
+  Task task = task_of(number, &plan);
+#pragma unroll
+  for (int u = 0; u < kUnits4; ++u) issue_unit(plan, u, run.own() + u * kUnitBytes);
+  block_sync();                          // everyone knows its task
+  while (true) {
+    const Layer& a = arguments();
+    const int tn = task.tn, p = task.panel;
+    const int from16 = first16 + p * share + (p < larger ? p : larger);
+    const int end = (from16 + share + (p < larger ? 1 : 0)) * 16;
+    const Panel panel = {from16 * 16, (end < a.rows ? end : a.rows) - from16 * 16};
+    uint32_t* const counters = a.counters + (size_t)(kGroups + (group * a.panels + p) * 3) * kLine;
+    const uint32_t times = a.layer + 1;
+    Task coming = {tasks, 0, 0, 0};
+    Plan then = {};
+    auto look_ahead = [&]() {
+      coming.number = (int)(__builtin_amdgcn_readfirstlane(*run.taken) - before);
+      if (coming.number >= tasks) return;
+      coming = task_of(coming.number, &then);
+    };
+    // Once the stores are on their way the next weights follow them; wait_vm counts what may
+    // still be in flight when the stores have arrived.
+    auto stores_first = [] {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto ahead_of_sum = [&](int step) {
+      if (step == 0) return look_ahead();
+      stores_first();
+      if (then.units == kUnits4) {
+#pragma unroll
+        for (int u = 0; u < kUnits4 - 1; ++u)
+          issue_unit(then, u, run.own() + kSumBytes + u * kUnitBytes);
+        wait_vm<(kUnits4 - 1) * kUnitLoads>();
+      } else {
+        issue_unit(then, 0, run.own() + kSumBytes);
+        wait_vm<0>();
+      }
+    };
+    auto ahead_of_norm = [&](int step) {
+      if (step == 0) return look_ahead();
+      if (step == 1) {
+        issue_unit(then, 0, lds + NormPlaces::of(0, run.wave()));
+        issue_unit(then, 1, lds + NormPlaces::of(1, run.wave()));
+        issue_half(then, 3, 0, lds + NormPlaces::of(3, run.wave()));
+        return;
+      }
+      stores_first();
+      if (then.units == kUnits4) {
+        issue_unit(then, 2, lds + NormPlaces::of(2, run.wave()));
+        issue_half(then, 3, 1, lds + NormPlaces::rest_of_last(run.wave()));
+        wait_vm<kUnitLoads + kUnitLoads / 2>();
+      } else {
+        wait_vm<0>();
+      }
+    };
+    const bool sum = (task.stage & 1) == 0;
+    uint32_t* raise = nullptr;
+    if (task.stage == 0) {
+      residual_task<1, false>(run, plan, panel, tn, a.att, a.proj, nullptr, a.x, a.y1,
+                              a.parts1, nullptr, 0, ahead_of_sum,
+                              std::make_integer_sequence<int, 1>{});
+      raise = counters;
+    } else if (task.stage == 1) {
+      const Shared x2(a.x2 + (size_t)panel.row0 * kD, panel.rows * kD * 2);
+      const Shared out(a.h + (size_t)panel.row0 * a.inner, panel.rows * a.inner * 2);
+      norm_task(
+          run, panel, tn, a.product[1].tasks, a.y1, a.norm1, counters, times * kResTasks,
+          [&](int r, int chunk, const u32x4& v) { x2.store16((r * kD + chunk * 8) * 2, v); },
+          [&](int col) { return *reinterpret_cast<const u32x4*>(a.ff1_b + col); },
+          [&](int r, int col, f32x4 left, f32x4 right, const u32x4& bias) {
+            left += unpack_bf16x4(u32x2{bias[0], bias[1]});
+            right += unpack_bf16x4(u32x2{bias[2], bias[3]});
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {                      // a NaN stays one
+              left[e] = left[e] < 0.0f ? 0.0f : left[e];
+              right[e] = right[e] < 0.0f ? 0.0f : right[e];
+            }
+            out.store16((r * a.inner + col) * 2, pack_bf16x8(left, right));
+          },
+          ahead_of_norm);
+      raise = counters + kLine;
+    } else if (task.stage == 2) {
+      residual_task<kUnits4, true>(run, plan, panel, tn, a.h, a.inner, a.ff2_b, a.x2, a.y2,
+                                   a.parts2, counters + kLine, times * a.product[1].tasks,
+                                   ahead_of_sum, std::make_integer_sequence<int, kUnits4>{});
+      raise = counters + 2 * kLine;
+    } else {
+      norm_task(
+          run, panel, tn, a.product[3].tasks, a.y2, a.norm2, counters + 2 * kLine,
+          times * kResTasks,
+          [&](int r, int chunk, const u32x4& v) { put_row(a.rows_out, panel.row0 + r, chunk, v); },
+          [&](int col) { return a.qkv.needs(col); },
+          [&](int r, int col, const f32x4& left, const f32x4& right, const QkvEpi::Needs& biases) {
+            if (r < panel.rows) a.qkv(panel.row0 + r, col, left, right, biases);
+          },
+          ahead_of_norm);
+    }
+    block_sync();                        // every wave's stores have arrived
+    if (raise && threadIdx.x == 0)
+      __hip_atomic_fetch_add(raise, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (coming.number >= tasks) return;
+    // the sums have been read: room for the last unit
+    if (sum) issue_unit(then, kUnits4 - 1, run.own());
+    run.place = sum ? Place::kBehindSum : Place::kBehindNorm;
+    task = coming;
+    plan = then;
+  }
 }
 
 // hidden = LN(y), one wave for four rows.
@@ -626,7 +1196,7 @@ __global__ __launch_bounds__(kThreads) void txl_norm_kernel(const float* y, Norm
   const int row = blockIdx.x * (kThreads / 16) + (threadIdx.x >> 4);
   const int at = row < M ? row : M - 1;
   NormRow in;
-  NormWeights weights;
+  NormWeights<4> weights;
   u32x4 v[4];
   in.load(y, norm, at, threadIdx.x & 15);
   weights.load(norm, threadIdx.x & 15);
@@ -637,9 +1207,11 @@ __global__ __launch_bounds__(kThreads) void txl_norm_kernel(const float* y, Norm
     *reinterpret_cast<u32x4*>(hidden + (size_t)row * kD + ((threadIdx.x & 15) + 16 * j) * 8) = v[j];
 }
 
-// table[distance] = [sin, cos](distance * 10000^(-2c/512)), bf16.
-__global__ __launch_bounds__(kD / 2) void txl_positions_kernel(uint16_t* table) {
+// table[distance] = [sin, cos](distance * 10000^(-2c/512)), bf16; and the counters at zero.
+__global__ __launch_bounds__(kD / 2) void txl_positions_kernel(uint16_t* table,
+                                                               uint32_t* counters, int count) {
   const int c = threadIdx.x;
+  for (int i = blockIdx.x * (kD / 2) + c; i < count; i += gridDim.x * (kD / 2)) counters[i] = 0;
   const double rate = exp2(-13.287712379549449391 * (2.0 * c / kD));   // log2(10000)
   const double angle = blockIdx.x * rate;
   const uint32_t v = pack_bf16((float)sin(angle), (float)cos(angle));
@@ -1483,10 +2055,15 @@ struct Pieces {
   }
 };
 
+size_t tiles(size_t n, size_t tile) { return (n + tile - 1) / tile; }
+
 struct Buffers {
-  uint16_t *x, *x2, *qu, *qv, *att, *h, *kv_x, *kv_mem, *table, *r;
-  float* y;
-  float2* parts;
+  uint16_t *x[2], *x2, *qu, *qv, *att, *h, *kv_x, *kv_mem, *table, *r;
+  float *y, *y2;
+  float2 *parts, *parts2;
+  uint32_t* counters;
+  int panels;                // a group of a layer launch has at most
+  size_t counts;
   size_t bytes;
 };
 
@@ -1497,7 +2074,13 @@ Buffers buffers_of(const orion_txl_dims& d, void* base) {
   Buffers b;
   b.y = p.take<float>(rows * kD);
   b.parts = p.take<float2>(rows * kParts);
-  b.x = p.take<uint16_t>(rows * kD);
+  b.y2 = p.take<float>(rows * kD);
+  b.parts2 = p.take<float2>(rows * kParts);
+  b.panels = (int)tiles(tiles(tiles(rows, 16), kGroups), kPanelTiles16);
+  b.counts = (size_t)kLine * kGroups * (1 + 3 * (size_t)b.panels);
+  b.counters = p.take<uint32_t>(b.counts);
+  b.x[0] = p.take<uint16_t>(rows * kD);
+  b.x[1] = p.take<uint16_t>(rows * kD);
   b.x2 = p.take<uint16_t>(rows * kD);
   b.qu = p.take<uint16_t>(rows * proj);
   b.qv = p.take<uint16_t>(rows * proj);
@@ -1519,8 +2102,6 @@ bool dims_fit(const orion_txl_dims& d) {
          d.inner <= (1 << 20) && ((int64_t)d.q_len + d.m_len) * d.batch < (1 << 24) &&
          d.q_len <= kMostQueries;
 }
-
-size_t tiles(size_t n, size_t tile) { return (n + tile - 1) / tile; }
 
 bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
   if (a->rows <= 0 || a->rows >= (1 << 24) || a->tails < 0 || a->tails > kMaxTails) return false;
@@ -1588,7 +2169,8 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
   const int proj = d.heads * kHead;
   typedef const uint16_t* In;
 
-  hipLaunchKernelGGL(txl_positions_kernel, dim3(k_len), dim3(kD / 2), 0, s, w.table);
+  hipLaunchKernelGGL(txl_positions_kernel, dim3(k_len), dim3(kD / 2), 0, s, w.table,
+                     w.counters, (int)w.counts);
   Jobs jobs;
   jobs.count = 0;
   uint64_t blocks = 0;
@@ -1613,29 +2195,30 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
   }
   flush();
 
-  const TileMap qkv_map(tiles(rows, 64), 3 * proj / 96), ff_map(tiles(rows, 64), d.inner / 128);
-  const TileMap res_map(tiles(rows, kResM), kD / kResN);
+  const TileMap qkv_map(tiles(rows, 64), 3 * proj / 96);
+  // a group has as many workgroups as a product has tasks there: with more, some would take
+  // two tasks of one product while others wait for them
+  size_t panel_tasks = kResTasks;
+  for (size_t columns : {(size_t)d.inner, 3 * (size_t)proj})
+    if (columns / kNormCols > panel_tasks) panel_tasks = columns / kNormCols;
+  const size_t row_tiles = tiles(rows, 16), groups = row_tiles < kGroups ? row_tiles : kGroups;
+  const size_t group_tasks = panel_tasks * tiles(tiles(row_tiles, groups), kPanelTiles16);
+  const size_t layer_blocks = groups * (group_tasks < kGroupMost ? group_tasks : kGroupMost);
   for (int i = 0; i < d.layers; ++i) {
     const orion_txl_layer& p = layers[i];
-    // x_i also goes into the memory's last rows
-    RowsOut out = {};
-    if (new_mems) {
-      out.mem = (uint16_t*)new_mems + i * new_mem_stride;
-      out.mem_from = (d.q_len - mem_rows_out) * d.batch;
-    }
-    const QkvEpi qkv = {w.qu, w.qv, w.kv_x, (In)u, (In)v, proj};
-    In x = (In)x0;
-    if (i == 0) {
-      hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 96, false, QkvEpi>), dim3(qkv_map.blocks()),
-                         dim3(kPanelThreads), 0, s, x0, (In)p.qkv, rows, qkv_map, Norm{},
-                         out, qkv);
-    } else {
-      x = out.x = w.x;
-      const Norm norm = {(In)layers[i - 1].norm2_w, (In)layers[i - 1].norm2_b, w.parts, d.eps};
-      hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 96, true, QkvEpi>), dim3(qkv_map.blocks()),
-                         dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.qkv, rows,
-                         qkv_map, norm, out, qkv);
-    }
+    // a layer's input also goes into the memory's last rows
+    auto rows_out = [&](int layer) {
+      RowsOut out = {};
+      if (new_mems) {
+        out.mem = (uint16_t*)new_mems + layer * new_mem_stride;
+        out.mem_from = (d.q_len - mem_rows_out) * d.batch;
+      }
+      return out;
+    };
+    if (i == 0)
+      hipLaunchKernelGGL((txl_panel_gemm_kernel<64, 96, QkvEpi>), dim3(qkv_map.blocks()),
+                         dim3(kPanelThreads), 0, s, (In)x0, (In)p.qkv, rows, qkv_map,
+                         rows_out(0), QkvEpi{w.qu, w.qv, w.kv_x, (In)u, (In)v, proj});
     const size_t attn_blocks = (size_t)d.heads * d.batch * tiles(d.q_len, kQ);
     Coming coming = {};
     size_t left = attn_blocks < kUnits ? (kUnits - attn_blocks) * kTouchBytes : 0, ahead = 0;
@@ -1661,22 +2244,47 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
                          (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
                          d.heads, (uint32_t)first, coming);
     }
-    hipLaunchKernelGGL(txl_residual_gemm_kernel, dim3(res_map.blocks()), dim3(2 * kThreads), 0, s,
-                       (In)w.att, (In)p.out, proj, (In) nullptr, x, w.y, w.parts, rows, res_map);
-    const Norm norm = {(In)p.norm1_w, (In)p.norm1_b, w.parts, d.eps};
-    RowsOut out2 = {};
-    out2.x = w.x2;
-    hipLaunchKernelGGL((txl_ln_gemm_kernel<64, 128, true, ReluEpi>), dim3(ff_map.blocks()),
-                       dim3(kPanelThreads), 0, s, (const void*)w.y, (In)p.ff1_w, rows,
-                       ff_map, norm, out2, ReluEpi{w.h, (In)p.ff1_b, d.inner});
-    hipLaunchKernelGGL(txl_residual_gemm_kernel, dim3(res_map.blocks()), dim3(2 * kThreads), 0, s,
-                       (In)w.h, (In)p.ff2_w, d.inner, (In)p.ff2_b, (In)w.x2, w.y, w.parts, rows,
-                       res_map);
+    Layer a = {};
+    auto product = [&](int stage, const void* W, int ld, int columns, int tasks) {
+      a.product[stage] = {(In)W, ld, columns, tasks, ~0u / (uint32_t)tasks};
+    };
+    product(0, p.out, proj, kResCols, kResTasks);
+    product(1, p.ff1_w, kD, kNormCols, d.inner / kNormCols);
+    product(2, p.ff2_w, d.inner, kResCols, kResTasks);
+    product(3, i + 1 < d.layers ? layers[i + 1].qkv : nullptr, kD, kNormCols,
+            3 * proj / kNormCols);
+    a.products = i + 1 < d.layers ? 4 : 3;
+    a.ff1_b = (In)p.ff1_b;
+    a.ff2_b = (In)p.ff2_b;
+    a.layer = i;
+    a.inner = d.inner;
+    a.proj = proj;
+    a.panels = w.panels;
+    a.rows = rows;
+    a.att = w.att;
+    a.x = i == 0 ? (In)x0 : w.x[i & 1];
+    a.norm1 = Norm{(In)p.norm1_w, (In)p.norm1_b, w.parts, d.eps};
+    a.norm2 = Norm{(In)p.norm2_w, (In)p.norm2_b, w.parts2, d.eps};
+    a.parts1 = w.parts;
+    a.parts2 = w.parts2;
+    a.y1 = w.y;
+    a.y2 = w.y2;
+    a.x2 = w.x2;
+    a.h = w.h;
+    if (i + 1 < d.layers) {
+      a.rows_out = rows_out(i + 1);
+      a.rows_out.x = w.x[(i + 1) & 1];
+      a.qkv = {w.qu, w.qv, w.kv_x, (In)u, (In)v, proj};
+    }
+    a.counters = w.counters;
+    a.groups = (int)groups;
+    hipLaunchKernelGGL(txl_layer_kernel, dim3((unsigned)layer_blocks), dim3(kLayerThreads), 0, s,
+                       a);
   }
   const orion_txl_layer& last = layers[d.layers - 1];
   hipLaunchKernelGGL(txl_norm_kernel, dim3((unsigned)tiles(rows, kThreads / 16)), dim3(kThreads), 0,
-                     s, (const float*)w.y,
-                     (Norm{(In)last.norm2_w, (In)last.norm2_b, w.parts, d.eps}),
+                     s, (const float*)w.y2,
+                     (Norm{(In)last.norm2_w, (In)last.norm2_b, w.parts2, d.eps}),
                      (uint16_t*)hidden, rows);
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
 }

@@ -246,6 +246,60 @@ def test_edges_of_query_blocks_and_of_the_kept_weights_rows(q_len, m_len, batch)
     assert _off(new, want_new) <= 1.25 * _off(old_new, want_new) + 1e-4
 
 
+@pytest.mark.parametrize("q_len,batch", [
+    # one group of workgroups, and eight with one row tile more or less: 16 rows each
+    (1, 1), (15, 1), (17, 1), (127, 1), (43, 3), (20, 7),
+    # panels of one, two and three row tiles in a group, of 47 to 49 rows a panel, several panels
+    (77, 5), (128, 3), (129, 3), (96, 8), (110, 7), (193, 8), (512, 7)])
+@pytest.mark.parametrize("n_head,d_inner", [(4, 256), (2, 128), (8, 2176)])
+def test_edges_of_row_panels(q_len, batch, n_head, d_inner):
+    """Panels of up to 48 rows in up to eight groups; 128 columns or 32 a task; 512 or 2048 of a
+    product's depth at a time (2, 4, 8, 34 k-tiles)."""
+    changes = dict(n_head=n_head, d_inner=d_inner, n_layer=2)
+    model = _model(**changes)
+    inputs = _inputs(model, q_len, 0, batch)
+    nll, new = _fused(model, *inputs)
+    old_nll, old_new = _operations(model, *inputs)
+    double = txl.MemTransformerLM(**dict(CONFIG, **changes))
+    double.load_state_dict(model.state_dict())
+    double = double.eval().to(DEV, torch.float64)
+    with torch.no_grad():
+        want_nll, want_new = double(*inputs)
+    # bf16 computations in another order, within their noise of each other
+    assert _off(nll, want_nll) <= 1.25 * _off(old_nll, want_nll) + 1e-4
+    assert _off(new, want_new) <= 1.25 * _off(old_new, want_new) + 1e-4
+
+
+def test_more_rows_than_a_launch_has_workgroups_for():
+    # 28 and 29 panels a group: every workgroup takes several tasks of each product
+    model = _model(n_layer=2)
+    inputs = _inputs(model, 217, 5, 50)
+    (nll, new), (old_nll, old_new) = _fused(model, *inputs), _operations(model, *inputs)
+    assert _off(nll, old_nll.double()) < 1e-2 and _off(new, old_new.double()) < 1e-2
+    again = _fused(model, *inputs)
+    assert torch.equal(again[0], nll) and torch.equal(again[1], new)
+
+
+def test_requests_on_few_compute_units_and_beside_each_other():
+    """Workgroups of a launch wait for each other's results: with one compute unit an XCD for
+    all of them, and with several requests at a time on streams that share units."""
+    model = _model(n_head=8, d_inner=2048)
+    torch.cuda.synchronize()
+    for shape in ((192, 192, 4), (50, 100, 3), (9, 0, 1)):
+        inputs = _inputs(model, *shape)
+        want_nll, want_new = _fused(model, *inputs)
+        torch.cuda.synchronize()
+        streams = [kernels.cu_masked_stream(cus) for cus in (8, 16, 32, 0, 0)]
+        got = []
+        for _ in range(3):
+            for stream in streams:
+                with torch.cuda.stream(stream):
+                    got.append(_fused(model, *inputs))
+        torch.cuda.synchronize()
+        for nll, new in got:
+            assert torch.equal(nll, want_nll) and torch.equal(new, want_new)
+
+
 def _losses_in_64_bits(hidden, target, weight, bias, tail_weight, tail_bias, edges):
     hidden, weight, bias, tail_weight, tail_bias = (
         t.double() for t in (hidden, weight, bias, tail_weight, tail_bias))
