@@ -11,6 +11,7 @@ import os
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 
 KERNELS_LIB = os.path.join(PKG_DIR, "liborion_kernels.so")
+KERNEL_CALLS = os.path.join(PKG_DIR, "kernel_calls.so")     # a Python module
 POLICY_LIB = os.path.join(PKG_DIR, "liborion_policy.so")
 CAPTURE_LIB = os.path.join(PKG_DIR, "libinttemp.so")
 SCHEDULER_LIB = os.path.join(PKG_DIR, "scheduler_eval.so")

@@ -14,6 +14,11 @@ from torch.autograd import forward_ad
 
 from . import _lib
 
+try:
+    from . import kernel_calls as _calls       # csrc/calls: the same calls for plain tensors
+except ImportError:
+    _calls = None
+
 STATUS = {0: "ok", 1: "bad argument", 2: "shape not a multiple of the tile",
           3: "pointer not 16-byte aligned", 4: "launch rejected"}
 
@@ -67,6 +72,9 @@ def lib():
         handle.orion_stream_destroy.argtypes = [ctypes.c_void_p]
         handle.orion_stream_destroy.restype = ctypes.c_int
         handle._orion_typed = True
+        if _calls is not None:
+            _calls.entries(*(ctypes.cast(entry, ctypes.c_void_p).value for entry in (
+                handle.orion_triad_f32, handle.orion_gemm_bf16_nt)))
     return handle
 
 
@@ -117,6 +125,8 @@ def _shutdown():
     while _streams:
         handle.orion_stream_destroy(ctypes.c_void_p(_streams.pop()))
     if _profiler_attached():
+        if _calls is not None:
+            _calls.entries(0, 0)
         _lib.unload(_lib.KERNELS_LIB)
 
 
@@ -148,6 +158,9 @@ _TENSOR_TYPES = (torch.Tensor, torch.nn.Parameter)
 
 def triad(a, b, c, s, grid_blocks=0, stream=None):
     """a = b + s * c (fp32, one FMA per element), in place into ``a``."""
+    done = _calls and _calls.triad(a, b, c, s, grid_blocks, stream)
+    if done is not None:
+        return done
     _check_device(a, b, c)
     if not (a.dtype == b.dtype == c.dtype == torch.float32):
         raise ValueError("triad is fp32")
@@ -164,6 +177,9 @@ def triad(a, b, c, s, grid_blocks=0, stream=None):
 
 def gemm_bf16_nt(a, b, out=None, out_dtype=torch.bfloat16, stream=None):
     """out[M,N] = a[M,K] @ b[N,K].T with bf16 inputs and fp32 accumulation."""
+    done = _calls and _calls.gemm(a, b, out, out_dtype, stream)
+    if done is not None:
+        return done
     _check_device(a, b)
     if a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16:
         raise ValueError("gemm_bf16_nt takes bf16 operands")
