@@ -11,9 +11,14 @@
 // all stayed on chip would move; as separate element-wise operations it is 100.
 //
 // Measured on the 16-layer, 267,735-token Transformer-XL (188 M parameters, 182
-// tensors): 1.30 ms a step, 5.8 TB/s over the 40 bytes, against 5.2 ms for the
-// element-wise operations.  Four 16-byte accesses per lane and array in
-// workgroups of 256 lanes; two per lane are 4 % slower, eight 9 %, 512 lanes 7 %.
+// tensors): 1.25 ms a step, 6.0 TB/s over the 40 bytes (1.31 with a contiguous chunk a
+// workgroup, cached accesses and the tensor found by a vector load), against 5.2 ms for
+// the element-wise operations.  The first pass has one 16-byte access per lane and array
+// in flight and every wavefront a compute unit can hold (37 registers): 715 us for 188 M
+// elements in launches of 5120 workgroups, 6.3 TB/s; four accesses a lane need 88
+// registers, hold five wavefronts a SIMD and reach the same only bare of everything else
+// (725).  The second is fastest with four (64 registers, 468 us, 6.4 TB/s), 10 % slower
+// with one.  Both lose 2 to 4 us a launch on its beginning and end.
 // Taking the tensors in groups small enough for the memory-side cache gains
 // nothing over the launches it adds, so a group is as many tensors as the arguments
 // hold, and its launches are cut by time only (kMomentsBlocks).
@@ -30,42 +35,72 @@
 
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kMomentsThreads = 1024, kThreads = 256;
 constexpr int kUnroll = 4;                            // 16-byte accesses per lane and array
 constexpr int kChunk = kThreads * 4 * kUnroll;        // elements per workgroup
-constexpr int kMaxTensors = 64;                       // one lane of a wavefront each
+static_assert(kChunk == kMomentsThreads * 4, "");
+constexpr int kMaxTensors = 64;
 constexpr int kReduceThreads = 1024;
 // Workgroups of one launch of each pass.  A launch cannot be held back once it has
 // begun, and best-effort kernels run on budgets of 100 us and more, so none takes longer
-// than that: 5120 (21 M elements) are 89 us of the first pass, 8192 (34 M) 87 us of the
-// second.  The step on the 188 M parameters: 1.286 ms in as few launches as the
-// arguments allow (0.54 ms the longest), 1.305 so, 1.343 with 4096 in both passes.
+// than that: 5120 (21 M elements) are 81 us of the first pass, 8192 (34 M) 84 us of the
+// second.
 constexpr uint64_t kMomentsBlocks = 5120, kUpdateBlocks = 8192;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// One launch's tensors, by value in the kernel's arguments (2.8 KiB): nothing to
+// The tensors of some launches, by value in the kernel's arguments (2.9 KiB): nothing to
 // upload, nothing that has to outlive the call.
 struct Group {
   orion_lamb_tensor t[kMaxTensors];
-  uint32_t first_block[kMaxTensors + 1];   // workgroups before tensor i
-  int count;
+  uint32_t first_block[kMaxTensors];       // workgroups before tensor i; past the last one all
+  uint32_t every8[8];                      // first_block[8 * i]
+  uint32_t blocks;
 };
 
 struct Coefs {
   float b1, b1c, b2, b2c, eps, decay;
 };
 
-// Tensor of this workgroup: every lane compares one entry of first_block.
-__device__ __forceinline__ int tensor_of_block(const Group& g, uint32_t block) {
-  const int lane = threadIdx.x & 63;
-  const bool before = lane < g.count && g.first_block[lane] <= block;
-  return __builtin_amdgcn_readfirstlane(__popcll(__ballot(before)) - 1);
+// Tensor of this workgroup, between the launch's first one and its last one.  All of it stays
+// in scalar registers and the scalar cache: a vector load, in which every lane compares an
+// entry, waits behind the arrays' (a step 1.28 ms so instead of 1.26).
+__device__ __forceinline__ int tensor_of_block(const Group& g, uint32_t block, int low, int high) {
+  if (low == high) return low;
+  int eight = 0, ti = 0;
+#pragma unroll
+  for (int i = 1; i < 8; ++i) eight += g.every8[i] <= block;
+#pragma unroll
+  for (int i = 1; i < 8; ++i) ti += g.first_block[eight * 8 + i] <= block;
+  return eight * 8 + ti;
 }
 
 __device__ __forceinline__ bool aligned16(const orion_lamb_tensor& t) {
   return ((((uintptr_t)t.w | (uintptr_t)t.g | (uintptr_t)t.m | (uintptr_t)t.v) & 15u) == 0);
 }
+
+// Where a workgroup's elements lie: kChunk / 256 pieces of one wavefront's access each, `step`
+// elements apart, U neighbours to a wavefront.  Eight workgroups in a row, which run on the
+// eight XCDs, share a window of 8 * kChunk elements piece by piece, so that what is under way
+// at a time lies close together in every array.  The accesses alone reach 6.4 TB/s so in the
+// first pass and 6.6 in the second; with a chunk a workgroup 6.1 and 6.4, and with cached
+// accesses 5.6 and 5.6.  A tensor's windows are counted from its start; in the last,
+// incomplete one every workgroup has a chunk.
+template <int U>
+struct Pieces {
+  uint64_t begin;                  // of the workgroup
+  uint32_t step;
+  bool whole;                      // no piece reaches past the tensor
+  __device__ __forceinline__ Pieces(uint32_t block, uint64_t n) {
+    const bool window = (uint64_t)((block | 7u) + 1) * kChunk <= n;
+    begin = window ? (uint64_t)(block & ~7u) * kChunk + (block & 7u) * 256 : (uint64_t)block * kChunk;
+    step = window ? 8 * 256 : 256;
+    whole = (uint64_t)(block + 1) * kChunk <= n;
+  }
+  __device__ __forceinline__ uint64_t at(int u) const {
+    return begin + ((threadIdx.x >> 6) * U + u) * step + (threadIdx.x & 63) * 4;
+  }
+};
 
 // Without decay the weight is not in the update at all: 0 * w would be a NaN for an
 // infinite weight, and through the norm for its whole tensor.
@@ -81,43 +116,35 @@ __device__ __forceinline__ void moments(float g, float& m, float& v, const Coefs
 }
 
 template <bool kDecay>
-__global__ __launch_bounds__(kThreads) void lamb_moments_kernel(Group g, Coefs c, uint32_t first,
-                                                                float2* partials) {
+__global__ __launch_bounds__(kMomentsThreads) void lamb_moments_kernel(
+    uint32_t first, int low, int high, float2* partials, Coefs c, Group g) {
   const uint32_t block = first + blockIdx.x;
-  const int ti = tensor_of_block(g, block);
+  const int ti = tensor_of_block(g, block, low, high);
   const orion_lamb_tensor t = g.t[ti];
-  const uint64_t base = (uint64_t)(block - g.first_block[ti]) * kChunk;
+  const Pieces<1> pieces(block - g.first_block[ti], t.n);
   float sw = 0.0f, su = 0.0f;
-  if (base + kChunk <= t.n && aligned16(t)) {
-    f32x4 vg[kUnroll], vm[kUnroll], vv[kUnroll], vw[kUnroll];
+  if (pieces.whole && aligned16(t)) {
+    const uint64_t i = pieces.at(0);
+    const f32x4 vg = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.g + i));
+    f32x4 vm = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.m + i));
+    f32x4 vv = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.v + i));
+    const f32x4 vw = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.w + i));
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const uint64_t i = base + (u * kThreads + threadIdx.x) * 4;
-      // the gradient is read once in a step: it must not push the others out
-      vg[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.g + i));
-      vm[u] = *reinterpret_cast<const f32x4*>(t.m + i);
-      vv[u] = *reinterpret_cast<const f32x4*>(t.v + i);
-      vw[u] = *reinterpret_cast<const f32x4*>(t.w + i);
+    for (int e = 0; e < 4; ++e) {
+      float m = vm[e], v = vv[e];
+      moments(vg[e], m, v, c);
+      vm[e] = m;
+      vv[e] = v;
+      const float w = vw[e], up = update_of<kDecay>(w, m, v, c);
+      sw = __builtin_fmaf(w, w, sw);
+      su = __builtin_fmaf(up, up, su);
     }
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const uint64_t i = base + (u * kThreads + threadIdx.x) * 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        float m = vm[u][e], v = vv[u][e];
-        moments(vg[u][e], m, v, c);
-        vm[u][e] = m;
-        vv[u][e] = v;
-        const float w = vw[u][e], up = update_of<kDecay>(w, m, v, c);
-        sw = __builtin_fmaf(w, w, sw);
-        su = __builtin_fmaf(up, up, su);
-      }
-      *reinterpret_cast<f32x4*>(t.m + i) = vm[u];
-      *reinterpret_cast<f32x4*>(t.v + i) = vv[u];
-    }
+    __builtin_nontemporal_store(vm, reinterpret_cast<f32x4*>(t.m + i));
+    __builtin_nontemporal_store(vv, reinterpret_cast<f32x4*>(t.v + i));
   } else {
+    const uint64_t base = (uint64_t)(block - g.first_block[ti]) * kChunk;
     const uint64_t end = base + kChunk < t.n ? base + kChunk : t.n;
-    for (uint64_t i = base + threadIdx.x; i < end; i += kThreads) {
+    for (uint64_t i = base + threadIdx.x; i < end; i += kMomentsThreads) {
       float m = t.m[i], v = t.v[i];
       moments(t.g[i], m, v, c);
       t.m[i] = m;
@@ -132,12 +159,12 @@ __global__ __launch_bounds__(kThreads) void lamb_moments_kernel(Group g, Coefs c
     sw += __shfl_xor(sw, d);
     su += __shfl_xor(su, d);
   }
-  __shared__ float2 wave_sums[kThreads / 64];
+  __shared__ float2 wave_sums[kMomentsThreads / 64];
   if ((threadIdx.x & 63) == 0) wave_sums[threadIdx.x >> 6] = make_float2(sw, su);
   __syncthreads();
   if (threadIdx.x == 0) {
     float2 s = wave_sums[0];
-    for (int w = 1; w < kThreads / 64; ++w) {
+    for (int w = 1; w < kMomentsThreads / 64; ++w) {
       s.x += wave_sums[w].x;
       s.y += wave_sums[w].y;
     }
@@ -147,11 +174,11 @@ __global__ __launch_bounds__(kThreads) void lamb_moments_kernel(Group g, Coefs c
 
 // One workgroup per tensor: the factor that the update is added with.
 __global__ __launch_bounds__(kReduceThreads) void lamb_ratio_kernel(
-    Group g, const float2* __restrict__ partials, float* __restrict__ factor, double lr,
-    double eps) {
+    const float2* __restrict__ partials, float* __restrict__ factor, double lr, double eps,
+    Group g) {
   const int ti = blockIdx.x;
   double sw = 0.0, su = 0.0;
-  const uint32_t end = g.first_block[ti + 1];
+  const uint32_t end = ti + 1 < kMaxTensors ? g.first_block[ti + 1] : g.blocks;
   uint32_t b = g.first_block[ti] + threadIdx.x;
   // eight loads in flight: one after the other they are a chain of cache misses
   // (52 us for the 33,000 partial sums of a 137M-element tensor)
@@ -190,32 +217,32 @@ __global__ __launch_bounds__(kReduceThreads) void lamb_ratio_kernel(
 }
 
 template <bool kDecay>
-__global__ __launch_bounds__(kThreads) void lamb_update_kernel(Group g, Coefs c, uint32_t first,
-                                                               const float* __restrict__ factor) {
-  // the first pass's last data first
-  const uint32_t block = g.first_block[kMaxTensors] - 1 - (first + blockIdx.x);
-  const int ti = tensor_of_block(g, block);
+__global__ __launch_bounds__(kMomentsThreads) void lamb_update_kernel(
+    uint32_t last, int low, int high, const float* __restrict__ factor, Coefs c, Group g) {
+  const uint32_t block = last - blockIdx.x;        // the first pass's last data first
+  const int ti = tensor_of_block(g, block, low, high);
   const orion_lamb_tensor t = g.t[ti];
-  const uint64_t base = (uint64_t)(block - g.first_block[ti]) * kChunk;
+  const Pieces<kUnroll> pieces(block - g.first_block[ti], t.n);
   const float f = factor[ti];
-  if (base + kChunk <= t.n && aligned16(t)) {
+  if (pieces.whole && aligned16(t)) {
     f32x4 vm[kUnroll], vv[kUnroll], vw[kUnroll];
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-      const uint64_t i = base + (u * kThreads + threadIdx.x) * 4;
+      const uint64_t i = pieces.at(u);
       vm[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.m + i));
       vv[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.v + i));
       vw[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.w + i));
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
-      const uint64_t i = base + (u * kThreads + threadIdx.x) * 4;
+      const uint64_t i = pieces.at(u);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         vw[u][e] = __builtin_fmaf(f, update_of<kDecay>(vw[u][e], vm[u][e], vv[u][e], c), vw[u][e]);
       __builtin_nontemporal_store(vw[u], reinterpret_cast<f32x4*>(t.w + i));
     }
   } else {
+    const uint64_t base = (uint64_t)(block - g.first_block[ti]) * kChunk;
     const uint64_t end = base + kChunk < t.n ? base + kChunk : t.n;
     for (uint64_t i = base + threadIdx.x; i < end; i += kThreads)
       t.w[i] = __builtin_fmaf(f, update_of<kDecay>(t.w[i], t.m[i], t.v[i], c), t.w[i]);
@@ -259,28 +286,38 @@ extern "C" int orion_lamb_step(const orion_lamb_tensor* tensors, int count, doub
   Group g;
   int next = 0;
   while (next < count) {
-    g.count = 0;
+    int tensors_in = 0;
     uint64_t blocks = 0;
-    for (; next < count && g.count < kMaxTensors; ++next) {
+    for (; next < count && tensors_in < kMaxTensors; ++next) {
       const orion_lamb_tensor& t = tensors[next];
       if (t.n == 0) continue;
-      g.t[g.count] = t;
-      g.first_block[g.count] = (uint32_t)blocks;
-      ++g.count;
+      g.t[tensors_in] = t;
+      g.first_block[tensors_in++] = (uint32_t)blocks;
       blocks += blocks_of(t.n);
     }
-    if (g.count == 0) break;
-    for (int i = g.count; i <= kMaxTensors; ++i) g.first_block[i] = (uint32_t)blocks;
-    for (uint64_t at = 0; at < blocks; at += kMomentsBlocks)
+    if (tensors_in == 0) break;
+    for (int i = tensors_in; i < kMaxTensors; ++i) g.first_block[i] = (uint32_t)blocks;
+    for (int i = 0; i < 8; ++i) g.every8[i] = g.first_block[8 * i];
+    g.blocks = (uint32_t)blocks;
+    auto tensor_at = [&](uint64_t block) {
+      return (int)(std::upper_bound(g.first_block, g.first_block + tensors_in, (uint32_t)block) -
+                   g.first_block) - 1;
+    };
+    for (uint64_t at = 0; at < blocks; at += kMomentsBlocks) {
+      const uint64_t n = std::min(kMomentsBlocks, blocks - at);
       hipLaunchKernelGGL(decay != 0.0 ? lamb_moments_kernel<true> : lamb_moments_kernel<false>,
-                         dim3((unsigned)std::min(kMomentsBlocks, blocks - at)), dim3(kThreads), 0,
-                         s, g, c, (uint32_t)at, partials);
-    hipLaunchKernelGGL(lamb_ratio_kernel, dim3((unsigned)g.count), dim3(kReduceThreads), 0, s, g,
-                       (const float2*)partials, factor, lr, eps);
-    for (uint64_t at = 0; at < blocks; at += kUpdateBlocks)
+                         dim3((unsigned)n), dim3(kMomentsThreads), 0, s, (uint32_t)at, tensor_at(at),
+                         tensor_at(at + n - 1), partials, c, g);
+    }
+    hipLaunchKernelGGL(lamb_ratio_kernel, dim3((unsigned)tensors_in), dim3(kReduceThreads), 0, s,
+                       (const float2*)partials, factor, lr, eps, g);
+    for (uint64_t end = blocks; end > 0;) {
+      const uint64_t n = std::min(kUpdateBlocks, end);
       hipLaunchKernelGGL(decay != 0.0 ? lamb_update_kernel<true> : lamb_update_kernel<false>,
-                         dim3((unsigned)std::min(kUpdateBlocks, blocks - at)), dim3(kThreads), 0,
-                         s, g, c, (uint32_t)at, (const float*)factor);
+                         dim3((unsigned)n), dim3(kThreads), 0, s, (uint32_t)(end - 1),
+                         tensor_at(end - n), tensor_at(end - 1), (const float*)factor, c, g);
+      end -= n;
+    }
   }
   return hipGetLastError() == hipSuccess ? ORION_OK : ORION_ERR_LAUNCH;
 }

@@ -63,6 +63,16 @@ def test_step_against_64_bits(sizes, offset, decay):
                                   atol=1e-6 * float(ref.abs().max()) if ref.numel() else 0)
 
 
+@pytest.mark.parametrize("offset", [0, 3])
+@pytest.mark.parametrize("sizes", [
+    # the last complete window of eight workgroups' 4096 elements, and what lies behind it
+    (32767, 32768, 32769, 36864, 65535, 65537, 98304 + 4095),
+    # every place of a tensor among the 64 of a launch, some of several workgroups
+    tuple(1 + 4099 * (i % 7) for i in range(129))])
+def test_windows_and_the_tensor_of_a_workgroup(sizes, offset):
+    test_step_against_64_bits(sizes, offset, 0.01)
+
+
 def test_same_bits_twice():
     runs = []
     for _ in range(2):
