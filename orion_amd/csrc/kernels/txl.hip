@@ -538,7 +538,7 @@ __global__ __launch_bounds__(kJobThreads, 1) void txl_jobs_kernel(Jobs jobs) {
 // counter says that they are done.  Its weights, 128 KiB, come meanwhile: a compute unit
 // takes in 60 to 100 KiB a us, and as much again of rows.  (16 rows more a panel and half the
 // columns a task than 32 rows and 64 or 256, which need twice the weights: 772 us a request
-// instead of 803.)  Panels are dealt out to up to eight groups of workgroups (with eight one
+// instead of 803.)  Panels are dealt out to one to eight groups of workgroups (with eight one
 // an XCD, which get workgroups in turn), evenly by 16 rows.
 //
 // Every wait ends, on any number of compute units and beside any other kernel: a group's
@@ -555,7 +555,7 @@ __global__ __launch_bounds__(kJobThreads, 1) void txl_jobs_kernel(Jobs jobs) {
 // stage whose 192 workgroups hand on 32 KiB a panel takes 1.6 us so (2.0 with a panel's
 // workgroups on all XCDs), 4.3 (6.8) with release and acquire fences, 2.5 to 2.9 as a launch.
 constexpr int kLayerThreads = 512;
-constexpr int kGroups = 8, kGroupMost = 32;          // workgroups of a group, one a compute unit
+constexpr int kGroups = 8;
 constexpr int kPanelTiles16 = 3, kPanelRows = 16 * kPanelTiles16;
 constexpr int kRowTileBytes = kPanelRows * kRowBytes;        // a panel's k-tile
 constexpr int kUnits4 = 4, kUnitCols = 32;           // a wave's weights: four k-tiles of 32 columns
@@ -2062,10 +2062,29 @@ struct Buffers {
   float *y, *y2;
   float2 *parts, *parts2;
   uint32_t* counters;
-  int panels;                // a group of a layer launch has at most
   size_t counts;
   size_t bytes;
 };
+
+// Panels of the largest of so many groups.
+size_t group_panels(size_t rows, size_t groups) {
+  return tiles(tiles(tiles(rows, 16), groups), kPanelTiles16);
+}
+
+// Groups of a layer launch, eight (an XCD each), four, two or one: those whose panels are the
+// fewest, since a panel that is not full takes as long as a full one and reads all weights;
+// as many as that allows.  us a request behind 192 tokens of memory on 32, 64, 128 and 256
+// compute units, by eight groups (or as many as there are tiles of 16 rows) and so: batch 1, 64
+// tokens 1120 and 880, 662 and 673, 580 and 590, 568 and 578; batch 2, 64 tokens 1618 and 1095,
+// 944 and 710, 626 and 624, 600 and 598; batch 1, 192 tokens 1740 and 1311, 1017 and 767, 656
+// and 646, 636 and 627; batch 3, 150 tokens 3350 and 2722, 1811 and 1487, 1060 and 887, 701
+// and 699.  Three, five to seven groups are no better: XCDs share theirs unevenly.
+size_t groups_of(size_t rows) {
+  size_t best = kGroups;
+  for (size_t g = kGroups; g > 0; g /= 2)
+    if (g * group_panels(rows, g) < best * group_panels(rows, best)) best = g;
+  return best;
+}
 
 Buffers buffers_of(const orion_txl_dims& d, void* base) {
   const size_t rows = (size_t)d.q_len * d.batch, mem_rows = (size_t)d.m_len * d.batch;
@@ -2076,8 +2095,8 @@ Buffers buffers_of(const orion_txl_dims& d, void* base) {
   b.parts = p.take<float2>(rows * kParts);
   b.y2 = p.take<float>(rows * kD);
   b.parts2 = p.take<float2>(rows * kParts);
-  b.panels = (int)tiles(tiles(tiles(rows, 16), kGroups), kPanelTiles16);
-  b.counts = (size_t)kLine * kGroups * (1 + 3 * (size_t)b.panels);
+  const size_t groups = groups_of(rows);
+  b.counts = (size_t)kLine * (kGroups + 3 * groups * group_panels(rows, groups));
   b.counters = p.take<uint32_t>(b.counts);
   b.x[0] = p.take<uint16_t>(rows * kD);
   b.x[1] = p.take<uint16_t>(rows * kD);
@@ -2201,9 +2220,9 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
   size_t panel_tasks = kResTasks;
   for (size_t columns : {(size_t)d.inner, 3 * (size_t)proj})
     if (columns / kNormCols > panel_tasks) panel_tasks = columns / kNormCols;
-  const size_t row_tiles = tiles(rows, 16), groups = row_tiles < kGroups ? row_tiles : kGroups;
-  const size_t group_tasks = panel_tasks * tiles(tiles(row_tiles, groups), kPanelTiles16);
-  const size_t layer_blocks = groups * (group_tasks < kGroupMost ? group_tasks : kGroupMost);
+  const size_t groups = groups_of(rows), panels = group_panels(rows, groups);
+  const size_t group_tasks = panel_tasks * panels, most = kUnits / groups;
+  const size_t layer_blocks = groups * (group_tasks < most ? group_tasks : most);
   for (int i = 0; i < d.layers; ++i) {
     const orion_txl_layer& p = layers[i];
     // a layer's input also goes into the memory's last rows
@@ -2259,7 +2278,7 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
     a.layer = i;
     a.inner = d.inner;
     a.proj = proj;
-    a.panels = w.panels;
+    a.panels = (int)panels;
     a.rows = rows;
     a.att = w.att;
     a.x = i == 0 ? (In)x0 : w.x[i & 1];

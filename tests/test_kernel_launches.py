@@ -178,18 +178,20 @@ def test_no_workgroup_of_a_layers_products_is_empty(run, q_len, batch):
     # the scheduler reads a launch's need of compute units from its number of workgroups
     ((rc, launches, _),) = run(TXL, [(2, 8, 2048, q_len, 192, batch, 256)])
     assert rc == 0
-    # rows go to up to eight groups of workgroups, evenly by 16, and in a group to panels of up
-    # to 48; a panel has 16 tasks of each product, and a group as many workgroups, at most 32
+    # rows go to eight, four, two or one groups of workgroups, evenly by 16, and in a group to
+    # panels of up to 48, the fewest in all; a panel has 16 tasks of each product, and a group
+    # as many workgroups, at most its share of 256
     tiles = -(-q_len * batch // 16)
-    groups = min(tiles, 8)
-    panels = -(-(-(-tiles // groups)) // 3)
+    panels_of = {groups: -(-(-(-tiles // groups)) // 3) for groups in (8, 4, 2, 1)}
+    groups = min(panels_of, key=lambda groups: groups * panels_of[groups])
+    panels, most = panels_of[groups], 256 // groups
     grids = {part: [grid for name, grid, _ in launches if part in name]
              for part in ("panel_gemm_kernelILi64ELi96E", "txl_layer_kernel")}
     assert grids == {"panel_gemm_kernelILi64ELi96E": [-(-q_len * batch // 64) * 3 * 8 * 64 // 96],
-                     "txl_layer_kernel": [groups * min(32, panels * 16)] * 2}
+                     "txl_layer_kernel": [groups * min(most, panels * 16)] * 2}
     # the smallest group's tasks of the last layer, which has three products
     fewest = -(-(tiles // groups) // 3) * 3 * 16
-    assert fewest >= min(32, panels * 16)
+    assert fewest >= min(most, panels * 16)
 
 
 @pytest.mark.parametrize("inner,q_len,batch,own,ahead", [
