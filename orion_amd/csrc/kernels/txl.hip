@@ -401,10 +401,15 @@ __global__ __launch_bounds__(kJobThreads, 1) void txl_jobs_kernel(Jobs jobs) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
-  const bool before = lane < jobs.count && jobs.first_block[lane] <= blockIdx.x;
+  // Each XCD (they get workgroups in turn) takes a contiguous share of the jobs, so that a
+  // layer's memory and weights go to one or two of them: with workgroups in order a batch-4
+  // request took 714 us, 709 so.
+  const unsigned xcd = blockIdx.x % 8, each = gridDim.x / 8, extra = gridDim.x % 8;
+  const unsigned block = xcd * each + (xcd < extra ? xcd : extra) + blockIdx.x / 8;
+  const bool before = lane < jobs.count && jobs.first_block[lane] <= block;
   const int i = __builtin_amdgcn_readfirstlane(__popcll(__ballot(before)) - 1);
   const Job job = jobs.job[i];
-  const int local = blockIdx.x - jobs.first_block[i];
+  const int local = block - jobs.first_block[i];
   const int tiles_n = (job.N + kJobN - 1) / kJobN;
   const int tn = local % tiles_n, row0 = local / tiles_n * (kJobPanels * kJobM);
   const int want = tn * kJobN + wave * kJobWaveN;
