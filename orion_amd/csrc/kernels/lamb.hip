@@ -11,7 +11,7 @@
 // all stayed on chip would move; as separate element-wise operations it is 100.
 //
 // Measured on the 16-layer, 267,735-token Transformer-XL (188 M parameters, 182
-// tensors): 1.25 ms a step, 6.0 TB/s over the 40 bytes (1.31 with a contiguous chunk a
+// tensors): 1.21 ms a step, 6.2 TB/s over the 40 bytes (1.31 with a contiguous chunk a
 // workgroup, cached accesses and the tensor found by a vector load), against 5.2 ms for
 // the element-wise operations.  The first pass has one 16-byte access per lane and array
 // in flight and every wavefront a compute unit can hold (37 registers): 715 us for 188 M
@@ -46,6 +46,13 @@ constexpr int kReduceThreads = 1024;
 // than that: 5120 (21 M elements) are 81 us of the first pass, 8192 (34 M) 84 us of the
 // second.
 constexpr uint64_t kMomentsBlocks = 5120, kUpdateBlocks = 8192;
+// The second pass begins with the first one's last data, so the launches that hold a group's
+// last 21 M elements leave the moments in the memory-side cache (168 MB of its 256); all
+// other accesses pass it by, gradients and weights among them.  us a step, nothing cached,
+// and so: 13.7 M parameters 97 and 89, 23.9 M 165 and 152, 85 M 585 and 555, 192 M 1290 and
+// 1245; the moments of all launches 1281, the second pass's accesses too 1366, the first
+// one's weights too 1251.  The same rule serves groups of any size, the smallest whole.
+constexpr uint64_t kKeptBlocks = 5120;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -115,7 +122,20 @@ __device__ __forceinline__ void moments(float g, float& m, float& v, const Coefs
   v = __builtin_fmaf(c.b2c * g, g, c.b2 * v);
 }
 
-template <bool kDecay>
+// Through the caches, or past them.
+template <bool kCached>
+__device__ __forceinline__ f32x4 load16(const float* p) {
+  const f32x4* from = reinterpret_cast<const f32x4*>(p);
+  return kCached ? *from : __builtin_nontemporal_load(from);
+}
+template <bool kCached>
+__device__ __forceinline__ void store16(const f32x4& v, float* p) {
+  f32x4* to = reinterpret_cast<f32x4*>(p);
+  if (kCached) *to = v;
+  else __builtin_nontemporal_store(v, to);
+}
+
+template <bool kDecay, bool kKept>
 __global__ __launch_bounds__(kMomentsThreads) void lamb_moments_kernel(
     uint32_t first, int low, int high, float2* partials, Coefs c, Group g) {
   const uint32_t block = first + blockIdx.x;
@@ -125,10 +145,10 @@ __global__ __launch_bounds__(kMomentsThreads) void lamb_moments_kernel(
   float sw = 0.0f, su = 0.0f;
   if (pieces.whole && aligned16(t)) {
     const uint64_t i = pieces.at(0);
-    const f32x4 vg = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.g + i));
-    f32x4 vm = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.m + i));
-    f32x4 vv = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.v + i));
-    const f32x4 vw = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.w + i));
+    const f32x4 vg = load16<false>(t.g + i);
+    f32x4 vm = load16<kKept>(t.m + i);
+    f32x4 vv = load16<kKept>(t.v + i);
+    const f32x4 vw = load16<false>(t.w + i);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       float m = vm[e], v = vv[e];
@@ -139,8 +159,8 @@ __global__ __launch_bounds__(kMomentsThreads) void lamb_moments_kernel(
       sw = __builtin_fmaf(w, w, sw);
       su = __builtin_fmaf(up, up, su);
     }
-    __builtin_nontemporal_store(vm, reinterpret_cast<f32x4*>(t.m + i));
-    __builtin_nontemporal_store(vv, reinterpret_cast<f32x4*>(t.v + i));
+    store16<kKept>(vm, t.m + i);
+    store16<kKept>(vv, t.v + i);
   } else {
     const uint64_t base = (uint64_t)(block - g.first_block[ti]) * kChunk;
     const uint64_t end = base + kChunk < t.n ? base + kChunk : t.n;
@@ -229,9 +249,9 @@ __global__ __launch_bounds__(kMomentsThreads) void lamb_update_kernel(
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       const uint64_t i = pieces.at(u);
-      vm[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.m + i));
-      vv[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.v + i));
-      vw[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(t.w + i));
+      vm[u] = load16<false>(t.m + i);
+      vv[u] = load16<false>(t.v + i);
+      vw[u] = load16<false>(t.w + i);
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
@@ -239,7 +259,7 @@ __global__ __launch_bounds__(kMomentsThreads) void lamb_update_kernel(
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         vw[u][e] = __builtin_fmaf(f, update_of<kDecay>(vw[u][e], vm[u][e], vv[u][e], c), vw[u][e]);
-      __builtin_nontemporal_store(vw[u], reinterpret_cast<f32x4*>(t.w + i));
+      store16<false>(vw[u], t.w + i);
     }
   } else {
     const uint64_t base = (uint64_t)(block - g.first_block[ti]) * kChunk;
@@ -305,7 +325,11 @@ extern "C" int orion_lamb_step(const orion_lamb_tensor* tensors, int count, doub
     };
     for (uint64_t at = 0; at < blocks; at += kMomentsBlocks) {
       const uint64_t n = std::min(kMomentsBlocks, blocks - at);
-      hipLaunchKernelGGL(decay != 0.0 ? lamb_moments_kernel<true> : lamb_moments_kernel<false>,
+      const bool kept = at + n + kKeptBlocks > blocks;
+      hipLaunchKernelGGL(decay != 0.0 ? (kept ? lamb_moments_kernel<true, true>
+                                              : lamb_moments_kernel<true, false>)
+                                      : (kept ? lamb_moments_kernel<false, true>
+                                              : lamb_moments_kernel<false, false>),
                          dim3((unsigned)n), dim3(kMomentsThreads), 0, s, (uint32_t)at, tensor_at(at),
                          tensor_at(at + n - 1), partials, c, g);
     }
