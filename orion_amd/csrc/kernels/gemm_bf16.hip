@@ -352,8 +352,9 @@ __global__ __launch_bounds__(GROUPS * 256, 1) void gemm_bf16_nt_tile_kernel(
   if constexpr (HALVES)
     stream_product_halves<TM, TN, NS>(acc, lds, K / kTileK, a, b, wm, wn, lane);
   else
-    stream_product<TM, TN, NS>(acc, lds + group * kGroupLds, K / (GROUPS * kTileK),
-                               GROUPS * kTileK, a, b, wm, wn, lane);
+    stream_product<TM, TN, NS, (GROUPS > 1)>(
+        acc, lds + group * kGroupLds, (K / kTileK + GROUPS - 1) / GROUPS, GROUPS * kTileK, a, b, wm,
+        wn, lane, (K / kTileK - group + GROUPS - 1) / GROUPS);
   block_sync();                        // the stages are free
   if (GROUPS > 1) {
     f32x4* other = reinterpret_cast<f32x4*>(lds) + wave * 64 + lane;
@@ -426,20 +427,26 @@ struct Cost {
   double fixed, per_tile;
 };
 struct TileCost {
-  int tm, tn, k;          // k: what the depth has to be a multiple of
+  int tm, tn, groups;     // of waves, which take turns at the k-tiles
   Cost whole, limited;
 };
 constexpr Cost kUnmeasured = {0.0, 0.0};
 constexpr TileCost kTiles[] = {
-    {256, 256, 64, {4.65, 0.958}, {4.0, 1.10}},
-    {256, 128, 64, {3.44, 0.584}, kUnmeasured},
-    {192, 128, 64, {3.92, 0.470}, kUnmeasured},
-    {128, 128, 64, {2.80, 0.336}, {2.0, 0.42}},
-    {96, 128, 64, {3.33, 0.305}, kUnmeasured},
-    {128, 64, 64, {1.7, 0.28}, {1.7, 0.28}},
-    {64, 64, 64, {1.5, 0.19}, {1.5, 0.19}},
-    {32, 64, 128, {1.5, 0.125}, {1.5, 0.125}},   // two groups of waves
+    {256, 256, 1, {4.65, 0.958}, {4.0, 1.10}},
+    {256, 128, 1, {3.44, 0.584}, kUnmeasured},
+    {192, 128, 1, {3.92, 0.470}, kUnmeasured},
+    {128, 128, 1, {2.80, 0.336}, {2.0, 0.42}},
+    {96, 128, 1, {3.33, 0.305}, kUnmeasured},
+    {128, 64, 1, {1.7, 0.28}, {1.7, 0.28}},
+    {64, 64, 1, {1.5, 0.19}, {1.5, 0.19}},
+    {32, 64, 2, {1.5, 0.125}, {1.5, 0.125}},
 };
+
+// k-tiles from which on a group of waves may have one less than the other.  By 64 x 64 tiles
+// and by 32 x 64, us: 512 x 1024 x 320 3.7 and 3.9, 256 x 512 x 448 3.8 and 3.8, 512 x 512 x
+// 576 4.1 and 4.0, 512 x 1024 x 1088 5.4 and 5.2, 512 x 512 x 2112 7.4 and 5.9, 256 x 1280 x
+// 4160 11.6 and 9.0, 256 x 512 x 8128 24.7 and 17.1.
+constexpr int kLeastUneven = 9;
 
 int tile_for(int M, int N, int K, int cus) {
   int best = 0;
@@ -447,9 +454,10 @@ int tile_for(int M, int N, int K, int cus) {
   for (int i = 0; i < (int)(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
     const TileCost& t = kTiles[i];
     const Cost& c = cus == stream_units::kWholeGpu ? t.whole : t.limited;
-    if (K % t.k != 0 || c.per_tile == 0.0) continue;
+    if ((K / BK % t.groups != 0 && K / BK < kLeastUneven) || c.per_tile == 0.0) continue;
     const long long blocks = (long long)((M + t.tm - 1) / t.tm) * ((N + t.tn - 1) / t.tn);
-    const double us = 1.5 + (double)((blocks + cus - 1) / cus) * (c.fixed + c.per_tile * (K / BK));
+    const int k_tiles = (K / BK + t.groups - 1) / t.groups * t.groups;
+    const double us = 1.5 + (double)((blocks + cus - 1) / cus) * (c.fixed + c.per_tile * k_tiles);
     if (i == 0 || us < best_us) {
       best = i;
       best_us = i == 0 ? 0.9 * us : us;

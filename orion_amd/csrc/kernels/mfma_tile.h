@@ -198,16 +198,20 @@ __device__ __forceinline__ void clear(f32x4 (&acc)[I][J]) {
 // staged through NS stages at `lds`.  The fragments of a whole k-tile are read
 // while the one before it is multiplied: behind the barrier the next tile has
 // landed, and every wave has this one in registers, so its stage is filled again.
-template <int BM, int BN, int NS>
+// kShared: groups of waves that meet at the same barriers take turns at the k-tiles, and
+// this one has `own` of them, KT or KT - 1 and at least one; for the one that it lacks it
+// loads its last one again, and does not multiply it.
+template <int BM, int BN, int NS, bool kShared = false>
 __device__ __forceinline__ void stream_product(f32x4 (&acc)[BM / 32][BN / 32],
                                                unsigned char* lds, int KT, int k_step,
                                                const Rows<BM>& a, const Rows<BN>& b, int wm,
-                                               int wn, int lane) {
+                                               int wn, int lane, int own = 0) {
   constexpr int kStage = Rows<BM>::kBytes + Rows<BN>::kBytes;
   constexpr int kLoads = Rows<BM>::kLoads + Rows<BN>::kLoads;
+  auto k_of = [&](int kt) { return (kShared && kt >= own ? own - 1 : kt) * k_step; };
   auto issue = [&](int kt, unsigned char* s) {
-    a.issue(kt * k_step, s);
-    b.issue(kt * k_step, s + Rows<BM>::kBytes);
+    a.issue(k_of(kt), s);
+    b.issue(k_of(kt), s + Rows<BM>::kBytes);
   };
   auto read = [&](Fragments<BM, BN>& f, unsigned char* s) {
     f.read(s, s + Rows<BM>::kBytes, wm, wn, lane);
@@ -236,8 +240,8 @@ __device__ __forceinline__ void stream_product(f32x4 (&acc)[BM / 32][BN / 32],
         acc, now,
         [&](int r) { next.read_one(r, cur, cur + Rows<BM>::kBytes, wm, wn, lane); },
         [&](int l) {
-          if (l < Rows<BM>::kLoads) a.issue_one(l, (kt + NS) * k_step, freed);
-          else b.issue_one(l - Rows<BM>::kLoads, (kt + NS) * k_step, freed + Rows<BM>::kBytes);
+          if (l < Rows<BM>::kLoads) a.issue_one(l, k_of(kt + NS), freed);
+          else b.issue_one(l - Rows<BM>::kLoads, k_of(kt + NS), freed + Rows<BM>::kBytes);
         });
   };
   // between these parts the compiler may move accumulators and fragments
@@ -259,7 +263,7 @@ __device__ __forceinline__ void stream_product(f32x4 (&acc)[BM / 32][BN / 32],
     even = odd;
   }
   settle(acc);
-  multiply(acc, even);
+  if (!kShared || own == KT) multiply(acc, even);
   settle(acc);
 }
 

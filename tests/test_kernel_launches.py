@@ -98,6 +98,13 @@ def test_gemm_edge_cases_run_on_the_tiles_that_they_name(run):
     assert {m % 96 for tile, (m, _, _) in EDGE_TILES if tile == "96x128"} == {0, 32, 64}
 
 
+def test_gemm_two_wave_groups_take_uneven_depths_from_nine_k_tiles_on(run):
+    from tests.test_kernels_gpu import UNEVEN_DEPTHS
+    for depths, tile in ((UNEVEN_DEPTHS, "ILi32ELi64E"), ((64, 192, 320, 448), "ILi64ELi64E")):
+        for rc, ((name, _, _),), _ in run(GEMM, [(256, 512, k, 256, True) for k in depths]):
+            assert rc == 0 and f"tile_kernel{tile}" in name
+
+
 def test_gemm_on_limited_streams_by_costs_measured_there(run):
     # 128 x 128 tiles 5 to 18 % faster than the 256 x 256 that the whole GPU's costs ask for
     cases = [(768, 2816, 384, 128, 132), (2048, 1792, 448, 128, 224), (512, 4352, 448, 128, 136),

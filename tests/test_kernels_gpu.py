@@ -227,6 +227,24 @@ def test_gemm_two_wave_groups_exact_on_small_integers(k):
         assert torch.equal(kernels.gemm_bf16_nt(ta, tb, out_dtype=dtype), want.to(dtype))
 
 
+# one group has a k-tile less: 4 to 8 and 63 of them; test_kernel_launches.py holds them to the tile
+UNEVEN_DEPTHS = [576, 704, 832, 960, 1088, 8128]
+
+
+@pytest.mark.parametrize("k", UNEVEN_DEPTHS)
+def test_gemm_two_wave_groups_of_uneven_depth_exact_on_small_integers(k):
+    """As above; what lies around the operands is infinite and reaches no result."""
+    g = torch.Generator(device=DEV).manual_seed(k)
+    around = [torch.full((rows + 512, k), float("inf"), device=DEV, dtype=torch.bfloat16)
+              for rows in (256, 512)]
+    ta, tb = (t[256:-256] for t in around)
+    for t in (ta, tb):
+        t.copy_(torch.randint(-4, 5, t.shape, device=DEV, generator=g))
+    want = ta.float() @ tb.float().t()
+    for dtype in (torch.float32, torch.bfloat16):
+        assert torch.equal(kernels.gemm_bf16_nt(ta, tb, out_dtype=dtype), want.to(dtype))
+
+
 # Depths around the stages of the tiles by k-steps, and partial last tiles of those that do
 # not divide 256; test_kernel_launches.py holds each shape to its tile.
 EDGE_TILES = [
