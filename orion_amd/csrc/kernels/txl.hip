@@ -1025,20 +1025,30 @@ struct Layer {
   RowsOut rows_out;                       // the next layer's input
   QkvEpi qkv;
   uint32_t* counters;                     // kLine apart: 8 of tasks, then 3 a panel
-  int layer, rows, inner, proj, groups, panels;   // panels a group has counters for
+  int rows, inner, proj, panels;          // panels a group has counters for
 };
 
-// The kernel's arguments, read anew where they are needed (from the scalar cache): sixty
+// What a workgroup needs before it has a task comes first, by value, in registers; the
+// workgroup asks for its first task with it and reads the rest meanwhile (a batch-4 request
+// 669 us so and 684 with all of it in the structure, batch 1, 16 tokens 519 and 531).
+struct alignas(8) LayerStart {
+  uint32_t* counters;
+  int group_mask, group_shift;            // of 1, 2, 4 or 8 groups
+  int tiles16, layer;                     // tiles of 16 rows; of the layers
+};
+// The other arguments, read anew where they are needed (from the scalar cache): sixty
 // registers of them do not fit, and the compiler would keep them in lanes of vector ones.
 __device__ __forceinline__ const Layer& arguments() {
-  auto at = (const __attribute__((address_space(4))) Layer*)__builtin_amdgcn_kernarg_segment_ptr();
+  auto at = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(at));
-  return *(const Layer*)at;
+  return *(const Layer*)(at + sizeof(LayerStart));
 }
 
-__global__ __launch_bounds__(kLayerThreads, 1) void txl_layer_kernel(Layer) {
+__global__ __launch_bounds__(kLayerThreads, 1) void txl_layer_kernel(
+    uint32_t* all_counters, int group_mask, int group_shift, int all16, int layer, Layer) {
+  // LayerStart, which has to arrive in registers, and behind it the structure
   __shared__ __attribute__((aligned(16))) unsigned char lds[kLayerLds + 16];
-  const int group = blockIdx.x % arguments().groups;
+  const int group = blockIdx.x & group_mask;
   // this group's share of the row tiles, and its panels': even ones
   int first16, tiles16, panels;
   int ff1_at, ff2_at, qkv_at, tasks;     // tasks before each product's
@@ -1047,11 +1057,12 @@ __global__ __launch_bounds__(kLayerThreads, 1) void txl_layer_kernel(Layer) {
   run.lds = lds;
   run.taken = reinterpret_cast<uint32_t*>(lds + kLayerLds);
   run.place = Place::kFirst;
+  run.next = all_counters + group * kLine;
+  uint32_t first_taken = 0;
+  if (threadIdx.x == 0) first_taken = run.take();
   {
     const Layer& a = arguments();
-    run.next = a.counters + group * kLine;
-    if (threadIdx.x == 0) *run.taken = run.take();
-    const int all16 = (a.rows + 15) / 16, each = all16 / a.groups, extra = all16 % a.groups;
+    const int each = all16 >> group_shift, extra = all16 & group_mask;
     tiles16 = each + (group < extra ? 1 : 0);
     first16 = group * each + (group < extra ? group : extra);
     panels = (tiles16 + kPanelTiles16 - 1) / kPanelTiles16;
@@ -1060,10 +1071,19 @@ __global__ __launch_bounds__(kLayerThreads, 1) void txl_layer_kernel(Layer) {
     qkv_at = ff2_at + ff1_at;
     const int all = qkv_at + panels * a.product[3].tasks;
     tasks = a.products == 4 ? all : qkv_at;
-    // every workgroup takes one task more than there are
-    before = (uint32_t)a.layer * (all + gridDim.x / a.groups);
+    before = (uint32_t)layer * (all + (gridDim.x >> group_shift));
+    // every cache line of the arguments
+    auto line = [&](int i) {
+      return *reinterpret_cast<const int*>(reinterpret_cast<const char*>(&a) + 64 * i);
+    };
+    static_assert(sizeof(Layer) > 5 * 64 && sizeof(Layer) <= 6 * 64, "six lines");
+    asm volatile("" ::"s"(line(0)), "s"(line(1)), "s"(line(2)), "s"(line(3)), "s"(line(4)),
+                 "s"(line(5)));
   }
-  const int share = tiles16 / panels, larger = tiles16 - share * panels;
+  if (threadIdx.x == 0) *run.taken = first_taken;
+  // tiles16 / panels, of the fewest panels that hold them
+  const int share = panels == 1 ? tiles16 : kPanelTiles16 - (tiles16 < kPanelTiles16 * panels);
+  const int larger = tiles16 - share * panels;
   struct Task {
     int number, stage, panel, tn;
   };
@@ -1097,7 +1117,7 @@ __global__ __launch_bounds__(kLayerThreads, 1) void txl_layer_kernel(Layer) {
     const int end = (from16 + share + (p < larger ? 1 : 0)) * 16;
     const Panel panel = {from16 * 16, (end < a.rows ? end : a.rows) - from16 * 16};
     uint32_t* const counters = a.counters + (size_t)(kGroups + (group * a.panels + p) * 3) * kLine;
-    const uint32_t times = a.layer + 1;
+    const uint32_t times = layer + 1;
     Task coming = {tasks, 0, 0, 0};
     Plan then = {};
     auto look_ahead = [&]() {
@@ -2280,7 +2300,6 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
     a.products = i + 1 < d.layers ? 4 : 3;
     a.ff1_b = (In)p.ff1_b;
     a.ff2_b = (In)p.ff2_b;
-    a.layer = i;
     a.inner = d.inner;
     a.proj = proj;
     a.panels = (int)panels;
@@ -2301,9 +2320,9 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
       a.qkv = {w.qu, w.qv, w.kv_x, (In)u, (In)v, proj};
     }
     a.counters = w.counters;
-    a.groups = (int)groups;
     hipLaunchKernelGGL(txl_layer_kernel, dim3((unsigned)layer_blocks), dim3(kLayerThreads), 0, s,
-                       a);
+                       w.counters, (int)groups - 1, __builtin_ctz((unsigned)groups),
+                       (int)tiles(rows, 16), i, a);
   }
   const orion_txl_layer& last = layers[d.layers - 1];
   hipLaunchKernelGGL(txl_norm_kernel, dim3((unsigned)tiles(rows, kThreads / 16)), dim3(kThreads), 0,
