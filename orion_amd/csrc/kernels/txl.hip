@@ -96,6 +96,17 @@ __device__ __forceinline__ float sum_over_rows(float v) {
   return over_rows(v, [](float a, float b) { return a + b; });
 }
 
+// n / d and n % d in scalar registers, given ~0u / d; the compiler's own division begins with
+// a reciprocal in vector ones and takes four times as many instructions.
+struct Divided {
+  uint32_t quotient, rest;
+};
+__device__ __forceinline__ Divided divide(uint32_t n, uint32_t d, uint32_t inverse) {
+  uint32_t q = __umulhi(n, inverse);               // or one more
+  if (n - q * d >= d) ++q;
+  return {q, n - q * d};
+}
+
 struct Norm {
   const uint16_t* w;
   const uint16_t* b;
@@ -1014,7 +1025,7 @@ struct Layer {
     const uint16_t* W;
     int ld, columns;                      // of a task
     int tasks;                            // of a panel
-    uint32_t inverse;                     // 2^32 over them
+    uint32_t inverse;                     // ~0u over them
   } product[4];                           // out, ff1, ff2, the next layer's qkv
   int products;                           // 4, in the last layer 3
   const uint16_t *att, *x, *ff1_b, *ff2_b;
@@ -1092,15 +1103,14 @@ __global__ __launch_bounds__(kLayerThreads, 1) void txl_layer_kernel(
     const unsigned at =
         number - (stage < 2 ? (stage == 0 ? 0 : ff1_at) : stage == 2 ? ff2_at : qkv_at);
     const Layer::Product& product = arguments().product[stage];
-    unsigned panel = __umulhi(at, product.inverse);    // or one more
-    if (at - panel * product.tasks >= (unsigned)product.tasks) ++panel;
-    const int tn = (int)(at - panel * product.tasks), wave = run.wave();
+    const Divided by_tasks = divide(at, product.tasks, product.inverse);
+    const int panel = by_tasks.quotient, tn = by_tasks.rest, wave = run.wave();
     const int col0 = tn * product.columns + (stage & 1 ? (wave & 3) * kUnitCols : 0);
     // a sum's waves share the depth, a norm's two halves
     const int first = stage == 0 ? wave : (stage == 2 ? wave : wave >> 2) * kUnits4;
     *plan = plan_of(product.W + (size_t)col0 * product.ld, product.ld, first,
                     stage == 0 ? 1 : kUnits4, thread_of_task() & 63);
-    return Task{number, stage, (int)panel, tn};
+    return Task{number, stage, panel, tn};
   };
   block_sync();
   const int number = (int)(__builtin_amdgcn_readfirstlane(*run.taken) - before);
@@ -1264,7 +1274,10 @@ __global__ __launch_bounds__(kD / 2) void txl_positions_kernel(uint16_t* table,
 // Bound by LDS and by the softmax's arithmetic, of two waves a SIMD: at batch 4 (192
 // workgroups, 384 keys, 3 stages) a stage takes 1.6 us of every wave and a
 // launch 8.2; with 64 queries a workgroup, 96 of them, 2.1 and 10.1.  The next stage's rows
-// travel through registers while this one is worked on.
+// travel through registers while this one is worked on.  The arguments that the first stage's
+// loads need are the leading ones, which arrive in registers (fourteen of them); the queries
+// are asked for behind those loads (a batch-4 request 658 us so, 671 with a wait for arguments
+// before the first load and two divisions there; batch 1, 16 tokens 515 and 520).
 constexpr int kAttnThreads = 512;
 constexpr int kQ = 32, kKeys = 128;
 constexpr int kParts4 = 4, kPartKeys = kKeys / kParts4;
@@ -1295,12 +1308,11 @@ constexpr uint32_t kTouchBytes = 192 << 10, kUnits = 256;
 struct Coming {
   const uint16_t* p[4];
   uint32_t bytes[4];                   // multiples of 16
-  uint32_t first_block;                // of the launch
 };
-__device__ __forceinline__ void touch(const Coming& coming) {
+__device__ __forceinline__ void touch(const Coming& coming, uint32_t first_block) {
   constexpr uint32_t kEach = kAttnThreads * 16, kUnroll = 4;
-  const uint32_t step = (gridDim.x - coming.first_block) * kEach;
-  const uint32_t mine = (blockIdx.x - coming.first_block) * kEach + threadIdx.x * 16;
+  const uint32_t step = (gridDim.x - first_block) * kEach;
+  const uint32_t mine = (blockIdx.x - first_block) * kEach + threadIdx.x * 16;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const char* p = reinterpret_cast<const char*>(coming.p[i]);
@@ -1318,21 +1330,24 @@ __device__ __forceinline__ void touch(const Coming& coming) {
 }
 
 __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
-    const uint16_t* __restrict__ qu, const uint16_t* __restrict__ qv,
     const uint16_t* __restrict__ kv_mem, const uint16_t* __restrict__ kv_x,
-    const uint16_t* __restrict__ r, uint16_t* __restrict__ out, int qlen, int mlen, int batch,
-    int heads, uint32_t first, Coming coming) {
+    const uint16_t* __restrict__ r, int qlen, int mlen, int batch, int heads, uint32_t first,
+    uint32_t own, uint32_t inverse_heads, uint32_t inverse_batch,
+    const uint16_t* __restrict__ qu, const uint16_t* __restrict__ qv, uint16_t* __restrict__ out,
+    Coming coming) {
   __shared__ __attribute__((aligned(16))) unsigned char lds[kAttnLds];
-  if (blockIdx.x >= coming.first_block) {
-    touch(coming);
+  if (blockIdx.x >= own) {
+    touch(coming, own);
     return;
   }
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
   const uint32_t block = first + blockIdx.x;
-  const int head = block % heads, b = block / heads % batch;
-  const int q0 = block / heads / batch * kQ;
+  const Divided by_heads = divide(block, heads, inverse_heads);
+  const Divided by_batch = divide(by_heads.quotient, batch, inverse_batch);
+  const int head = by_heads.rest, b = by_batch.rest;
+  const int q0 = by_batch.quotient * kQ;
   const int klen = mlen + qlen;
   const int proj = heads * kHead;
   const int qt = wave & 1, part = wave >> 1;
@@ -1389,6 +1404,8 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
     }
   };
 
+  fetch(0);
+  __builtin_amdgcn_sched_barrier(0);
   const int qi = q0 + qt * 16 + l16;            // this lane's query
   bf16x8 fqu[2], fqv[2];
   {
@@ -1412,7 +1429,6 @@ __global__ __launch_bounds__(kAttnThreads, 1) void txl_attention_kernel(
   float m = -__builtin_inff(), l = 0.0f;
   const int last_query = q0 + kQ <= qlen ? q0 + kQ - 1 : qlen - 1;
   const int stages = (mlen + last_query) / kKeys + 1;
-  fetch(0);
   for (int st = 0; st < stages; ++st) {
     const int j0 = st * kKeys;
     if (st > 0) block_sync();                   // everyone is done with the last stage
@@ -2280,13 +2296,12 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
     if (i + 1 < d.layers) add_coming(layers[i + 1].qkv, 3 * (size_t)proj);
     for (size_t first = 0; first < attn_blocks; first += kAttnMost) {
       const size_t own = attn_blocks - first < kAttnMost ? attn_blocks - first : kAttnMost;
-      coming.first_block = (uint32_t)own;
       hipLaunchKernelGGL(txl_attention_kernel,
                          dim3((unsigned)(own + tiles(ahead, kTouchBytes))), dim3(kAttnThreads), 0,
-                         s, (In)w.qu, (In)w.qv,
-                         (In)(w.kv_mem + (size_t)i * mem_rows * 2 * proj), (In)w.kv_x,
-                         (In)(w.r + (size_t)i * k_len * proj), w.att, d.q_len, d.m_len, d.batch,
-                         d.heads, (uint32_t)first, coming);
+                         s, (In)(w.kv_mem + (size_t)i * mem_rows * 2 * proj), (In)w.kv_x,
+                         (In)(w.r + (size_t)i * k_len * proj), d.q_len, d.m_len, d.batch, d.heads,
+                         (uint32_t)first, (uint32_t)own, ~0u / (uint32_t)d.heads,
+                         ~0u / (uint32_t)d.batch, (In)w.qu, (In)w.qv, w.att, coming);
     }
     Layer a = {};
     auto product = [&](int stage, const void* W, int ld, int columns, int tasks) {
