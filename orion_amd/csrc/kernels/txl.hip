@@ -546,8 +546,8 @@ __global__ __launch_bounds__(kJobThreads, 1) void txl_jobs_kernel(Jobs jobs) {
 // the next layer's queries, keys and values.  As launches of their own, with 64 x 96, 64 x
 // 128 and 32 x 64 tiles, the four products took 32 us of a batch-4 request's layer: a launch
 // begins 2 us after the last one ends, waits 2 us for its first data and reads weights only
-// then.  So 24: 4 for the first product, 6.5, 5.5 and 5.5 for the others (a request 694 us
-// instead of 801; batch 1, 16 tokens 555 and 660; batch 16 2050 and 2183).
+// then.  So 24: 4 for the first product, 6.5, 5.5 and 5.5 for the others (a request 664 us
+// instead of 801; batch 1, 16 tokens without memory 529 and 644).
 //
 // Rows come in panels of up to 48.  The work is a list of tasks, 32 or 128 columns of a
 // product for a panel; a task that reads what others of its panel write waits until a
@@ -1273,7 +1273,7 @@ __global__ __launch_bounds__(kD / 2) void txl_positions_kernel(uint16_t* table,
 //
 // Bound by LDS and by the softmax's arithmetic, of two waves a SIMD: at batch 4 (192
 // workgroups, 384 keys, 3 stages) a stage takes 1.6 us of every wave and a
-// launch 8.2; with 64 queries a workgroup, 96 of them, 2.1 and 10.1.  The next stage's rows
+// launch 8.0; with 64 queries a workgroup, 96 of them, 2.1 and 10.1.  The next stage's rows
 // travel through registers while this one is worked on.  The arguments that the first stage's
 // loads need are the leading ones, which arrive in registers (fourteen of them); the queries
 // are asked for behind those loads (a batch-4 request 658 us so, 671 with a wait for arguments

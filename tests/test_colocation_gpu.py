@@ -440,7 +440,7 @@ def test_transformer_xl_bf16_inference_client(tmp_path, best_effort):
     with open(filled[mine]["kernel_file"]) as f:
         rows = [line.split(",") for line in f.read().splitlines()[1:]]
     own = [r for r in rows if "txl_" in r[0] or "crit_" in r[0]]
-    assert len(own) == 2 + 5 * small["n_layer"] + 1 + 3
+    assert len(own) == 3 + 2 * small["n_layer"] + 1 + 3
     assert {int(r[1]) for r in own if "txl_" in r[0] and "positions" not in r[0]} <= {0, 1}
 
     with cc.MODEL_INIT_LOCK:
