@@ -2118,11 +2118,16 @@ size_t group_panels(size_t rows, size_t groups) {
 // compute units, by eight groups (or as many as there are tiles of 16 rows) and so: batch 1, 64
 // tokens 1120 and 880, 662 and 673, 580 and 590, 568 and 578; batch 2, 64 tokens 1618 and 1095,
 // 944 and 710, 626 and 624, 600 and 598; batch 1, 192 tokens 1740 and 1311, 1017 and 767, 656
-// and 646, 636 and 627; batch 3, 150 tokens 3350 and 2722, 1811 and 1487, 1060 and 887, 701
-// and 699.  Three, five to seven groups are no better: XCDs share theirs unevenly.
+// and 646, 636 and 627; batch 3, 150 tokens 3350 and 2921, 1811 and 1618, 1060 and 959, 701
+// and 701.  Three, five to seven groups are no better: XCDs share theirs unevenly.  Two or one
+// are for rows that eight full panels hold: with more of them every XCD has work of every panel,
+// and requests on the whole GPU take longer (by four groups and by one: batch 4, 100 tokens 617
+// and 642, 120 tokens 635 and 682, batch 3, 160 tokens 641 and 709; batch 40, 200 tokens
+// without memory 4539 and 4680).
 size_t groups_of(size_t rows) {
+  const bool few = rows <= kGroups * kPanelRows;
   size_t best = kGroups;
-  for (size_t g = kGroups; g > 0; g /= 2)
+  for (size_t g = kGroups; g >= (few ? 1u : kGroups / 2); g /= 2)
     if (g * group_panels(rows, g) < best * group_panels(rows, best)) best = g;
   return best;
 }

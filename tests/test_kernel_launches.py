@@ -185,11 +185,11 @@ def test_no_workgroup_of_a_layers_products_is_empty(run, q_len, batch):
     # the scheduler reads a launch's need of compute units from its number of workgroups
     ((rc, launches, _),) = run(TXL, [(2, 8, 2048, q_len, 192, batch, 256)])
     assert rc == 0
-    # rows go to eight, four, two or one groups of workgroups, evenly by 16, and in a group to
-    # panels of up to 48, the fewest in all; a panel has 16 tasks of each product, and a group
-    # as many workgroups, at most its share of 256
+    # rows go to eight, four, or where eight panels hold them two or one groups of workgroups,
+    # evenly by 16, and in a group to panels of up to 48, the fewest in all; a panel has 16
+    # tasks of each product, and a group as many workgroups, at most its share of 256
     tiles = -(-q_len * batch // 16)
-    panels_of = {groups: -(-(-(-tiles // groups)) // 3) for groups in (8, 4, 2, 1)}
+    panels_of = {groups: -(-(-(-tiles // groups)) // 3) for groups in ((8, 4, 2, 1) if tiles <= 24 else (8, 4))}
     groups = min(panels_of, key=lambda groups: groups * panels_of[groups])
     panels, most = panels_of[groups], 256 // groups
     grids = {part: [grid for name, grid, _ in launches if part in name]
