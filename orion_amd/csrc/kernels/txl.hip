@@ -566,7 +566,7 @@ __global__ __launch_bounds__(kJobThreads, 1) void txl_jobs_kernel(Jobs jobs) {
 // What one workgroup writes and another reads within the launch is written through to
 // memory (sc1, agent scope), and a counter is raised when its workgroup's stores have been
 // acknowledged.  Readers may cache it: a line of it holds one panel's values of one product
-// only, no one reads it in this launch before the counter says so, and caches start a launch
+// only (Pieces), no one reads it in this launch before the counter says so, and caches start a launch
 // without lines of the launches before.  So nothing depends on where a workgroup runs.  A
 // stage whose 192 workgroups hand on 32 KiB a panel takes 1.6 us so (2.0 with a panel's
 // workgroups on all XCDs), 4.3 (6.8) with release and acquire fences, 2.5 to 2.9 as a launch.
@@ -2084,10 +2084,15 @@ __global__ __launch_bounds__(kThreads) void crit_losses_kernel(Crit c, uint16_t*
   if (lane == 0) nll[row] = (uint16_t)pack_bf16(loss, 0.0f);
 }
 
-// Pieces of a workspace, 256-byte aligned; with no base only their sizes add up.
+// Pieces of a workspace, each in cache lines of its own whatever the workspace's alignment (16
+// bytes at least): a layer launch's visibility needs that.  With no base only their sizes add up.
 struct Pieces {
+  static constexpr size_t kAlign = 128;
   char* base;
   size_t used = 0;
+  explicit Pieces(void* workspace)
+      : base((char*)(((uintptr_t)workspace + kAlign - 1) & ~(uintptr_t)(kAlign - 1))) {}
+  size_t bytes() const { return used + kAlign - 16; }
   template <typename T>
   T* take(size_t count) {
     T* p = base ? reinterpret_cast<T*>(base + used) : nullptr;
@@ -2135,7 +2140,7 @@ size_t groups_of(size_t rows) {
 Buffers buffers_of(const orion_txl_dims& d, void* base) {
   const size_t rows = (size_t)d.q_len * d.batch, mem_rows = (size_t)d.m_len * d.batch;
   const size_t proj = (size_t)d.heads * kHead, k_len = (size_t)d.q_len + d.m_len;
-  Pieces p{(char*)base};
+  Pieces p(base);
   Buffers b;
   b.y = p.take<float>(rows * kD);
   b.parts = p.take<float2>(rows * kParts);
@@ -2155,7 +2160,7 @@ Buffers buffers_of(const orion_txl_dims& d, void* base) {
   b.kv_mem = p.take<uint16_t>(d.layers * mem_rows * 2 * proj);
   b.table = p.take<uint16_t>(k_len * kD);
   b.r = p.take<uint16_t>(d.layers * k_len * proj);
-  b.bytes = p.used;
+  b.bytes = p.bytes();
   return b;
 }
 
@@ -2186,7 +2191,7 @@ bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
   const size_t head = tiles(a->rows, kCritM) * tiles(a->edges[1], kCritN);
   const size_t least = tiles(head, kCritBlocks);
   c->least = (int)(least < kCritLeast ? kCritLeast : least > kCritMost ? kCritMost : least);
-  Pieces p{(char*)base};
+  Pieces p(base);
   c->plan = p.take<CritPlan>(1);
   c->count = p.take<int>(kMaxTails);
   c->place = p.take<int>(a->rows);
@@ -2195,7 +2200,7 @@ bool lay_out(const orion_nll* a, void* base, Crit* c, size_t* bytes) {
     c->stride[k] = (int)tiles((size_t)c->edge[k + 1] - c->edge[k], kCritN * c->least);
     c->pairs[k] = p.take<float2>((size_t)a->rows * c->stride[k]);
   }
-  *bytes = p.used;
+  *bytes = p.bytes();
   return true;
 }
 

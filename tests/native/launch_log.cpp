@@ -14,6 +14,7 @@ struct Dim3 {
 struct Launch {
   std::string name;
   Dim3 grid, block;
+  std::vector<uint64_t> words;      // of the watched argument
 };
 struct Config {
   Dim3 grid, block;
@@ -26,6 +27,10 @@ std::map<const void*, std::string>& names() {
 }
 std::vector<Launch> launches;
 Config pushed;
+// the leading words of an argument of the kernels whose names contain a text
+std::string watched;
+int watched_argument = 0;
+size_t watched_words = 0;
 int compute_units = 256;      // of every stream; 0: the query fails
 int queries = 0;
 int last_error = 0;
@@ -38,6 +43,13 @@ const char* launch_log_name(int i) { return launches[i].name.c_str(); }
 unsigned launch_log_grid(int i) { return launches[i].grid.x * launches[i].grid.y; }
 unsigned launch_log_block(int i) { return launches[i].block.x; }
 void launch_log_set_compute_units(int n) { compute_units = n; }
+void launch_log_watch(const char* name, int argument, int words) {
+  watched = name;
+  watched_argument = argument;
+  watched_words = words;
+}
+int launch_log_words(int i) { return (int)launches[i].words.size(); }
+uint64_t launch_log_word(int i, int k) { return launches[i].words[k]; }
 int launch_log_queries() { return queries; }
 int launch_log_kernels() { return (int)names().size(); }
 const char* launch_log_kernel(int i) {
@@ -66,8 +78,12 @@ int __hipPopCallConfiguration(Dim3* grid, Dim3* block, size_t* shmem, void** str
   *stream = pushed.stream;
   return 0;
 }
-int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void**, size_t, void*) {
-  launches.push_back({names().count(f) ? names()[f] : "unknown", grid, block});
+int hipLaunchKernel(const void* f, Dim3 grid, Dim3 block, void** args, size_t, void*) {
+  launches.push_back({names().count(f) ? names()[f] : "unknown", grid, block, {}});
+  if (watched_words && launches.back().name.find(watched) != std::string::npos) {
+    launches.back().words.resize(watched_words);
+    memcpy(launches.back().words.data(), args[watched_argument], watched_words * 8);
+  }
   return 0;
 }
 int hipExtStreamGetCUMask(void*, uint32_t words, uint32_t* mask) {

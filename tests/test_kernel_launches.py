@@ -226,6 +226,33 @@ def test_no_launch_of_attention_has_more_threads_than_a_grid_can_have(run):
     assert all(grid * block < 1 << 32 for grid, block in attention)
 
 
+WORKSPACE = """
+log.launch_log_watch(b"txl_layer", 5, 40)          # the structure's first 320 bytes
+log.launch_log_word.restype = ctypes.c_uint64
+out = []
+for base in json.loads(sys.argv[3])[0]:
+    dims = Dims(2, 8, 2048, 150, 192, 3, 1e-5)
+    size = lib.orion_txl_workspace_bytes(ctypes.byref(dims))
+    rc = lib.orion_txl_hidden(ctypes.byref(dims), (P * 22)(*[AT] * 22), AT, AT, AT, AT,
+                              192 * 3 * 512, None, 0, 0, AT, base, size, None)
+    words = [log.launch_log_word(i, k) for i in range(log.launch_log_size())
+             for k in range(log.launch_log_words(i))]
+    out.append((rc, size, [w - base for w in words if base <= w < base + size]))
+    log.launch_log_clear()
+print(json.dumps(out))
+"""
+
+
+def test_a_layers_arrays_begin_on_cache_lines_in_any_workspace(run):
+    # caches may hold lines of them that another workgroup has written whole
+    bases = [(1 << 41) + at for at in (0, 16, 64, 112, 128, 240)]
+    body = TXL[:TXL.index("out = []")] + WORKSPACE
+    for base, (rc, size, places) in zip(bases, run(body, bases)):
+        assert rc == 0 and len(set(places)) > 10
+        assert {(base + at) % 128 for at in places} == {0}
+    assert run(body, [(1 << 41) + 8])[0][0] == 3
+
+
 KERNELS = """
 print(json.dumps([log.launch_log_kernel(i).decode() for i in range(log.launch_log_kernels())]))
 """
