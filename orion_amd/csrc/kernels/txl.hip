@@ -565,9 +565,11 @@ __global__ __launch_bounds__(kJobThreads, 1) void txl_jobs_kernel(Jobs jobs) {
 //
 // What one workgroup writes and another reads within the launch is written through to
 // memory (sc1, agent scope), and a counter is raised when its workgroup's stores have been
-// acknowledged.  Readers may cache it: a line of it holds one panel's values of one product
-// only (Pieces), no one reads it in this launch before the counter says so, and caches start a launch
-// without lines of the launches before.  So nothing depends on where a workgroup runs.  A
+// acknowledged.  Readers may cache it: a line of it is one workgroup's (Pieces), no one reads
+// it in this launch before the counter says so, and caches start a launch without lines of the
+// launches before.  Only the means and squares of a row's parts lie sixteen workgroups to a
+// line; a cache that holds the line because it wrote a part of it must not answer for the
+// others, so they are read past the caches.  So nothing depends on where a workgroup runs.  A
 // stage whose 192 workgroups hand on 32 KiB a panel takes 1.6 us so (2.0 with a panel's
 // workgroups on all XCDs), 4.3 (6.8) with release and acquire fences, 2.5 to 2.9 as a launch.
 constexpr int kLayerThreads = 512;
@@ -594,6 +596,10 @@ struct Shared {
   }
   __device__ __forceinline__ u32x2 load8(int at) const {
     return __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, 0);
+  }
+  // past the caches, for lines that several workgroups write a part of
+  __device__ __forceinline__ u32x2 fresh8(int at) const {
+    return __builtin_amdgcn_raw_buffer_load_b64(r, at, 0, kCoherent);
   }
   __device__ __forceinline__ void store16(int at, const u32x4& v) const {
     __builtin_amdgcn_raw_buffer_store_b128(v, r, at, 0, kCoherent);
@@ -924,7 +930,7 @@ __device__ __forceinline__ void norm_task(Run& run, const Panel& panel, int tn, 
 #pragma unroll
     for (int h = 0; h < 2; ++h)
       part[h] = __builtin_bit_cast(
-          f32x2, sums.load8(((first + (h ? 4 + (lq & 1) : lq)) * kParts + l16) * 8));
+          f32x2, sums.fresh8(((first + (h ? 4 + (lq & 1) : lq)) * kParts + l16) * 8));
     f32x4 v[kPasses][2][2];
 #pragma unroll
     for (int it = 0; it < kPasses; ++it)
