@@ -7,7 +7,8 @@
 // (us a call: triad of 1,000,003 elements 5.3 so, 3.6 here; gemm 256 x 512 x 256 with its
 // output allocated 7.2, 4.5).  Every other call, and every refusal, returns None and is
 // made, or raised, by the Python code, so nothing is decided in two places but what is taken
-// here.
+// here.  Only the runtime's error is raised here: it is found behind the launch, which must
+// not be made again.
 #include <Python.h>
 
 #include <ATen/ops/empty.h>
@@ -17,6 +18,8 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include "orion_kernels.h"
 
 namespace {
 
@@ -63,6 +66,20 @@ PyObject* none() {
   Py_RETURN_NONE;
 }
 
+// What an entry point answered that has not taken the call: argument, shape and alignment are
+// checked before anything is launched, and the Python code is refused in the same way.
+PyObject* refused(const char* entry, int code) {
+  if (code < ORION_ERR_LAUNCH) return none();
+  PyObject* kernels = PyImport_ImportModule("orion_amd.kernels");
+  PyObject* error = kernels ? PyObject_GetAttrString(kernels, "KernelError") : nullptr;
+  PyObject* raised = error ? PyObject_CallFunction(error, "si", entry, code) : nullptr;
+  if (raised) PyErr_SetObject(error, raised);
+  Py_XDECREF(raised);
+  Py_XDECREF(error);
+  Py_XDECREF(kernels);
+  return nullptr;
+}
+
 // entries(triad, gemm): addresses of the C entry points, 0 for none.
 PyObject* entries(PyObject*, PyObject* const* args, Py_ssize_t count) {
   if (count != 2) {
@@ -101,7 +118,7 @@ PyObject* triad(PyObject*, PyObject* const* args, Py_ssize_t count) {
     Py_BEGIN_ALLOW_THREADS
     rc = triad_entry(pa, pb, pc, (float)s, n, (int)grid_blocks, stream);
     Py_END_ALLOW_THREADS
-    if (rc != 0) return none();          // refused: the Python code is refused too, and says so
+    if (rc != ORION_OK) return refused("orion_triad_f32", rc);
   } catch (...) {
     return none();
   }
@@ -140,7 +157,7 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t count) {
     Py_BEGIN_ALLOW_THREADS
     rc = gemm_entry(pa, pb, po, (int)m, (int)n, (int)k, wide, stream);
     Py_END_ALLOW_THREADS
-    if (rc != 0) return none();
+    if (rc != ORION_OK) return refused("orion_gemm_bf16_nt", rc);
     if (made.defined()) return THPVariable_Wrap(std::move(made));
   } catch (...) {
     return none();

@@ -1,6 +1,11 @@
 """Calls that go to the kernels without Python in between against the same calls made in
 Python: which ones are taken, what they give, and how the others are refused."""
 
+import json
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -44,6 +49,73 @@ def test_module_is_built_and_leaves_host_tensors_to_python():
         kernels.triad(x, x, x, 1.0)
     with pytest.raises(ValueError, match="device tensors"):
         kernels.gemm_bf16_nt(bf, bf)
+
+
+# Entry points that answer with a code, and tensors "on the GPU" over addresses that nothing
+# reads: in a process of its own, since torch then takes the GPU runtime for initialised.
+STUBS = """
+import ctypes, json, sys, types
+import torch
+torch.cuda._lazy_init = lambda: None
+from orion_amd import kernels
+P, I, F, Z = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_size_t
+
+class DLTensor(ctypes.Structure):
+    _fields_ = [("data", P), ("device_type", I), ("device_id", I), ("ndim", I),
+                ("type", ctypes.c_uint8 * 4), ("shape", P), ("strides", P),
+                ("offset", ctypes.c_uint64), ("context", P), ("deleter", P)]
+
+capsule = ctypes.pythonapi.PyCapsule_New
+capsule.restype, capsule.argtypes = ctypes.py_object, [P, ctypes.c_char_p, P]
+held = []
+
+def tensor(shape, code, bits):
+    sizes = (ctypes.c_int64 * len(shape))(*shape)
+    managed = DLTensor(1 << 40, 10, 0, len(shape), (code, bits, 1, 0), ctypes.addressof(sizes))
+    held.extend((sizes, managed))
+    return torch.utils.dlpack.from_dlpack(capsule(ctypes.addressof(managed), b"dltensor", None))
+
+made, answer = [], 0
+def native(*args):
+    made.append("native")
+    return answer
+def in_python(*args):
+    made.append("python")
+    return answer
+stubs = (ctypes.CFUNCTYPE(I, P, P, P, F, Z, I, P)(native),
+         ctypes.CFUNCTYPE(I, P, P, P, I, I, I, I, P)(native))
+kernels.lib = lambda: types.SimpleNamespace(orion_triad_f32=in_python,
+                                            orion_gemm_bf16_nt=in_python)
+kernels._calls.entries(*(ctypes.cast(s, P).value for s in stubs))
+stream = types.SimpleNamespace(cuda_stream=0)
+x, m, out = tensor((1003,), 2, 32), tensor((256, 64), 4, 16), tensor((256, 256), 2, 32)
+seen = []
+for answer in range(6):
+    for call, result in ((lambda: kernels.triad(x, x, x, 2.0, stream=stream), x),
+                         (lambda: kernels.gemm_bf16_nt(m, m, out=out, stream=stream), out)):
+        del made[:]
+        try:
+            got = call() is result
+        except kernels.KernelError as e:
+            got = (e.code, str(e))
+        seen.append((answer, got, list(made)))
+kernels._calls.entries(0, 0)
+print(json.dumps(seen))
+"""
+
+
+def test_the_runtimes_error_is_raised_and_the_kernel_not_launched_again():
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    out = subprocess.run([sys.executable, "-c", STUBS], cwd=root, check=True, timeout=120,
+                         capture_output=True, text=True).stdout
+    for answer, got, made in json.loads(out):
+        if answer == 0:
+            assert got is True and made == ["native"]
+            continue
+        code, text = got
+        assert code == answer and text.startswith("orion_")
+        # 1 to 3 come before the launch and are said again by the Python code
+        assert made == (["native"] if answer >= 4 else ["native", "python"])
 
 
 def _outcome(call):
