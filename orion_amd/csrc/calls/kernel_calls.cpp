@@ -23,10 +23,8 @@
 
 namespace {
 
-typedef int (*Triad)(void*, const void*, const void*, float, size_t, int, void*);
-typedef int (*Gemm)(const void*, const void*, void*, int, int, int, int, void*);
-Triad triad_entry = nullptr;
-Gemm gemm_entry = nullptr;
+decltype(&orion_triad_f32) triad_entry = nullptr;
+decltype(&orion_gemm_bf16_nt) gemm_entry = nullptr;
 
 // Modes, transforms and tracers that see operations: for the Python code.
 bool plain() {
@@ -89,8 +87,8 @@ PyObject* entries(PyObject*, PyObject* const* args, Py_ssize_t count) {
   void* triad = PyLong_AsVoidPtr(args[0]);
   void* gemm = PyLong_AsVoidPtr(args[1]);
   if (PyErr_Occurred()) return nullptr;
-  triad_entry = reinterpret_cast<Triad>(triad);
-  gemm_entry = reinterpret_cast<Gemm>(gemm);
+  triad_entry = reinterpret_cast<decltype(triad_entry)>(triad);
+  gemm_entry = reinterpret_cast<decltype(gemm_entry)>(gemm);
   Py_RETURN_NONE;
 }
 
@@ -111,8 +109,9 @@ PyObject* triad(PyObject*, PyObject* const* args, Py_ssize_t count) {
     void* stream;
     if (PyErr_Occurred() || grid_blocks != (int)grid_blocks || !stream_of(args[5], &stream))
       return none();
-    void* pa = a->data_ptr();
-    const void *pb = b->data_ptr(), *pc = c->data_ptr();
+    float* pa = static_cast<float*>(a->data_ptr());
+    const float* pb = static_cast<const float*>(b->data_ptr());
+    const float* pc = static_cast<const float*>(c->data_ptr());
     const size_t n = (size_t)a->numel();
     int rc;
     Py_BEGIN_ALLOW_THREADS

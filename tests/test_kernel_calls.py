@@ -12,9 +12,11 @@ import torch
 from torch.overrides import TorchFunctionMode
 from torch.utils._python_dispatch import TorchDispatchMode
 
-from orion_amd import kernels
+from orion_amd import _lib, kernels
 
 DEV = "cuda:0"
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "orion_amd", "csrc")
 
 
 class Sub(torch.Tensor):
@@ -105,8 +107,7 @@ print(json.dumps(seen))
 
 
 def test_the_runtimes_error_is_raised_and_the_kernel_not_launched_again():
-    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    out = subprocess.run([sys.executable, "-c", STUBS], cwd=root, check=True, timeout=120,
+    out = subprocess.run([sys.executable, "-c", STUBS], cwd=ROOT, check=True, timeout=120,
                          capture_output=True, text=True).stdout
     for answer, got, made in json.loads(out):
         if answer == 0:
@@ -116,6 +117,24 @@ def test_the_runtimes_error_is_raised_and_the_kernel_not_launched_again():
         assert code == answer and text.startswith("orion_")
         # 1 to 3 come before the launch and are said again by the Python code
         assert made == (["native"] if answer >= 4 else ["native", "python"])
+
+
+def test_the_calls_follow_the_headers_of_the_entry_points(tmp_path):
+    plan = subprocess.run(["make", "-C", CSRC, "-n", "-B", _lib.KERNEL_CALLS], check=True,
+                          capture_output=True, text=True).stdout
+    (command,) = [line.split() for line in plan.split("\n") if "kernel_calls.cpp" in line]
+    with open(os.path.join(ROOT, "include", "orion_kernels.h")) as f:
+        header = f.read()
+    for was, becomes, compiles in (("", "", True),
+                                   ("size_t n, int grid_blocks", "size_t n, int* grid_blocks", False),
+                                   ("int K, int out_is_f32", "int K, int* out_is_f32", False)):
+        changed = header.replace(was, becomes) if was else header
+        assert compiles or changed != header
+        # first among the folders of headers
+        (tmp_path / "orion_kernels.h").write_text(changed)
+        done = subprocess.run([command[0], "-fsyntax-only", f"-I{tmp_path}", *command[1:]],
+                              cwd=CSRC, capture_output=True, text=True, timeout=300)
+        assert (done.returncode == 0) == compiles, done.stderr[-2000:]
 
 
 def _outcome(call):
