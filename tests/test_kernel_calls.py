@@ -137,6 +137,18 @@ def test_the_calls_follow_the_headers_of_the_entry_points(tmp_path):
         assert (done.returncode == 0) == compiles, done.stderr[-2000:]
 
 
+def test_without_python_or_torch_headers_the_rest_is_built():
+    def plan(*settings):
+        return subprocess.run(["make", "-C", CSRC, "-n", "-B", *settings, "all"], check=True,
+                              capture_output=True, text=True)
+    assert "kernel_calls.cpp" in plan().stdout
+    for settings in (("PYTHON=false",), ("PYTHON=echo",), ("PYINC=/nowhere",), ("TORCH=/nowhere",)):
+        made = plan(*settings)
+        assert "kernel_calls.cpp" not in made.stdout and "kernel_calls.so is left out" in made.stdout
+        assert all(lib in made.stdout for lib in ("liborion_kernels.so", "scheduler_eval.so"))
+        assert "Traceback" not in made.stderr
+
+
 def _outcome(call):
     try:
         got = call()
