@@ -8,6 +8,8 @@ Transformer-XL client: ``transformer_xl.py`` asks here which calls they take).
 
 import atexit
 import ctypes
+import os
+import warnings
 
 import torch
 from torch.autograd import forward_ad
@@ -16,8 +18,11 @@ from . import _lib
 
 try:
     from . import kernel_calls as _calls       # csrc/calls: the same calls for plain tensors
-except ImportError:
+except ImportError as error:
     _calls = None
+    if os.path.exists(_lib.KERNEL_CALLS):      # built, for another PyTorch or Python perhaps
+        warnings.warn(f"{_lib.KERNEL_CALLS} does not load, so small kernels are called at up to "
+                      f"1.6 times the time: {error}", RuntimeWarning, stacklevel=2)
 
 STATUS = {0: "ok", 1: "bad argument", 2: "shape not a multiple of the tile",
           3: "pointer not 16-byte aligned", 4: "launch rejected"}
@@ -97,7 +102,6 @@ def _profiler_attached():
     names it in ROCP_TOOL_LIBRARIES and LD_PRELOAD and it shows in the process's
     maps.  (``librocprofiler-register.so`` does not count: the HIP runtime maps
     it in every process, profiled or not.)"""
-    import os
     named = os.environ.get("ROCP_TOOL_LIBRARIES", "") + ":" + os.environ.get("LD_PRELOAD", "")
     if "rocprofiler-sdk-tool" in named:
         return True

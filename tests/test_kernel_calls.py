@@ -149,6 +149,26 @@ def test_without_python_or_torch_headers_the_rest_is_built():
         assert "Traceback" not in made.stderr
 
 
+BROKEN = """
+import sys, warnings
+from orion_amd import _lib
+_lib.KERNEL_CALLS = sys.argv[1]
+sys.modules["orion_amd.kernel_calls"] = None       # importing it is an ImportError
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    from orion_amd import kernels
+assert kernels._calls is None
+print(sum("does not load" in str(w.message) for w in seen))
+"""
+
+
+@pytest.mark.parametrize("path,warned", [(_lib.KERNEL_CALLS, 1), ("/nowhere/kernel_calls.so", 0)])
+def test_a_module_that_does_not_load_is_named(path, warned):
+    out = subprocess.run([sys.executable, "-c", BROKEN, path], cwd=ROOT, check=True, timeout=120,
+                         capture_output=True, text=True).stdout
+    assert int(out) == warned
+
+
 def _outcome(call):
     try:
         got = call()
