@@ -32,6 +32,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "kernels.h"
@@ -2143,6 +2144,25 @@ size_t groups_of(size_t rows) {
   return best;
 }
 
+// Rows of one layer launch, a multiple of what full panels of all groups hold.  A launch cannot
+// be held back once it has begun, and best-effort kernels run on budgets of 100 us and more, so
+// none takes longer than that on the whole GPU: 3072 rows 79 us, 3840 96, 4608 114, 6144 145.
+// What is cut off costs its beginning and end, us a request behind 192 tokens of memory in one
+// launch a layer and so: batch 20 (3840 rows) 2555 and 2551, 21 2700 and 2884, 32 3877 and 4006,
+// 40 4758 and 4888, 64 7556 and 7946.  A launch may be issued to another stream than its call
+// names, so a stream's units are not asked: batch 4 takes 136 us a launch on 32 of them, 72 on
+// 64.  (The logits' launch, which is not cut, takes 4 to 5 times as long as a layer's.)
+constexpr size_t kFullRows = kGroups * kPanelRows, kLaunchRows = 10 * kFullRows;
+size_t launch_rows(size_t rows) {
+  return tiles(tiles(rows, tiles(rows, kLaunchRows)), kFullRows) * kFullRows;
+}
+
+// Counters of a layer launch of so many rows.
+size_t counters_of(size_t rows) {
+  const size_t groups = groups_of(rows);
+  return kLine * (kGroups + 3 * groups * group_panels(rows, groups));
+}
+
 Buffers buffers_of(const orion_txl_dims& d, void* base) {
   const size_t rows = (size_t)d.q_len * d.batch, mem_rows = (size_t)d.m_len * d.batch;
   const size_t proj = (size_t)d.heads * kHead, k_len = (size_t)d.q_len + d.m_len;
@@ -2152,8 +2172,8 @@ Buffers buffers_of(const orion_txl_dims& d, void* base) {
   b.parts = p.take<float2>(rows * kParts);
   b.y2 = p.take<float>(rows * kD);
   b.parts2 = p.take<float2>(rows * kParts);
-  const size_t groups = groups_of(rows);
-  b.counts = (size_t)kLine * (kGroups + 3 * groups * group_panels(rows, groups));
+  const size_t most = launch_rows(rows), rest = rows % most;
+  b.counts = rows / most * counters_of(most) + (rest ? counters_of(rest) : 0);
   b.counters = p.take<uint32_t>(b.counts);
   b.x[0] = p.take<uint16_t>(rows * kD);
   b.x[1] = p.take<uint16_t>(rows * kD);
@@ -2277,9 +2297,7 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
   size_t panel_tasks = kResTasks;
   for (size_t columns : {(size_t)d.inner, 3 * (size_t)proj})
     if (columns / kNormCols > panel_tasks) panel_tasks = columns / kNormCols;
-  const size_t groups = groups_of(rows), panels = group_panels(rows, groups);
-  const size_t group_tasks = panel_tasks * panels, most = kUnits / groups;
-  const size_t layer_blocks = groups * (group_tasks < most ? group_tasks : most);
+  const size_t rows_each = launch_rows(rows);
   for (int i = 0; i < d.layers; ++i) {
     const orion_txl_layer& p = layers[i];
     // a layer's input also goes into the memory's last rows
@@ -2333,27 +2351,36 @@ extern "C" int orion_txl_hidden(const orion_txl_dims* dims, const orion_txl_laye
     a.ff2_b = (In)p.ff2_b;
     a.inner = d.inner;
     a.proj = proj;
-    a.panels = (int)panels;
-    a.rows = rows;
-    a.att = w.att;
-    a.x = i == 0 ? (In)x0 : w.x[i & 1];
-    a.norm1 = Norm{(In)p.norm1_w, (In)p.norm1_b, w.parts, d.eps};
-    a.norm2 = Norm{(In)p.norm2_w, (In)p.norm2_b, w.parts2, d.eps};
-    a.parts1 = w.parts;
-    a.parts2 = w.parts2;
-    a.y1 = w.y;
-    a.y2 = w.y2;
-    a.x2 = w.x2;
-    a.h = w.h;
-    if (i + 1 < d.layers) {
-      a.rows_out = rows_out(i + 1);
-      a.rows_out.x = w.x[(i + 1) & 1];
-      a.qkv = {w.qu, w.qv, w.kv_x, (In)u, (In)v, proj};
+    uint32_t* counters = w.counters;
+    for (size_t row0 = 0; row0 < (size_t)rows; row0 += rows_each) {
+      const size_t n = std::min(rows_each, rows - row0);
+      const size_t groups = groups_of(n), panels = group_panels(n, groups);
+      a.panels = (int)panels;
+      a.rows = (int)n;
+      a.att = w.att + row0 * proj;
+      a.x = (i == 0 ? (In)x0 : w.x[i & 1]) + row0 * kD;
+      a.parts1 = w.parts + row0 * kParts;
+      a.parts2 = w.parts2 + row0 * kParts;
+      a.norm1 = Norm{(In)p.norm1_w, (In)p.norm1_b, a.parts1, d.eps};
+      a.norm2 = Norm{(In)p.norm2_w, (In)p.norm2_b, a.parts2, d.eps};
+      a.y1 = w.y + row0 * kD;
+      a.y2 = w.y2 + row0 * kD;
+      a.x2 = w.x2 + row0 * kD;
+      a.h = w.h + row0 * d.inner;
+      if (i + 1 < d.layers) {
+        a.rows_out = rows_out(i + 1);
+        a.rows_out.x = w.x[(i + 1) & 1] + row0 * kD;
+        a.rows_out.mem_from -= (int)row0;
+        a.qkv = {w.qu + row0 * proj, w.qv + row0 * proj, w.kv_x + row0 * 2 * proj, (In)u, (In)v,
+                 proj};
+      }
+      a.counters = counters;
+      const size_t group_blocks = std::min(panel_tasks * panels, kUnits / groups);
+      hipLaunchKernelGGL(txl_layer_kernel, dim3((unsigned)(groups * group_blocks)),
+                         dim3(kLayerThreads), 0, s, counters, (int)groups - 1,
+                         __builtin_ctz((unsigned)groups), (int)tiles(n, 16), i, a);
+      counters += counters_of(n);
     }
-    a.counters = w.counters;
-    hipLaunchKernelGGL(txl_layer_kernel, dim3((unsigned)layer_blocks), dim3(kLayerThreads), 0, s,
-                       w.counters, (int)groups - 1, __builtin_ctz((unsigned)groups),
-                       (int)tiles(rows, 16), i, a);
   }
   const orion_txl_layer& last = layers[d.layers - 1];
   hipLaunchKernelGGL(txl_norm_kernel, dim3((unsigned)tiles(rows, kThreads / 16)), dim3(kThreads), 0,

@@ -201,6 +201,27 @@ def test_no_workgroup_of_a_layers_products_is_empty(run, q_len, batch):
     assert fewest >= min(most, panels * 16)
 
 
+@pytest.mark.parametrize("q_len,batch,launches_a_layer", [
+    (1, 1, 1), (192, 4, 1), (3840, 1, 1), (3841, 1, 2), (192, 32, 2), (200, 40, 3), (217, 50, 3),
+    (65537, 16, 274)])
+def test_no_launch_of_a_layers_products_is_long(run, q_len, batch, launches_a_layer):
+    # a launch once begun cannot be held back: best-effort inference has to leave gaps
+    rows = q_len * batch
+    ((rc, _, layer_launches),) = run(TXL[:TXL.index("out = []")] + ROWS, [(q_len, batch)])
+    assert rc == 0 and len(layer_launches) == 2 * launches_a_layer
+    for layer in (layer_launches[:launches_a_layer], layer_launches[launches_a_layer:]):
+        begin = min(at for at, _, _ in layer)
+        shares = sorted((at - begin, own) for at, _, own in layer)
+        # every row once: means and squares lie 128 bytes to a row
+        assert [at for at, _ in shares] == [128 * sum(n for _, n in shares[:i])
+                                            for i in range(launches_a_layer)]
+        assert sum(own for _, own in shares) == rows and max(own for _, own in shares) <= 3840
+        # each with counters of its own: eight of tasks, and three a panel of up to 48 rows
+        counters = sorted(at for _, at, _ in layer)
+        assert all(b - a >= 128 * (8 + 3 * -(-own // 48)) for a, b, (_, own) in
+                   zip(counters, counters[1:], shares))
+
+
 @pytest.mark.parametrize("inner,q_len,batch,own,ahead", [
     # 192 KiB of the coming weights a workgroup: 6 MiB of a layer, 4.5 of the last
     (2048, 192, 4, 192, [32, 24]), (2048, 16, 1, 8, [32, 24]),
@@ -224,6 +245,24 @@ def test_no_launch_of_attention_has_more_threads_than_a_grid_can_have(run):
     attention = [(grid, block) for name, grid, block in launches if "attention" in name]
     assert sum(grid for grid, _ in attention) == 32 * 200_000 * 2
     assert all(grid * block < 1 << 32 for grid, block in attention)
+
+
+# Where a launch's means and squares lie, its counters and how many rows it has: words of the
+# layer kernel's structure.
+ROWS = """
+log.launch_log_watch(b"txl_layer", 5, 42)
+log.launch_log_word.restype = ctypes.c_uint64
+((q_len, batch),) = json.loads(sys.argv[3])[0]
+dims = Dims(2, 8, 2048, q_len, 0, batch, 1e-5)
+size = lib.orion_txl_workspace_bytes(ctypes.byref(dims))
+base = 1 << 41
+rc = lib.orion_txl_hidden(ctypes.byref(dims), (P * 22)(*[AT] * 22), AT, AT, AT, None, 0, None,
+                          0, 0, AT, base, size, None)
+launches = [[log.launch_log_word(i, k) for k in (27, 40, 41)] for i in range(log.launch_log_size())
+            if log.launch_log_words(i)]
+print(json.dumps([(rc, size, [(parts, counters, rows & 0xffffffff)
+                              for parts, counters, rows in launches])]))
+"""
 
 
 WORKSPACE = """

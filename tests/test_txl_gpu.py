@@ -271,13 +271,30 @@ def test_edges_of_row_panels(q_len, batch, n_head, d_inner):
 
 
 def test_more_rows_than_a_launch_has_workgroups_for():
-    # 28 and 29 panels a group: every workgroup takes several tasks of each product
+    # three launches a layer, ten and nine panels a group: workgroups take several tasks of
+    # each product
     model = _model(n_layer=2)
     inputs = _inputs(model, 217, 5, 50)
     (nll, new), (old_nll, old_new) = _fused(model, *inputs), _operations(model, *inputs)
     assert _off(nll, old_nll.double()) < 1e-2 and _off(new, old_new.double()) < 1e-2
     again = _fused(model, *inputs)
     assert torch.equal(again[0], nll) and torch.equal(again[1], new)
+
+
+@pytest.mark.parametrize("q_len,m_len,batch", [(192, 60, 21), (3841, 0, 1), (40, 192, 200)])
+def test_a_layers_products_in_several_launches(q_len, m_len, batch):
+    """More rows than a launch takes: a row's result is the same in a request of fewer."""
+    model = _model(n_layer=3)
+    data, target, mems = _inputs(model, q_len, m_len, batch)
+    nll, new = _fused(model, data, target, mems)
+    old_nll, old_new = _operations(model, data, target, mems)
+    assert _off(nll, old_nll.double()) < 1e-2 and _off(new, old_new.double()) < 1e-2
+    few = max(1, 3000 // q_len)
+    for b in range(0, batch - few + 1 if batch > 1 else 0, few):
+        own = slice(b, b + few)
+        _, part = _fused(model, data[:, own].contiguous(), target[:, own].contiguous(),
+                         mems[:, :, own].contiguous() if m_len else None)
+        assert torch.equal(part, new[:, :, own])
 
 
 def test_requests_on_few_compute_units_and_beside_each_other():
