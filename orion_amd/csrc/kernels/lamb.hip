@@ -237,7 +237,7 @@ __global__ __launch_bounds__(kReduceThreads) void lamb_ratio_kernel(
 }
 
 template <bool kDecay>
-__global__ __launch_bounds__(kMomentsThreads) void lamb_update_kernel(
+__global__ __launch_bounds__(kThreads) void lamb_update_kernel(
     uint32_t last, int low, int high, const float* __restrict__ factor, Coefs c, Group g) {
   const uint32_t block = last - blockIdx.x;        // the first pass's last data first
   const int ti = tensor_of_block(g, block, low, high);

@@ -158,6 +158,17 @@ def test_no_launch_of_a_lamb_step_is_long(run, counts):
     assert sum(ratios) == sum(n > 0 for n in counts)
 
 
+def test_the_passes_of_a_lamb_step_are_launched_as_they_are_built(run):
+    # sixteen wavefronts a workgroup in the first pass, four in the second
+    _, launches = run(LAMB, [70001])
+    assert {name.split("lamb_")[1].split("_")[0]: block for name, _, block in launches} == {
+        "moments": 1024, "ratio": 1024, "update": 256}
+    source = open(os.path.join(ROOT, "orion_amd", "csrc", "kernels", "lamb.hip")).read()
+    for kernel, threads in (("moments", "kMomentsThreads"), ("ratio", "kReduceThreads"),
+                            ("update", "kThreads")):
+        assert f"__launch_bounds__({threads}) void lamb_{kernel}_kernel" in source
+
+
 TXL = """
 I = ctypes.c_int
 class Dims(ctypes.Structure):
