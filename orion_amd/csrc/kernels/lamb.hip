@@ -46,12 +46,16 @@ constexpr int kReduceThreads = 1024;
 // than that: 5120 (21 M elements) are 81 us of the first pass, 8192 (34 M) 84 us of the
 // second.
 constexpr uint64_t kMomentsBlocks = 5120, kUpdateBlocks = 8192;
-// The second pass begins with the first one's last data, so the launches that hold a group's
-// last 21 M elements leave the moments in the memory-side cache (168 MB of its 256); all
-// other accesses pass it by, gradients and weights among them.  us a step, nothing cached,
-// and so: 13.7 M parameters 97 and 89, 23.9 M 165 and 152, 85 M 585 and 555, 192 M 1290 and
-// 1245; the moments of all launches 1281, the second pass's accesses too 1366, the first
-// one's weights too 1251.  The same rule serves groups of any size, the smallest whole.
+// The second pass begins with the first one's last data, so a group's last launch of the first
+// pass and the full one before it, 21 to 42 M elements, leave the moments (168 to 335 MB) in the
+// memory-side cache (256 MB); all other accesses pass it by, gradients and weights among them.
+// Where that is more than the cache holds, what it still has is what comes first.  us a step,
+// nothing cached, and so: 13.7 M parameters 97 and 89, 23.9 M 165 and 152, 85 M 585 and 555,
+// 192 M 1290 and 1245; the moments of all launches 1281, the second pass's accesses too 1366,
+// the first one's weights too 1251.  With only the last launch's moments, with those of exactly
+// the last 21 M elements, and so (eight tensors): 21.4 M 144, 134, 134; 41.5 M 260, 260, 256;
+// 61.6 M 383, 384, 380; 88 M 566, 556, 554; 146 M 928, 931, 927.  The same rule serves groups of
+// any size, the smallest whole.
 constexpr uint64_t kKeptBlocks = 5120;
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));

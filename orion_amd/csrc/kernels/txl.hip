@@ -6,9 +6,9 @@
 //
 // A request is small (768 token rows at batch 4: 0.2 TFLOP, half of it in the
 // vocabulary) and a chain of 16 layers, so what bounds it is the number of
-// dependent steps and the latency inside each, not a rate.  Two launches a
-// layer; whatever does not depend on the chain runs before it, for all layers at
-// once:
+// dependent steps and the latency inside each, not a rate.  Two launches a layer (of
+// at most 3840 rows); whatever does not depend on the chain runs before it, for all
+// layers at once:
 //
 //   before      positions (sinusoids); keys and values of the memory and the
 //               projected positions of every layer; [q k v] = x_0 Wqkv^T
@@ -1301,16 +1301,17 @@ constexpr size_t kAttnMost = (1u << 23) - 1024;   // workgroups: a grid has less
 
 // Weights of the launches that follow, read by workgroups of their own on compute units
 // that attention leaves idle, so that they come from the memory-side cache then: a
-// request's vocabulary has pushed them out since they were last used (a batch-4 request
-// takes 801 us so, 866 without; batch 1, 16 tokens 630 and 689).  Each of these workgroups
-// reads 192 KiB, about what fits attention's time: 32 of them a layer of the client's, more
-// for wider ones while units are left (all of the weights by 32 workgroups took 830 us
-// instead of 728 at an inner width of 65536, 731 so).  How many follows attention's size
-// alone, not the compute units of the stream: they are the last of the grid, and on streams
-// of 32 to 128 units, where they wait for attention's own, requests take between 10 % less
-// and 0.1 % more time than without.  Beside a GEMM or a triad on another stream (16 pairs)
-// requests take 0 to 11 % less, in one pair 2 % more, and the other's rate changes by -2 to
-// +8 %.
+// request's vocabulary has pushed them out since they were last used.  A layer launch reads its
+// weights a task ahead, but its first ones and each product's would come from memory.  us a
+// request so and without: batch 4, 192 tokens 688 and 712, 2 x 192 650 and 675, 1 x 64 579 and
+// 608, 1 x 16 without memory 530 and 528.  Each of these workgroups reads 192 KiB, about what
+// fits attention's time: 32 of them a layer of the client's, more for wider ones while units
+// are left (at an inner width of 65536, two layers, batch 4 797 so and 805 without, 1 x 64 462
+// and 457).  How many follows attention's size alone, not the compute units of the stream: they
+// are the last of the grid, and on streams of 32 to 128 units, where they wait for attention's
+// own, requests take between 4 % less (2 x 192 on 64) and 6 % more (2 x 64 on 32) time than
+// without.  Beside a GEMM or a triad on another stream (16 pairs of masks and sizes) they take
+// between 3 % less and 8 % more, the other's rate is the same within 4 %.
 constexpr uint32_t kTouchBytes = 192 << 10, kUnits = 256;
 struct Coming {
   const uint16_t* p[4];
