@@ -281,6 +281,40 @@ def test_more_rows_than_a_launch_has_workgroups_for():
     assert torch.equal(again[0], nll) and torch.equal(again[1], new)
 
 
+def _norms_alone(x, norms, n_layer, eps):
+    """``txl_hidden`` of rows ``x`` [rows, 512] in layers whose products are all zero: the
+    hidden states and the layers' inputs."""
+    def zeros(*shape):
+        return torch.zeros(shape, dtype=torch.bfloat16, device=DEV)
+    layer = (zeros(384, 512), zeros(128, 512), zeros(512, 128), *norms[:2], zeros(128, 512),
+             zeros(128), zeros(512, 128), zeros(512), *norms[2:])
+    hidden, new = kernels.txl_hidden(x[:, None].contiguous(), None, zeros(2, 64), zeros(2, 64),
+                                     [layer] * n_layer, 128, eps, len(x))
+    return hidden[:, 0], new[:, :, 0]
+
+
+def _random_rows(*sizes, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(n, generator=g).to(DEV, torch.bfloat16) for n in sizes]
+
+
+def test_rows_far_from_zero_are_normalised_by_what_they_differ_in():
+    w1, b1, w2, b2 = norms = _random_rows(512, 512, 512, 512)
+    far = torch.tensor([0, 1, 3, 100, -1000, 3000, 1e5, 1.004e6, -1e10, 1e20, 1e30, 3e36],
+                       device=DEV).to(torch.bfloat16)
+    x = far[:, None].expand(-1, 512)
+    # nothing is left of the first norm but its bias
+    want = torch.nn.functional.layer_norm(b1.double(), (512,), w2.double(), b2.double(), 1e-5)
+    for got in (_norms_alone(x, norms, 1, 1e-5)[0], _norms_alone(x, norms, 2, 1e-5)[1][1]):
+        # one rounding to eight bits
+        assert float((got.double() - want).abs().div(want.abs()).max()) < 2 ** -8
+    for c in far:
+        norms = (w1, c.expand(512).contiguous(), w2, b2)     # and nothing of the second
+        hidden, _ = _norms_alone(x, norms, 1, 1e-5)
+        _, inputs = _norms_alone(x, norms, 2, 1e-5)
+        assert torch.equal(hidden, b2.expand(12, 512)) and torch.equal(inputs[1], hidden)
+
+
 @pytest.mark.parametrize("q_len,m_len,batch", [(192, 60, 21), (3841, 0, 1), (40, 192, 200)])
 def test_a_layers_products_in_several_launches(q_len, m_len, batch):
     """More rows than a launch takes: a row's result is the same in a request of fewer."""
