@@ -125,13 +125,15 @@ __device__ __forceinline__ float2 row_stats(const float2& part, float eps) {
   const float d = part.x - mean;
   const float squares = sum16(__builtin_fmaf((float)kPartLen * d, d, part.y));
   const float variance = squares * (1.0f / kD) + eps;
-  // one step of Newton's from the instruction's value (zero for an infinite variance, where
-  // the step has none): two roundings as a square root and a division have, a tenth of the
-  // instructions
-  const float r = __builtin_amdgcn_rsqf(variance);
-  const float off = __builtin_fmaf(-variance * r, r, 1.0f);
-  const float rstd = r == 0.0f ? r : __builtin_fmaf(0.5f * r, off, r);
-  return make_float2(mean, rstd);
+  // one step of Newton's from the instruction's value (but from zero and infinity, of an
+  // infinite variance and of none): two roundings as a square root and a division have, a
+  // tenth of the instructions.  The instruction takes a subnormal variance for zero.
+  const bool small = variance < 0x1p-126f;
+  const float scaled = small ? variance * 0x1p48f : variance;
+  const float r = __builtin_amdgcn_rsqf(scaled);
+  const float off = __builtin_fmaf(-scaled * r, r, 1.0f);
+  const float rstd = r == 0.0f || r == __builtin_inff() ? r : __builtin_fmaf(0.5f * r, off, r);
+  return make_float2(mean, small ? rstd * 0x1p24f : rstd);
 }
 
 // Eight elements of a row, normalised.  The mean comes off before the scale: as x * rstd -

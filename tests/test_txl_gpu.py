@@ -315,6 +315,29 @@ def test_rows_far_from_zero_are_normalised_by_what_they_differ_in():
         assert torch.equal(hidden, b2.expand(12, 512)) and torch.equal(inputs[1], hidden)
 
 
+@pytest.mark.parametrize("eps", [0.0, 1e-40])
+def test_rows_whose_variance_is_subnormal(eps):
+    w1, b1, w2, b2 = norms = _random_rows(512, 512, 512, 512, seed=1)
+    b1.zero_()
+    # variances from 1e-36, which is normal, to 1e-42, of 700 steps
+    scale = torch.tensor([1e-18, 1.2e-19, 1e-19, 1e-20, 1e-21], device=DEV)
+    x = (scale[:, None] * _random_rows(512, seed=2)[0].float()).to(torch.bfloat16)
+
+    def norm(x, w, b):                 # in 64 bits: eps as the kernels have it
+        eps32 = float(torch.tensor(eps))
+        off = x.double() - x.double().mean(-1, keepdim=True)
+        return off / (off.pow(2).mean(-1, keepdim=True) + eps32).sqrt() * w.double() + b.double()
+    want = norm(norm(x, w1, b1).to(torch.bfloat16), w2, b2)
+    for got in (_norms_alone(x, norms, 1, eps)[0], _norms_alone(x, norms, 2, eps)[1][1]):
+        # a value may round to another neighbour between the norms and is rounded behind them
+        off = (got.double() - want).norm(dim=-1) / want.norm(dim=-1)
+        assert float(off.max()) < 2 ** -8 + 2 ** -9
+    # rows of one value have no variance at all, of which only the first norm's bias is left
+    # where eps allows it
+    flat = _norms_alone(torch.full_like(x, 3.0), norms, 1, eps)[0]
+    assert torch.isnan(flat).all() if eps == 0 else torch.equal(flat, b2.expand(5, 512))
+
+
 @pytest.mark.parametrize("q_len,m_len,batch", [(192, 60, 21), (3841, 0, 1), (40, 192, 200)])
 def test_a_layers_products_in_several_launches(q_len, m_len, batch):
     """More rows than a launch takes: a row's result is the same in a request of fewer."""
