@@ -629,6 +629,8 @@ struct Plan {
   int units;                    // of the four that there are
 };
 
+// The range check counts `at`, the scalar offset, too (seen on the device, to LDS and to
+// registers): a row of a panel that is not full is not read wherever it would lie.
 __device__ __forceinline__ void buffer_to_lds(const Shared& from, int lane_at, int at,
                                               unsigned char* to) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(
